@@ -151,6 +151,25 @@ int jh_launch_repeat(jh_function fn, uint32_t grid_x, uint32_t grid_y, uint32_t 
                      uint32_t block_y, uint32_t block_z, uint32_t shared_bytes, void **args, int count);
 
 /*
+ * Queue a list of launches in order: what a compiled jit program dispatches (`JitProgram.execute`,
+ * src/frontend/jit.ts:111-162) in one call, without host work of the caller's language between the launches.  The
+ * arguments of all steps lie one after the other in `args`: an argument is the 64-bit `value` itself, or, when `buffer`
+ * is not negative, the address `value` bytes behind `buffers[buffer]`.  Empty grids are skipped.  Stops at the first
+ * launch that fails.  At most 128 arguments per step.
+ */
+typedef struct {
+  jh_function fn;
+  uint32_t grid[3], block[3];
+  uint32_t shared_bytes;
+  uint32_t num_args;
+} jh_step;
+typedef struct {
+  uint64_t value;
+  int64_t buffer;
+} jh_arg;
+int jh_launch_list(const jh_step *steps, uint32_t num_steps, const jh_arg *args, const uint64_t *buffers);
+
+/*
  * Record a sequence of launches once and replay it with one call.  Everything queued with `jh_launch` between
  * `jh_graph_begin` and `jh_graph_end` is captured into a HIP graph instead of running; `jh_graph_launch`
  * then replays the whole sequence in order on the stream.  This is how a compiled jit program

@@ -397,6 +397,24 @@ int jh_launch_repeat(jh_function fn, uint32_t gx, uint32_t gy, uint32_t gz, uint
   return 0;
 }
 
+int jh_launch_list(const jh_step *steps, uint32_t num_steps, const jh_arg *args, const uint64_t *buffers) {
+  JH_NEED_INIT();
+  if (num_steps && (!steps || !args || !buffers)) return fail(-5, "null launch list");
+  constexpr uint32_t kMaxArgs = 128;
+  uint64_t cells[kMaxArgs];
+  void *argv[kMaxArgs];
+  for (uint32_t i = 0; i < kMaxArgs; ++i) argv[i] = &cells[i];
+  for (uint32_t s = 0; s < num_steps; ++s) {
+    const jh_step &st = steps[s];
+    if (st.num_args > kMaxArgs) return fail(-5, "step %u takes %u arguments, at most %u are supported", s, st.num_args, kMaxArgs);
+    for (uint32_t i = 0; i < st.num_args; ++i) cells[i] = (args[i].buffer >= 0 ? buffers[args[i].buffer] : 0) + args[i].value;
+    args += st.num_args;
+    int rc = jh_launch(st.fn, st.grid[0], st.grid[1], st.grid[2], st.block[0], st.block[1], st.block[2], st.shared_bytes, argv);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 int jh_graph_begin(void) {
   JH_NEED_INIT();
   JH_HIP(hipStreamBeginCapture(g_rt.stream, hipStreamCaptureModeThreadLocal));

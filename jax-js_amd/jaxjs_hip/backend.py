@@ -34,7 +34,9 @@ from .alu import Kernel, byteWidth
 from .errors import HipRuntimeError, SlotError, UnsupportedRoutineError
 from .kernelgen import NUMERICS, KernelSource, generate
 from .routine import Routine
+from .rowchain import RowChain, gen_rows
 from .runtime import Device, check, compile_source, pack_args
+from .schedule import Schedule
 
 
 class Executable:
@@ -115,6 +117,13 @@ def routineKey(routine: Routine) -> tuple:
             tuple(str(d) for d in t.outputDtypes), _freeze(routine.params))
 
 
+def programKey(prog) -> tuple:
+    """Structural identity of a jit program: its dispatches and how they are wired."""
+    return (prog.nargs, tuple(prog.outputs), tuple(
+        (s.kind, s.output, s.size) if s.kind != "execute" else
+        (s.kernel.key(), s.output, *s.inputs) if s.routine is None else (routineKey(s.routine), *s.outputs, *s.inputs) for s in prog.steps))
+
+
 class HipBackend:
     """MI355X backend.  `numerics="wasm"` evaluates transcendentals with the reference Wasm backend's polynomials,
     operation for operation (f32 maps within 2 ulp of the parity oracle); the default `"fast"` is the same except that
@@ -123,6 +132,7 @@ class HipBackend:
     libm."""
 
     type = "hip"
+    _releases = 0  # executables released so far: holders of prepared executables look again when it changes
     maxArgs = 64  # kernel parameters are plain pointers; same bound as the Wasm backend (src/backend/wasm.ts:38)
 
     def __init__(self, device: int = 0, numerics: str = "fast"):
@@ -140,6 +150,8 @@ class HipBackend:
         self._pool_limit = 8 << 30
         self._exes: "OrderedDict[tuple, Executable]" = OrderedDict()
         self.cacheLimit = 4096
+        self._programs: "OrderedDict[tuple, Schedule]" = OrderedDict()
+        self.programLimit = 512
         self._preparing: Dict[tuple, "asyncio.Future"] = {}  # prepares in flight, by cache key
         self._compile_pool = None
         self._staging: Dict[int, List[int]] = {}  # capacity -> free pinned host buffers for asynchronous reads
@@ -300,6 +312,7 @@ class HipBackend:
             # objects and writes its scratch without coming through dispatch)
             for k in [k for k, e in self._exes.items() if not e.data.pins and e is not exe][:len(self._exes) - self.cacheLimit]:
                 self._exes.pop(k).data.release(self.dev)
+                self._releases += 1
         return exe
 
     def clearCache(self) -> None:
@@ -307,6 +320,7 @@ class HipBackend:
         graph, which stay prepared until the graph is closed."""
         for k in [k for k, e in self._exes.items() if not e.data.pins]:
             self._exes.pop(k).data.release(self.dev)
+            self._releases += 1
 
     def pin(self, exe: Executable) -> None:
         """Keep `exe` prepared until `unpin`: for holders that launch it outside `dispatch` (a captured graph)."""
@@ -383,6 +397,56 @@ class HipBackend:
         key = ("routine", routineKey(routine), self.numerics)
         return await self._prepare_async(key, routine, lambda: generateRoutine(routine, self.numerics))
 
+    def prepareSync(self, source) -> Executable:
+        """`prepareKernelSync` / `prepareRoutineSync` / a chain of Kernels over the same rows, by the source's type."""
+        if isinstance(source, Kernel):
+            return self.prepareKernelSync(source)
+        if isinstance(source, Routine):
+            return self.prepareRoutineSync(source)
+        key = (source.key(), self.numerics)
+        return self._cached(key) or self._remember(key, self._build(source, gen_rows(source, self.numerics)))
+
+    def scheduleProgram(self, prog) -> Schedule:
+        """The schedule of a jit program, cached by the program's structure like the executables it consists of."""
+        key = programKey(prog)
+        found = self._programs.get(key)
+        if found is not None and found.live():
+            self._programs.move_to_end(key)
+            return found
+        found = self._programs[key] = Schedule(self, prog)
+        while len(self._programs) > self.programLimit:  # a schedule owns no device memory: only the host's lists go
+            self._programs.popitem(last=False)
+        return found
+
+    def _dispatch_chain(self, exe: Executable, ins, outs) -> None:
+        chain, prep = exe.source, exe.data
+        if prep.released:
+            raise ValueError("executable was released (evicted from the backend's cache): prepare it again")
+        if len(ins) != len(chain.inputs) or len(outs) != len(chain.outputs):
+            raise ValueError(f"the chain takes {len(chain.inputs)} inputs and {len(chain.outputs)} outputs")
+        for gid, need in prep.ks.min_input_bytes.items():
+            if ins[gid]["size"] < need:
+                raise ValueError(f"input {gid} holds {ins[gid]['size']} bytes, the chain addresses {need}")
+        for s, j in zip(outs, chain.outputs):
+            if s["size"] < chain.stages[j].kernel.bytes:
+                raise ValueError(f"output slot holds {s['size']} bytes, the chain writes {chain.stages[j].kernel.bytes}")
+        self._launch_steps(prep, ins, outs)
+
+    def _launch_steps(self, prep: _Prepared, ins, outs) -> None:
+        for step, fn, head, (cells, argv, patch) in zip(prep.ks.steps, prep.functions, prep.launch_head, prep.bound):
+            for c, kind, i in patch:
+                cells[c] = (ins if kind == "in" else outs)[i]["ptr"]
+            if self.trace is not None:
+                e0, e1 = self.dev.event(), self.dev.event()
+                self.dev.record(e0)
+                self.dev.launch(fn, step.grid, step.block, step.shared, argv)
+                self.dev.record(e1)
+                self.trace.append((f"{prep.ks.klass}:{step.name}", e0, e1))
+                continue
+            rc = self.dev.lib.jh_launch(*head, argv)
+            if rc:
+                check(rc, "jh_launch")
+
     def _dispatch_routine(self, exe: Executable, ins, outs) -> None:
         """Launch a routine's native plan (several kernels on the one in-order stream)."""
         routine: Routine = exe.source
@@ -402,13 +466,7 @@ class HipBackend:
                     need = prep.ks.min_input_bytes[i]
                 if s["size"] < need:
                     raise ValueError(f"{what} {i} holds {s['size']} bytes, the routine addresses {need}")
-        jh_launch = self.dev.lib.jh_launch
-        for head, (cells, argv, patch) in zip(prep.launch_head, prep.bound):
-            for c, kind, i in patch:
-                cells[c] = (ins if kind == "in" else outs)[i]["ptr"]
-            rc = jh_launch(*head, argv)
-            if rc:
-                check(rc, "jh_launch")
+        self._launch_steps(prep, ins, outs)
 
     # -- profiler hook (src/backend/webgpu/tracing.ts: a timestamp pair around every pass) -----------
     def _trace_begin(self):
@@ -462,6 +520,9 @@ class HipBackend:
         outs = [self._get(s) for s in outputs]
         if isinstance(exe.source, Routine):
             self._dispatch_routine(exe, ins, outs)
+            return
+        if isinstance(exe.source, RowChain):
+            self._dispatch_chain(exe, ins, outs)
             return
 
         kernel: Kernel = exe.source

@@ -1225,6 +1225,11 @@ class JitProgram:
         by the caller; inputs stay owned by the caller."""
         if len(inputs) != self.nargs:
             raise ValueError(f"jit program takes {self.nargs} inputs, got {len(inputs)}")
+        schedule = getattr(prepared, "schedule", None)
+        if prepared is None and hasattr(backend, "scheduleProgram"):
+            schedule = backend.scheduleProgram(self)
+        if schedule is not None and schedule.backend is backend:
+            return schedule.run(inputs)
         scope: Dict[int, int] = {i: s for i, s in enumerate(inputs)}
         for k, step in enumerate(self.steps):
             if step.kind == "malloc":
@@ -1242,6 +1247,10 @@ class JitProgram:
         return [scope[o] for o in self.outputs]
 
     def prepare(self, backend) -> Dict[int, Any]:
+        """Everything `execute` needs from `backend`, compiled and loaded: pass it as `prepared`."""
+        if hasattr(backend, "scheduleProgram"):
+            from .schedule import PreparedProgram
+            return PreparedProgram(backend, self)
         return {k: (backend.prepareRoutineSync(s.routine) if s.routine is not None else backend.prepareKernelSync(s.kernel))
                 for k, s in enumerate(self.steps) if s.kind == "execute"}
 

@@ -47,6 +47,17 @@ class DeviceInfo(ctypes.Structure):
     ]
 
 
+class LaunchStepC(ctypes.Structure):
+    """`jh_step`: one launch of a list."""
+    _fields_ = [("fn", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3), ("block", ctypes.c_uint32 * 3), ("shared_bytes", ctypes.c_uint32),
+                ("num_args", ctypes.c_uint32)]
+
+
+class LaunchRef(ctypes.Structure):
+    """`jh_arg`: one kernel argument of a list, `value` or (buffer >= 0) an address `value` bytes into that buffer."""
+    _fields_ = [("value", ctypes.c_uint64), ("buffer", ctypes.c_int64)]
+
+
 _SIGNATURES = {
     "jh_abi_version": (ctypes.c_int, []),
     "jh_last_error": (ctypes.c_char_p, []),
@@ -76,6 +87,7 @@ _SIGNATURES = {
     "jh_static_scratch_bytes": (ctypes.c_int, [ctypes.POINTER(ctypes.c_size_t)]),
     "jh_launch_repeat": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_uint32] * 7 +
                          [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int]),
+    "jh_launch_list": (ctypes.c_int, [ctypes.POINTER(LaunchStepC), ctypes.c_uint32, ctypes.POINTER(LaunchRef), ctypes.POINTER(ctypes.c_uint64)]),
     "jh_sync": (ctypes.c_int, []),
     "jh_graph_begin": (ctypes.c_int, []),
     "jh_graph_end": (ctypes.c_int, [ctypes.POINTER(ctypes.c_void_p)]),

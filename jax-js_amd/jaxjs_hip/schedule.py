@@ -1,0 +1,222 @@
+"""How a jit program runs on the `hip` backend: its dispatches as one list of native launches.
+
+A `JitProgram` (src/frontend/jit.ts:111-162) is a fixed list of allocations, dispatches and releases.  `Schedule` prepares
+it once: neighbouring Kernels over the same rows become one launch (`rowchain.py`), every intermediate gets a place in one
+workspace that is taken from the backend's pool for the call (places are used again as soon as their buffer is dead), and
+the launches of all steps go to the stream in one native call (`jh_launch_list`).  Per call the host looks up the input
+slots, allocates the output slots and makes that call; dispatching step by step cost 6 us of host time per launch, which
+is more than most launches of a small program take on the device.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import threading
+from typing import Any, Dict, List, Optional, Sequence
+
+from . import tracing
+from .alu import Kernel, byteWidth
+from .errors import SlotError
+from .routine import Routine
+from .rowchain import collect_chain
+from .runtime import LaunchRef, LaunchStepC, check
+from .shape import prod
+
+
+class Unit:
+    """One dispatch of the schedule: an executable, the buffer ids it reads and the ones it writes."""
+
+    def __init__(self, source, inputs: Sequence[int], outputs: Sequence[int]):
+        self.source, self.inputs, self.outputs = source, list(inputs), list(outputs)
+        self.exe = None
+
+
+def plan_units(prog) -> List[Unit]:
+    """The program's dispatches with runs of Kernels over the same rows joined."""
+    steps = [s for s in prog.steps if s.kind == "execute"]
+    last_read: Dict[int, int] = {}
+    for k, s in enumerate(steps):
+        for i in s.inputs:
+            last_read[i] = k
+    kept = set(prog.outputs)
+    view = [(s.kernel, s.inputs, s.output) if s.routine is None else (None, s.inputs, -1) for s in steps]
+    units: List[Unit] = []
+    k = 0
+    while k < len(steps):
+        s = steps[k]
+        found = collect_chain(view, k, lambda o, last: o in kept or last_read.get(o, -1) > last)
+        if found is not None:
+            chain, n = found
+            units.append(Unit(chain, chain.inputs, [steps[k + j].output for j in chain.outputs]))
+            k += n
+            continue
+        units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs))
+        k += 1
+    return units
+
+
+_ALIGN = 256
+
+
+def place_intermediates(units: Sequence[Unit], sizes: Dict[int, int], keep) -> Dict[int, int]:
+    """Byte offsets of the buffers that live only inside the program, and the workspace's size under -1: each buffer takes
+    the lowest gap that is free from its first write to its last use."""
+    first: Dict[int, int] = {}
+    last: Dict[int, int] = {}
+    for k, u in enumerate(units):
+        for b in u.outputs:
+            first.setdefault(b, k)
+            last[b] = k
+        for b in u.inputs:
+            if b in first:
+                last[b] = k
+    placed: Dict[int, int] = {-1: 0}
+    for b in sorted((b for b in first if b not in keep), key=lambda b: (first[b], -sizes[b])):
+        need = (sizes[b] + _ALIGN - 1) // _ALIGN * _ALIGN
+        busy = sorted((placed[o], placed[o] + (sizes[o] + _ALIGN - 1) // _ALIGN * _ALIGN) for o in placed
+                      if o >= 0 and first[o] <= last[b] and first[b] <= last[o])
+        at = 0
+        for lo, hi in busy:
+            if at + need <= lo:
+                break
+            at = max(at, hi)
+        placed[b] = at
+        placed[-1] = max(placed[-1], at + need)
+    return placed
+
+
+class Schedule:
+    """A jit program prepared for one backend."""
+
+    def __init__(self, backend, prog):
+        self.backend, self.prog = backend, prog
+        self.units = plan_units(prog)
+        for u in self.units:
+            u.exe = backend.prepareSync(u.source)
+        self._sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
+        self._made = list(dict.fromkeys(o for o in prog.outputs if o >= prog.nargs))
+        self._increfs = [s.output for s in prog.steps if s.kind == "incref"]
+        self._work = place_intermediates(self.units, self._sizes, set(self._made))
+        self._lock = threading.Lock()
+        self._bind()
+
+    def _bind(self) -> None:
+        """The native launch list.  Buffer table: inputs, outputs made here, workspace."""
+        self._releases = self.backend._releases
+        n = self.prog.nargs
+        table = {i: i for i in range(n)}
+        table.update({o: n + k for k, o in enumerate(self._made)})
+        self._workspace = n + len(self._made)
+        self._need: Dict[int, int] = {}
+        steps, refs = [], []
+        for u in self.units:
+            prep = u.exe.data
+            if isinstance(u.source, Kernel) and u.source.size == 0:
+                continue
+            needs = dict(prep.ks.min_input_bytes)
+            if isinstance(u.source, Routine):
+                t = u.source.type
+                needs = {i: needs.get(i, prod(s) * byteWidth(d)) for i, (s, d) in enumerate(zip(t.inputShapes, t.inputDtypes))}
+            for gid, need in needs.items():
+                b = u.inputs[gid]
+                if b < n:
+                    self._need[b] = max(self._need.get(b, 0), need)
+                elif self._sizes[b] < need:
+                    raise ValueError(f"buffer {b} holds {self._sizes[b]} bytes, its reader addresses {need}")
+            for step, fn in zip(prep.ks.steps, prep.functions):
+                c = LaunchStepC(fn, (ctypes.c_uint32 * 3)(*step.grid), (ctypes.c_uint32 * 3)(*step.block), step.shared, len(step.args))
+                steps.append(c)
+                for kind, i in step.args:
+                    if kind in ("in", "out"):
+                        b = (u.inputs if kind == "in" else u.outputs)[i]
+                        refs.append(LaunchRef(0, table[b]) if b in table else LaunchRef(self._work[b], self._workspace))
+                    else:
+                        refs.append(LaunchRef(prep.scratch[i] if kind == "scratch" else int(i), -1))
+        self._n_steps = len(steps)
+        self._steps = (LaunchStepC * max(len(steps), 1))(*steps)
+        self._refs = (LaunchRef * max(len(refs), 1))(*refs)
+        self._buffers = (ctypes.c_uint64 * (self._workspace + 1))()
+        self._inputs = [(i, self._need.get(i, 0)) for i in range(n)]
+        self._zeroed = any(u.exe.data.ks.zeroed_scratch for u in self.units)
+
+    def live(self) -> bool:
+        """False once an executable of the schedule was released (evicted from the backend's cache)."""
+        if self._releases != self.backend._releases:
+            if any(u.exe.data.released for u in self.units):
+                return False
+            self._releases = self.backend._releases
+        return True
+
+    def run(self, inputs: Sequence[int]) -> List[int]:
+        be, prog = self.backend, self.prog
+        if len(inputs) != prog.nargs:
+            raise ValueError(f"jit program takes {prog.nargs} inputs, got {len(inputs)}")
+        if not self.live():
+            raise ValueError("executable was released (evicted from the backend's cache): prepare the program again")
+        if be.trace is not None or (tracing.isTracing() and not be.capturing):
+            return self._run_by_unit(inputs)
+        slots = be._slots
+        made = [be.malloc(self._sizes[o]) for o in self._made]
+        space = be._alloc(self._work[-1])
+        try:
+            with self._lock:
+                buf = self._buffers
+                for i, need in self._inputs:
+                    s = slots.get(inputs[i])
+                    if s is None:
+                        raise SlotError(inputs[i])
+                    if s["size"] < need:
+                        raise ValueError(f"input {i} holds {s['size']} bytes, the program addresses {need}")
+                    buf[i] = s["ptr"]
+                for k, m in enumerate(made):
+                    buf[prog.nargs + k] = slots[m]["ptr"]
+                buf[self._workspace] = space
+                rc = be.dev.lib.jh_launch_list(self._steps, self._n_steps, self._refs, buf)
+                if rc:
+                    if self._zeroed and not be.capturing:
+                        for u in self.units:
+                            u.exe.data.rezero(be.dev)
+                    check(rc, "jh_launch_list")
+        except BaseException:
+            for m in made:
+                be.decRef(m)
+            raise
+        finally:
+            be._release(space, self._work[-1])  # a later owner's work is queued behind this program's on the one stream
+        scope = dict(zip(self._made, made))
+        for o in self._increfs:
+            be.incRef(scope[o] if o in scope else inputs[o])
+        return [scope[o] if o in scope else inputs[o] for o in prog.outputs]
+
+    def _run_by_unit(self, inputs: Sequence[int]) -> List[int]:
+        """The same dispatches one at a time, for per-dispatch timestamps."""
+        be, prog = self.backend, self.prog
+        scope = dict(enumerate(inputs))
+        owned = []
+        for u in self.units:
+            for o in u.outputs:
+                scope[o] = be.malloc(self._sizes[o])
+                if o not in self._made:
+                    owned.append(scope[o])
+            be.dispatch(u.exe, [scope[i] for i in u.inputs], [scope[o] for o in u.outputs])
+        for s in owned:
+            be.decRef(s)
+        for o in self._increfs:
+            be.incRef(scope[o])
+        return [scope[o] for o in prog.outputs]
+
+
+class PreparedProgram(dict):
+    """What `JitProgram.prepare` hands out for the `hip` backend: the schedule, and under a step's index the executable of
+    that step alone, prepared when it is asked for."""
+
+    def __init__(self, backend, prog):
+        super().__init__()
+        self.prog, self.schedule = prog, backend.scheduleProgram(prog)
+
+    def __missing__(self, k: int) -> Any:
+        s = self.prog.steps[k]
+        if s.kind != "execute":
+            raise KeyError(k)
+        self[k] = exe = self.schedule.backend.prepareSync(s.kernel if s.routine is None else s.routine)
+        return exe

@@ -14,6 +14,7 @@ from dataclasses import dataclass, field
 from typing import Callable, List, Optional, Tuple
 
 from .alu import Kernel
+from .rowchain import RowChain
 
 _enabled = False
 _flush: List[Callable[[], None]] = []
@@ -77,6 +78,10 @@ def traceSourceInfo(source) -> TraceInfo:
         else:
             color = "secondary"
             props.append(("reduction", f"{source.reduction.op}:{source.reduction.size}"))
+    elif isinstance(source, RowChain):
+        color = "secondary"
+        label = f"Rows[{humanSize(source.R)}x{humanSize(source.C)}]"
+        props += [("kernels", str(len(source.stages))), ("size", str(source.R * source.C))]
     else:
         color = "tertiary"
         label = str(source.name)

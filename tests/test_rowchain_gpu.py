@@ -1,0 +1,68 @@
+"""Runs of Kernels over the same rows in one launch, against the same program on the CPU checker, at row lengths around the
+vector width, the lane counts and the register limit."""
+import numpy as np
+import pytest
+
+from gpu_util import WARM_ONLY, backend
+from jaxjs_hip import DType
+from jaxjs_hip import jit as J
+from jaxjs_hip import library as L
+from jaxjs_hip import workloads as W
+from jaxjs_hip.jit import ShapedArray
+from jaxjs_hip.rowchain import RowChain, gen_rows
+from jaxjs_hip.schedule import plan_units
+from jit_util import run_program
+from oracle.backend import OracleBackend
+
+pytestmark = pytest.mark.gpu
+OPS = {"softmax": lambda x: L.softmax(x, -1), "logsoftmax": lambda x: L.logSoftmax(x, -1), "standardize": lambda x: L.standardize(x, -1),
+       "argmax": lambda x: L.argmax(x, -1), "softmax_of_masked": lambda x: L.softmax(J.where(L.tri_const(x.shape[-2], x.shape[-1], 0), x, -1e30), -1)}
+SHAPES = [(1, 2), (3, 7), (64, 10), (5, 64), (300, 66), (2, 33, 257), (1100, 1024), (7, 4097), (3, 50257)]
+
+
+def check(prog, arrays, f16, chained=True):
+    chains = [u.source for u in plan_units(prog) if isinstance(u.source, RowChain)]
+    assert len(chains) == 1 or not chained, [type(u.source).__name__ for u in plan_units(prog)]
+    if WARM_ONLY:
+        from jaxjs_hip.runtime import compile_source
+        for c in chains:
+            compile_source(gen_rows(c, "wasm").sources[0])
+        pytest.skip("warm-up run: compiled only")
+    be = backend()
+    before = be.live_slots()
+    got, want = run_program(be, prog, arrays), run_program(OracleBackend(), prog, arrays)
+    assert be.live_slots() == before
+    for g, w in zip(got, want):
+        if g.dtype.kind in "iu":
+            np.testing.assert_array_equal(g, w)
+        else:
+            np.testing.assert_allclose(g.astype(np.float64), w.astype(np.float64), rtol=1e-2 if f16 else 2e-5, atol=2e-3 if f16 else 2e-6)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("dtype", [DType.Float32, DType.Float16], ids=lambda d: d.value)
+@pytest.mark.parametrize("op", list(OPS))
+def test_row_chains(op, dtype, shape):
+    if op == "softmax_of_masked" and shape[-1] > 5000:
+        pytest.skip("the mask constant alone is large")
+    f16 = dtype == DType.Float16
+    x = np.random.default_rng(shape[-1]).standard_normal(shape).astype(np.float16 if f16 else np.float32)
+    check(J.jit(OPS[op], [ShapedArray(tuple(shape), dtype)]), [x], f16)
+
+
+def test_a_chain_keeps_what_is_read_behind_it():
+    """Results of the middle of a chain that the program returns or a later Kernel reads are stored as well."""
+    def f(x, w):
+        m = x.max(-1, keepdims=True)
+        e = J.exp(x.sub(m))
+        s = e.sum(-1, keepdims=True)
+        y = e.div(s)
+        return [y, m.reshape([40]), e, L.matmul(y, w)]
+    rng = np.random.default_rng(3)
+    x, w = rng.standard_normal((40, 96)).astype(np.float32), rng.standard_normal((96, 48)).astype(np.float32)
+    check(J.jit(f, [ShapedArray(x.shape, DType.Float32), ShapedArray(w.shape, DType.Float32)]), [x, w], False, chained=False)
+
+
+def test_row_statistics_of_the_benchmark_program():
+    x = np.random.default_rng(1).standard_normal((333, 4096)).astype(np.float32)
+    check(W.rowSoftmaxArgmaxProgram(333, 4096), [x], False)

@@ -1,0 +1,54 @@
+"""Host logic of a jit program's schedule: index forms against direct evaluation, placement of intermediates."""
+import numpy as np
+import pytest
+
+from jaxjs_hip.alu import AluExp, DType
+from jaxjs_hip.rowchain import index_form
+from jaxjs_hip.schedule import Unit, place_intermediates
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_index_form_has_the_value_of_its_expression(seed):
+    rng = np.random.default_rng(seed)
+    R, C = int(rng.integers(1, 30)), int(rng.integers(1, 40))
+    row, col = AluExp.special(DType.Int32, "gidx", R), AluExp.special(DType.Int32, "ridx", C)
+    flat = AluExp.add(AluExp.mul(row, AluExp.i32(C)), col)
+    e = flat
+    for _ in range(int(rng.integers(1, 5))):
+        n = int(rng.choice([1, 2, 3, 5, C, 2 * C, C * R, max(1, C // 2)]))
+        e = [lambda: AluExp.mod(e, AluExp.i32(n)), lambda: AluExp.idiv(e, AluExp.i32(n)),
+             lambda: AluExp.add(AluExp.mul(AluExp.idiv(flat, AluExp.i32(n)), AluExp.i32(n)), AluExp.mod(flat, AluExp.i32(n))),
+             lambda: AluExp.add(AluExp.mul(e, AluExp.i32(n)), row)][int(rng.integers(0, 4))]()
+    f = index_form(e, {"gidx": R, "ridx": C})
+    if f is None:
+        return
+    for r in range(R):
+        for c in range(C):
+            got = sum(v * (1 if k is None else (r if k[0] == "gidx" else c) // k[1]) for k, v in f.items())
+            assert got == e.evaluate({"gidx": r, "ridx": c}), (str(e), f, r, c)
+
+
+def test_unravelled_and_ravelled_positions_have_the_form_of_the_position():
+    R, C = 98304, 1024
+    row, col = AluExp.special(DType.Int32, "gidx", R), AluExp.special(DType.Int32, "ridx", C)
+    i = lambda e, n: AluExp.idiv(e, AluExp.i32(n))  # noqa: E731
+    m = lambda e, n: AluExp.mul(e, AluExp.i32(n))  # noqa: E731
+    flat = AluExp.add(m(row, C), col)
+    e = AluExp.add(m(i(flat, 12 * C * C), 12 * C * C), AluExp.add(m(AluExp.mod(i(flat, C * C), AluExp.i32(12)), C * C),
+                                                                 AluExp.add(m(AluExp.mod(row, AluExp.i32(C)), C), col)))
+    assert index_form(e, {"gidx": R, "ridx": C}) == {("gidx", 1): C, ("ridx", 1): 1}
+
+
+def test_intermediates_that_are_alive_together_do_not_overlap():
+    rng = np.random.default_rng(5)
+    for _ in range(30):
+        n = int(rng.integers(2, 14))
+        sizes = {k: int(rng.integers(0, 4000)) for k in range(n)}
+        units = [Unit(None, [int(x) for x in rng.choice(k, min(k, 2), replace=False)] if k else [], [k]) for k in range(n)]
+        placed = place_intermediates(units, sizes, {n - 1})
+        last = {k: max([k] + [j for j, u in enumerate(units) if k in u.inputs]) for k in range(n)}
+        for a in range(n - 1):
+            assert placed[a] % 256 == 0 and placed[a] + sizes[a] <= placed[-1]
+            for b in range(a):
+                if last[b] >= a:  # b is still read when a is written
+                    assert placed[a] + sizes[a] <= placed[b] or placed[b] + sizes[b] <= placed[a], (a, b)
