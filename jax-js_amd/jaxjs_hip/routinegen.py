@@ -7,7 +7,7 @@ time, which is what the Backend interface prescribes for a routine a backend lac
   Sort, Argsort                               `sort.hip.inc`     32-bit, float16 and float64 keys
   Scatter                                     `scatter.hip.inc`  float32/float16/float64/int32/uint32/bool updates
   TriangularSolve, Cholesky, LU, JacobiEigh   `linalg.hip.inc`   float32/float64/float16 (arithmetic in double, as the reference)
-  Fft                                         `fft.hip.inc`      float32/float64/float16
+  Fft                                         `fft_pass.hip.inc`, `fft.hip.inc` (large prime factors)  float32/float64/float16
   Attention (extension, not in the reference) `attention.hip.inc` float16, head size 32 / 64 / 128, any L and S
 """
 
@@ -247,6 +247,10 @@ def _gen_fft(routine: Routine, numerics: str) -> Optional[KernelSource]:
     rows = prod(shape[:-1])
     if rows == 0:
         return _empty("fft", n=n, rows=rows)
+    if "singleLaunch" not in params:
+        ks = _fft_passes(n, rows, ctype, eb, bool(params.get("inverse")), numerics, factors)
+        if ks is not None:
+            return ks
     # Rows that fit the LDS twice over (16 bytes per point) run in one launch, one workgroup per row, unless there are
     # too few rows for that to use the chip (a single long row is quicker spread over many workgroups per stage).
     S = len(factors)
@@ -283,6 +287,163 @@ def _gen_fft(routine: Routine, numerics: str) -> Optional[KernelSource]:
         prev *= radix
     scratch = [rows * n * eb, rows * n * eb, max(offsets[-1], 1) * 16] if S >= 1 else [8, 8, 16]
     return KernelSource([src], steps, scratch, "fft", need, dict(n=n, rows=rows, factors=factors, launches=len(steps), fused=False))
+
+
+FFT_PASS_RADIX_MAX = 13       # larger prime factors: one thread per output of a stage (fft.hip.inc)
+FFT_PASS_POINTS = 8192        # points a workgroup keeps in LDS, twice (128 KiB as float pairs)
+
+
+def _fft_radices(L: int) -> Optional[list]:
+    """L as a product of butterfly sizes, powers of two in eights and sixteens; None when a prime factor is too large."""
+    out, two = [], 0
+    while L % 2 == 0:
+        L, two = L // 2, two + 1
+    while two:  # 2^4k and 2^3k first choice; 2, 4 only for what is left
+        step = 3 if two in (3, 6, 9) else 4 if two >= 4 else two
+        out.append(1 << step)
+        two -= step
+    for p in (3, 5, 7, 11, 13):
+        while L % p == 0:
+            out.append(p)
+            L //= p
+    return out if L == 1 else None
+
+
+def _fft_lengths(n: int, limit: int) -> Optional[list]:
+    """n as a product of one, two or three pass lengths up to `limit`, as equal as its divisors allow."""
+    if n <= limit:
+        return [n]
+    divisors = [d for i in range(1, int(n ** 0.5) + 1) if n % i == 0 for d in (i, n // i)]
+    for passes in (2, 3):
+        best = None
+        for a in divisors:
+            if a > limit:
+                continue
+            rest = n // a
+            tails = [[rest]] if passes == 2 else [[b, rest // b] for b in divisors if b <= limit and rest % b == 0]
+            for tail in tails:
+                if max(tail) <= limit and (best is None or max([a] + tail) < max(best)):
+                    best = sorted([a] + tail, reverse=True)
+        if best is not None:
+            return best
+    return None
+
+
+def _fft_columns(L: int, total: int, points: int, alone: bool) -> int:
+    """Columns a workgroup transforms side by side: up to a whole line of them (16 floats), fewer while that leaves CUs
+    without a workgroup, but four where they are adjacent in memory (n = 10^6 in passes of 1000: two columns 26.3 us, four
+    20.9, eight 23.7; three passes of 100 with 4 to 32 columns 23.4 to 26.9)."""
+    cols = 1
+    while cols < (64 if alone else 16) and 2 * cols * L <= min(points, 4096 if alone else points // 2) and (total // (2 * cols) >= 256 or (not alone and cols < 4)):
+        cols *= 2
+    return cols
+
+
+def _fft_butterfly(R: int, sign: float) -> str:
+    """`jh_dft` for R points in place: sums over pairs q, R - q for odd R, two nested transforms for 2^k."""
+    import math
+    lines = [f"JH_DEV void jh_dft(jh_c (&v)[{R}]) {{"]
+    lit = lambda x: float(x).hex()  # noqa: E731
+    if R == 2:
+        lines.append("  const jh_c a = v[0], b = v[1]; v[0] = jh_c{a.re + b.re, a.im + b.im}; v[1] = jh_c{a.re - b.re, a.im - b.im};")
+    elif R == 4:
+        s = "" if sign > 0 else "-"
+        lines += ["  const jh_c a = jh_c{v[0].re + v[2].re, v[0].im + v[2].im}, b = jh_c{v[0].re - v[2].re, v[0].im - v[2].im};",
+                  "  const jh_c c = jh_c{v[1].re + v[3].re, v[1].im + v[3].im}, d = jh_c{v[1].re - v[3].re, v[1].im - v[3].im};",
+                  f"  const jh_c e = jh_c{{{'-' if sign > 0 else ''}d.im, {s}d.re}};",  # d times +-i
+                  "  v[0] = jh_c{a.re + c.re, a.im + c.im}; v[1] = jh_c{b.re + e.re, b.im + e.im};",
+                  "  v[2] = jh_c{a.re - c.re, a.im - c.im}; v[3] = jh_c{b.re - e.re, b.im - e.im};"]
+    elif R in (8, 16):
+        A, B = R // 4, 4  # v[a + A*b]: transforms over b, twiddles, transforms over a
+        lines.append(f"  jh_c t[{A}][4];")
+        for a in range(A):
+            lines.append(f"  {{ jh_c x[4] = {{v[{a}], v[{a + A}], v[{a + 2 * A}], v[{a + 3 * A}]}}; jh_dft(x);")
+            for k in range(4):
+                ang = sign * 2 * math.pi * a * k / R
+                lines.append(f"    t[{a}][{k}] = " + (f"x[{k}];" if a * k == 0 else f"jh_mul(x[{k}], jh_c{{{lit(math.cos(ang))}, {lit(math.sin(ang))}}});"))
+            lines.append("  }")
+        for k in range(4):
+            lines.append(f"  {{ jh_c x[{A}] = {{{', '.join(f't[{a}][{k}]' for a in range(A))}}}; jh_dft(x); " + " ".join(f"v[{k + 4 * a}] = x[{a}];" for a in range(A)) + " }")
+    else:
+        H = (R - 1) // 2
+        for q in range(1, H + 1):
+            lines.append(f"  const jh_c s{q} = jh_c{{v[{q}].re + v[{R - q}].re, v[{q}].im + v[{R - q}].im}}, d{q} = jh_c{{v[{q}].re - v[{R - q}].re, v[{q}].im - v[{R - q}].im}};")
+        lines.append("  const jh_c z = v[0];")
+        lines.append("  v[0] = jh_c{z.re + " + " + ".join(f"s{q}.re" for q in range(1, H + 1)) + ", z.im + " + " + ".join(f"s{q}.im" for q in range(1, H + 1)) + "};")
+        for p in range(1, H + 1):
+            cs = [math.cos(2 * math.pi * (q * p % R) / R) for q in range(1, H + 1)]
+            sn = [sign * math.sin(2 * math.pi * (q * p % R) / R) for q in range(1, H + 1)]
+            even = lambda part: "z." + part + "".join(f" + {lit(c)} * s{q}.{part}" for q, c in enumerate(cs, 1))  # noqa: E731
+            odd = lambda part: " + ".join(f"{lit(s)} * d{q}.{part}" for q, s in enumerate(sn, 1))  # noqa: E731
+            lines.append(f"  {{ const double er = {even('re')}, ei = {even('im')}, orr = {odd('re')}, oi = {odd('im')};")
+            lines.append(f"    v[{p}] = jh_c{{er - oi, ei + orr}}; v[{R - p}] = jh_c{{er + oi, ei - orr}}; }}")
+    lines.append("}")
+    return "\n".join(lines)
+
+
+def _fft_passes(n: int, rows: int, ctype: str, eb: int, inverse: bool, numerics: str, factors: list) -> Optional[KernelSource]:
+    """The transform in as few passes over memory as its length allows (fft_pass.hip.inc); None for lengths with a prime
+    factor above FFT_PASS_RADIX_MAX."""
+    import numpy as np
+
+    if n < 2 or _fft_radices(n) is None:
+        return None
+    points = FFT_PASS_POINTS * 8 // (2 * max(eb, 4))
+    # Alone in a workgroup a row may fill its LDS; the passes of a longer one take columns side by side, at least four.
+    lengths = _fft_lengths(n, points) if n <= points else _fft_lengths(n, points // 4)
+    if lengths is None:
+        return None
+    sign = 1.0 if inverse else -1.0
+    exchange = "double" if ctype == "double" else "float"
+
+    def table(count: int, of: int, step: int = 1) -> str:
+        """exp(sign 2 pi i m step / of) for m < count, each angle reduced to the first eighth of the circle exactly."""
+        m = (np.arange(count, dtype=np.int64) * step) % of
+        oct_, rem = (8 * m) // of, None
+        ang = 2 * np.pi * np.where(oct_ % 2 == 0, m * 8 - oct_ * of, (oct_ + 1) * of - m * 8).astype(np.float64) / (8.0 * of)
+        c, s = np.cos(ang), np.sin(ang)
+        swap = np.isin(oct_ % 8, (1, 2, 5, 6))
+        re, im = np.where(swap, s, c), np.where(swap, c, s)
+        re, im = np.where(np.isin(oct_ % 8, (2, 3, 4, 5)), -re, re), sign * np.where(np.isin(oct_ % 8, (4, 5, 6, 7)), -im, im)
+        return ", ".join(f"{{{float(a).hex()}, {float(b).hex()}}}" for a, b in zip(re, im))
+
+    sources, steps = [], []
+    S = 1
+    for i, Ln in enumerate(lengths):
+        D = n // S // Ln
+        final = D == 1
+        alone = len(lengths) == 1
+        total = rows * S * D
+        cols = _fft_columns(Ln, total, points, alone)
+        radices = _fft_radices(Ln) or [1]
+        threads = _round64(max(Ln // r for r in radices) * cols, 512 if max(radices) > 8 else 1024)
+        low_bits = max(1, (Ln * D - 1).bit_length() // 2)
+        kinds = sorted({r for r in radices} | ({4} if any(r in (8, 16) for r in radices) else set()) | ({2} if 8 in radices else set()))
+        blocks = -(-total // cols)
+        # Neighbouring tiles of columns share the lines of the rows they cut: neighbours go to one XCD (workgroups are handed
+        # to the eight XCDs in turn), whose L2 then serves the second of them.
+        grid = blocks if alone else -(-blocks // 8) * 8
+        tile = "JH_DEV int jh_tile() { return " + ("(int)blockIdx.x" if alone else f"(int)(blockIdx.x % 8) * {grid // 8} + (int)(blockIdx.x / 8)") + "; }"
+        calls, NS = [], 1
+        for s, r in enumerate(radices):
+            src, dst = (s + 1) & 1, s & 1
+            calls.append(f"  jh_stage<{r}, {NS}, {'true' if s == 0 else 'false'}, {'true' if s == len(radices) - 1 else 'false'}>(in_re, in_im, out_re, out_im, re[{src}], im[{src}], re[{dst}], im[{dst}]);")
+            if s < len(radices) - 1:
+                calls.append("  __syncthreads();")
+            NS *= r
+        sources.append(_prelude(numerics) + fill(template("fft_pass.hip.inc"), dict(
+            N=n, L=Ln, COLS=cols, THREADS=threads, S=S, D=D, TOTAL=total, GUARD=1 if grid * cols != total else 0, L1=lengths[0], L2=lengths[1] if len(lengths) == 3 else 1,
+            POINTS_FIRST=1 if final else 0, POINTS_LAST=1 if alone else 0, SCALE=repr(1.0 / n) if inverse and final else "1.0", LOW_BITS=low_bits,
+            INDEX="int" if rows * n + cols * n < (1 << 31) else "long long", ELEM=ctype, EXCHANGE=exchange, TWIDDLES=table(Ln, Ln), HIGH=table(((Ln * D - 1) >> low_bits) + 1, Ln * D, 1 << low_bits) if not final else "{1.0, 0.0}",
+            LOW=table(1 << low_bits, Ln * D) if not final else "{1.0, 0.0}", BUTTERFLIES=tile + "\n" + "\n".join(_fft_butterfly(r, sign) for r in kinds),
+            NAME=f"jh_fft_pass{i}", STAGES=len(radices), STAGE_CALLS="\n".join(calls))))
+        src_pair = [("in", 0), ("in", 1)] if i == 0 else [("scratch", 2 * ((i - 1) % 2)), ("scratch", 2 * ((i - 1) % 2) + 1)]
+        dst_pair = [("out", 0), ("out", 1)] if final else [("scratch", 2 * (i % 2)), ("scratch", 2 * (i % 2) + 1)]
+        steps.append(LaunchStep(f"jh_fft_pass{i}", (grid, 1, 1), (threads, 1, 1), 0, src_pair + dst_pair, module=i))
+        S *= Ln
+    scratch = [rows * n * eb] * (2 * (len(lengths) - 1))
+    need = {0: rows * n * eb, 1: rows * n * eb}
+    return KernelSource(sources, steps, scratch, "fft", need, dict(n=n, rows=rows, factors=factors, launches=len(steps), passes=lengths))
 
 
 _SCATTER_KINDS = {DType.Float32: (0, "float"), DType.Float16: (1, "jh_f16"), DType.Int32: (2, "int"), DType.Uint32: (3, "jh_u32"),

@@ -179,6 +179,21 @@ def test_fft_single_launch_and_staged_paths_give_the_same_bits(shape):
         assert_bits(a, b, f"{shape} inverse={inverse}")
 
 
+@pytest.mark.parametrize("shape", [(2,), (3, 16), (5, 143), (9, 2310), (1, 8192), (300, 4096), (2, 12288), (3, 70875), (1, 4 * 11 * 13 * 49), (1, 1 << 23)], ids=str)
+@pytest.mark.parametrize("dt", [F32, np.float64, np.float16], ids=lambda d: np.dtype(d).name)
+def test_fft_in_passes(shape, dt):
+    """One, two and three passes over memory, lone and many rows, every butterfly size, against numpy in double."""
+    if dt != F32 and shape[-1] > 100000:
+        pytest.skip("the pass structure does not depend on the element type")
+    re, im = RNG.standard_normal(shape).astype(dt), RNG.standard_normal(shape).astype(dt)
+    for inverse in (False, True):
+        got, ks = R.run_gpu(R.fft(re, im, inverse), [re, im])
+        z = re.astype(np.complex128) + 1j * im.astype(np.complex128)
+        want = np.fft.ifft(z) if inverse else np.fft.fft(z)
+        err = np.abs(got[0].astype(np.complex128) + 1j * got[1] - want).max() / np.abs(want).max()
+        assert "passes" in ks.info and err < {"float32": 5e-7, "float64": 1e-14, "float16": 2e-3}[np.dtype(dt).name], (ks.info, err)
+
+
 def test_fft_factor_orders_and_validation():
     re, im = RNG.standard_normal((2, 60)).astype(F32), RNG.standard_normal((2, 60)).astype(F32)
     for factors in ([4, 3, 5], [5, 3, 4], [2, 2, 15], [60]):
