@@ -25,7 +25,7 @@ _SORT_KINDS = {DType.Float32: (0, "float"), DType.Float16: (1, "jh_f16"), DType.
                DType.Uint32: (3, "jh_u32"), DType.Bool: (2, "int"), DType.Float64: (4, "double")}
 SORT_TILE = 8192  # 64 KB of LDS in 8-byte words: rows up to 8192 elements never leave the CU (4096 in 16-byte words)
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
-CHOLESKY_PANEL_FROM = 192  # matrix order from which Cholesky runs panel by panel over the whole chip
+CHOLESKY_PANEL_FROM = 192  # matrix order from which one panel's launch spans many CUs (smaller ones: a few workgroups)
 
 
 def _next_pow2(n: int) -> int:
@@ -84,39 +84,32 @@ def _gen_cholesky(routine: Routine, numerics: str) -> Optional[KernelSource]:
     batch = prod(shape[:-2])
     if batch == 0 or n == 0:
         return _empty("cholesky", n=n, batch=batch)
-    if n >= CHOLESKY_PANEL_FROM and batch * n * n * 8 <= CHOLESKY_RIGHT_LOOKING_MAX_BYTES:
-        # Large matrices, right-looking: the running sums of the whole triangle in a double-precision scratch copy; per
-        # 32-column panel one launch that finishes the panel and one that updates the trailing triangle (bit-identical).
-        src = _linalg_source(numerics, ROUTINE=5, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
-        grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
-        steps = [LaunchStep("jh_chol_init", grid1(batch * n * n), (256, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0)])]
+    if n <= 64 or batch * n * n * 8 <= CHOLESKY_RIGHT_LOOKING_MAX_BYTES:  # (two panels need no copy)
+        # Right-looking: the running sums of the whole triangle in a double-precision scratch copy, one launch per
+        # 32-column panel that finishes the panel and subtracts the one before it from the rest.
+        src = _linalg_source(numerics, ROUTINE=5, N=n, ELEM=ctype, CMP=cmp_t)
+        steps = []
         for j0 in range(0, n, 32):
             after = max(0, n - j0 - 32)
-            steps.append(LaunchStep("jh_chol_panel", (batch * max(1, (after + 63) // 64), 1, 1), (64, 1, 1), 0,
-                                    [("scratch", 0), ("out", 0), ("const", j0)]))
-            if after > 0:
-                T = (after + 63) // 64
-                steps.append(LaunchStep("jh_chol_update", (batch * T * T, 1, 1), (256, 1, 1), 0, [("out", 0), ("scratch", 0), ("const", j0)]))
-        return KernelSource([src], steps, [batch * n * n * 8], "cholesky", {0: batch * n * n * eb},
-                            dict(n=n, batch=batch, panels=(n + 31) // 32, launches=len(steps), variant="right-looking"))
-    if n >= CHOLESKY_PANEL_FROM and batch * n * n < (1 << 31):
-        # Large matrices: 32-column panels, two launches each, every launch spread over the chip; the same sums in the
-        # same order as the single-workgroup kernel (bit-identical results).
-        src = _linalg_source(numerics, ROUTINE=4, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
-        grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
-        steps = [LaunchStep("jh_chol_zero", grid1(batch * n * n), (256, 1, 1), 0, [("out", 0)])]
-        for j0 in range(0, n, 32):
-            steps.append(LaunchStep("jh_chol_bulk", (batch * ((n - j0 + 63) // 64), 1, 1), (256, 1, 1), 0,
-                                    [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
-            after = max(0, n - j0 - 32)
-            steps.append(LaunchStep("jh_chol_panel", (batch * max(1, (after + 63) // 64), 1, 1), (64, 1, 1), 0,
-                                    [("scratch", 0), ("out", 0), ("const", j0)]))
-        return KernelSource([src], steps, [batch * n * 32 * 8], "cholesky", {0: batch * n * n * eb},
-                            dict(n=n, batch=batch, panels=(n + 31) // 32, launches=len(steps)))
-    threads = _round64(n)
-    src = _linalg_source(numerics, ROUTINE=0, N=n, THREADS=threads, ELEM=ctype, CMP=cmp_t)
-    steps = [LaunchStep("jh_cholesky", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0)])]
-    return KernelSource([src], steps, [batch * n * n * eb], "cholesky", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=threads))
+            T = (after + 63) // 64
+            blocks = max(1, (after + 31) // 32) + (T * (T + 1) // 2 if j0 else 0)
+            steps.append(LaunchStep("jh_chol_step", (batch * blocks, 1, 1), (256, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
+        info = dict(n=n, batch=batch, launches=len(steps), variant="right-looking")
+        if n >= CHOLESKY_PANEL_FROM:
+            info["panels"] = len(steps)
+        return KernelSource([src], steps, [batch * n * n * 8 if n > 64 else 8], "cholesky", {0: batch * n * n * eb}, info)
+    # Left-looking where that copy would be too large: 32-column panels, two launches each; the same sums in the same order.
+    src = _linalg_source(numerics, ROUTINE=4, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
+    grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
+    steps = [LaunchStep("jh_chol_zero", grid1(batch * n * n), (256, 1, 1), 0, [("out", 0)])]
+    for j0 in range(0, n, 32):
+        steps.append(LaunchStep("jh_chol_bulk", (batch * ((n - j0 + 63) // 64), 1, 1), (256, 1, 1), 0,
+                                [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
+        after = max(0, n - j0 - 32)
+        steps.append(LaunchStep("jh_chol_panel", (batch * max(1, (after + 63) // 64), 1, 1), (64, 1, 1), 0,
+                                [("scratch", 0), ("out", 0), ("const", j0)]))
+    return KernelSource([src], steps, [batch * n * 32 * 8], "cholesky", {0: batch * n * n * eb},
+                        dict(n=n, batch=batch, panels=(n + 31) // 32, launches=len(steps)))
 
 
 def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
