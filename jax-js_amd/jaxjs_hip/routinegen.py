@@ -205,12 +205,19 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     params = routine.params or {}
     threads = _round64(n)
     in_lds = 1 if 2 * n * n * eb <= 150 * 1024 else 0  # both matrices in the CU's 160 KB of LDS: n <= 138 in float32
+    blocks = (n + 7) // 8
+    if n >= JACOBI_BLOCKS_FROM and eb * (n * (n + 1) // 2 + n * n) + 16 * (blocks + 1) * n + 1024 <= 160 * 1024:
+        # the pivot rows pipelined through blocks of 8 indices, everything in LDS
+        src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=1024, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (1024, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1)])]
+        return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=1024, in_lds=bool(in_lds), blocks=blocks))
     src = _linalg_source(numerics, ROUTINE=3, N=n, THREADS=threads, IN_LDS=in_lds, MAX_SWEEPS=int(params["maxSweeps"]),
                          TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
     steps = [LaunchStep("jh_jacobi", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1)])]
     return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=threads, in_lds=bool(in_lds)))
 
 
+JACOBI_BLOCKS_FROM = 9        # below, one block holds the whole matrix
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS
 TRISOLVE_AHEAD = 8       # entries of a row that a right-hand side's thread fetches ahead of its subtraction chain
