@@ -205,19 +205,20 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     params = routine.params or {}
     threads = _round64(n)
     in_lds = 1 if 2 * n * n * eb <= 150 * 1024 else 0  # both matrices in the CU's 160 KB of LDS: n <= 138 in float32
-    blocks = (n + 7) // 8
-    if n >= JACOBI_BLOCKS_FROM and eb * (n * (n + 1) // 2 + n * n) + 16 * (blocks + 1) * n + 1024 <= 160 * 1024:
-        # the pivot rows pipelined through blocks of 8 indices, everything in LDS
-        src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=1024, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
-        steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (1024, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1)])]
-        return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=1024, in_lds=bool(in_lds), blocks=blocks))
+    for size in (4, 8):  # indices per block; the triangle and the rotations under way have to fit the LDS
+        blocks = -(-n // size)
+        if JACOBI_BLOCKS_FROM <= n <= 192 and eb * (n * (n + 1) // 2) + 16 * (blocks + 1) * n + 32 * blocks + 512 <= 160 * 1024:
+            src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=512, RB=size, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
+            steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (512, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("scratch", 0)])]
+            return KernelSource([src], steps, [batch * n * n * eb], "jacobi", {0: batch * n * n * eb},
+                                dict(n=n, batch=batch, threads=512, in_lds=bool(in_lds), block=size))
     src = _linalg_source(numerics, ROUTINE=3, N=n, THREADS=threads, IN_LDS=in_lds, MAX_SWEEPS=int(params["maxSweeps"]),
                          TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
     steps = [LaunchStep("jh_jacobi", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1)])]
     return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=threads, in_lds=bool(in_lds)))
 
 
-JACOBI_BLOCKS_FROM = 9        # below, one block holds the whole matrix
+JACOBI_BLOCKS_FROM = 13       # the step of a block costs more than the few rotations of a smaller matrix (12: 183 against 178 us, 16: 272 against 324)
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS
 TRISOLVE_AHEAD = 8       # entries of a row that a right-hand side's thread fetches ahead of its subtraction chain

@@ -136,6 +136,19 @@ def test_jacobi_eigh(shape):
     assert_bits(got, want, f"jacobi_eigh {shape} {ks.info}")
 
 
+@pytest.mark.parametrize("n", [12, 13, 15, 17, 65, 129, 139, 160])
+def test_jacobi_eigh_by_blocks_at_ragged_orders(n):
+    """Partial last blocks, one to three waves of chains, both block sizes; and pairs that are left alone (zeros, negative
+    zeros among them) beside pairs that turn."""
+    a = RNG.standard_normal((2, n, n))
+    sym = (a + np.swapaxes(a, -1, -2)).astype(F32)
+    sym[1, : n // 2, n // 2:] = sym[1, n // 2:, : n // 2] = -0.0
+    sym[1, 1, :1] = sym[1, :1, 1] = 0.0
+    got, want, ks = both(R.jacobi_eigh(sym, 3, 0.0), [sym])
+    assert ("block" in ks.info) == (n >= 13)
+    assert_bits(got, want, f"jacobi_eigh {n} {ks.info}")
+
+
 def test_jacobi_eigh_sweep_limits_and_special_values():
     a = RNG.standard_normal((3, 12, 12))
     sym = (a + np.swapaxes(a, -1, -2)).astype(F32)
