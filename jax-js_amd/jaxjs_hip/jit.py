@@ -1211,6 +1211,7 @@ class JitProgram:
     nargs: int
     outputs: List[int]
     consts: List[ConstArray]
+    jaxpr: Optional[Jaxpr] = field(default=None, repr=False, compare=False)  # what it was compiled from
 
     @property
     def kernels(self) -> List[Kernel]:
@@ -1427,7 +1428,7 @@ def jitCompile(jaxpr: Jaxpr, consts: Sequence[ConstArray] = (), maxArgs: int = 6
             for i in dict.fromkeys(s.inputs + written(s)):
                 if i >= nargs and i not in outputs and last_use.get(i) == k:
                     final.append(JitStep("free", output=i))
-    return JitProgram(final, nargs, outputs, list(consts))
+    return JitProgram(final, nargs, outputs, list(consts), jaxpr)
 
 
 def jit(fn: Callable[..., Any], avals: Sequence[ShapedArray], maxArgs: int = 64) -> JitProgram:

@@ -219,6 +219,7 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
 
 
 JACOBI_BLOCKS_FROM = 13       # the step of a block costs more than the few rotations of a smaller matrix (12: 183 against 178 us, 16: 272 against 324)
+ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which every query is a workgroup of its own and not a row of a 128-row tile
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS
 TRISOLVE_AHEAD = 8       # entries of a row that a right-hand side's thread fetches ahead of its subtraction chain
@@ -592,6 +593,19 @@ def _gen_attention(routine: Routine, numerics: str) -> Optional[KernelSource]:
             lay.append((sb, sp, sn, v["offset"]))
             need[i] = v["elements"] * 2
     (qb, ql, qn, qo), (kb, ksp, kn, ko), (vb, vsp, vn, vo) = lay
+    if L <= ATTENTION_FEW_QUERIES:
+        lanes = H // 8
+        threads = 128
+        while threads < 1024 and threads < S * lanes // 2:
+            threads *= 2
+        passes = -(-S // (threads // lanes))
+        rounds = -(-passes // 10)  # ten keys and values of 16 bytes each in flight per thread
+        src = _prelude(numerics) + fill(template("attention_few.hip.inc"), dict(
+            NH=N, L=L, S=S, H=H, CAUSAL=1 if params.get("isCausal") else 0, SCALE_LOG2E=repr(scale * math.log2(math.e)), THREADS=threads,
+            PASSES=-(-passes // rounds), ROUNDS=rounds, QB=qb, QL=ql, QN=qn, QOFF=qo, KB=kb, KS=ksp, KN=kn, KOFF=ko, VB=vb, VS=vsp, VN=vn, VOFF=vo,
+            OB=L * N * H, OL=N * H, ON=H))
+        steps = [LaunchStep("jh_attention_few", (B * L * N, 1, 1), (threads, 1, 1), 0, [("in", 0), ("in", 1), ("in", 2), ("out", 0)])]
+        return KernelSource([src], steps, [], "attention", need, dict(B=B, L=L, S=S, N=N, H=H, causal=bool(params.get("isCausal")), blocks=B * L * N, threads=threads))
     src = _prelude(numerics) + fill(template("attention.hip.inc"), dict(
         B=B, NH=N, L=L, S=S, H=H, CAUSAL=1 if params.get("isCausal") else 0, SCALE_LOG2E=repr(scale * math.log2(math.e)),
         FOLD_SCALE=1 if 0 < scale < float("inf") else 0,

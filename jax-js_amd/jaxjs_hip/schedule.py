@@ -89,6 +89,12 @@ class Schedule:
     """A jit program prepared for one backend."""
 
     def __init__(self, backend, prog):
+        from .jit import jitCompile
+        from .rewrite import fuse_attention
+
+        fused = fuse_attention(prog.jaxpr, prog.consts) if prog.jaxpr is not None else None
+        if fused is not None:
+            prog = jitCompile(fused, prog.consts, backend.maxArgs)
         self.backend, self.prog = backend, prog
         self.units = plan_units(prog)
         for u in self.units:

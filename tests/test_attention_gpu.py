@@ -43,6 +43,21 @@ def test_attention_matches_float64(case, causal):
     np.testing.assert_allclose(got[0].astype(np.float64), want[0].astype(np.float64), rtol=1e-2, atol=3e-3, err_msg=str(ks.info))
 
 
+@pytest.mark.parametrize("case", [(2, 1, 1, 3, 64), (1, 2, 2, 1, 32), (3, 1, 63, 2, 128), (2, 4, 129, 2, 64), (8, 1, 1025, 12, 64), (1, 3, 1281, 2, 64), (1, 1, 5000, 2, 32)],
+                         ids=lambda c: "B%d_L%d_S%d_N%d_H%d" % c)
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+def test_attention_of_few_queries(case, causal):
+    """One workgroup per query: one pass and several, several rounds, key counts around the passes, every head size."""
+    B, L, S, N, H = case
+    rng = np.random.default_rng(S + H)
+    q, k, v = [rng.standard_normal((B, T, N, H)).astype(np.float16) for T in (L, S, S)]
+    routine = attention_routine(B, L, S, N, causal, H=H)
+    got, ks = R.run_gpu(routine, [q, k, v])
+    want = R.run_oracle(routine, [q, k, v])
+    assert ks.info["blocks"] == B * L * N
+    np.testing.assert_allclose(got[0].astype(np.float64), want[0].astype(np.float64), rtol=2e-3, atol=1e-3, err_msg=str(ks.info))
+
+
 def test_attention_is_stable_for_large_scores_and_peaked_rows():
     rng = np.random.default_rng(4)
     q, k, v = [rng.standard_normal((1, 256, 2, 64)).astype(np.float16) for _ in range(3)]
@@ -167,3 +182,40 @@ def test_gpt2_block_with_fused_attention():
     want = block_reference(arrs["x"].astype(np.float64), {n: arrs[n].astype(np.float64) for n in order[1:]}, heads)
     np.testing.assert_allclose(y.astype(np.float64).reshape(batch, seq, d), want, rtol=3e-2, atol=3e-2)
     np.testing.assert_allclose(y.astype(np.float64), y0.astype(np.float64), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("shape", [(2, 40, 40, 3, 32), (1, 1, 77, 4, 64), (2, 130, 65, 1, 128)], ids=str)
+def test_composed_attention_runs_as_the_routine(shape, causal):
+    """The front-end's composition is recognised when a program is scheduled: same result within float16."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L_
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import Schedule
+    from oracle.backend import OracleBackend
+    B, L, S, N, H = shape
+    rng = np.random.default_rng(S)
+    arrays = [rng.standard_normal((B, T, N, H)).astype(np.float16) for T in (L, S, S)]
+    prog = J.jit(lambda q, k, v: L_.dotProductAttention(q, k, v, isCausal=causal), [ShapedArray(a.shape, F16) for a in arrays])
+    assert not prog.routines
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    be = backend()
+    names = [str(getattr(u.source, "name", "")) for u in Schedule(be, prog).units]
+    assert names == ["Attention"], names
+    got, want = run_program(be, prog, arrays), run_program(OracleBackend(), prog, arrays)
+    np.testing.assert_allclose(got[0].astype(np.float64), want[0].astype(np.float64), rtol=1e-2, atol=3e-3)
+
+
+def test_a_chain_whose_scores_are_used_elsewhere_stays_as_it_is():
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L_
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rewrite import fuse_attention
+
+    def f(q, k, v):
+        scores = L_.einsum("BLNH,BSNH->BNLS", q, k)
+        p = L_.softmax(scores, -1)
+        return [L_.einsum("BNLS,BSNH->BLNH", p, v), p]
+    prog = J.jit(f, [ShapedArray((1, 8, 2, 32), F16)] * 3)
+    assert fuse_attention(prog.jaxpr, prog.consts) is None
