@@ -15,6 +15,7 @@ from .alu import AluExp, AluOp, DType, Kernel, byteWidth
 from .codegen import CTYPE, STORAGE_CTYPE, HipExpCodegen, strip_parens
 from .kernelgen import KernelSource, LaunchStep, _Body, _min_bytes, _prelude, _used_args, epilogue_compile_options, fill, template
 from . import tuner
+from .fewgen import gen_few, plan_few
 from .tuner import TuneResult, classify_loads
 
 
@@ -545,7 +546,8 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
     re = kernel.reduction
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
-    tile = dict() if ("BM" in override or "BN" in override) else choose_tile(g)
+    few = plan_few(g) if not override else None
+    tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g)
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
         raise ValueError("a tile override must give both BM and BN")
@@ -584,7 +586,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
 
     # An operand off the 16-byte grid that a pre-pass copies into scratch (see `_repack_operand`): from here on it is a
     # dense [K][rows_pad] operand named `jh_repack`.
-    repack = _repack_operand(g) if split == 1 and tile.get("REPACK", 1) else None
+    repack = _repack_operand(g) if split == 1 and tile.get("REPACK", 1) and not few else None
     load_rows = dict(a=g["M"], b=g["N"])
     repack_src = {}
     if repack:
@@ -639,6 +641,21 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
         src_options = ""
         epi_fn = f"static __device__ __forceinline__ float jh_epilogue(float acc, int row, int col, int b0, int b1, int b2{epi_params}) {{\n  return acc;\n}}"
     epi_args = "".join(f", {n}" for n in names)
+
+    if few:
+        lines = ["  {", "    int rem = batch;"]
+        for k, (size, sa, sb, sc) in reversed(list(enumerate(g["batch"]))):
+            lines.append(f"    jh_b{k} = rem % {size}; rem /= {size};")
+            lines.append(f"    a_base += (long long)jh_b{k} * {sa}ll; b_base += (long long)jh_b{k} * {sb}ll; c_base += (long long)jh_b{k} * {sc}ll;")
+        lines.append("  }")
+        text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "")
+        need = _min_bytes(t.epilogue)
+        for tg in ("a", "b"):
+            need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * 2)
+        step = LaunchStep(name, grid, block, 0, [("in", i) for i in range(kernel.nargs)] + [("out", 0)])
+        return KernelSource([src_options + _prelude(numerics) + text], [step], [], "gemm", need,
+                            dict(few=True, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0], waves=few["waves"], columns=16 * few["VN"],
+                                 along_k=few["along_k"], splitk=1))
 
     # Element loaders for gather operands: the operand's lowered expression (masked load through its view
     # chain) with the flat output index rebuilt from (tile row, batch coordinates) and ridx = k.

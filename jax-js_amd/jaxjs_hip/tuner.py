@@ -689,10 +689,18 @@ def _gemm_worthwhile(g: dict) -> bool:
     thin = min(g["M"], g["N"])
     # (A convolution's gathered operand makes the reduction classes walk its window arithmetic once per output; it
     # pays to pad even a 27-long k axis -- 3 channels x 3 x 3 -- to one slab: 83 -> 14 us.)
-    if g["K"] < (GEMM_MIN_K // 2 if g.get("a_gather") or g.get("b_gather") else GEMM_MIN_K) or thin < 2:
-        return False  # one row or column is a matvec: the reduction classes stream it at the HBM rate
-    if thin < GEMM_MIN_ROWS and (max(g["M"], g["N"]) < 128 or g["K"] < 256 or max(g["M"], g["N"]) * g["K"] < (1 << 20)):
+    if g["K"] < (GEMM_MIN_K // 2 if g.get("a_gather") or g.get("b_gather") else GEMM_MIN_K):
         return False
+    wide = max(g["M"], g["N"])
+    # one row or column is a matvec: the reduction classes stream a large operand at the HBM rate
+    reduces = thin < 2 or (thin < GEMM_MIN_ROWS and (wide < 128 or g["K"] < 256 or wide * g["K"] < (1 << 20)))
+    if reduces:
+        # ... but one of half a megabyte to 16 that runs along the outputs is cut over k there, with a second launch for the
+        # fold, where the kernel for few rows takes one: 1 x 768 x 768 6.3 -> 3.1 us, 8 x 512 x 512 5.7 -> 2.7,
+        # 1 x 4096 x 2048 8.4 -> 4.2.  Along k the reductions are as fast (1 x 768 x 3072 3.0 us against 4.9).
+        if (g["dtype"] != DType.Float16 or g.get("a_gather") or g.get("b_gather") or wide < 128 or not 256 <= g["K"] < 4096 or not (1 << 18) <= wide * g["K"] <= (8 << 20)
+                or (g["b_sk"] if g["M"] <= g["N"] else g["a_sk"]) == 1):
+            return False
     # (2..31 rows against a large operand -- a linear layer on a handful of tokens -- do go to the matrix cores: as
     # separate dot products the large operand is read once per row, 202 us for 16 x 14336 x 4096 against 25 us.)
     vec = 8 if g["dtype"] == DType.Float16 else 4
@@ -718,6 +726,11 @@ def _gemm_worthwhile(g: dict) -> bool:
 
     # (Gather operands take any k extent: the element loader and the row-vector loader check every k, and the block
     # loaders of the tap-major order are only chosen when k is a multiple of 8.)
-    return ((g.get("a_gather") or operand_ok("a", g["a_sk"], g["a_sm"], g["M"], g["a_off"], bstr_a, g["a_k0"]))
+    fits = ((g.get("a_gather") or operand_ok("a", g["a_sk"], g["a_sm"], g["M"], g["a_off"], bstr_a, g["a_k0"]))
             and (g.get("b_gather") or operand_ok("b", g["b_sk"], g["b_sn"], g["N"], g["b_off"], bstr_b, g["b_k0"]))
             and split_ok(g["a_k0"], g["a_sk"], g["a_sk1"]) and split_ok(g["b_k0"], g["b_sk"], g["b_sk1"]))
+    if not (fits and reduces):
+        return fits
+    from .fewgen import plan_few
+
+    return plan_few(g) is not None

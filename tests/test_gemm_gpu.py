@@ -441,6 +441,20 @@ def test_gemm_with_a_handful_of_rows_runs_on_the_matrix_cores(dt, M, N, K, bt, w
     np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), A.astype(np.float32) @ B.astype(np.float32), err_msg=str(ks.info))
 
 
+@pytest.mark.parametrize("M,N,K,bt", [(1, 512, 512, False), (2, 777, 1000, False), (16, 1024, 1024, True), (17, 1001, 1530, False), (33, 640, 96, True), (64, 2000, 999, False),
+                                      (48, 515, 1026, True), (1, 2049, 1023, False), (9, 4096, 2048, True), (4100, 20, 257, True)])
+def test_gemm_f16_with_few_rows_on_one_side(M, N, K, bt):
+    """Up to 64 rows (or columns) against a matrix that streams straight into the matrix instructions: ragged column tiles,
+    k axes off the 32-step and off the 16-byte grid, both orders of the matrix."""
+    A, B = RNG.integers(-2, 3, (M, K)).astype(np.float16), RNG.integers(-2, 3, (K, N)).astype(np.float16)
+    A[:, RNG.random(K) < 0.7] = 0  # keep every sum an exact float16
+    got, ks = device_run(matmulKernel(M, N, K, DType.Float16, b_transposed=bt), [A, np.ascontiguousarray(B.T) if bt else B])
+    assert ks.klass == "gemm" and ks.info.get("few"), (ks.klass, ks.info)
+    want = A.astype(np.float32) @ B.astype(np.float32)
+    assert np.abs(want).max() <= 2048
+    np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), want, err_msg=str(ks.info))
+
+
 def test_single_rows_and_small_operands_stay_with_the_reduction_classes():
     from jaxjs_hip.tuner import tuneHip
     for M, N, K in ((1, 14336, 4096), (14336, 1, 4096), (5, 300, 700), (16, 64, 64), (8, 100, 2048)):
