@@ -24,26 +24,26 @@ class GraphedProgram:
         for s in inputs:
             backend.incRef(s)
             self._owned.append(s)
-        steps = [s for s in prog.steps if s.kind == "execute"]
-        # compile + load before any capture; a routine step is several launches and outputs, recorded the same way
-        exes = [backend.prepareRoutineSync(s.routine) if s.routine is not None else backend.prepareKernelSync(s.kernel) for s in steps]
+        # The units of the program's schedule, compiled and loaded before any capture; a routine is several launches and
+        # outputs, recorded the same way.
+        schedule = backend.scheduleProgram(prog)
+        prog, units = schedule.prog, schedule.units
         # The graph launches these executables' code objects and writes their scratch buffers without going through
         # dispatch: pin them so that neither cache eviction nor clearCache() can release them under a replay.
         self._exes = []
-        for exe in exes:
-            backend.pin(exe)
-            self._exes.append(exe)
+        for u in units:
+            backend.pin(u.exe)
+            self._exes.append(u.exe)
         sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
-        for s in steps:
-            for o in (s.outputs if s.routine is not None else [s.output]):
+        for u in units:
+            for o in u.outputs:
                 slot = backend.malloc(sizes[o])
                 self._slots[o] = slot
                 self._owned.append(slot)
 
         def issue():
-            for s, exe in zip(steps, exes):
-                outs = s.outputs if s.routine is not None else [s.output]
-                backend.dispatch(exe, [self._slots[i] for i in s.inputs], [self._slots[o] for o in outs])
+            for u in units:
+                backend.dispatch(u.exe, [self._slots[i] for i in u.inputs], [self._slots[o] for o in u.outputs])
 
         issue()  # one eager pass: every code object is resident before the capture starts
         backend.dev.sync()
@@ -59,7 +59,7 @@ class GraphedProgram:
         finally:
             backend.trace, backend.capturing = trace, False
         self.outputs = [self._slots[o] for o in prog.outputs]
-        self.kernels = len(steps)
+        self.kernels = len(units)
 
     def launch(self) -> None:
         """Queue one replay of the whole program (asynchronous, in order with everything else)."""
