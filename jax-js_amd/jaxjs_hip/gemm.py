@@ -546,7 +546,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
     re = kernel.reduction
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
-    few = plan_few(g) if not override else None
+    few = plan_few(g, lambda: choose_tile(g)) if not override and _repack_operand(g) is None else None
     tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g)
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
@@ -651,10 +651,10 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
         text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "")
         need = _min_bytes(t.epilogue)
         for tg in ("a", "b"):
-            need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * 2)
+            need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * byteWidth(g["dtype"]))
         step = LaunchStep(name, grid, block, 0, [("in", i) for i in range(kernel.nargs)] + [("out", 0)])
         return KernelSource([src_options + _prelude(numerics) + text], [step], [], "gemm", need,
-                            dict(few=True, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0], waves=few["waves"], columns=16 * few["VN"],
+                            dict(few=True, direct_lds=False, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0], waves=few["waves"], columns=16 * few["VN"],
                                  along_k=few["along_k"], splitk=1))
 
     # Element loaders for gather operands: the operand's lowered expression (masked load through its view

@@ -695,11 +695,15 @@ def _gemm_worthwhile(g: dict) -> bool:
     # one row or column is a matvec: the reduction classes stream a large operand at the HBM rate
     reduces = thin < 2 or (thin < GEMM_MIN_ROWS and (wide < 128 or g["K"] < 256 or wide * g["K"] < (1 << 20)))
     if reduces:
-        # ... but one of half a megabyte to 16 that runs along the outputs is cut over k there, with a second launch for the
-        # fold, where the kernel for few rows takes one: 1 x 768 x 768 6.3 -> 3.1 us, 8 x 512 x 512 5.7 -> 2.7,
-        # 1 x 4096 x 2048 8.4 -> 4.2.  Along k the reductions are as fast (1 x 768 x 3072 3.0 us against 4.9).
-        if (g["dtype"] != DType.Float16 or g.get("a_gather") or g.get("b_gather") or wide < 128 or not 256 <= g["K"] < 4096 or not (1 << 18) <= wide * g["K"] <= (8 << 20)
-                or (g["b_sk"] if g["M"] <= g["N"] else g["a_sk"]) == 1):
+        # ... but an operand that runs along the outputs is walked there one output a lane, or cut over k with a second launch
+        # for the fold, where the kernel for few rows takes one launch: float16 1 x 768 x 768 6.3 -> 3.1 us, 8 x 512 x 512
+        # 5.7 -> 2.7, 1 x 4096 x 2048 8.4 -> 4.2, 12 x 54 x 576 5.6 -> 2.7; float32 22 x 407 x 329 5.6 -> 2.8,
+        # 11 x 768 x 183 3.9 -> 2.7.  Along k the reductions are as fast (1 x 768 x 3072 3.0 us against 4.9), and a small
+        # float16 operand with a longer k axis stays with them.
+        f32 = g["dtype"] == DType.Float32
+        size = wide * g["K"]
+        if (g["dtype"] not in (DType.Float16, DType.Float32) or g.get("a_gather") or g.get("b_gather") or not 96 <= g["K"] < 4096 or size > (8 << 20)
+                or (g["b_sk"] if g["M"] <= g["N"] else g["a_sk"]) == 1 or not (f32 or g["K"] < 640 or (size >= 1 << 18 and wide >= 128))):
             return False
     # (2..31 rows against a large operand -- a linear layer on a handful of tokens -- do go to the matrix cores: as
     # separate dot products the large operand is read once per row, 202 us for 16 x 14336 x 4096 against 25 us.)

@@ -441,15 +441,21 @@ def test_gemm_with_a_handful_of_rows_runs_on_the_matrix_cores(dt, M, N, K, bt, w
     np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), A.astype(np.float32) @ B.astype(np.float32), err_msg=str(ks.info))
 
 
-@pytest.mark.parametrize("M,N,K,bt", [(1, 512, 512, False), (2, 777, 1000, False), (16, 1024, 1024, True), (17, 1001, 1530, False), (33, 640, 96, True), (64, 2000, 999, False),
-                                      (48, 515, 1026, True), (1, 2049, 1023, False), (9, 4096, 2048, True), (4100, 20, 257, True)])
-def test_gemm_f16_with_few_rows_on_one_side(M, N, K, bt):
-    """Up to 64 rows (or columns) against a matrix that streams straight into the matrix instructions: ragged column tiles,
-    k axes off the 32-step and off the 16-byte grid, both orders of the matrix."""
-    A, B = RNG.integers(-2, 3, (M, K)).astype(np.float16), RNG.integers(-2, 3, (K, N)).astype(np.float16)
+@pytest.mark.parametrize("dt,M,N,K,bt", [
+    (DType.Float16, 1, 512, 512, False), (DType.Float16, 2, 777, 1000, False), (DType.Float16, 16, 1024, 1024, True), (DType.Float16, 17, 1001, 1530, False),
+    (DType.Float16, 33, 640, 96, True), (DType.Float16, 64, 2000, 999, False), (DType.Float16, 48, 515, 1026, True), (DType.Float16, 4100, 20, 257, True),
+    (DType.Float16, 9, 4096, 2048, True), (DType.Float16, 322, 1025, 412, False), (DType.Float32, 64, 256, 784, False), (DType.Float32, 40, 74, 767, False),
+    (DType.Float32, 1, 130, 97, False), (DType.Float32, 128, 315, 565, True), (DType.Float32, 209, 56, 33, False), (DType.Float32, 2650, 128, 309, False),
+], ids=lambda v: v.value if isinstance(v, DType) else str(v))
+def test_gemm_too_small_for_tiles(dt, M, N, K, bt):
+    """Few rows, or few tiles, against a matrix that streams straight into the matrix instructions: ragged row and column
+    tiles, k axes off the step and off the 16-byte grid, both orders of the matrix."""
+    npdt = np.float16 if dt == DType.Float16 else np.float32
+    A, B = RNG.integers(-2, 3, (M, K)).astype(npdt), RNG.integers(-2, 3, (K, N)).astype(npdt)
     A[:, RNG.random(K) < 0.7] = 0  # keep every sum an exact float16
-    got, ks = device_run(matmulKernel(M, N, K, DType.Float16, b_transposed=bt), [A, np.ascontiguousarray(B.T) if bt else B])
+    got, ks = device_run(matmulKernel(M, N, K, dt, b_transposed=bt), [A, np.ascontiguousarray(B.T) if bt else B])
     assert ks.klass == "gemm" and ks.info.get("few"), (ks.klass, ks.info)
+    assert ks.min_input_bytes == {0: A.nbytes, 1: B.nbytes}  # what the kernel addresses, so that a short buffer is an error
     want = A.astype(np.float32) @ B.astype(np.float32)
     assert np.abs(want).max() <= 2048
     np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), want, err_msg=str(ks.info))
