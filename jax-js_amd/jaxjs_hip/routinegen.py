@@ -23,7 +23,16 @@ from .shape import prod
 
 _SORT_KINDS = {DType.Float32: (0, "float"), DType.Float16: (1, "jh_f16"), DType.Int32: (2, "int"),
                DType.Uint32: (3, "jh_u32"), DType.Bool: (2, "int"), DType.Float64: (4, "double")}
-SORT_TILE = 8192  # 64 KB of LDS in 8-byte words: rows up to 8192 elements never leave the CU (4096 in 16-byte words)
+SORT_TILE = 8192  # LDS tile in 8-byte words (64 KB): 16384 4-byte words, 4096 16-byte words
+SORT_REGISTERS = 256  # bytes of words a lane holds in the register network
+SORT_WAVES = 2048     # waves (two per SIMD) from which 16 lanes per row are enough; with fewer, a row takes up to 64
+# Rows of more than 64 x 16 words in fewer than 256 waves: short register runs on many lanes, then LDS (float32 1 x 4096:
+# 9.6 us against 11.2 with runs of 1024 words; 600 x 3000 stays in registers, 21.7 us).
+SORT_FEW, SORT_FEW_WAVES = 16, 256
+# Fewer tiles than a quarter of the chip: smaller ones, which cost a launch per stage but work side by side (float32
+# 1 x 20000: 58 us with tiles of 16384, 36 of 8192, 33 of 4096, 37 of 2048; 100 x 16384 stays at 16384, 42.5 against 45.6).
+SORT_SMALL_TILE, SORT_FEW_TILES = 4096, 64
+SORT_LOCAL, SORT_TILES = 16, 1024  # words of a lane in a tile's register runs, from 1024 tiles on
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
 CHOLESKY_PANEL_FROM = 192  # matrix order from which one panel's launch spans many CUs (smaller ones: a few workgroups)
 
@@ -530,30 +539,43 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
         return None
     P = max(_next_pow2(n), 2)
     kind, ctype = _SORT_KINDS[dtype]
-    word = (8 if argsort else 4) * (2 if dtype == DType.Float64 else 1)  # bytes per keyed word
-    tile = min(P, SORT_TILE * 8 // max(word, 8))
-    # A thread moves eight words per pass (three strides at once, or its register group), so tile / 8 threads keep
-    # every lane busy and leave room for several blocks per CU, whose barriers then overlap; with few tiles in the
-    # launch the wider block (tile / 2) finishes its one tile sooner.
-    threads = max(1, min(tile // 2, 1024))
-    if rows * (P // tile) >= 8 * 256 and tile >= 512:
-        threads = min(tile // 8, 1024)
-    src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(N=n, P=P, ROWS=rows, TILE=tile, ARGSORT=1 if argsort else 0,
-                                                                   KIND=kind, T=ctype, THREADS=threads, GROUP=SORT_GROUP if P > 256 else 4))
-    tiles = rows * (P // tile)
+    short = argsort and dtype == DType.Float16 and n <= 65536  # key and position in 32 bits
+    word = (8 if argsort and not short else 4) * (2 if dtype == DType.Float64 else 1)  # bytes per keyed word
+    most = SORT_REGISTERS // word
+    values = dict(N=n, P=P, ROWS=rows, ARGSORT=1 if argsort else 0, KIND=kind, T=ctype, GROUP=SORT_GROUP if P > 256 else 4)
+    need = {0: rows * n * byteWidth(dtype)}
     outs = [("out", 0), ("out", 1)] if argsort else [("out", 0), ("out", 0)]
+    if P <= 64 * most:
+        # 16 lanes per row pair most words inside a lane and reach every other one by DPP; with few rows up to 64, since the
+        # launch then waits for one wave's chain.
+        E = min(max(2, P // 16), most)
+        while E > max(2, P // 64) and rows * (P // E) < SORT_WAVES * 64:
+            E //= 2
+        E = max(E, P // 64, 1)
+        if E <= SORT_FEW or rows * (P // E) >= SORT_FEW_WAVES * 64:
+            src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, TILE=P, THREADS=256, E=E, W=P))
+            steps = [LaunchStep("jh_sort_rows", (-(-rows * (P // E) // 256), 1, 1), (256, 1, 1), 0, [("in", 0)] + outs)]
+            return KernelSource([src], steps, [], "sort", need, dict(n=n, rows=rows, P=P, tile=P, argsort=argsort, launches=1))
+    tile = min(P, SORT_TILE * 8 // word)
+    while tile > SORT_SMALL_TILE and rows * (P // tile) < SORT_FEW_TILES:
+        tile //= 2
+    # With few tiles the block is as wide as it gets, which finishes its one tile sooner; else longer register runs.
+    E = max(min(SORT_LOCAL, most // 2) if rows * (P // tile) >= SORT_TILES else 4, tile // 1024)
+    threads = tile // E
+    src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, TILE=tile, THREADS=threads, E=E, W=64 * E))
+    tiles = rows * (P // tile)
     steps = [LaunchStep("jh_sort_local", (tiles, 1, 1), (threads, 1, 1), 0, [("in", 0), ("scratch", 0)] + outs)]
-    pair_blocks = max(1, min((rows * (P // 2) + 255) // 256, 1 << 20))
     k = tile * 2
     while k <= P:
         j = k // 2
         while j >= tile:
-            steps.append(LaunchStep("jh_sort_global", (pair_blocks, 1, 1), (256, 1, 1), 0, [("scratch", 0), ("const", k), ("const", j)]))
-            j //= 2
+            count = min(3, (j // tile).bit_length())
+            blocks = max(1, min((rows * (P >> count) + 255) // 256, 1 << 20))
+            steps.append(LaunchStep("jh_sort_global", (blocks, 1, 1), (256, 1, 1), 0, [("scratch", 0), ("const", k), ("const", j), ("const", count)]))
+            j >>= count
         steps.append(LaunchStep("jh_sort_merge", (tiles, 1, 1), (threads, 1, 1), 0, [("in", 0), ("scratch", 0)] + outs + [("const", k)]))
         k *= 2
     scratch = [rows * P * word] if P > tile else [16]
-    need = {0: rows * n * byteWidth(dtype)}
     return KernelSource([src], steps, scratch, "sort", need, dict(n=n, rows=rows, P=P, tile=tile, argsort=argsort, launches=len(steps)))
 
 

@@ -122,6 +122,34 @@ def test_argsort_matches_host_routine(shape, dtype):
     np.testing.assert_array_equal(v.view(np.uint8), wv.view(np.uint8))
 
 
+# Edges of the register network: lanes 1 to 64 per row and 2 to 64 words per lane (row lengths around powers of two, few and
+# many rows), rows past the last whole workgroup, runs of a tile in LDS, tiles chosen for few and for many rows, fused
+# strides over memory, and the longest float16 row whose key and position share a word.
+@pytest.mark.parametrize("shape,dtype", [((70, 16), DType.Float32), ((33, 17), DType.Float16), ((1000, 33), DType.Int32), ((3, 129), DType.Float32),
+                                         ((2100, 1024), DType.Float32), ((300, 1000), DType.Float64), ((9000, 130), DType.Float32), ((260, 4095), DType.Float32),
+                                         ((3, 4096), DType.Float32), ((70, 8192), DType.Int32), ((1030, 16384), DType.Float32), ((2, 40000), DType.Float32),
+                                         ((1, 140000), DType.Float16), ((1, 65536), DType.Float16), ((1, 65537), DType.Float16)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v.value)
+@pytest.mark.parametrize("name", [Routines.Sort, Routines.Argsort], ids=lambda n: n.value)
+def test_sort_register_network(name, shape, dtype):
+    x = _data(shape, dtype)
+    be = backend()
+    if WARM_ONLY:
+        run(name, x, dtype)
+    exe = be.prepareRoutineSync(make(name, shape, dtype))
+    src, out, idx = be.malloc(x.nbytes, x.tobytes()), be.malloc(x.nbytes), be.malloc(x.size * 4)
+    be.dispatch(exe, [src], [out] if name == Routines.Sort else [out, idx])
+    y = np.frombuffer(be.readSync(out), dtype=x.dtype).reshape(shape)
+    if name == Routines.Sort:
+        np.testing.assert_array_equal(y, np.sort(x, -1))
+    else:
+        want = np.argsort(x, -1, kind="stable")
+        np.testing.assert_array_equal(np.frombuffer(be.readSync(idx), dtype=np.int32).reshape(shape), want)
+        np.testing.assert_array_equal(y.view(np.uint8), np.take_along_axis(x, want, -1).view(np.uint8))
+    for s in (src, out, idx):
+        be.decRef(s)
+
+
 def test_zero_sized_rows_and_unsupported_dtype_path():
     if WARM_ONLY:
         pytest.skip("nothing to compile")
