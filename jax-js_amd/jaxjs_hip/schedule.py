@@ -15,12 +15,13 @@ import threading
 from typing import Any, Dict, List, Optional, Sequence
 
 from . import tracing
-from .alu import Kernel, byteWidth
+from .alu import AluExp, AluOp, DType, Kernel, Reduction, byteWidth
 from .errors import SlotError
 from .routine import Routine
-from .rowchain import collect_chain
+from .rowchain import _tidy, collect_chain, index_form
 from .runtime import LaunchRef, LaunchStepC, check
 from .shape import prod
+from .tuner import match_gemm
 
 
 class Unit:
@@ -31,9 +32,59 @@ class Unit:
         self.exe = None
 
 
+def join_epilogue(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int]) -> Optional[Kernel]:
+    """The contraction `product`, which writes `buffer`, with the elementwise `following` (reading `inputs`) as the rest of
+    its epilogue, or None.  `following` has to read nothing but `buffer`, each element at its own position.  The product's
+    value keeps the type it was stored in, so results keep their bits.
+
+    A value that is used more than once ends the front-end's fusion (src/frontend/jit.ts:572-789): gelu behind a linear
+    layer was a launch of its own that read and wrote the whole activation again (float16 [8192, 3072]: 24 us)."""
+    re = product.reduction
+    if re is None or following.reduction is not None or following.size != product.size or product.size == 0:
+        return None
+    gidx = AluExp.special(DType.Int32, "gidx", product.size)
+    exp = following.exp.substitute({"gidx": gidx}).rewriteGlobalViews().reduceExactIndex().simplify()
+    loads = exp.collect(lambda n: n.op == AluOp.GlobalIndex)
+    own = _tidy({("gidx", 1): 1}, {"gidx": product.size})
+    if not loads or any(inputs[n.arg[0]] != buffer or n.dtype != re.epilogue.dtype or index_form(n.src[0], {"gidx": product.size}) != own for n in loads):
+        return None
+    if match_gemm(product) is None:
+        return None
+    exp = exp.rewrite(lambda n: re.epilogue if n.op == AluOp.GlobalIndex else None)
+    return Kernel(product.nargs, product.size, product.exp_raw, Reduction(re.dtype, re.op, re.size, exp))
+
+
+class _Dispatch:
+    """One dispatch of a program: `kernel` or `routine`, and buffer ids."""
+
+    def __init__(self, kernel, routine, inputs, output, outputs):
+        self.kernel, self.routine, self.inputs, self.output, self.outputs = kernel, routine, inputs, output, outputs
+
+
+def plan_dispatches(prog) -> List[_Dispatch]:
+    """The program's dispatches, elementwise Kernels behind a contraction joined to it where nothing else reads its result."""
+    made = [_Dispatch(s.kernel, s.routine, s.inputs, s.output, s.outputs) for s in prog.steps if s.kind == "execute"]
+    reads: Dict[int, int] = {}
+    for d in made:
+        for i in set(d.inputs):
+            reads[i] = reads.get(i, 0) + 1
+    kept = set(prog.outputs)
+    out: List[_Dispatch] = []
+    for d in made:
+        before = out[-1] if out else None
+        if before is not None and before.kernel is not None and d.kernel is not None and before.output in d.inputs \
+                and reads[before.output] == 1 and before.output not in kept:
+            joined = join_epilogue(before.kernel, before.output, d.kernel, d.inputs)
+            if joined is not None:
+                out[-1] = _Dispatch(joined, None, before.inputs, d.output, d.outputs)
+                continue
+        out.append(d)
+    return out
+
+
 def plan_units(prog) -> List[Unit]:
     """The program's dispatches with runs of Kernels over the same rows joined."""
-    steps = [s for s in prog.steps if s.kind == "execute"]
+    steps = plan_dispatches(prog)
     last_read: Dict[int, int] = {}
     for k, s in enumerate(steps):
         for i in s.inputs:

@@ -66,3 +66,13 @@ def test_a_chain_keeps_what_is_read_behind_it():
 def test_row_statistics_of_the_benchmark_program():
     x = np.random.default_rng(1).standard_normal((333, 4096)).astype(np.float32)
     check(W.rowSoftmaxArgmaxProgram(333, 4096), [x], False)
+
+
+@pytest.mark.parametrize("mnk", [(8, 512, 256), (130, 257, 100), (512, 512, 256), (128, 128, 2048), (1, 96, 64)], ids=str)
+@pytest.mark.parametrize("dtype", [DType.Float32, DType.Float16], ids=lambda d: d.value)
+def test_an_elementwise_kernel_in_a_contractions_epilogue(dtype, mnk):
+    m, n, k = mnk
+    rng, t = np.random.default_rng(m), np.float16 if dtype == DType.Float16 else np.float32
+    arrays = [rng.standard_normal((m, k)).astype(t), (rng.standard_normal((k, n)) * k ** -0.5).astype(t), rng.standard_normal(n).astype(t)]
+    prog = J.jit(lambda x, w, b: L.gelu(L.matmul(x, w).add(b)), [ShapedArray(a.shape, dtype) for a in arrays])
+    check(prog, arrays, dtype == DType.Float16, chained=False)

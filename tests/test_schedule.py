@@ -52,3 +52,19 @@ def test_intermediates_that_are_alive_together_do_not_overlap():
             for b in range(a):
                 if last[b] >= a:  # b is still read when a is written
                     assert placed[a] + sizes[a] <= placed[b] or placed[b] + sizes[b] <= placed[a], (a, b)
+
+
+def test_an_elementwise_kernel_joins_the_contraction_that_only_it_reads():
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import plan_units
+    avals = [ShapedArray(s, DType.Float16) for s in ((64, 128), (128, 256), (256,))]
+
+    def count(f):
+        return len(plan_units(J.jit(f, avals)))
+
+    hidden = lambda x, w, b: L.matmul(x, w).add(b)  # noqa: E731
+    assert count(lambda x, w, b: L.gelu(hidden(x, w, b))) == 1
+    assert count(lambda x, w, b: (lambda h: [L.gelu(h), h])(hidden(x, w, b))) == 2            # the product is kept
+    assert count(lambda x, w, b: (lambda h: h.mul(h).mul(L.swapaxes(h, 0, 1)))(L.matmul(x, L.swapaxes(x, 0, 1)))) == 2  # read at another position too
