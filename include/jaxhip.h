@@ -104,7 +104,7 @@ int jh_host_free(void *ptr);
  * malloc'd code object to release with `jh_code_free`; on failure `log` (if non-NULL) receives
  * the compiler output, truncated to `log_size`.  A source may ask for options of its own in leading lines of the form
  * `// hiprtc-option: <option>`: they are added to `options` when they are on the library's fixed list
- * (`-fno-slp-vectorize`, which the generator puts on float16 kernels) and make the call fail when they are not.
+ * (`-fno-slp-vectorize`, which the generator puts on float16 kernels, `-ffinite-math-only` on sorts) and make the call fail when they are not.
  */
 int jh_compile(const char *source, const char *name, const char *const *options, int num_options,
                void **code, size_t *code_size, char *log, size_t log_size);

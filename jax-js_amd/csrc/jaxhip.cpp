@@ -261,11 +261,12 @@ int jh_compile(const char *source, const char *name, const char *const *options,
   hiprtcResult r = hiprtcCreateProgram(&prog, source, name ? name : "kernel.hip", 0, nullptr, nullptr);
   if (r != HIPRTC_SUCCESS) return fail((int)r, "hiprtcCreateProgram: %s", hiprtcGetErrorString(r));
   // Options the source asks for itself: leading lines of the form "// hiprtc-option: <option>", honoured for the
-  // options on a fixed list (the generator marks float16 kernels that the SLP vectorizer makes the compiler abort on).
+  // options on a fixed list (the generator marks float16 kernels that the SLP vectorizer makes the compiler abort on, and
+  // sorts whose only floating-point values are finite ones made from integer keys).
   std::vector<std::string> asked;
   {
     static const char kMark[] = "// hiprtc-option: ";
-    static const char *const kAllowed[] = {"-fno-slp-vectorize"};
+    static const char *const kAllowed[] = {"-fno-slp-vectorize", "-ffinite-math-only"};
     const char *line = source;
     while (strncmp(line, kMark, sizeof(kMark) - 1) == 0) {
       const char *begin = line + sizeof(kMark) - 1;

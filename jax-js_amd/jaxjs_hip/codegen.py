@@ -20,7 +20,7 @@ from .errors import UnsupportedOpError
 # A generated source may open with lines of this form; `runtime.compile_source` adds the named option (from a fixed
 # list) to the compiler's command line for that source alone.
 SOURCE_OPTION = "// hiprtc-option: "
-SOURCE_OPTIONS_ALLOWED = ("-fno-slp-vectorize",)
+SOURCE_OPTIONS_ALLOWED = ("-fno-slp-vectorize", "-ffinite-math-only")
 
 CTYPE = {
     DType.Float32: "float",

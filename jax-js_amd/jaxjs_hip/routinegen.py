@@ -16,6 +16,7 @@ from __future__ import annotations
 from typing import Optional
 
 from .alu import DType, byteWidth
+from .codegen import SOURCE_OPTION
 from .kernelgen import KernelSource, LaunchStep, _prelude, fill, template
 from .errors import UnsupportedRoutineError
 from .routine import Routine, Routines, ScatterOp
@@ -545,15 +546,17 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
     values = dict(N=n, P=P, ROWS=rows, ARGSORT=1 if argsort else 0, KIND=kind, T=ctype, GROUP=SORT_GROUP if P > 256 else 4)
     need = {0: rows * n * byteWidth(dtype)}
     outs = [("out", 0), ("out", 1)] if argsort else [("out", 0), ("out", 0)]
-    if P <= 64 * most:
+    if P <= (64 if word == 4 and not argsort else 32 if short else 16) * most:
         # 16 lanes per row pair most words inside a lane and reach every other one by DPP; with few rows up to 64, since the
-        # launch then waits for one wave's chain.
+        # launch then waits for one wave's chain.  Sorts gain from registers up to 64 lanes (8000 x 4000 float32: 118 us
+        # against 134 through LDS); wider words pay for every lane exchange twice and argsort gathers its values (argsort
+        # float32 4000 x 2000: 95 us in 64 lanes, 54 through LDS; 30000 x 1000: 206 in 32, 154; float16 8000 x 4000: 183 and 144).
         E = min(max(2, P // 16), most)
         while E > max(2, P // 64) and rows * (P // E) < SORT_WAVES * 64:
             E //= 2
         E = max(E, P // 64, 1)
         if E <= SORT_FEW or rows * (P // E) >= SORT_FEW_WAVES * 64:
-            src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, TILE=P, THREADS=256, E=E, W=P))
+            src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=0, TILE=P, THREADS=256, E=E, W=P))
             steps = [LaunchStep("jh_sort_rows", (-(-rows * (P // E) // 256), 1, 1), (256, 1, 1), 0, [("in", 0)] + outs)]
             return KernelSource([src], steps, [], "sort", need, dict(n=n, rows=rows, P=P, tile=P, argsort=argsort, launches=1))
     tile = min(P, SORT_TILE * 8 // word)
@@ -561,8 +564,13 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
         tile //= 2
     # With few tiles the block is as wide as it gets, which finishes its one tile sooner; else longer register runs.
     E = max(min(SORT_LOCAL, most // 2) if rows * (P // tile) >= SORT_TILES else 4, tile // 1024)
+    E = min(E, P // 128)  # (runs shorter than the row, of 64 lanes)
     threads = tile // E
-    src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, TILE=tile, THREADS=threads, E=E, W=64 * E))
+    # Words that are doubles where they go through LDS (float32 2000 x 7000: 204 -> 179 us; the register network alone
+    # loses by them, 30000 x 1000 in 32 lanes: 206 -> 243).
+    doubles = argsort and dtype in (DType.Float32, DType.Int32, DType.Uint32, DType.Bool) and n <= 1 << 20
+    opening = SOURCE_OPTION + "-ffinite-math-only\n" if doubles else ""
+    src = opening + _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=1 if doubles else 0, TILE=tile, THREADS=threads, E=E, W=64 * E))
     tiles = rows * (P // tile)
     steps = [LaunchStep("jh_sort_local", (tiles, 1, 1), (threads, 1, 1), 0, [("in", 0), ("scratch", 0)] + outs)]
     k = tile * 2

@@ -128,7 +128,7 @@ def test_argsort_matches_host_routine(shape, dtype):
 @pytest.mark.parametrize("shape,dtype", [((70, 16), DType.Float32), ((33, 17), DType.Float16), ((1000, 33), DType.Int32), ((3, 129), DType.Float32),
                                          ((2100, 1024), DType.Float32), ((300, 1000), DType.Float64), ((9000, 130), DType.Float32), ((260, 4095), DType.Float32),
                                          ((3, 4096), DType.Float32), ((70, 8192), DType.Int32), ((1030, 16384), DType.Float32), ((2, 40000), DType.Float32),
-                                         ((1, 140000), DType.Float16), ((1, 65536), DType.Float16), ((1, 65537), DType.Float16)],
+                                         ((1, 140000), DType.Float16), ((1, 1 << 20), DType.Int32), ((1, (1 << 20) + 1), DType.Float32), ((1, 65536), DType.Float16), ((1, 65537), DType.Float16)],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v.value)
 @pytest.mark.parametrize("name", [Routines.Sort, Routines.Argsort], ids=lambda n: n.value)
 def test_sort_register_network(name, shape, dtype):
