@@ -118,8 +118,9 @@ def routineKey(routine: Routine) -> tuple:
 
 
 def programKey(prog) -> tuple:
-    """Structural identity of a jit program: its dispatches and how they are wired."""
-    return (prog.nargs, tuple(prog.outputs), tuple(
+    """Structural identity of a jit program: its dispatches, how they are wired, and the constants it closes over, whose
+    values a schedule may be specialised on (a mask that is the lower triangle)."""
+    return (prog.nargs, tuple(prog.outputs), tuple((tuple(c.shape), c.dtype, c.exp) for c in prog.consts), tuple(
         (s.kind, s.output, s.size) if s.kind != "execute" else
         (s.kernel.key(), s.output, *s.inputs) if s.routine is None else (routineKey(s.routine), *s.outputs, *s.inputs) for s in prog.steps))
 

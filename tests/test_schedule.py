@@ -68,3 +68,50 @@ def test_an_elementwise_kernel_joins_the_contraction_that_only_it_reads():
     assert count(lambda x, w, b: L.gelu(hidden(x, w, b))) == 1
     assert count(lambda x, w, b: (lambda h: [L.gelu(h), h])(hidden(x, w, b))) == 2            # the product is kept
     assert count(lambda x, w, b: (lambda h: h.mul(h).mul(L.swapaxes(h, 0, 1)))(L.matmul(x, L.swapaxes(x, 0, 1)))) == 2  # read at another position too
+
+
+def _stand_in(limit=4096):
+    """A backend without a device: kernels are generated, not compiled, and launch lists are kept instead of launched."""
+    from collections import OrderedDict
+
+    from jaxjs_hip import backend as B
+    from test_backend_cache import make_backend
+    be = make_backend(limit)
+    be.numerics, be._programs, be.programLimit, be.trace, be._slots, be._next_slot = "fast", OrderedDict(), 512, None, {}, 1
+    be._pool, be._pool_bytes, be._pool_limit = {}, 0, 1 << 30
+    made = []
+
+    def build(source, ks, blobs=None):
+        made.append(B.Executable(source, B._Prepared(ks, [100 + len(made)] * len(ks.steps), [7] * len(ks.scratch_bytes), [1])))
+        return made[-1]
+    be._build = build
+    return be
+
+
+_MASKS = {"tril": 0, "one above": 1, "one below": -1, "argument": None}
+
+
+def _masked_attention(k, shape=(1, 48, 48, 2, 32)):
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    B, l, s, n, h = shape
+
+    def attend(mask, q, key, v):
+        scores = L.einsum("BLNH,BSNH->BNLS", q, key).mul(h ** -0.5)
+        return L.einsum("BNLS,BSNH->BLNH", L.softmax(J.where(mask, scores, -np.inf), -1), v)
+    operands = [ShapedArray((B, t, n, h), DType.Float16) for t in (l, s, s)]
+    if k is None:
+        return J.jit(attend, [ShapedArray((l, s), DType.Bool)] + operands)
+    return J.jit(lambda q, key, v: attend(L.tri_const(l, s, k), q, key, v), operands)
+
+
+@pytest.mark.parametrize("order", [list(_MASKS), list(_MASKS)[::-1]], ids=["tril first", "tril last"])
+def test_a_schedule_is_found_again_only_for_the_constants_it_was_made_for(order):
+    """Four programs with the same dispatches: only the one whose mask is the lower triangle has a causal attention."""
+    be = _stand_in()
+    for _ in range(2):
+        for name in order:
+            units = be.scheduleProgram(_masked_attention(_MASKS[name])).units
+            assert any(getattr(u.source, "params", None) for u in units) == (name == "tril"), name
+    assert len(be._programs) == 4
