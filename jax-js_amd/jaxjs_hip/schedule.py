@@ -143,6 +143,7 @@ class Schedule:
         from .jit import jitCompile
         from .rewrite import fuse_attention
 
+        self.source = prog  # its expressions, which name it in the backend's cache, live as long as the schedule
         fused = fuse_attention(prog.jaxpr, prog.consts) if prog.jaxpr is not None else None
         if fused is not None:
             prog = jitCompile(fused, prog.consts, backend.maxArgs)

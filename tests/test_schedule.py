@@ -115,3 +115,16 @@ def test_a_schedule_is_found_again_only_for_the_constants_it_was_made_for(order)
             units = be.scheduleProgram(_masked_attention(_MASKS[name])).units
             assert any(getattr(u.source, "params", None) for u in units) == (name == "tril"), name
     assert len(be._programs) == 4
+
+
+def test_a_schedule_keeps_the_program_that_its_key_was_made_from():
+    """The key names expressions by identity: they have to live as long as it does, rewritten program or not."""
+    import gc
+    import weakref
+    be = _stand_in()
+    prog = _masked_attention(0)
+    nodes = [weakref.ref(k.exp) for k in prog.kernels]
+    be.scheduleProgram(prog)
+    del prog
+    gc.collect()
+    assert all(n() is not None for n in nodes)
