@@ -63,12 +63,14 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
     if tuple(p.aval.shape) != (B, N, L, 1, S) or tuple(z.aval.shape) != (B, N, 1, H, S) or S < 2 or B * N * L * S * H == 0:
         return None
     share = g.by(g.through(p, "Reshape"), "Mul")
-    if share is None or tuple(share.outBinders[0].aval.shape) != (B, N, L, S):
+    # Operands broadcast, and reshapes are looked through: a value per row has to be read as one, next to whole rows.
+    rows, row = (B, N, L, S), (B, N, L, 1)
+    if share is None or tuple(share.outBinders[0].aval.shape) != rows:
         return None
     for e, r in (share.inputs, share.inputs[::-1]):  # exp(...) times 1 / its sum
         inverse = g.by(r, "Reciprocal")
         exp = g.by(e, "Exp", uses=2)
-        if inverse is not None and exp is not None:
+        if inverse is not None and exp is not None and tuple(r.aval.shape) == row and tuple(e.aval.shape) == rows:
             break
     else:
         return None
@@ -80,7 +82,7 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
         return None
     for scores, m in (shifted.inputs, shifted.inputs[::-1]):  # scores minus their maximum
         minus = g.by(m, "Neg")
-        if minus is not None:
+        if minus is not None and tuple(m.aval.shape) == row and tuple(scores.aval.shape) == rows:
             break
     else:
         return None
@@ -91,7 +93,7 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
     where = g.by(x, "Where", uses=2)
     if where is not None:
         mask, x, floor = where.inputs
-        if not (isinstance(floor, Lit) and floor.value == -np.inf and _lower_triangle(mask, jaxpr, consts, L, S)):
+        if tuple(x.aval.shape) != rows or not (isinstance(floor, Lit) and floor.value == -np.inf and _lower_triangle(mask, jaxpr, consts, L, S)):
             return None
         causal = True
     scale, reads = 1.0, 1 if causal else 2
@@ -101,7 +103,7 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
         x = next((i for i in scaled.inputs if not isinstance(i, Lit)), None)
         scale, reads = float(np.float16(lit.value)), 1
     dot = g.by(x, "Dot", uses=reads)
-    if dot is None:
+    if dot is None or tuple(x.aval.shape) != rows:
         return None
     q, k = dot.inputs
     if not isinstance(q, Var) or not isinstance(k, Var) or tuple(q.aval.shape) != (B, N, L, 1, H) or tuple(k.aval.shape) != (B, N, 1, S, H):

@@ -128,3 +128,24 @@ def test_a_schedule_keeps_the_program_that_its_key_was_made_from():
     del prog
     gc.collect()
     assert all(n() is not None for n in nodes)
+
+
+@pytest.mark.parametrize("total,top", [("row", "row"), ("column", "row"), ("row", "column"), ("column", "column")])
+@pytest.mark.parametrize("masked", [False, True], ids=["full", "causal"])
+def test_a_softmax_that_uses_a_row_s_sum_or_maximum_along_the_columns_stays_as_it_is(masked, total, top):
+    """With as many queries as keys the sums of the rows fit the columns as well: that is another function."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rewrite import fuse_attention
+    B, T, N, H = 2, 24, 3, 64
+    spread = {"row": [B, N, T, 1], "column": [B, N, 1, T]}
+
+    def f(q, k, v):
+        scores = L.einsum("BLNH,BSNH->BNLS", q, k).mul(0.125)
+        if masked:
+            scores = J.where(L.tri_const(T, T, 0), scores, -np.inf)
+        e = J.exp(scores.sub(J.stopGradient(scores.max(-1).reshape(spread[top]))))
+        return L.einsum("BNLS,BSNH->BLNH", e.div(e.sum(-1).reshape(spread[total])), v)
+    prog = J.jit(f, [ShapedArray((B, T, N, H), DType.Float16)] * 3)
+    assert (fuse_attention(prog.jaxpr, prog.consts) is not None) == (total == top == "row")
