@@ -149,14 +149,21 @@ class Schedule:
             prog = jitCompile(fused, prog.consts, backend.maxArgs)
         self.backend, self.prog = backend, prog
         self.units = plan_units(prog)
-        for u in self.units:
-            u.exe = backend.prepareSync(u.source)
         self._sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
         self._made = list(dict.fromkeys(o for o in prog.outputs if o >= prog.nargs))
         self._increfs = [s.output for s in prog.steps if s.kind == "incref"]
         self._work = place_intermediates(self.units, self._sizes, set(self._made))
         self._lock = threading.Lock()
-        self._bind()
+        pinned = []
+        try:  # a unit that is prepared here must not push out one that was prepared before it
+            for u in self.units:
+                u.exe = backend.prepareSync(u.source)
+                backend.pin(u.exe)
+                pinned.append(u.exe)
+            self._bind()
+        finally:
+            for exe in pinned:
+                backend.unpin(exe)
 
     def _bind(self) -> None:
         """The native launch list.  Buffer table: inputs, outputs made here, workspace."""
@@ -169,6 +176,8 @@ class Schedule:
         steps, refs = [], []
         for u in self.units:
             prep = u.exe.data
+            if prep.released:
+                raise ValueError("executable was released (evicted from the backend's cache): prepare it again")
             if isinstance(u.source, Kernel) and u.source.size == 0:
                 continue
             needs = dict(prep.ks.min_input_bytes)

@@ -149,3 +149,43 @@ def test_a_softmax_that_uses_a_row_s_sum_or_maximum_along_the_columns_stays_as_i
         return L.einsum("BNLS,BSNH->BLNH", e.div(e.sum(-1).reshape(spread[total])), v)
     prog = J.jit(f, [ShapedArray((B, T, N, H), DType.Float16)] * 3)
     assert (fuse_attention(prog.jaxpr, prog.consts) is not None) == (total == top == "row")
+
+
+@pytest.mark.parametrize("limit", [1, 2, 3])
+def test_a_schedule_of_more_executables_than_the_cache_holds_launches_all_of_them(limit):
+    """Nothing that a schedule is made of is evicted while the rest of it is prepared; afterwards it is, as anything else."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    be = _stand_in(limit)
+    avals = [ShapedArray(s, DType.Float32) for s in ((64, 128), (128, 256), (256, 512), (512, 64))]
+    prog = J.jit(lambda x, a, b, c: L.matmul(L.matmul(L.matmul(x, a), b), c), avals)
+    s = be.scheduleProgram(prog)
+    assert len(s.units) == 3 and s.live() and s._n_steps == sum(len(u.exe.data.ks.steps) for u in s.units) >= 3
+    assert not any(u.exe.data.pins or u.exe.data.released for u in s.units)
+    assert be.scheduleProgram(prog) is s
+    be.prepareKernelSync(J.jit(lambda x: L.matmul(x, x), [ShapedArray((96, 96), DType.Float32)]).kernels[0])
+    assert len(be._exes) <= limit and not s.live()
+    again = be.scheduleProgram(prog)
+    assert again is not s and again.live() and again._n_steps == s._n_steps
+    with pytest.raises(ValueError, match="released"):
+        s.run([0, 1, 2, 3])
+
+
+def test_a_schedule_that_cannot_be_prepared_leaves_nothing_pinned():
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    be = _stand_in()
+    prog = J.jit(lambda x, a, b: L.matmul(L.matmul(x, a), b), [ShapedArray(s, DType.Float32) for s in ((64, 128), (128, 256), (256, 64))])
+    build, calls = be._build, []
+
+    def second_fails(*a):
+        calls.append(a)
+        if len(calls) == 2:
+            raise RuntimeError("no memory")
+        return build(*a)
+    be._build = second_fails
+    with pytest.raises(RuntimeError, match="no memory"):
+        be.scheduleProgram(prog)
+    assert not be._programs and [e.data.pins for e in be._exes.values()] == [0]
