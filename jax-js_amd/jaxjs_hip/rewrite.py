@@ -101,7 +101,10 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
     if scaled is not None and any(isinstance(i, Lit) for i in scaled.inputs):
         lit = next(i for i in scaled.inputs if isinstance(i, Lit))
         x = next((i for i in scaled.inputs if not isinstance(i, Lit)), None)
-        scale, reads = float(np.float16(lit.value)), 1
+        with np.errstate(over="ignore"):
+            scale, reads = float(np.float16(lit.value)), 1
+        if not np.isfinite(scale):  # the routine's source holds it as a number
+            return None
     dot = g.by(x, "Dot", uses=reads)
     if dot is None or tuple(x.aval.shape) != rows:
         return None

@@ -189,3 +189,20 @@ def test_a_schedule_that_cannot_be_prepared_leaves_nothing_pinned():
     with pytest.raises(RuntimeError, match="no memory"):
         be.scheduleProgram(prog)
     assert not be._programs and [e.data.pins for e in be._exes.values()] == [0]
+
+
+@pytest.mark.parametrize("scale", [float("inf"), -float("inf"), float("nan"), 70000.0, 0.125, -2.0, 0.0])
+def test_attention_under_a_scale_that_is_not_a_finite_float16_stays_as_it_is(scale):
+    """The routine's source holds the scale as a number; the composition multiplies by whatever it is given."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rewrite import fuse_attention
+    from jaxjs_hip.routinegen import generateRoutine
+    from jaxjs_hip.runtime import compile_source
+    prog = J.jit(lambda q, k, v: L.dotProductAttention(q, k, v, scale=scale), [ShapedArray((1, 40, 2, 32), DType.Float16)] * 3)
+    fused = fuse_attention(prog.jaxpr, prog.consts)
+    assert (fused is not None) == (abs(scale) < 65520)
+    if fused is not None:
+        for source in generateRoutine(J.jitCompile(fused, prog.consts).routines[0], "fast").sources:
+            compile_source(source)
