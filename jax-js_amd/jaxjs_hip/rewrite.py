@@ -4,7 +4,8 @@
 around scale, mask and softmax, seven Kernels over a [B, N, L, S] score tensor) and puts the backend's Attention routine in
 its place, which keeps scores in registers and in float32 where the composition rounds them to float16 and moves them
 through memory seven times.  Only what the routine computes: float16, head size 32, 64 or 128, no mask or the lower
-triangle, and no part of the chain used by anything else.
+triangle, and no part of the chain used by anything else; and only where the routine is the faster one
+(`routine_is_faster`): it never splits the keys, which the composition spreads over the whole chip.
 """
 
 from __future__ import annotations
@@ -113,7 +114,37 @@ def _match(g: _Graph, values: JaxprEqn, jaxpr: Jaxpr, consts: List[ConstArray]) 
         return None
     if any(v.aval.dtype != DType.Float16 for v in (q, k, z)):
         return None
+    if not routine_is_faster(B, N, L, S, H, causal):
+        return None
     return dict(q=q, k=k, z=z, B=B, N=N, L=L, S=S, H=H, scale=scale, causal=causal)
+
+
+# Microseconds per key that a workgroup of the tile kernel walks, by head size (16384 keys: 162, 206 and 304 us).
+_TILE_US_PER_KEY = {32: 0.0100, 64: 0.0126, 128: 0.0188}
+
+
+def routine_is_faster(B: int, N: int, L: int, S: int, H: int, causal: bool) -> bool:
+    """Whether the Attention routine beats the composition.  From both sides measured at B N = 1 .. 768, L = 1 .. 4096 and
+    S = 128 .. 65536 in all head sizes: of 646 shapes the rule takes the slower side by more than a fifth at five (by 1.54
+    at most, at S = 5001), where the routine everywhere would lose that much at 158, and up to 21 times.
+
+    Up to ATTENTION_FEW_QUERIES queries, a workgroup each: it reads keys and values at 100 GB/s, so 4096 keys of 64 take it
+    12 us and 65536 take 162, when the composition's launches and all CUs' reading take 14 and 33.  With many workgroups
+    both are bound by reading the cache, which the composition reads once for all queries of a head: from 50 million
+    multiplications (in heads of 64) on it is ahead by up to a tenth (384 heads x 2 x 2048: 57.5 against 51.5 us, 192 x 2 x
+    2048, at the line: 31.8 against 30.2, 96 x 2 x 2048: 16.9 against 21.4).
+
+    More queries: workgroups of 128 rows, one to a CU at first, that walk all keys they see (half of them on average under
+    the mask).  The composition costs 10 us of launches and moves the scores several times: 1.8 us per million of them, and
+    3.2 where its products' tiles of 64 rows are partly empty.  (12 x 64 x 2048 x 64: 27.6 against 16.3 us; 12 x 512 x 2048:
+    28.4 against 36; 96 x 128 x 4096: 54 against 106; 1 x 4096 x 4096, causal: 62 against 48.)"""
+    from .routinegen import ATTENTION_FEW_QUERIES
+    if L <= ATTENTION_FEW_QUERIES:
+        return S * H <= 4096 * 64 and B * N * L * S * max(H, 64) <= 3 << 24
+    tiles = B * N * -(-L // 128)
+    walked = min(S, L) if causal else S
+    routine = 2 + _TILE_US_PER_KEY[H] * walked * max(1.0, tiles * (0.6 if causal else 1.0) / 256)
+    return routine <= 10 + (3.2 if L <= 64 else 1.8) * B * N * max(L, 64) * S / 1e6
 
 
 def fuse_attention(jaxpr: Jaxpr, consts: List[ConstArray]) -> Optional[Jaxpr]:

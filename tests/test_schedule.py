@@ -206,3 +206,31 @@ def test_attention_under_a_scale_that_is_not_a_finite_float16_stays_as_it_is(sca
     if fused is not None:
         for source in generateRoutine(J.jitCompile(fused, prog.consts).routines[0], "fast").sources:
             compile_source(source)
+
+
+@pytest.mark.parametrize("heads,queries,keys,size,causal,routine", [
+    # decode: microseconds of the routine and of the composition at these shapes
+    (96, 1, 1025, 64, False, True),     # 6 and 14
+    (12, 4, 4096, 64, False, True),     # 12 and 17
+    (12, 1, 16384, 64, False, False),   # 52 and 20
+    (1, 4, 65536, 64, False, False),    # 162 and 36
+    (12, 1, 16384, 128, False, False),  # 99 and 27
+    (384, 2, 2048, 64, False, False),   # 57 and 51
+    # prefill
+    (12, 5, 512, 64, False, True),      # 8 and 12
+    (12, 5, 4096, 64, False, False),    # 52 and 17
+    (12, 128, 16384, 64, False, False),  # 204 and 55
+    (96, 128, 4096, 64, False, True),   # 54 and 106
+    (96, 16, 4096, 128, False, True),   # 79 and 179
+    (96, 1024, 1024, 64, True, True),   # 27 and 203
+    (1, 128, 16384, 64, True, True),    # 6 and 22: the mask hides all but 128 keys
+    (1, 1024, 1024, 64, True, False),   # 18 and 11
+], ids=str)
+def test_attention_runs_as_the_routine_where_that_is_the_faster_one(heads, queries, keys, size, causal, routine):
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rewrite import fuse_attention
+    shapes = [(1, t, heads, size) for t in (queries, keys, keys)]
+    prog = J.jit(lambda q, k, v: L.dotProductAttention(q, k, v, isCausal=causal), [ShapedArray(s, DType.Float16) for s in shapes])
+    assert (fuse_attention(prog.jaxpr, prog.consts) is not None) == routine
