@@ -130,7 +130,12 @@ class HipBackend:
     operation for operation (f32 maps within 2 ulp of the parity oracle); the default `"fast"` is the same except that
     `exp` and `reciprocal` run on the hardware's exp2 / rcp instructions (within rel 1e-5 of the oracle, the bar for f32
     maps), which is what keeps fused softmax-style rows bound by HBM instead of the VALU; `"native"` uses the device
-    libm."""
+    libm.
+
+    The modes are about Kernels.  A float16 attention that a jit program composes and that the schedule recognises
+    (`rewrite.fuse_attention`) runs as the Attention routine in every mode: hardware exp2, and scores in float32 that the
+    composition would round to float16 three times.  For the composition operation for operation, return the scores or
+    the probabilities from the program as well, or dispatch its steps one by one (`JitProgram.steps`)."""
 
     type = "hip"
     _releases = 0  # executables released so far: holders of prepared executables look again when it changes
