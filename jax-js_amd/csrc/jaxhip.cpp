@@ -262,7 +262,7 @@ int jh_compile(const char *source, const char *name, const char *const *options,
   if (r != HIPRTC_SUCCESS) return fail((int)r, "hiprtcCreateProgram: %s", hiprtcGetErrorString(r));
   // Options the source asks for itself: leading lines of the form "// hiprtc-option: <option>", honoured for the
   // options on a fixed list (the generator marks float16 kernels that the SLP vectorizer makes the compiler abort on, and
-  // sorts whose only floating-point values are finite ones made from integer keys).
+  // sorts whose only floating-point values are finite ones made from integer keys: elements are integers there).
   std::vector<std::string> asked;
   {
     static const char kMark[] = "// hiprtc-option: ";

@@ -22,8 +22,8 @@ from .errors import UnsupportedRoutineError
 from .routine import Routine, Routines, ScatterOp
 from .shape import prod
 
-_SORT_KINDS = {DType.Float32: (0, "float"), DType.Float16: (1, "jh_f16"), DType.Int32: (2, "int"),
-               DType.Uint32: (3, "jh_u32"), DType.Bool: (2, "int"), DType.Float64: (4, "double")}
+_SORT_KINDS = {DType.Float32: (0, "jh_u32"), DType.Float16: (1, "jh_u16"), DType.Int32: (2, "int"),
+               DType.Uint32: (3, "jh_u32"), DType.Bool: (2, "int"), DType.Float64: (4, "unsigned long long")}
 SORT_TILE = 8192  # LDS tile in 8-byte words (64 KB): 16384 4-byte words, 4096 16-byte words
 SORT_REGISTERS = 256  # bytes of words a lane holds in the register network
 SORT_WAVES = 2048     # waves (two per SIMD) from which 16 lanes per row are enough; with fewer, a row takes up to 64
