@@ -35,7 +35,8 @@ SORT_FEW, SORT_FEW_WAVES = 16, 256
 SORT_SMALL_TILE, SORT_FEW_TILES = 4096, 64
 SORT_LOCAL, SORT_TILES = 16, 1024  # words of a lane in a tile's register runs, from 1024 tiles on
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
-CHOLESKY_PANEL_FROM = 192  # matrix order from which one panel's launch spans many CUs (smaller ones: a few workgroups)
+CHOLESKY_PANEL_FROM = 192  # matrix order from which many matrices may take two launches a panel, and a plan counts its panels
+CHOLESKY_WAVE_BELOW = {2: 44, 4: 28, 8: 28}  # matrix order, by bytes per element, below which many matrices take a wave each
 
 
 def _next_pow2(n: int) -> int:
@@ -63,7 +64,7 @@ def _round64(n: int, cap: int = 1024) -> int:
     return max(64, min(cap, (n + 63) // 64 * 64))
 
 
-_LINALG_DEFAULTS = dict(ROUTINE=0, N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1,
+_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1,
                         ELEM="float", CMP="float")
 # Element types of the dense routines: C type, the type magnitudes are compared in, bytes per element.
 _FLOAT_ELEMS = {DType.Float32: ("float", "float", 4), DType.Float64: ("double", "double", 8), DType.Float16: ("jh_f16", "float", 2)}
@@ -77,6 +78,28 @@ def _float_elem(t):
     """(C type, comparison type, bytes) when every operand has one and the same floating-point type, else None."""
     d = t.inputDtypes[0]
     return _FLOAT_ELEMS.get(d) if all(x == d for x in t.inputDtypes) else None
+
+
+def _cholesky_plan(n: int, batch: int, eb: int) -> str:
+    """Which of the four plans factors `batch` matrices of order n; they give the same bits (float32, microseconds).
+
+    A launch per panel has the shortest chain, and a workgroup of 256 per 32 rows with 50 KB of LDS (68 in float64): three
+    (two) of them on a CU.  A wave per matrix holds 32 on a CU and is as fast alone up to order 8 (7.0 and 7.0); from there
+    its chain is longer and it takes batches to win (16: 256 matrices 14 against 7.7, 1536 20 and 18, 4096 24 and 42,
+    65536 282 and 623; 24: 4096 47 and 56), which it never does from order 28 on (28: 16384 266 against 249; in float16,
+    whose panels pay for conversions, to 40: 16384 473 against 634, 48: 768 against 725).
+    Two launches per panel do less work on a longer chain, and win where the panels' workgroups come 16 to a CU, 8 in
+    float64 (256: 512 matrices 662 against 635, 1024 1065 and 1189; 512: 128 1174 and 1000, 256 1739 and 1807)."""
+    from . import tuner
+    cus = tuner.CU_COUNT
+    many = 2 if eb == 8 and n <= 12 else min(n // 4, 6)  # matrices per CU
+    if n <= 8 or n < CHOLESKY_WAVE_BELOW[eb] and batch > cus * many:
+        return "wave per matrix"
+    if n > 64 and batch * n * n * 8 > CHOLESKY_RIGHT_LOOKING_MAX_BYTES:
+        return "left-looking"
+    if n >= CHOLESKY_PANEL_FROM and batch * (n // 32) >= cus * (8 if eb == 8 else 16):
+        return "two launches"
+    return "right-looking"
 
 
 def _gen_cholesky(routine: Routine, numerics: str) -> Optional[KernelSource]:
@@ -94,32 +117,47 @@ def _gen_cholesky(routine: Routine, numerics: str) -> Optional[KernelSource]:
     batch = prod(shape[:-2])
     if batch == 0 or n == 0:
         return _empty("cholesky", n=n, batch=batch)
-    if n <= 64 or batch * n * n * 8 <= CHOLESKY_RIGHT_LOOKING_MAX_BYTES:  # (two panels need no copy)
-        # Right-looking: the running sums of the whole triangle in a double-precision scratch copy, one launch per
+    plan = _cholesky_plan(n, batch, eb)
+    grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
+    need, panels = {0: batch * n * n * eb}, range(0, n, 32)
+    if plan == "wave per matrix":
+        src = _linalg_source(numerics, ROUTINE=8, N=n, ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_cholesky", (batch, 1, 1), (64, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0)])]
+        return KernelSource([src], steps, [batch * n * n * eb], "cholesky", need, dict(n=n, batch=batch, threads=64))
+    if plan == "right-looking":
+        # The running sums of the whole triangle in a double-precision scratch copy (two panels need none), one launch per
         # 32-column panel that finishes the panel and subtracts the one before it from the rest.
         src = _linalg_source(numerics, ROUTINE=5, N=n, ELEM=ctype, CMP=cmp_t)
         steps = []
-        for j0 in range(0, n, 32):
+        for j0 in panels:
             after = max(0, n - j0 - 32)
             T = (after + 63) // 64
             blocks = max(1, (after + 31) // 32) + (T * (T + 1) // 2 if j0 else 0)
             steps.append(LaunchStep("jh_chol_step", (batch * blocks, 1, 1), (256, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
-        info = dict(n=n, batch=batch, launches=len(steps), variant="right-looking")
-        if n >= CHOLESKY_PANEL_FROM:
-            info["panels"] = len(steps)
-        return KernelSource([src], steps, [batch * n * n * 8 if n > 64 else 8], "cholesky", {0: batch * n * n * eb}, info)
-    # Left-looking where that copy would be too large: 32-column panels, two launches each; the same sums in the same order.
-    src = _linalg_source(numerics, ROUTINE=4, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
-    grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
-    steps = [LaunchStep("jh_chol_zero", grid1(batch * n * n), (256, 1, 1), 0, [("out", 0)])]
-    for j0 in range(0, n, 32):
-        steps.append(LaunchStep("jh_chol_bulk", (batch * ((n - j0 + 63) // 64), 1, 1), (256, 1, 1), 0,
-                                [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
-        after = max(0, n - j0 - 32)
-        steps.append(LaunchStep("jh_chol_panel", (batch * max(1, (after + 63) // 64), 1, 1), (64, 1, 1), 0,
-                                [("scratch", 0), ("out", 0), ("const", j0)]))
-    return KernelSource([src], steps, [batch * n * 32 * 8], "cholesky", {0: batch * n * n * eb},
-                        dict(n=n, batch=batch, panels=(n + 31) // 32, launches=len(steps)))
+        scratch, info = [batch * n * n * 8 if n > 64 else 8], dict(variant=plan)
+    elif plan == "two launches":
+        src = _linalg_source(numerics, ROUTINE=9, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_chol_init", grid1(batch * n * n), (256, 1, 1), 0, [("in", 0), ("out", 0), ("scratch", 0)])]
+        for j0 in panels:
+            after = max(0, n - j0 - 32)
+            T = (after + 63) // 64
+            steps.append(LaunchStep("jh_chol_panel", (batch * max(1, T), 1, 1), (64, 1, 1), 0, [("scratch", 0), ("out", 0), ("const", j0)]))
+            if after:
+                steps.append(LaunchStep("jh_chol_update", (batch * T * T, 1, 1), (256, 1, 1), 0, [("out", 0), ("scratch", 0), ("const", j0)]))
+        scratch, info = [batch * n * n * 8], dict(variant=plan)
+    else:  # left-looking: 32-column panels, two launches each; the same sums in the same order
+        src = _linalg_source(numerics, ROUTINE=4, N=n, M=batch, ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_chol_zero", grid1(batch * n * n), (256, 1, 1), 0, [("out", 0)])]
+        for j0 in panels:
+            steps.append(LaunchStep("jh_chol_bulk", (batch * ((n - j0 + 63) // 64), 1, 1), (256, 1, 1), 0,
+                                    [("in", 0), ("out", 0), ("scratch", 0), ("const", j0)]))
+            after = max(0, n - j0 - 32)
+            steps.append(LaunchStep("jh_chol_panel", (batch * max(1, (after + 63) // 64), 1, 1), (64, 1, 1), 0,
+                                    [("scratch", 0), ("out", 0), ("const", j0)]))
+        scratch, info = [batch * n * 32 * 8], {}
+    if n >= CHOLESKY_PANEL_FROM:
+        info["panels"] = len(panels)
+    return KernelSource([src], steps, scratch, "cholesky", need, dict(n=n, batch=batch, launches=len(steps), **info))
 
 
 def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:

@@ -1,4 +1,6 @@
 """Plan generation on the host (no GPU): properties every kernel plan must have."""
+import pytest
+
 from jaxjs_hip import DType
 from jaxjs_hip.kernelgen import generate
 
@@ -218,3 +220,28 @@ def test_wide_load_of_a_looked_up_row_reads_what_the_guarded_element_loads_read(
     prog = J.jit(lambda t, i: Lb.take(t, i, 0), [ShapedArray((1000, 768), DType.Float16), ShapedArray((64,), DType.Int32)])
     from jaxjs_hip.tuner import tuneHip
     assert "vector_gm" in tuneHip(prog.kernels[0]).vector_loads.values()
+
+
+@pytest.mark.parametrize("order,batch,dtype,plan", [
+    # microseconds of a wave per matrix against a launch per panel
+    (8, 1, DType.Float32, "wave per matrix"), (8, 65536, DType.Float64, "wave per matrix"),              # 7 and 7; 36 and 143 (16384)
+    (12, 768, DType.Float32, "right-looking"), (12, 1024, DType.Float32, "wave per matrix"),             # 12 and 9; 12 and 15
+    (12, 512, DType.Float64, "right-looking"), (12, 768, DType.Float64, "wave per matrix"),              # 9 and 9; 9 and 16
+    (24, 1024, DType.Float32, "right-looking"), (24, 4096, DType.Float32, "wave per matrix"),            # 27 and 19; 47 and 56
+    (28, 16384, DType.Float32, "right-looking"), (28, 4096, DType.Float16, "wave per matrix"),           # 266 and 249; 65 and 99
+    (40, 4096, DType.Float16, "wave per matrix"), (48, 16384, DType.Float16, "right-looking"),           # 128 and 168; 768 and 725
+    (191, 1024, DType.Float32, "right-looking"),
+    # of two launches per panel against one
+    (192, 512, DType.Float32, "right-looking"), (192, 1024, DType.Float32, "two launches"),              # 379 and 327; 576 and 604
+    (512, 128, DType.Float32, "right-looking"), (512, 512, DType.Float32, "two launches"),               # 1174 and 1000; 3000 and 3501
+    (512, 128, DType.Float64, "two launches"), (1024, 32, DType.Float64, "right-looking"),               # 1188 and 1235; 2135 and 1896
+    (1024, 1, DType.Float32, "right-looking"), (1024, 256, DType.Float32, "left-looking"),               # (2 GiB of running sums)
+], ids=str)
+def test_cholesky_s_plan_follows_the_number_of_matrices(order, batch, dtype, plan):
+    from jaxjs_hip.alu import byteWidth
+    from jaxjs_hip.routine import Routine, Routines, RoutineType
+    from jaxjs_hip.routinegen import _cholesky_plan, generateRoutine
+    assert _cholesky_plan(order, batch, byteWidth(dtype)) == plan
+    shape = [batch, order, order]
+    first = generateRoutine(Routine(Routines.Cholesky, RoutineType([shape], [dtype], [shape], [dtype]))).steps[0].name
+    assert first == {"wave per matrix": "jh_cholesky", "right-looking": "jh_chol_step", "two launches": "jh_chol_init", "left-looking": "jh_chol_zero"}[plan]
