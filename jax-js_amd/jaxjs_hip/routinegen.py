@@ -233,6 +233,23 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, [], "lu", {0: batch * m * n * eb}, dict(m=m, n=n, batch=batch, threads=threads))
 
 
+def _jacobi_blocks_pay(n: int, batch: int, eb: int) -> bool:
+    """Whether JacobiEigh by blocks is faster than one rotation after the other for this many matrices (same bits).
+
+    By blocks, a matrix takes a CU for itself, so time goes with rounds of 256 matrices; one after the other, as many
+    share a CU as its LDS holds two copies of, at no cost to each other up to about one wave per SIMD.  One round is
+    faster by n / 16 (float32 order 16: 1.2 times, 32: 2.3, 48: 2.9, 64: 4.2), in float16, whose every value is
+    converted, by n / 28; past that many rounds the others have caught up, unless they wait for each other too (float32, ms:
+    16 x 512 0.42 against 0.63 by blocks, 32 x 512 2.41 and 1.93, 32 x 1024 2.2 and 3.4, 48 x 1024 5.4 and 6.8, 64 x 1024
+    14.2 and 9.9, 13 x 16384 1.8 and 16.2)."""
+    from . import tuner
+    rounds = -(-batch // tuner.CU_COUNT)
+    held = 150 * 1024 // (2 * n * n * eb)  # matrices on a CU when one rotation follows the other
+    if held == 0:  # too large for LDS: ten times slower alone, and more so together
+        return True
+    return rounds <= max(1.0, n / (28 if eb == 2 else 16)) * -(-rounds // held)
+
+
 def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     t = routine.type
     shape = list(t.inputShapes[0])
@@ -253,9 +270,10 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     params = routine.params or {}
     threads = _round64(n)
     in_lds = 1 if 2 * n * n * eb <= 150 * 1024 else 0  # both matrices in the CU's 160 KB of LDS: n <= 138 in float32
+    by_blocks = JACOBI_BLOCKS_FROM[eb] <= n <= 192 and _jacobi_blocks_pay(n, batch, eb)
     for size in (4, 8):  # indices per block; the triangle and the rotations under way have to fit the LDS
         blocks = -(-n // size)
-        if JACOBI_BLOCKS_FROM <= n <= 192 and eb * (n * (n + 1) // 2) + 16 * (blocks + 1) * n + 32 * blocks + 512 <= 160 * 1024:
+        if by_blocks and eb * (n * (n + 1) // 2) + 16 * (blocks + 1) * n + 32 * blocks + 512 <= 160 * 1024:
             src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=512, RB=size, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
             steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (512, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("scratch", 0)])]
             return KernelSource([src], steps, [batch * n * n * eb], "jacobi", {0: batch * n * n * eb},
@@ -266,7 +284,9 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=threads, in_lds=bool(in_lds)))
 
 
-JACOBI_BLOCKS_FROM = 13       # the step of a block costs more than the few rotations of a smaller matrix (12: 183 against 178 us, 16: 272 against 324)
+# The step of a block costs more than the few rotations of a smaller matrix (float32 12: 183 against 178 us, 13: 257 and 249,
+# 16: 272 and 324; float16 13: 437 and 402, 16: 525 and 622).
+JACOBI_BLOCKS_FROM = {2: 16, 4: 13, 8: 13}
 ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which every query is a workgroup of its own and not a row of a 128-row tile
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS

@@ -245,3 +245,22 @@ def test_cholesky_s_plan_follows_the_number_of_matrices(order, batch, dtype, pla
     shape = [batch, order, order]
     first = generateRoutine(Routine(Routines.Cholesky, RoutineType([shape], [dtype], [shape], [dtype]))).steps[0].name
     assert first == {"wave per matrix": "jh_cholesky", "right-looking": "jh_chol_step", "two launches": "jh_chol_init", "left-looking": "jh_chol_zero"}[plan]
+
+
+@pytest.mark.parametrize("order,batch,dtype,blocks", [
+    # milliseconds by blocks against one rotation after the other
+    (16, 256, DType.Float32, True), (16, 257, DType.Float32, False),      # 0.32 and 0.39; 0.64 and 0.42 (300)
+    (32, 512, DType.Float32, True), (32, 513, DType.Float32, False),      # 1.93 and 2.41; 2.54 and 2.18 (768)
+    (48, 768, DType.Float32, True), (48, 1024, DType.Float32, False),     # 4.5 and 4.7; 6.8 and 5.4
+    (64, 2048, DType.Float32, True), (128, 4096, DType.Float32, True),    # 19.7 and 27.9: those wait for each other too
+    (64, 2048, DType.Float64, True), (48, 1024, DType.Float64, False),    # 18.4 and 45.8; 5.7 and 5.3
+    (48, 512, DType.Float16, False), (64, 512, DType.Float16, True),      # 7.2 and 7.2; 11.9 and 15.0
+    (64, 1024, DType.Float16, False), (160, 4096, DType.Float32, True),   # 23.7 and 15.6; (too large for LDS)
+    (13, 2, DType.Float32, True), (13, 2, DType.Float16, False), (12, 1, DType.Float32, False),
+], ids=str)
+def test_jacobi_eigh_s_plan_follows_the_number_of_matrices(order, batch, dtype, blocks):
+    from jaxjs_hip.routine import Routine, Routines, RoutineType
+    from jaxjs_hip.routinegen import generateRoutine
+    shape = [batch, order, order]
+    ks = generateRoutine(Routine(Routines.JacobiEigh, RoutineType([shape], [dtype], [shape] * 2, [dtype] * 2), dict(maxSweeps=30, tolerance=1e-7)))
+    assert ks.steps[0].name == ("jh_jacobi_blocks" if blocks else "jh_jacobi") and ("block" in ks.info) == blocks

@@ -420,3 +420,13 @@ def test_cholesky_of_many_small_matrices(n, batch):
     got, want, ks = both(R.cholesky(x), [x])
     assert [s.name for s in ks.steps] == ["jh_cholesky"]
     assert_bits(got, want, f"cholesky {batch} x {n}")
+
+
+@pytest.mark.parametrize("n,batch", [(13, 256), (13, 257), (20, 300)])
+def test_jacobi_eigh_of_many_small_matrices(n, batch):
+    """Either side of the line between a matrix per CU, by blocks, and several that rotate one pair after the other."""
+    a = RNG.standard_normal((batch, n, n))
+    sym = (a + np.swapaxes(a, -1, -2)).astype(F32)
+    got, want, ks = both(R.jacobi_eigh(sym), [sym])
+    assert ("block" in ks.info) == (batch <= 256)
+    assert_bits(got, want, f"jacobi_eigh {batch} x {n}")
