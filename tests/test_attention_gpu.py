@@ -219,3 +219,16 @@ def test_a_chain_whose_scores_are_used_elsewhere_stays_as_it_is():
         return [L_.einsum("BNLS,BSNH->BLNH", p, v), p]
     prog = J.jit(f, [ShapedArray((1, 8, 2, 32), F16)] * 3)
     assert fuse_attention(prog.jaxpr, prog.consts) is None
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 77, 2, 64), (2, 3, 1025, 1, 32), (1, 40, 77, 2, 128), (1, 130, 65, 1, 64)], ids=str)
+def test_an_infinite_value_of_the_last_key_stays_one(shape):
+    """Keys past the last one are read from its row: their weight is zero, and zero times infinity is not."""
+    B, L, S, N, H = shape
+    rng = np.random.default_rng(L)
+    q, k, v = (rng.standard_normal((B, T, N, H)).astype(np.float16) for T in (L, S, S))
+    v[:, -1, :, 5], v[:, -1, :, 6] = np.inf, -np.inf
+    y = R.run_gpu(attention_routine(B, L, S, N, False, H=H), [q, k, v])[0][0]
+    assert (y[..., 5] == np.inf).all() and (y[..., 6] == -np.inf).all()
+    rest = [i for i in range(H) if i not in (5, 6)]
+    assert np.isfinite(y[..., rest]).all()
