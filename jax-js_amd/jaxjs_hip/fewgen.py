@@ -4,16 +4,14 @@ from __future__ import annotations
 
 from typing import Optional
 
+from . import tuner
 from .alu import DType
 from .kernelgen import fill, template
-from .tuner import CU_COUNT
 
 FEW_LDS = 128 * 1024  # float32 sums of all waves
-# Tile plans with at least this many workgroups stand, unless the operand along k has at most FEW_ROWS rows; with a float32
-# k axis of under 256 twice as many, with float16 off the 16-byte grid one for every CU, and any the direct-to-LDS path takes.
-FEW_WORKGROUPS = 64
-FEW_ROWS = 64
-FEW_DEEP = 4096       # longest k axis: each wave of a tile would walk too many steps
+FEW_ROWS = 64         # short operands up to this many rows are what the kernel is made for
+FEW_DEEP = 4096       # longest k axis for more rows, or across 16-byte lines: each wave of a tile would walk too many steps
+FEW_WORKGROUPS = 64   # tile plans with as many workgroups stand against more rows (see `_tiles_stand`)
 
 
 def _loads(g: dict, tag: str, along_k: bool) -> float:
@@ -24,18 +22,9 @@ def _loads(g: dict, tag: str, along_k: bool) -> float:
     return 3.0 if along_k else 1.5
 
 
-def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
-    """Workgroup shape for `g` (see tuner.match_gemm) if one operand runs along k, the other along either axis, and this
-    kernel is expected to beat the LDS tiles, else None.  `tiles_of()` gives the tile plan to compare with.
-
-    The estimates are fits to measurements (us, at 2.4 GHz).  Here: 2.6 for the launch; per step of a workgroup 28 cycles
-    for each 16-row piece of an operand and the matrix instructions of four SIMDs; 16 cycles per wave and 16 x 16 tile for the
-    sums; and W again from beyond the L2 for every row tile when it is more than 4 MB.  Tiles: 2.5 for the launch, 2 for
-    folding a k split, and a time per element of k: float32 0.026 for a 64 x 64 tile; float16 0.0045 on the direct-to-LDS
-    path, else 0.008 along k, 0.012 across and 0.025 across rows off the 16-byte grid.  They leave (before -> here):
-    float32 64 x 256 x 784 22.3 -> 4.0, 128 x 1000 x 1000 28.1 -> 7.0, 300 x 300 x 300 10.1 -> 3.4; float16 64 x 256 x 784
-    12.0 -> 2.9, 200 x 300 x 300 12.5 -> 2.6, 64 x 1024 x 1024 8.0 -> 3.3, 12 x 805 x 1906 47 -> 6.0, 3 x 9287 x 5632
-    46.5 -> 33; but 64 x 2048 x 4096 (10.2 against 11.9) and 16 x 14336 x 4096 (25.8 against 32) stay with the tiles."""
+def _operands(g: dict) -> Optional[dict]:
+    """The short operand, which has to run along k, the wide one, along k or along its rows, and their extents; None where
+    the kernel does not apply."""
     if g["dtype"] not in (DType.Float16, DType.Float32) or g.get("a_gather") or g.get("b_gather") or g["a_k0"] != g["K"] or g["b_k0"] != g["K"] or g["K"] < 32:
         return None
     nb = 1
@@ -43,8 +32,6 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
         nb *= b[0]
     if nb > 65535:
         return None
-    f32 = g["dtype"] == DType.Float32
-    eb = 4 if f32 else 2
     row, rows = {"a": "a_sm", "b": "b_sn"}, {"a": g["M"], "b": g["N"]}
     short = "a" if g["M"] <= g["N"] else "b"
     if g[short + "_sk"] != 1:
@@ -55,13 +42,23 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
     along_k = g[wide + "_sk"] == 1
     if not along_k and not (g[row[wide]] == 1 and g[wide + "_sk"] > 0):
         return None
+    loose = bool(g.get("a_loose") or g.get("b_loose"))
     R, C, K = rows[short], rows[wide], g["K"]
-    if R > FEW_ROWS and K > FEW_DEEP or along_k and K > FEW_DEEP and (g.get("a_loose") or g.get("b_loose")):
+    if K > FEW_DEEP and (R > FEW_ROWS or along_k and loose):
         return None
-    step = 64 // eb
-    steps = -(-K // step)
-    wx, ww = _loads(g, short, True), _loads(g, wide, along_k)
-    w_bytes = C * K * eb * nb
+    eb = 4 if g["dtype"] == DType.Float32 else 2
+    return dict(R=R, C=C, K=K, short=short, wide=wide, along_k=along_k, loose=loose, nbatch=nb, row=row, eb=eb, w_bytes=C * K * eb * nb)
+
+
+def _shape(g: dict, o: dict) -> Optional[dict]:
+    """The workgroup's tile (MT 16-row and VN 16-column pieces), its waves, and the launch's estimated microseconds: 2.6
+    to start; per step of a workgroup 28 cycles for each 16-row piece of an operand and the matrix instructions of four
+    SIMDs; 16 cycles per wave and 16 x 16 tile for the sums; and the wide operand again from beyond the L2 for every row
+    tile when it is more than 4 MB."""
+    f32, along_k, R, C = o["eb"] == 4, o["along_k"], o["R"], o["C"]
+    step = 64 // o["eb"]
+    steps = -(-o["K"] // step)
+    wx, ww = _loads(g, o["short"], True), _loads(g, o["wide"], along_k)
     best = None
     for MT in (1, 2, 4):
         if MT > 1 and 8 * MT >= R:
@@ -69,41 +66,77 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
         for VN in ((1, 2, 4) if f32 or along_k else (2, 4, 8)):
             if MT * VN > 16 or (not along_k and C < VN) or (VN > 1 and 8 * VN >= C and VN != 2):
                 continue
-            waves = max(1, min(16, K // step or 1, FEW_LDS // (MT * 16 * (16 * VN + 1) * 4)))
+            waves = max(1, min(16, o["K"] // step or 1, FEW_LDS // (MT * 16 * (16 * VN + 1) * 4)))
             row_tiles = -(-R // (16 * MT))
-            count = row_tiles * -(-C // (16 * VN)) * nb
+            count = row_tiles * -(-C // (16 * VN)) * o["nbatch"]
             cycles = steps * (28 * (MT * wx + VN * ww) + MT * VN * (32 if f32 else 4)) + waves * MT * VN * 16
-            us = 2.6 + max(1.0, count / CU_COUNT) * cycles / 2400 + (row_tiles * w_bytes / 10e6 if w_bytes > 4 << 20 else 0.0)
-            if row_tiles <= 65535 and (best is None or us < best[0]):
-                best = (us, MT, VN, waves)
+            work = max(1.0, count / tuner.CU_COUNT) * cycles / 2400
+            again = row_tiles * o["w_bytes"] / 10e6 if o["w_bytes"] > 4 << 20 else 0.0
+            if row_tiles <= 65535 and (best is None or 2.6 + work + again < best["us"]):
+                best = dict(us=2.6 + work + again, work=work, MT=MT, VN=VN, waves=waves)
+    return best
+
+
+def _tile_launch(g: dict, o: dict, tile: dict) -> dict:
+    """The tile plan's workgroups, whether it is on the direct-to-LDS path, and its estimated microseconds: 2.5 to start
+    (2.8 where whole 16-byte groups are staged through registers), 2 for folding a k split, and a time
+    per element of k that depends on the loader."""
+    BM, BN, split = tile["BM"], tile["BN"], tile.get("SPLITK", 1)
+    count = -(-g["M"] // BM) * -(-g["N"] // BN) * o["nbatch"] * split
+    direct = o["eb"] == 2 and BM >= 128 and BN >= 128 and o["K"] % 32 == 0 and not o["loose"]
+    start = 2.5 if direct or o["loose"] else 2.8
+    if o["eb"] == 4:
+        per_k = (0.026 if o["loose"] else 0.024) * BM * BN / 4096
+    elif direct:
+        per_k = 0.0045 * BM * BN / 16384
+    elif o["along_k"]:
+        per_k = 0.008 if o["loose"] else 0.0066
+    else:
+        per_k = 0.025 if g.get(o["wide"] + "_loose") else 0.012
+    us = start + (2.0 if split > 1 else 0.0) + max(1.0, count / tuner.CU_COUNT) * o["K"] / split * per_k
+    return dict(count=count, direct=direct, us=us)
+
+
+def _tiles_stand(o: dict, t: dict) -> bool:
+    """Tile plans that no estimate is asked about: with enough workgroups to hide their loads behind each other, against
+    more rows than a few (64; twice as many for float32 with a k axis of under 256, one per CU for float16 off the
+    16-byte grid, any on the direct-to-LDS path), or against weights that stream from memory anyway."""
+    if o["eb"] == 4:
+        many = 2 * FEW_WORKGROUPS if o["loose"] or o["K"] < 256 else FEW_WORKGROUPS
+    else:
+        many = 0 if t["direct"] else tuner.CU_COUNT if o["loose"] else FEW_WORKGROUPS
+    return t["count"] >= many and o["R"] > FEW_ROWS or t["count"] >= FEW_WORKGROUPS and o["w_bytes"] > 96 << 20 and not o["loose"]
+
+
+def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
+    """Workgroup shape for `g` (see tuner.match_gemm) if one operand runs along k, the other along either axis, and this
+    kernel is expected to beat the LDS tiles, else None.  `tiles_of()` gives the tile plan to compare with.
+
+    The choice is between two estimates that are fits to both sides measured at 1072 shapes (rows and columns up to 16384,
+    k up to 8192).  Of the 809 that take this kernel it is the slower side by more than a fifth at eleven, mostly wide
+    outputs of a short or ragged k axis (float16 3392 x 256 x 63: 10.1 us against 5.7, 106 x 8500 x 56: 8.6 and 5.9); the
+    estimate is raised by a third for more than 16 rows of whole 16-byte groups, where it was low and the tiles' was not.
+    microseconds, tiles -> here: float32 64 x 256 x 784 22.3 -> 4.0, 128 x 1000 x 1000 28.1 -> 7.0, 300 x 300 x 300
+    10.1 -> 3.4; float16 64 x 256 x 784 12.0 -> 2.9, 200 x 300 x 300 12.5 -> 2.6, 64 x 1024 x 1024 8.0 -> 3.3, 12 x 805 x
+    1906 47 -> 6.0, 3 x 9287 x 5632 46.5 -> 33.  With the tiles stay float16 64 x 2048 x 4096 (10.2 against 11.9),
+    16 x 14336 x 4096 (25.8 against 32), 64 x 10112 x 4416 of weights along k (30 against 53), 64 x 2304 x 5248 (20 against
+    29) and float32 45 x 2133 x 3712 (27 against 35), 61 x 10492 x 1444 (38 against 58)."""
+    o = _operands(g)
+    best = _shape(g, o) if o is not None else None
     if best is None:
         return None
-    us, MT, VN, waves = best
     if tiles_of is not None:
-        tile = tiles_of()
-        BM, BN, split = tile["BM"], tile["BN"], tile.get("SPLITK", 1)
-        count = -(-g["M"] // BM) * -(-g["N"] // BN) * nb * split
-        loose = g.get("a_loose") or g.get("b_loose")
-        direct = not f32 and BM >= 128 and BN >= 128 and K % 32 == 0 and not loose
-        many = 0 if direct else FEW_WORKGROUPS if not loose and not (f32 and K < 256) else FEW_WORKGROUPS * 2 if f32 else CU_COUNT
-        if count >= many and R > FEW_ROWS or count >= FEW_WORKGROUPS and w_bytes > 96 << 20 and not loose:
-            return None
-        if f32:
-            per_k = 0.026 * BM * BN / 4096
-        elif direct:
-            per_k = 0.0045 * BM * BN / 16384
-        else:
-            per_k = 0.008 if along_k else 0.012 if not g.get(wide + "_loose") else 0.025
-        tiles_us = 2.5 + (2.0 if split > 1 else 0.0) + max(1.0, count / CU_COUNT) * K / split * per_k
-        stream = w_bytes / 4.5e6
-        if max(us, stream) >= 0.95 * max(tiles_us, stream):
+        t = _tile_launch(g, o, tiles_of())
+        us = best["us"] + (0.35 * best["work"] if best["MT"] > 1 and not o["loose"] else 0.0)
+        stream = o["w_bytes"] / 4.5e6  # the weights from memory, which either waits for
+        if _tiles_stand(o, t) or max(us, stream) >= 0.95 * max(t["us"], stream):
             return None
     # Steps in equal shares for the waves, in equal batches of what the registers of a full workgroup hold in flight.
-    share = -(-max(1, K // step) // waves)
-    waves = -(-max(1, K // step) // share)
+    MT, VN, steps = best["MT"], best["VN"], max(1, o["K"] // (64 // o["eb"]))
+    share = -(-steps // best["waves"])
     most = max(1, (104 - 4 * MT * VN) // (4 * (MT + VN)))
-    batch = -(-share // -(-share // most))
-    return dict(R=R, MT=MT, C=C, short=short, wide=wide, along_k=along_k, VN=VN, waves=waves, batch=batch, nbatch=nb, row=row)
+    return dict(R=o["R"], MT=MT, C=o["C"], short=o["short"], wide=o["wide"], along_k=o["along_k"], VN=VN, waves=-(-steps // share),
+                batch=-(-share // -(-share // most)), nbatch=o["nbatch"], row=o["row"])
 
 
 def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_args: str, decode: str):

@@ -699,10 +699,11 @@ def _gemm_worthwhile(g: dict) -> bool:
         # for the fold, where the kernel for few rows takes one launch: float16 1 x 768 x 768 6.3 -> 3.1 us, 8 x 512 x 512
         # 5.7 -> 2.7, 1 x 4096 x 2048 8.4 -> 4.2, 12 x 54 x 576 5.6 -> 2.7; float32 22 x 407 x 329 5.6 -> 2.8,
         # 11 x 768 x 183 3.9 -> 2.7.  Along k the reductions are as fast (1 x 768 x 3072 3.0 us against 4.9), and a small
-        # float16 operand with a longer k axis stays with them.
+        # float16 operand with a longer k axis stays with them, as does a float32 one, whose matrix instructions are the chain
+        # then (22 x 452 x 1280 5.3 against 6.7 us, 30 x 94 x 1504 6.6 and 5.3, 26 x 128 x 3072 11.4 and 6.0).
         f32 = g["dtype"] == DType.Float32
         size = wide * g["K"]
-        if (g["dtype"] not in (DType.Float16, DType.Float32) or g.get("a_gather") or g.get("b_gather") or not 96 <= g["K"] < 4096 or size > (8 << 20)
+        if (g["dtype"] not in (DType.Float16, DType.Float32) or g.get("a_gather") or g.get("b_gather") or not 96 <= g["K"] < (1300 if f32 else 4096) or size > (8 << 20)
                 or (g["b_sk"] if g["M"] <= g["N"] else g["a_sk"]) == 1 or not (f32 or g["K"] < 640 or (size >= 1 << 18 and wide >= 128))):
             return False
     # (2..31 rows against a large operand -- a linear layer on a handful of tokens -- do go to the matrix cores: as

@@ -264,3 +264,38 @@ def test_jacobi_eigh_s_plan_follows_the_number_of_matrices(order, batch, dtype, 
     shape = [batch, order, order]
     ks = generateRoutine(Routine(Routines.JacobiEigh, RoutineType([shape], [dtype], [shape] * 2, [dtype] * 2), dict(maxSweeps=30, tolerance=1e-7)))
     assert ks.steps[0].name == ("jh_jacobi_blocks" if blocks else "jh_jacobi") and ("block" in ks.info) == blocks
+
+
+FEW = "few"  # gemm_few.hip.inc
+PRODUCT_PLANS = [
+    # dtype, M, N, K, B stored [N, K] -> the kernel that takes it, and microseconds of it and of what it is chosen over
+    (DType.Float32, 64, 256, 784, False, FEW),                # 4.0 and 22.3 in tiles
+    (DType.Float32, 300, 300, 300, False, FEW),               # 3.4 and 10.1
+    (DType.Float32, 45, 2133, 3712, True, "gemm"),            # 27 and 35
+    (DType.Float32, 61, 10492, 1444, True, "gemm"),           # 38 and 58
+    (DType.Float32, 56, 5248, 1856, False, "gemm"),           # 28 and 41
+    (DType.Float16, 64, 256, 784, False, FEW),                # 2.9 and 12.0
+    (DType.Float16, 64, 1024, 1024, False, FEW),              # 3.3 and 8.0
+    (DType.Float16, 64, 2048, 4096, False, "gemm+fold"),      # 10.2 and 11.9
+    (DType.Float16, 16, 14336, 4096, False, "gemm+fold"),     # 25.8 and 32
+    (DType.Float16, 3, 9287, 5632, False, FEW),               # 33 and 46.5: rows off the 16-byte grid
+    (DType.Float16, 64, 10112, 4416, True, "gemm"),           # 30 and 53
+    (DType.Float16, 40, 8896, 704, True, "gemm"),             # 7.2 and 9.6
+    (DType.Float16, 42, 10240, 512, False, FEW),              # 5.8 and 9.0
+    (DType.Float16, 64, 2304, 5248, True, "gemm+fold"),       # 20 and 29
+    # a handful of rows: of the reductions
+    (DType.Float16, 1, 768, 768, False, FEW),                 # 3.1 and 6.3
+    (DType.Float16, 1, 768, 3072, True, "reduce_row"),        # 3.0 and 4.9
+    (DType.Float16, 12, 54, 576, False, FEW),                 # 2.7 and 5.6
+    (DType.Float16, 1, 11008, 4096, False, "reduce_col+fold"),
+    (DType.Float32, 22, 452, 1280, False, FEW),               # 5.3 and 6.7
+    (DType.Float32, 30, 94, 1504, False, "reduce_col+fold"),  # 5.3 and 6.6
+    (DType.Float32, 26, 128, 3072, False, "reduce_col+fold"),  # 6.0 and 11.4
+]
+
+
+@pytest.mark.parametrize("dtype,m,n,k,transposed,taken", PRODUCT_PLANS, ids=str)
+def test_products_of_few_rows_or_tiles_take_the_kernel_that_was_measured_faster(dtype, m, n, k, transposed, taken):
+    from jaxjs_hip.lowering import matmulKernel
+    ks = generate(matmulKernel(m, n, k, dtype, b_transposed=transposed), "fast")
+    assert (FEW if ks.info.get("few") else ks.klass) == taken
