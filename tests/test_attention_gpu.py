@@ -232,3 +232,53 @@ def test_an_infinite_value_of_the_last_key_stays_one(shape):
     assert (y[..., 5] == np.inf).all() and (y[..., 6] == -np.inf).all()
     rest = [i for i in range(H) if i not in (5, 6)]
     assert np.isfinite(y[..., rest]).all()
+
+
+def _composed(mask, T, N, H, sums="row"):
+    """Attention under a mask that the program closes over (`mask` a diagonal) or takes (None), its softmax written out."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L_
+    from jaxjs_hip.jit import ShapedArray
+
+    def attend(m, q, k, v):
+        s = J.where(m, L_.einsum("BLNH,BSNH->BNLS", q, k).mul(H ** -0.5), -np.inf)
+        e = J.exp(s.sub(J.stopGradient(s.max(-1, keepdims=True))))
+        total = e.sum(-1).reshape([2, N, T, 1] if sums == "row" else [2, N, 1, T])
+        return L_.einsum("BNLS,BSNH->BLNH", e.div(total), v)
+    operands = [ShapedArray((2, T, N, H), F16)] * 3
+    if mask is None:
+        return J.jit(attend, [ShapedArray((T, T), DType.Bool)] + operands)
+    return J.jit(lambda q, k, v: attend(L_.tri_const(T, T, mask), q, k, v), operands)
+
+
+@pytest.mark.parametrize("order", [(0, 1, -1, None), (None, -1, 1, 0)], ids=["causal first", "causal last"])
+def test_masks_of_one_shape_do_not_run_as_each_other(order):
+    """Programs with the same dispatches on one backend: each under its own mask, whichever was prepared first."""
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    from oracle.backend import OracleBackend
+    be, (T, N, H) = backend(), (72, 2, 32)
+    be._programs.clear()
+    rng = np.random.default_rng(6)
+    qkv = [rng.standard_normal((2, T, N, H)).astype(np.float16) for _ in range(3)]
+    free = (rng.random((T, T)) < 0.5) | np.eye(T, dtype=bool)
+    for mask in order:
+        prog, arrays = _composed(mask, T, N, H), qkv if mask is not None else [free.astype(np.int32)] + qkv
+        got, want = run_program(be, prog, arrays)[0], run_program(OracleBackend(), prog, arrays)[0]
+        if mask == -1:  # the first row sees no key: NaN in both
+            assert np.isnan(want.reshape(2, T, -1)[:, 0]).all() and np.isnan(got.reshape(2, T, -1)[:, 0]).all()
+        np.testing.assert_allclose(got.astype(np.float64), want.astype(np.float64), rtol=1e-2, atol=3e-3, equal_nan=True, err_msg=str(mask))
+
+
+def test_sums_along_the_columns_are_not_taken_for_a_softmax():
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    from oracle.backend import OracleBackend
+    T, N, H = 64, 2, 64
+    rng = np.random.default_rng(8)
+    arrays = [rng.standard_normal((2, T, N, H)).astype(np.float16) for _ in range(3)]
+    row, column = _composed(0, T, N, H), _composed(0, T, N, H, "column")
+    got = [run_program(backend(), p, arrays)[0].astype(np.float64) for p in (row, column)]
+    want = run_program(OracleBackend(), column, arrays)[0].astype(np.float64)
+    np.testing.assert_allclose(got[1], want, rtol=1e-2, atol=3e-3 * np.abs(want).max())
+    assert np.abs(got[0] - got[1]).max() > 0.1
