@@ -234,3 +234,57 @@ def test_attention_runs_as_the_routine_where_that_is_the_faster_one(heads, queri
     shapes = [(1, t, heads, size) for t in (queries, keys, keys)]
     prog = J.jit(lambda q, k, v: L.dotProductAttention(q, k, v, isCausal=causal), [ShapedArray(s, DType.Float16) for s in shapes])
     assert (fuse_attention(prog.jaxpr, prog.consts) is not None) == routine
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_what_is_recognised_as_attention_computes_what_the_composition_does(seed, monkeypatch):
+    """Variations of the composition (along which axis sums and maxima go, masks, scales, operands in another order, values
+    used twice), with extents that coincide: whatever is rewritten gives the composition's results on the checker."""
+    import random
+
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip import rewrite
+    from jaxjs_hip.jit import ShapedArray, jitCompile
+    from jit_util import run_program
+    from oracle.backend import OracleBackend
+    monkeypatch.setattr(rewrite, "routine_is_faster", lambda *a: True)
+    rng, values = random.Random(seed), np.random.default_rng(seed)
+    mostly = lambda usual, *others: usual if rng.random() < 0.8 else rng.choice(others)  # noqa: E731
+    fused = 0
+    for _ in range(150):
+        B, N, H, T = rng.choice([1, 2]), rng.choice([1, 2, 3]), rng.choice([32, 64]), rng.choice([2, 5, 8])
+        S = mostly(T, 3, 9)
+        top, total = (mostly("row", "column", "all") for _ in range(2))
+        mask, scale, again = mostly(0, 1, None, "none"), mostly(0.125, -0.5, 1.0, "twice"), mostly("no", "probabilities", "scores")
+        order, shift = mostly("exp first", "sum first"), mostly("minus", "from")
+
+        def along(x, how):
+            return x.max() if how == "all" else x.reshape([B, N, 1, T] if how == "column" and T == S else [B, N, T, 1])
+
+        def f(*args):
+            q, k, v = args[-3:]
+            s = L.einsum("BLNH,BSNH->BNLS", q, k)
+            s = s.mul(0.5).mul(0.25) if scale == "twice" else s if scale == 1.0 else s.mul(scale)
+            if mask != "none":
+                s = J.where(args[0] if mask is None else L.tri_const(T, S, mask), s, -np.inf)
+            m = J.stopGradient(along(s.max(-1), top))
+            e = J.exp(s.sub(m) if shift == "minus" else m.sub(s))
+            r = J.reciprocal(along(e.sum(-1), total))
+            p = e.mul(r) if order == "exp first" else r.mul(e)
+            out = L.einsum("BNLS,BSNH->BLNH", p, v)
+            return [out, p] if again == "probabilities" else [out, s] if again == "scores" else [out]
+        avals = [ShapedArray((B, t, N, H), DType.Float16) for t in (T, S, S)]
+        arrays = [values.standard_normal(a.shape).astype(np.float16) for a in avals]
+        if mask is None:
+            avals = [ShapedArray((T, S), DType.Bool)] + avals
+            arrays = [((values.random((T, S)) < 0.6) | (np.arange(S) == 0)).astype(np.int32)] + arrays
+        prog = J.jit(f, avals)
+        other = rewrite.fuse_attention(prog.jaxpr, prog.consts)
+        if other is None:
+            continue
+        fused += 1
+        want, got = (run_program(OracleBackend(), p, arrays)[0].astype(np.float64) for p in (prog, jitCompile(other, prog.consts)))
+        what = (B, N, T, S, H, top, total, mask, scale, again, order, shift)
+        np.testing.assert_allclose(got, want, rtol=1e-2, atol=3e-3 * max(1.0, np.nanmax(np.abs(want))), equal_nan=True, err_msg=str(what))
+    assert fused >= 15
