@@ -17,6 +17,7 @@ from typing import Any, Dict, List, Optional, Sequence
 from . import tracing
 from .alu import AluExp, AluOp, DType, Kernel, Reduction, byteWidth
 from .errors import SlotError
+from .kernelgen import generate
 from .routine import Routine
 from .rowchain import _tidy, collect_chain, index_form
 from .runtime import LaunchRef, LaunchStepC, check
@@ -32,13 +33,22 @@ class Unit:
         self.exe = None
 
 
+_LONG_OPS = (AluOp.Erf, AluOp.Erfc, AluOp.Sin, AluOp.Cos, AluOp.Asin, AluOp.Atan)  # dozens of instructions each
+
+
 def join_epilogue(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int]) -> Optional[Kernel]:
     """The contraction `product`, which writes `buffer`, with the elementwise `following` (reading `inputs`) as the rest of
     its epilogue, or None.  `following` has to read nothing but `buffer`, each element at its own position.  The product's
     value keeps the type it was stored in, so results keep their bits.
 
     A value that is used more than once ends the front-end's fusion (src/frontend/jit.ts:572-789): gelu behind a linear
-    layer was a launch of its own that read and wrote the whole activation again (float16 [8192, 3072]: 24 us)."""
+    layer was a launch of its own that read and wrote the whole activation again (float16 [8192, 3072]: 24 us).
+
+    Where the epilogue is long it stays a launch of its own behind float16 tiles: a tile's few threads have it in front of
+    them when the product is done, and the product is quick (512 x 512 x 512, x erfc(x): 13.5 us joined, 8.7 in two
+    launches; sine 12.8 and 8.6; arc tangent 10.5 and 8.4; 8192 x 3072 x 768 78 and 73).  exp and log are short enough
+    (tanh, mish), float32 products long enough (1024 x 1024 x 1024: 35.4 and 33.8, 8000 x 1000 x 100 43 and 47), and a
+    short k axis or the kernel for few rows leaves room (2048 x 2048 x 64 12.7 and 15.5, 8 x 3072 x 768 5.7 and 8.7)."""
     re = product.reduction
     if re is None or following.reduction is not None or following.size != product.size or product.size == 0:
         return None
@@ -48,8 +58,13 @@ def join_epilogue(product: Kernel, buffer: int, following: Kernel, inputs: Seque
     own = _tidy({("gidx", 1): 1}, {"gidx": product.size})
     if not loads or any(inputs[n.arg[0]] != buffer or n.dtype != re.epilogue.dtype or index_form(n.src[0], {"gidx": product.size}) != own for n in loads):
         return None
-    if match_gemm(product) is None:
+    g = match_gemm(product)
+    if g is None:
         return None
+    if g["dtype"] == DType.Float16 and g["K"] >= 256 and exp.collect(lambda n: n.op in _LONG_OPS):
+        plan = generate(product)
+        if plan.klass.startswith("gemm") and not plan.info.get("few"):
+            return None
     exp = exp.rewrite(lambda n: re.epilogue if n.op == AluOp.GlobalIndex else None)
     return Kernel(product.nargs, product.size, product.exp_raw, Reduction(re.dtype, re.op, re.size, exp))
 

@@ -288,3 +288,27 @@ def test_what_is_recognised_as_attention_computes_what_the_composition_does(seed
         what = (B, N, T, S, H, top, total, mask, scale, again, order, shift)
         np.testing.assert_allclose(got, want, rtol=1e-2, atol=3e-3 * max(1.0, np.nanmax(np.abs(want))), equal_nan=True, err_msg=str(what))
     assert fused >= 15
+
+
+@pytest.mark.parametrize("shape,dtype,f,launches", [
+    # microseconds joined and in two launches
+    ((512, 512, 512), DType.Float16, "erfc", 2),     # 13.5 and 8.7
+    ((512, 512, 512), DType.Float16, "sin", 2),      # 12.8 and 8.6
+    ((512, 512, 512), DType.Float16, "atan", 2),     # 10.5 and 8.4
+    ((8192, 3072, 768), DType.Float16, "erfc", 2),   # 78 and 73
+    ((512, 512, 512), DType.Float16, "tanh", 1),     # 8.4 and 8.5 (gelu)
+    ((8192, 3072, 768), DType.Float16, "tanh", 1),
+    ((8, 3072, 768), DType.Float16, "erfc", 1),      # 5.7 and 8.7: the kernel for few rows
+    ((2048, 2048, 64), DType.Float16, "erfc", 1),    # 12.7 and 15.5
+    ((512, 512, 512), DType.Float32, "erfc", 1),     # 12.5 and 12.9
+    ((8000, 1000, 100), DType.Float32, "sin", 1),
+], ids=str)
+def test_a_long_epilogue_stays_a_launch_of_its_own_behind_float16_tiles(shape, dtype, f, launches):
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import plan_units
+    m, n, k = shape
+    act = dict(erfc=J.erfc, sin=J.sin, atan=J.atan, tanh=L.tanh)[f]
+    prog = J.jit(lambda x, w: (lambda h: h.mul(act(h)))(L.matmul(x, w)), [ShapedArray(s, dtype) for s in ((m, k), (k, n))])
+    assert len(plan_units(prog)) == launches
