@@ -128,22 +128,24 @@ def routine_is_faster(B: int, N: int, L: int, S: int, H: int, causal: bool) -> b
     S = 128 .. 65536 in all head sizes: of 646 shapes the rule takes the slower side by more than a fifth at five (by 1.54
     at most, at S = 5001), where the routine everywhere would lose that much at 158, and up to 21 times.
 
-    Up to ATTENTION_FEW_QUERIES queries, a workgroup each: it reads keys and values at 100 GB/s, so 4096 keys of 64 take it
-    12 us and 65536 take 162, when the composition's launches and all CUs' reading take 14 and 33.  With many workgroups
-    both are bound by reading the cache, which the composition reads once for all queries of a head: from 50 million
-    multiplications (in heads of 64) on it is ahead by up to a tenth (384 heads x 2 x 2048: 57.5 against 51.5 us, 192 x 2 x
-    2048, at the line: 31.8 against 30.2, 96 x 2 x 2048: 16.9 against 21.4).
+    A workgroup per query reads keys and values at 100 GB/s, so 4096 keys of 64 take it 12 us and 65536 take 162, when the
+    composition's launches and all CUs' reading take 14 and 33.  With many workgroups both are bound by reading the cache:
+    from 50 million multiplications (in heads of 64) on the composition is level (384 heads x 3072 55.5 against 54.6 us).
 
-    More queries: workgroups of 128 rows, one to a CU at first, that walk all keys they see (half of them on average under
-    the mask).  The composition costs 10 us of launches and moves the scores several times: 1.8 us per million of them, and
-    3.2 where its products' tiles of 64 rows are partly empty.  (12 x 64 x 2048 x 64: 27.6 against 16.3 us; 12 x 512 x 2048:
-    28.4 against 36; 96 x 128 x 4096: 54 against 106; 1 x 4096 x 4096, causal: 62 against 48.)"""
-    from .routinegen import ATTENTION_FEW_QUERIES
-    if L <= ATTENTION_FEW_QUERIES:
+    Workgroups of 128 rows, one to a CU at first, walk all keys they see (half of them on average under the mask).  The
+    composition costs 10 us of launches and moves the scores several times: 1.8 us per million of them, and 3.2 where its
+    products' tiles of 64 rows are partly empty (12 x 64 x 2048 x 64: 27.6 against 16.3 us; 12 x 512 x 2048: 28.4 against 36;
+    96 x 128 x 4096: 54 against 106; 1 x 4096 x 4096, causal: 62 against 48).  Up to four queries it has no such tiles and
+    reads the cache at 4.3 TB/s for two of them (192 x 2 x 2048 x 64: 28 against 30 us, 8192: 119 and 107; 4 x 8192: 118 and
+    152; 384 x 4 x 1024: 23 and 36)."""
+    from .routinegen import ATTENTION_FEW_QUERIES, attention_by_queries
+    if attention_by_queries(B * N, L, H):
         return S * H <= 4096 * 64 and B * N * L * S * max(H, 64) <= 3 << 24
     tiles = B * N * -(-L // 128)
     walked = min(S, L) if causal else S
     routine = 2 + _TILE_US_PER_KEY[H] * walked * max(1.0, tiles * (0.6 if causal else 1.0) / 256)
+    if L <= ATTENTION_FEW_QUERIES:
+        return 1.1 * routine <= 12 + (0.6 + 0.2 * L) * 4 * B * N * S * H / 4.3e6
     return routine <= 10 + (3.2 if L <= 64 else 1.8) * B * N * max(L, 64) * S / 1e6
 
 

@@ -287,7 +287,7 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
 # The step of a block costs more than the few rotations of a smaller matrix (float32 12: 183 against 178 us, 13: 257 and 249,
 # 16: 272 and 324; float16 13: 437 and 402, 16: 525 and 622).
 JACOBI_BLOCKS_FROM = {2: 16, 4: 13, 8: 13}
-ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which every query is a workgroup of its own and not a row of a 128-row tile
+ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which a query may be a workgroup of its own (`attention_by_queries`)
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS
 TRISOLVE_AHEAD = 8       # entries of a row that a right-hand side's thread fetches ahead of its subtraction chain
@@ -645,6 +645,18 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, scratch, "sort", need, dict(n=n, rows=rows, P=P, tile=tile, argsort=argsort, launches=len(steps)))
 
 
+def attention_by_queries(heads: int, queries: int, size: int) -> bool:
+    """Whether every query takes a workgroup of its own (attention_few.hip.inc) and not a row of a tile of 128.  `heads`
+    counts those of all sequences.  Alone on its CU a query reads its keys as fast as they come, where a tile walks 64 at a
+    time: 8 x 12 heads over 2048 keys of 64 10 us against 27.  But every query reads them for itself: from 128 heads on
+    two to four of them wait for memory, the tile of each head does not (11 x 12 heads, 4 queries, 2048 keys 32 us against
+    28, 32 x 12 67 against 41, 64 x 12 156 against 79).  One query stays ahead (64 x 12 71 against 80), in heads of 32
+    up to 512 of them (32 x 12 0.93 of the tile's time, 64 x 12 1.25)."""
+    if queries == 1:
+        return heads <= 512 or size > 32
+    return queries <= ATTENTION_FEW_QUERIES and heads <= 128
+
+
 def _gen_attention(routine: Routine, numerics: str) -> Optional[KernelSource]:
     """Fused attention over [B, L, N, H] / [B, S, N, H] float16 operands with H = 32, 64 or 128 and any L and S >= 1
     (contiguous, or strided views with unit stride along the head dimension)."""
@@ -681,7 +693,7 @@ def _gen_attention(routine: Routine, numerics: str) -> Optional[KernelSource]:
             lay.append((sb, sp, sn, v["offset"]))
             need[i] = v["elements"] * 2
     (qb, ql, qn, qo), (kb, ksp, kn, ko), (vb, vsp, vn, vo) = lay
-    if L <= ATTENTION_FEW_QUERIES:
+    if attention_by_queries(B * N, L, H):
         lanes = H // 8
         threads = 128
         while threads < 1024 and threads < S * lanes // 2:

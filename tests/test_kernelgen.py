@@ -299,3 +299,19 @@ def test_products_of_few_rows_or_tiles_take_the_kernel_that_was_measured_faster(
     from jaxjs_hip.lowering import matmulKernel
     ks = generate(matmulKernel(m, n, k, dtype, b_transposed=transposed), "fast")
     assert (FEW if ks.info.get("few") else ks.klass) == taken
+
+
+@pytest.mark.parametrize("heads,queries,size,by_queries", [
+    # microseconds of a workgroup per query and of tiles, 2048 keys
+    ((8, 12), 1, 64, True), ((64, 12), 1, 64, True), ((64, 12), 1, 128, True),     # 10 and 27; 71 and 80
+    ((32, 12), 1, 32, True), ((64, 12), 1, 32, False),                             # 0.93 and 1.25 of the tiles' time
+    ((8, 12), 4, 64, True), ((4, 32), 4, 64, True), ((11, 12), 4, 64, False),      # 21 and 27; 21 and 29; 32 and 28
+    ((32, 12), 2, 64, False), ((64, 12), 4, 128, False), ((1, 1), 5, 64, False),   # 57 and 43; 1.8 of the tiles' time
+], ids=str)
+def test_attention_takes_a_workgroup_per_query_only_for_few_queries_of_few_heads(heads, queries, size, by_queries):
+    from jaxjs_hip.routine import Routine, Routines, RoutineType
+    from jaxjs_hip.routinegen import generateRoutine
+    B, N = heads
+    shapes = [[B, t, N, size] for t in (queries, 2048, 2048)]
+    ks = generateRoutine(Routine(Routines.Attention, RoutineType(shapes, [DType.Float16] * 3, [shapes[0]], [DType.Float16]), dict(scale=0.125)))
+    assert [s.name for s in ks.steps] == ["jh_attention_few" if by_queries else "jh_attention"]

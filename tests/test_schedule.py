@@ -215,7 +215,10 @@ def test_attention_under_a_scale_that_is_not_a_finite_float16_stays_as_it_is(sca
     (12, 1, 16384, 64, False, False),   # 52 and 20
     (1, 4, 65536, 64, False, False),    # 162 and 36
     (12, 1, 16384, 128, False, False),  # 99 and 27
-    (384, 2, 2048, 64, False, False),   # 57 and 51
+    (384, 1, 8192, 64, False, False),   # 156 and 144
+    (384, 2, 2048, 64, False, True),    # 43 and 51: in tiles
+    (192, 2, 8192, 64, False, False),   # 119 and 107
+    (192, 4, 8192, 64, False, True),    # 118 and 152
     # prefill
     (12, 5, 512, 64, False, True),      # 8 and 12
     (12, 5, 4096, 64, False, False),    # 52 and 17
