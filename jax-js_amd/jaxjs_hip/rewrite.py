@@ -125,8 +125,8 @@ _TILE_US_PER_KEY = {32: 0.0100, 64: 0.0126, 128: 0.0188}
 
 def routine_is_faster(B: int, N: int, L: int, S: int, H: int, causal: bool) -> bool:
     """Whether the Attention routine beats the composition.  From both sides measured at B N = 1 .. 768, L = 1 .. 4096 and
-    S = 128 .. 65536 in all head sizes: of 646 shapes the rule takes the slower side by more than a fifth at five (by 1.54
-    at most, at S = 5001), where the routine everywhere would lose that much at 158, and up to 21 times.
+    S = 128 .. 65536 in all head sizes: of 640 shapes the rule takes the slower side by more than a fifth at five (by 1.54
+    at most, at S = 5001), where the routine everywhere would lose that much at 153, and up to 21 times.
 
     A workgroup per query reads keys and values at 100 GB/s, so 4096 keys of 64 take it 12 us and 65536 take 162, when the
     composition's launches and all CUs' reading take 14 and 33.  With many workgroups both are bound by reading the cache:
