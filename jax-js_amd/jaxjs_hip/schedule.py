@@ -238,9 +238,12 @@ class Schedule:
         if be.trace is not None or (tracing.isTracing() and not be.capturing):
             return self._run_by_unit(inputs)
         slots = be._slots
-        made = [be.malloc(self._sizes[o]) for o in self._made]
-        space = be._alloc(self._work[-1])
+        made: List[int] = []
+        space = 0
         try:
+            for o in self._made:
+                made.append(be.malloc(self._sizes[o]))
+            space = be._alloc(self._work[-1])
             with self._lock:
                 buf = self._buffers
                 for i, need in self._inputs:

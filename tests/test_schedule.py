@@ -315,3 +315,30 @@ def test_a_long_epilogue_stays_a_launch_of_its_own_behind_float16_tiles(shape, d
     act = dict(erfc=J.erfc, sin=J.sin, atan=J.atan, tanh=L.tanh)[f]
     prog = J.jit(lambda x, w: (lambda h: h.mul(act(h)))(L.matmul(x, w)), [ShapedArray(s, dtype) for s in ((m, k), (k, n))])
     assert len(plan_units(prog)) == launches
+
+
+@pytest.mark.parametrize("room", [0, 1, 2])
+def test_a_call_that_runs_out_of_memory_gives_back_what_it_took(room):
+    """Outputs and the workspace are taken one after the other; whichever fails, the call leaves no slot behind."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    be = _stand_in()
+    shapes = ((64, 128), (128, 256), (256, 64))
+    prog = J.jit(lambda x, a, b: (lambda h: [L.matmul(h, b), J.exp(x)])(L.matmul(x, a)), [ShapedArray(s, DType.Float32) for s in shapes])
+    taken = []
+
+    def malloc(n):
+        if len(taken) == room:
+            raise MemoryError(n)
+        taken.append(n)
+        return 4096 * len(taken)
+    be.dev.malloc = malloc
+    be._alloc = lambda n: malloc(n) if n else 0
+    schedule = be.scheduleProgram(prog)
+    assert schedule._work[-1] > 0 and len(schedule._made) == 2
+    be._slots = {i + 1: dict(ptr=1 << 20, size=1 << 20, ref=1) for i in range(3)}
+    be._next_slot = 4
+    with pytest.raises(MemoryError):
+        schedule.run([1, 2, 3])
+    assert list(be._slots) == [1, 2, 3] and sum(len(free) for free in be._pool.values()) == room
