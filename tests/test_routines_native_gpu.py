@@ -382,31 +382,32 @@ def test_outputs_are_fully_initialised_without_updates():
     assert_bits(got, want)
 
 
-@pytest.mark.parametrize("dt", [F32, np.float64, np.float16], ids=lambda d: np.dtype(d).name)
-@pytest.mark.parametrize("shape", [(70, 1, 1), (3, 8, 8), (5, 9, 9), (2, 3, 27, 27), (2, 43, 43), (4, 63, 63), (64, 64)], ids=str)
+@pytest.mark.parametrize("shape,dt", [((70, 1, 1), F32), ((5, 9, 9), F32), ((2, 3, 27, 27), F32), ((64, 64), F32), ((3, 8, 8), np.float64),
+                                      ((2, 27, 27), np.float64), ((2, 43, 43), np.float16), ((4, 63, 63), np.float16)], ids=str)
 def test_cholesky_with_a_wave_per_matrix(shape, dt, monkeypatch):
     """The plan of many small matrices, at every order that a wave can hold a row per lane of: the checker's bits."""
-    from gpu_util import backend
+    from gpu_util import WARM_ONLY, backend
     from jaxjs_hip import routinegen
     n = shape[-1]
     x = (spd(tuple(shape[:-2]), n).astype(np.float64) / n + np.triu(RNG.standard_normal(shape), 1)).astype(dt)
     monkeypatch.setattr(routinegen, "_cholesky_plan", lambda *a: "wave per matrix")
-    backend().clearCache()
+    if not WARM_ONLY:
+        backend().clearCache()  # prepared routines are cached by structure
     got, want, ks = both(R.cholesky(x), [x])
     backend().clearCache()
     assert [s.name for s in ks.steps] == ["jh_cholesky"]
     assert_bits(got, want, f"cholesky {shape} {np.dtype(dt).name}")
 
 
-@pytest.mark.parametrize("dt", [F32, np.float64, np.float16], ids=lambda d: np.dtype(d).name)
-@pytest.mark.parametrize("shape", [(192, 192), (3, 200, 200), (2, 333, 333)], ids=str)
+@pytest.mark.parametrize("shape,dt", [((192, 192), F32), ((2, 333, 333), F32), ((3, 200, 200), np.float64), ((2, 333, 333), np.float16)], ids=str)
 def test_cholesky_with_two_launches_per_panel(shape, dt, monkeypatch):
-    from gpu_util import backend
+    from gpu_util import WARM_ONLY, backend
     from jaxjs_hip import routinegen
     n = shape[-1]
     x = (spd(tuple(shape[:-2]), n).astype(np.float64) / n).astype(dt)
     monkeypatch.setattr(routinegen, "_cholesky_plan", lambda *a: "two launches")
-    backend().clearCache()
+    if not WARM_ONLY:
+        backend().clearCache()  # prepared routines are cached by structure
     got, want, ks = both(R.cholesky(x), [x])
     backend().clearCache()
     assert ks.info["variant"] == "two launches" and ks.info["panels"] == -(-n // 32)
