@@ -271,13 +271,16 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     threads = _round64(n)
     in_lds = 1 if 2 * n * n * eb <= 150 * 1024 else 0  # both matrices in the CU's 160 KB of LDS: n <= 138 in float32
     by_blocks = JACOBI_BLOCKS_FROM[eb] <= n <= 192 and _jacobi_blocks_pay(n, batch, eb)
+    # Waves for part 3 beside the chains' (three times n / 64), as many as leave a lane the registers it needs (float32 64:
+    # 1.87 ms with 8, 1.89 with 16; 128: 7.4 with 8, 7.1 with 12, 6.8 with 16; float64 96: 4.7 with 12, 5.1 with 16).
+    block_threads = 512 if n <= 64 else 768 if eb == 8 else 1024
     for size in (4, 8):  # indices per block; the triangle and the rotations under way have to fit the LDS
         blocks = -(-n // size)
         if by_blocks and eb * (n * (n + 1) // 2) + 16 * (blocks + 1) * n + 32 * blocks + 512 <= 160 * 1024:
-            src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=512, RB=size, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
-            steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (512, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("scratch", 0)])]
+            src = _linalg_source(numerics, ROUTINE=7, N=n, THREADS=block_threads, RB=size, MAX_SWEEPS=int(params["maxSweeps"]), TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
+            steps = [LaunchStep("jh_jacobi_blocks", (batch, 1, 1), (block_threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("scratch", 0)])]
             return KernelSource([src], steps, [batch * n * n * eb], "jacobi", {0: batch * n * n * eb},
-                                dict(n=n, batch=batch, threads=512, in_lds=bool(in_lds), block=size))
+                                dict(n=n, batch=batch, threads=block_threads, in_lds=bool(in_lds), block=size))
     src = _linalg_source(numerics, ROUTINE=3, N=n, THREADS=threads, IN_LDS=in_lds, MAX_SWEEPS=int(params["maxSweeps"]),
                          TOL=repr(float(params["tolerance"])), ELEM=ctype, CMP=cmp_t)
     steps = [LaunchStep("jh_jacobi", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1)])]

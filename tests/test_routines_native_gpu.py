@@ -149,6 +149,19 @@ def test_jacobi_eigh_by_blocks_at_ragged_orders(n):
     assert_bits(got, want, f"jacobi_eigh {n} {ks.info}")
 
 
+@pytest.mark.parametrize("scale", [1e-44, 1e-30, 1e30, 1e38])
+@pytest.mark.parametrize("n", [14, 65])
+def test_jacobi_eigh_at_the_ends_of_the_element_range(n, scale):
+    """Rotations without scaled quotients: elements that are denormal, and elements that overflow on the way (the result then
+    holds infinities and NaNs, the same ones); a widely graded diagonal makes the smallest and largest angles."""
+    a = RNG.uniform(-1, 1, (3, n, n)) * 10.0 ** RNG.integers(-6, 1, (3, 1, n))
+    a[2] += np.diag(3.0 * 10.0 ** RNG.integers(-12, 1, n))
+    with np.errstate(over="ignore"):
+        sym = ((a + np.swapaxes(a, -1, -2)) * scale).astype(F32)
+    got, want, _ = both(R.jacobi_eigh(sym, 4, 0.0), [sym])
+    assert_bits(got, want, f"jacobi_eigh {n} scale {scale}")
+
+
 def test_jacobi_eigh_sweep_limits_and_special_values():
     a = RNG.standard_normal((3, 12, 12))
     sym = (a + np.swapaxes(a, -1, -2)).astype(F32)
