@@ -83,13 +83,14 @@ def _float_elem(t):
 def _cholesky_plan(n: int, batch: int, eb: int) -> str:
     """Which of the four plans factors `batch` matrices of order n; they give the same bits (float32, microseconds).
 
-    A launch per panel has the shortest chain, and a workgroup of 256 per 32 rows with 50 KB of LDS (68 in float64): three
-    (two) of them on a CU.  A wave per matrix holds 32 on a CU and is as fast alone up to order 8 (7.0 and 7.0); from there
-    its chain is longer and it takes batches to win (16: 256 matrices 14 against 7.7, 1536 20 and 18, 4096 24 and 42,
-    65536 282 and 623; 24: 4096 47 and 56), which it never does from order 28 on (28: 16384 266 against 249; in float16,
-    whose panels pay for conversions, to 40: 16384 473 against 634, 48: 768 against 725).
-    Two launches per panel do less work on a longer chain, and win where the panels' workgroups come 16 to a CU, 8 in
-    float64 (256: 512 matrices 662 against 635, 1024 1065 and 1189; 512: 128 1174 and 1000, 256 1739 and 1807)."""
+    A launch per panel has the shortest chain, and a workgroup of 256 per 32 rows with 36 KB of LDS (55 in float64): four (two)
+    of them on a CU.  A wave per matrix holds 32 on a CU and is as fast alone up to order 8 (9 and 10); from there its chain
+    is longer and it takes batches to win (16: 256 matrices 16.6 against 9.9, 1536 20.9 and 13.9, 4096 26 and 30, 65536 298
+    and 397; 24: 4096 48 and 39), which it does not from order 28 on (28: 16384 271 against 153; in float16, whose panels pay
+    for conversions, 40: 16384 482 against 441, 48: 791 against 497).
+    Two launches per panel take less room in LDS; the lines between them and a launch per panel date from a slower kernel for
+    the latter, which is now the faster one on both sides (256: 512 matrices 439 against 688, 1024 826 and 1096; 512: 128
+    712 and 1199, 512 2261 and 3030)."""
     from . import tuner
     cus = tuner.CU_COUNT
     many = 2 if eb == 8 and n <= 12 else min(n // 4, 6)  # matrices per CU

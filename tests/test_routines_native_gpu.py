@@ -62,6 +62,30 @@ def test_cholesky_left_looking_panels_when_the_double_copy_is_too_large(shape, m
     assert_bits(left, right, f"cholesky variants {shape}")
 
 
+@pytest.mark.parametrize("dt", [F32, np.float16, np.float64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("n", [9, 32, 33, 70])
+def test_cholesky_pivots_that_are_no_ordinary_numbers(n, dt):
+    """Roots and quotients without the compiler's scaling and special cases: zero, negative, infinite and undefined pivots, and
+    elements at either end of the range, in the first columns, inside a panel, at its end and behind it."""
+    x = RNG.standard_normal((8, n, n))
+    base = (x @ np.swapaxes(x, -1, -2) / n + np.eye(n)).astype(dt)
+    tiny, big = np.finfo(dt).tiny, np.finfo(dt).max
+    mats = []
+    for at in sorted({0, 1, 2, 3, n // 2, min(31, n - 1), n - 1}):
+        for value in (0.0, -0.0, -1.0, np.inf, -np.inf, np.nan, tiny, tiny / 4, big):
+            m = base[at % 8].copy()
+            m[at, at] = value
+            if value in (0.0, -1.0):
+                m[at, :at] = m[:at, at] = 0
+            mats.append(m)
+    scales = [tiny / 8, tiny * 4, big / 64]
+    with np.errstate(over="ignore", under="ignore"):
+        mats += [(base[i].astype(np.float64) * s).astype(dt) for i, s in enumerate(scales)]
+    a = np.stack(mats)
+    got, want, _ = both(R.cholesky(a), [a])
+    assert_bits(got, want, f"cholesky {n} {np.dtype(dt).name}")
+
+
 def test_cholesky_not_positive_definite_and_empty():
     x = np.array([[[1, 2], [2, 1]], [[4, 2], [2, 3]]], F32)
     got, want, _ = both(R.cholesky(x), [x])
