@@ -403,10 +403,10 @@ class HipBackend:
         key = ("routine", routineKey(routine), self.numerics)
         return await self._prepare_async(key, routine, lambda: generateRoutine(routine, self.numerics))
 
-    def prepareSync(self, source) -> Executable:
+    def prepareSync(self, source, **tune_opts) -> Executable:
         """`prepareKernelSync` / `prepareRoutineSync` / a chain of Kernels over the same rows, by the source's type."""
         if isinstance(source, Kernel):
-            return self.prepareKernelSync(source)
+            return self.prepareKernelSync(source, **tune_opts)
         if isinstance(source, Routine):
             return self.prepareRoutineSync(source)
         key = (source.key(), self.numerics)

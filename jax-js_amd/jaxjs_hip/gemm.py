@@ -17,6 +17,7 @@ from .kernelgen import KernelSource, LaunchStep, _Body, _min_bytes, _prelude, _u
 from . import tuner
 from .fewgen import gen_few, plan_few
 from .tuner import TuneResult, classify_loads
+from .wgradgen import gen_wgrad
 
 
 def choose_tile(g: dict) -> Dict[str, int]:
@@ -562,7 +563,8 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
     # Split of the k axis over blockIdx.y: every slice is the same kernel on K / split, its f32 accumulators go to a
     # scratch buffer [slice][output] and a generated fold Kernel adds the slices in order and applies the epilogue
     # (deterministic: no float atomics).  For launches that would otherwise leave most CUs without a workgroup.
-    split = int(tile.get("SPLITK", 1))
+    wgrad = t.params.get("wgrad") if not override else None  # a filter cotangent with a kernel of its own
+    split = 1 if wgrad else int(tile.get("SPLITK", 1))
     K_full = g["K"]
     two_stride = dict(a=g["a_k0"] != K_full, b=g["b_k0"] != K_full)  # of the whole k axis, before any slicing
     if split > 1:
@@ -586,7 +588,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
 
     # An operand off the 16-byte grid that a pre-pass copies into scratch (see `_repack_operand`): from here on it is a
     # dense [K][rows_pad] operand named `jh_repack`.
-    repack = _repack_operand(g) if split == 1 and tile.get("REPACK", 1) and not few else None
+    repack = _repack_operand(g) if split == 1 and tile.get("REPACK", 1) and not few and not wgrad else None
     load_rows = dict(a=g["M"], b=g["N"])
     repack_src = {}
     if repack:
@@ -641,6 +643,8 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
         src_options = ""
         epi_fn = f"static __device__ __forceinline__ float jh_epilogue(float acc, int row, int col, int b0, int b1, int b2{epi_params}) {{\n  return acc;\n}}"
     epi_args = "".join(f", {n}" for n in names)
+    if wgrad:
+        return gen_wgrad(kernel, g, wgrad, numerics, name, params, names, out_t, epi_fn, epi_params, epi_args, _min_bytes(t.epilogue), src_options)
 
     if few:
         lines = ["  {", "    int rem = batch;"]

@@ -23,13 +23,15 @@ from .rowchain import _tidy, collect_chain, index_form
 from .runtime import LaunchRef, LaunchStepC, check
 from .shape import prod
 from .tuner import match_gemm
+from .wgradgen import is_filter_cotangent
 
 
 class Unit:
-    """One dispatch of the schedule: an executable, the buffer ids it reads and the ones it writes."""
+    """One dispatch of the schedule: an executable (of `source`, prepared with `options`), the buffer ids it reads and the ones
+    it writes."""
 
-    def __init__(self, source, inputs: Sequence[int], outputs: Sequence[int]):
-        self.source, self.inputs, self.outputs = source, list(inputs), list(outputs)
+    def __init__(self, source, inputs: Sequence[int], outputs: Sequence[int], **options):
+        self.source, self.inputs, self.outputs, self.options = source, list(inputs), list(outputs), options
         self.exe = None
 
 
@@ -116,7 +118,8 @@ def plan_units(prog) -> List[Unit]:
             units.append(Unit(chain, chain.inputs, [steps[k + j].output for j in chain.outputs]))
             k += n
             continue
-        units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs))
+        options = dict(filter_bands=True) if s.routine is None and is_filter_cotangent(s.kernel) else {}
+        units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))
         k += 1
     return units
 
@@ -172,7 +175,7 @@ class Schedule:
         pinned = []
         try:  # a unit that is prepared here must not push out one that was prepared before it
             for u in self.units:
-                u.exe = backend.prepareSync(u.source)
+                u.exe = backend.prepareSync(u.source, **u.options)
                 backend.pin(u.exe)
                 pinned.append(u.exe)
             self._bind()

@@ -490,8 +490,9 @@ def match_transposed_map(kernel: Kernel) -> Optional[dict]:
 def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True,
             gemm_tile: Optional[tuple] = None, col_strip: Optional[tuple] = None,
             row_lanes: Optional[int] = None, row_unroll: Optional[int] = None, row_nt: Optional[int] = None, col_nt: Optional[int] = None,
-            map_unroll: Optional[int] = None, map_nt: Optional[int] = None) -> TuneResult:
-    """Pick the kernel class and its parameters for one Kernel on MI355X."""
+            map_unroll: Optional[int] = None, map_nt: Optional[int] = None, filter_bands: bool = False) -> TuneResult:
+    """Pick the kernel class and its parameters for one Kernel on MI355X.  `filter_bands`: a convolution's filter cotangent
+    takes the kernel of `wgradgen.py` where that covers it."""
     t = tuneNullopt(kernel)
     re = kernel.reduction
     size = kernel.size
@@ -531,12 +532,17 @@ def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True
     R = re.size
     if allow_gemm and GEMM_ENABLED:
         g = match_gemm(kernel)
-        if g is not None and _gemm_worthwhile(g):
-            t.klass = "gemm"
-            t.gemm = g
-            if gemm_tile:
-                t.params["gemm_tile"] = dict(gemm_tile)
-            return t
+        if g is not None:
+            if filter_bands:
+                from .wgradgen import find_wgrad
+
+                t.params["wgrad"] = find_wgrad(kernel, t, g)
+            if t.params.get("wgrad") or _gemm_worthwhile(g):
+                t.klass = "gemm"
+                t.gemm = g
+                if gemm_tile:
+                    t.params["gemm_tile"] = dict(gemm_tile)
+                return t
 
     loads = _load_nodes(t.exp)
     Vr = _pick_vector_width(kernel, t, R)

@@ -1,0 +1,108 @@
+"""The filter cotangent of a convolution with its bands in LDS (`wgrad_f16.hip.inc`): which Kernels it is chosen for, and its
+sums against the definition, tap by tap."""
+import numpy as np
+import pytest
+
+from gpu_util import device_run
+from jaxjs_hip import DType, jit as J
+from jaxjs_hip.convolution import ConvParams
+from jaxjs_hip.jit import ShapedArray
+from jaxjs_hip.kernelgen import generate
+from jaxjs_hip.schedule import plan_units
+
+RNG = np.random.default_rng(11)
+
+
+def cotangent_program(batch, cin, cout, h, w, kh, kw, pad, stride=1, dtype=DType.Float16, dilation=1):
+    """(program of the filter's cotangent, shape of the cotangent); pad: ((top, bottom), (left, right))."""
+    p = ConvParams(0, [stride] * 2, list(pad), [1, 1], [dilation] * 2)
+    oh = (h + sum(pad[0]) - (kh - 1) * dilation - 1) // stride + 1
+    ow = (w + sum(pad[1]) - (kw - 1) * dilation - 1) // stride + 1
+    avals = [ShapedArray((batch, cin, h, w), dtype), ShapedArray((batch, cout, oh, ow), dtype)]
+    prog = J.jit(lambda x, ct: J.convTransposeRhs(x, ct, [cout, cin, kh, kw], p), avals)
+    return prog, (batch, cout, oh, ow)
+
+
+def cotangent_kernel(*args, **kw):
+    prog, shape = cotangent_program(*args, **kw)
+    return [s.kernel for s in prog.steps if s.kind == "execute"][0], shape
+
+
+SAME = lambda k: ((k // 2, k // 2),) * 2  # noqa: E731
+
+CASES = [
+    # batch, cin, cout, h, w, kh, kw, padding        what it reaches
+    (2, 64, 64, 16, 16, 3, 3, SAME(3)),              # whole groups of eight, one launch
+    (2, 40, 72, 20, 24, 3, 3, SAME(3)),              # channels past the last tile of either operand
+    (4, 33, 31, 37, 41, 3, 3, SAME(3)),              # rows that are no whole groups, bands with fewer rows at the end
+    (3, 32, 64, 28, 28, 5, 5, SAME(5)),              # a workgroup per window row, two dwords' worth of padding
+    (2, 64, 48, 20, 20, 5, 5, ((0, 0), (0, 0))),     # no padding: the image is wider than the cotangent
+    (6, 48, 48, 33, 9, 3, 3, ((0, 0), (1, 0))),      # padding on one side, nine columns
+    (9, 32, 32, 9, 57, 3, 2, ((1, 1), (0, 1))),      # an even window, odd numbers of groups
+    (2, 64, 64, 24, 24, 4, 4, ((3, 3), (3, 3))),     # full padding: the cotangent is wider than the image
+    (9, 64, 96, 56, 56, 3, 3, SAME(3)),              # slices over the bands, more of them than a multiple of eight
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_plan_covers_the_case(case):
+    kernel, _ = cotangent_kernel(*case)
+    info = generate(kernel, filter_bands=True).info
+    assert "wgrad" in info, info
+    assert "wgrad" not in generate(kernel).info  # by itself it keeps the general templates
+    assert plan_units(cotangent_program(*case)[0])[0].options == dict(filter_bands=True)
+
+
+@pytest.mark.parametrize("kw", [dict(stride=2), dict(dilation=2), dict(dtype=DType.Float32), dict(w=7), dict(kh=1), dict(batch=1, cin=16, cout=16)], ids=str)
+def test_what_the_kernel_does_not_cover_stays_where_it_was(kw):
+    args = dict(dict(batch=4, cin=64, cout=64, h=24, w=24, kh=3, kw=3, pad=SAME(3)), **kw)
+    kernel, _ = cotangent_kernel(**args)
+    assert "wgrad" not in generate(kernel, filter_bands=True).info
+    assert plan_units(cotangent_program(**args)[0])[0].options == {}
+
+
+def reference(x, ct, kh, kw, pad):
+    """sums[c, o, ky, kx] in 64 bits and the sums of the terms' magnitudes."""
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0)) + tuple(pad))
+    c64 = ct.astype(np.float64).transpose(1, 0, 2, 3).reshape(ct.shape[1], -1)
+    oh, ow = ct.shape[2:]
+    want, scale = (np.empty((x.shape[1], ct.shape[1], kh, kw)) for _ in range(2))
+    for ky in range(kh):
+        for kx in range(kw):
+            win = xp[:, :, ky:ky + oh, kx:kx + ow].transpose(1, 0, 2, 3).reshape(x.shape[1], -1)
+            with np.errstate(invalid="ignore"):
+                want[:, :, ky, kx], scale[:, :, ky, kx] = win @ c64.T, np.abs(win) @ np.abs(c64).T
+    return want, scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_sums_against_the_definition(case):
+    batch, cin, cout, h, w, kh, kw, pad = case
+    kernel, cts = cotangent_kernel(*case)
+    x = RNG.standard_normal((batch, cin, h, w)).astype(np.float16)
+    ct = RNG.standard_normal(cts).astype(np.float16)
+    got = device_run(kernel, [x.reshape(-1), ct.reshape(-1)], filter_bands=True)[0].reshape(cin, cout, kh, kw).astype(np.float64)
+    want, scale = reference(x, ct, kh, kw, pad)
+    # float32 sums of exact products (n terms: at most n half-ulps of the running sum), one rounding to float16
+    n = batch * cts[2] * cts[3]
+    bound = np.abs(want) * 2.0 ** -11 + scale * n * 2.0 ** -24 + 2.0 ** -25
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [24, 29])
+def test_infinities_and_nans_reach_the_taps_that_see_them(size):
+    """A pixel or a cotangent that is no finite number spoils exactly the sums it is a term of: what lies beside a row in LDS, or
+    past the end of a group of eight, is a term of none.  (Padding is a zero that is multiplied.)"""
+    case = (2, 40, 40, size, size, 3, 3, SAME(3))
+    kernel, cts = cotangent_kernel(*case)
+    x = RNG.integers(-3, 4, (2, 40, size, size)).astype(np.float16)
+    ct = RNG.integers(1, 4, cts).astype(np.float16)
+    for c, (y, xx) in enumerate([(0, 0), (0, size - 1), (size - 1, 0), (size - 1, size - 1), (7, 8), (8, 7), (5, size - 1), (11, 0), (0, 12)]):
+        x[c % 2, c, y, xx] = [np.inf, -np.inf, np.nan][c % 3]
+    ct[0, 37, 0, 0], ct[1, 38, size - 1, size - 1] = np.inf, np.nan
+    got = device_run(kernel, [x.reshape(-1), ct.reshape(-1)], filter_bands=True)[0].reshape(40, 40, 3, 3).astype(np.float64)
+    want, _ = reference(x, ct, 3, 3, SAME(3))
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)].astype(np.float16).astype(np.float64))
