@@ -86,19 +86,30 @@ def _table(cond, idx, k, tap):
 
 
 def match_wgrad(g: dict, exps: dict) -> Optional[dict]:
-    """Geometry of the window walk and the operands' tags, or None."""
-    if g["dtype"] != DType.Float16 or len(g["batch"]) != 1 or not (g.get("a_gather") or g.get("b_gather")):
-        return None
-    T, K = g["batch"][0][0], g["K"]
-    if T < 2:
+    """Geometry of the window walk and the operands' tags, or None.  The taps are the batch axis, or (`joined`) the image
+    operand's rows are channel * taps + tap."""
+    if g["dtype"] != DType.Float16 or len(g["batch"]) > 1:
         return None
     for img, ct in (("a", "b"), ("b", "a")):
         if not g.get(img + "_gather"):
             continue
-        found = _match(T, K, exps[img], exps[ct], g["M"] if img == "a" else g["N"], g["N"] if img == "a" else g["M"])
-        if found is not None:
-            return dict(found, img=img, ct=ct)
+        C, O = (g["M"], g["N"]) if img == "a" else (g["N"], g["M"])
+        forms = [(g["batch"][0][0], C, exps[img], False)] if g["batch"] else _split_rows(exps[img], C)
+        for T, channels, image, joined in forms:
+            found = _match(T, g["K"], image, exps[ct], channels, O) if T > 1 else None
+            if found is not None:
+                return dict(found, img=img, ct=ct, joined=joined)
     return None
+
+
+def _split_rows(image: AluExp, rows: int):
+    """Ways to read the image operand's rows as channel * T + tap: (T, channels, the operand with `row` the channel and `b0` the
+    tap, True)."""
+    divisors = {int(x.src[1].arg) for x in image.collect(lambda x: x.op == AluOp.Idiv and x.src[1].op == AluOp.Const)}
+    for T in sorted(divisors, reverse=True):
+        if 1 < T < rows and rows % T == 0:
+            row = AluExp.add(AluExp.mul(AluExp.special(DType.Int32, "row", rows // T), AluExp.i32(T)), AluExp.special(DType.Int32, "b0", T))
+            yield T, rows // T, image.rewrite(lambda n, row=row: row if n.op == AluOp.Special and n.arg[0] == "row" else None).reduceExactIndex().simplify(), True
 
 
 def _match(T: int, K: int, image: AluExp, cotangent: AluExp, C: int, O: int) -> Optional[dict]:
@@ -215,9 +226,9 @@ def find_wgrad(kernel, t, g: dict) -> Optional[dict]:
     [8,256,14,14] 256 91.6 -> 15, [16,128,28,28] 128 34 -> 18, [3,32,28,28] 64 5x5 22.6 -> 10.5.  Odd sizes and few channels, which
     went element by element: [6,72,40,40] 72 439 -> 15, [2,64,57,57] 64 197 -> 11.5, [32,16,56,56] 16 1937 -> 29.  Below the line the
     differences are within a microsecond of a launch ([8,24,9,9] 40 8.9 and 10.9, [1,64,12,12] 64 9.9 and 7.3)."""
-    if g["dtype"] != DType.Float16 or len(g["batch"]) != 1 or not (g.get("a_gather") or g.get("b_gather")):
+    if g["dtype"] != DType.Float16 or len(g["batch"]) > 1 or not (g.get("a_gather") or g.get("b_gather")):
         return None
-    if g["M"] * g["N"] * g["batch"][0][0] * g["K"] < WGRAD_WORK:
+    if g["M"] * g["N"] * (g["batch"][0][0] if g["batch"] else 1) * g["K"] < WGRAD_WORK:
         return None
     exps = operand_exps(kernel, t, g)
     m = match_wgrad(g, exps) if exps is not None else None
@@ -240,11 +251,12 @@ def gen_wgrad(kernel, g: dict, w: dict, numerics: str, name: str, params: str, n
 
     aligned = all(v % 8 == 0 for v in (w["W"], w["OW"], w["SC"], w["SB"], w["CTO"], w["CTB"], w["IMG_OFF"], w["CT_OFF"]))
     image_rows = w["img"] == "a"
+    c_row = f"c * {w['T']} + tap" if w["joined"] else "c"
     src = src_options + _prelude(numerics) + fill(template("wgrad_f16.hip.inc"), dict(
         {k: w[k] for k in ("C", "O", "W", "H", "OW", "OH", "KW", "KY", "GROUPS", "PH", "PW", "SC", "SB", "CTO", "CTB", "R", "NB", "IC", "PI", "PC", "IMG_OFF", "CT_OFF")},
         SLICES=w["slices"], ALIGN=16 if aligned else 2, EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, IMG_PTR=names[g["gid_" + w["img"]]],
-        CT_PTR=names[g["gid_" + w["ct"]]], ROW="c" if image_rows else "o", COL="o" if image_rows else "c",
-        C_SM=g["c_sm"], C_SN=g["c_sn"], C_ST=g["batch"][0][3], OUT_T=out_t, EPILOGUE_PARAMS=epi_params, EPILOGUE_ARGS=epi_args))
+        CT_PTR=names[g["gid_" + w["ct"]]], ROW=c_row if image_rows else "o", COL="o" if image_rows else c_row,
+        C_SM=g["c_sm"], C_SN=g["c_sn"], C_ST=0 if w["joined"] else g["batch"][0][3], B0="0" if w["joined"] else "tap", OUT_T=out_t, EPILOGUE_PARAMS=epi_params, EPILOGUE_ARGS=epi_args))
     args = [("in", i) for i in range(kernel.nargs)] + [("out", 0)]
     pieces, scratch = w["tiles"] * w["KY"] * w["KW"] * 256, []
     steps = [LaunchStep(name, (w["tiles"] * w["slices"], 1, 1), (256, 1, 1), 0, args)]

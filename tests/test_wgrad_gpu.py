@@ -3,7 +3,7 @@ sums against the definition, tap by tap."""
 import numpy as np
 import pytest
 
-from gpu_util import device_run
+from gpu_util import WARM_ONLY, backend, device_run
 from jaxjs_hip import DType, jit as J
 from jaxjs_hip.convolution import ConvParams
 from jaxjs_hip.jit import ShapedArray
@@ -50,7 +50,23 @@ def test_plan_covers_the_case(case):
     info = generate(kernel, filter_bands=True).info
     assert "wgrad" in info, info
     assert "wgrad" not in generate(kernel).info  # by itself it keeps the general templates
-    assert plan_units(cotangent_program(*case)[0])[0].options == dict(filter_bands=True)
+    units = plan_units(cotangent_program(*case)[0])
+    assert [u.options for u in units] == [dict(filter_bands=True)]  # and the exchange of its channels goes with it
+    joined = generate(units[0].source, filter_bands=True).info
+    assert joined["wgrad"] == info["wgrad"]
+
+
+def test_an_exchange_that_is_more_than_one_stays_a_launch():
+    """What reads the cotangent besides its own transpose, or reads it at other positions, is not joined."""
+    case = CASES[0]
+    _, cts = cotangent_program(*case)
+    p = ConvParams(0, [1, 1], list(case[7]), [1, 1], [1, 1])
+    avals = [ShapedArray((case[0], case[1], case[3], case[4]), DType.Float16), ShapedArray(cts, DType.Float16)]
+    ws = [case[2], case[1], case[5], case[6]]
+    flipped = J.jit(lambda x, ct: J.flip(J.convTransposeRhs(x, ct, ws, p), [2]), avals)
+    assert len(plan_units(flipped)) == 2
+    scaled = J.jit(lambda x, ct: J.convTransposeRhs(x, ct, ws, p).mul(J.convTransposeRhs(x, ct, ws, p)), avals)
+    assert all(u.options == dict(filter_bands=True) or u.options == {} for u in plan_units(scaled))
 
 
 @pytest.mark.parametrize("kw", [dict(stride=2), dict(dilation=2), dict(dtype=DType.Float32), dict(w=7), dict(kh=1), dict(batch=1, cin=16, cout=16)], ids=str)
@@ -88,6 +104,25 @@ def test_sums_against_the_definition(case):
     n = batch * cts[2] * cts[3]
     bound = np.abs(want) * 2.0 ** -11 + scale * n * 2.0 ** -24 + 2.0 ** -25
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES[:5] + CASES[-1:], ids=str)
+def test_a_program_gets_the_filters_own_order(case):
+    batch, cin, cout, h, w, kh, kw, pad = case
+    prog, cts = cotangent_program(*case)
+    x = RNG.standard_normal((batch, cin, h, w)).astype(np.float16)
+    ct = RNG.standard_normal(cts).astype(np.float16)
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    be = backend()
+    slots = [be.malloc(v.nbytes, np.ascontiguousarray(v).tobytes()) for v in (x, ct)]
+    outs = prog.execute(be, slots, prog.prepare(be))
+    got = np.frombuffer(be.readSync(outs[0]), np.float16).reshape(cout, cin, kh, kw).astype(np.float64)
+    for s in slots + outs:
+        be.decRef(s)
+    want, scale = (v.transpose(1, 0, 2, 3) for v in reference(x, ct, kh, kw, pad))
+    assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + scale * batch * cts[2] * cts[3] * 2.0 ** -24 + 2.0 ** -25)
 
 
 @pytest.mark.gpu
