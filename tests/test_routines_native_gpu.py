@@ -244,6 +244,20 @@ def test_fft_in_passes(shape, dt):
         assert "passes" in ks.info and err < {"float32": 5e-7, "float64": 1e-14, "float16": 2e-3}[np.dtype(dt).name], (ks.info, err)
 
 
+@pytest.mark.parametrize("shape", [(1, 6), (3, 9), (2, 10), (5, 12), (1, 14), (7, 15), (2, 90), (3, 140 * 15), (1, 10 * 12 * 14 * 15), (2, 9 ** 5)], ids=str)
+def test_fft_butterflies_made_of_two_smaller_ones(shape):
+    """Every such size first, last and alone; more butterflies than threads, with twiddles read ahead for the first of them."""
+    from jaxjs_hip.routinegen import FFT_NESTED, _fft_radices
+    assert any(r in FFT_NESTED for r in _fft_radices(shape[-1]) or ()) or shape[-1] > 8192
+    re, im = RNG.standard_normal(shape).astype(F32), RNG.standard_normal(shape).astype(F32)
+    for inverse in (False, True):
+        got, ks = R.run_gpu(R.fft(re, im, inverse), [re, im])
+        z = re.astype(np.complex128) + 1j * im.astype(np.complex128)
+        want = np.fft.ifft(z) if inverse else np.fft.fft(z)
+        # a rounding to float32 a stage, of values as large as the result's, over a handful of stages
+        assert np.abs(got[0].astype(np.complex128) + 1j * got[1] - want).max() <= 5e-7 * np.abs(want).max(), ks.info
+
+
 def test_fft_factor_orders_and_validation():
     re, im = RNG.standard_normal((2, 60)).astype(F32), RNG.standard_normal((2, 60)).astype(F32)
     for factors in ([4, 3, 5], [5, 3, 4], [2, 2, 15], [60]):
