@@ -288,6 +288,14 @@ def plan_rows(chain: RowChain) -> Optional[dict]:
     return dict(V=V, T=T, iters=iters, full=full, block=block, grid=-(-chain.R * T // block))
 
 
+def _fold_text(op: AluOp, dtype: DType, halves: bool) -> str:
+    """One step of a fold.  float32 maxima and minima are the instruction that lets a NaN through (`jh_row_max`); where a
+    chain has float16 values this compiler's instruction selection can fail on it, and the select around `fmax` stays."""
+    if dtype == DType.Float32 and op in (AluOp.Max, AluOp.Min) and not halves:
+        return f"jh_row_{'max' if op == AluOp.Max else 'min'}(a, b)"
+    return _reduce_text(op, dtype)
+
+
 def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSource:
     p = plan_rows(chain)
     V, T = p["V"], p["T"]
@@ -347,7 +355,7 @@ def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSou
             if what not in folds:
                 lane_body, value = _lane_accumulate(body, lane_loads, st.exp, re, acc_t, f"a{j}")
                 value = value.replace("JH_REDUCE(", f"jh_op{j}(", 1) if value.startswith("JH_REDUCE(") else value
-                text.append(f"  const auto jh_op{j} = [](const {acc_t} a, const {acc_t} b) {{ return ({acc_t})({_reduce_text(re.op, re.dtype)}); }};")
+                text.append(f"  const auto jh_op{j} = [](const {acc_t} a, const {acc_t} b) {{ return ({acc_t})({_fold_text(re.op, re.dtype, halves)}); }};")
                 text.append(f"  {acc_t} a{j} = {const_literal(re.dtype, re.identity)};")
                 text += loop + [hoisted, "#pragma unroll", "      for (int lane = 0; lane < JH_V; ++lane) {", "        const int ridx = c0 + lane;", "        (void)ridx;",
                                 lane_body, f"        a{j} = {value};", "      }"] + end

@@ -76,3 +76,33 @@ def test_an_elementwise_kernel_in_a_contractions_epilogue(dtype, mnk):
     arrays = [rng.standard_normal((m, k)).astype(t), (rng.standard_normal((k, n)) * k ** -0.5).astype(t), rng.standard_normal(n).astype(t)]
     prog = J.jit(lambda x, w, b: L.gelu(L.matmul(x, w).add(b)), [ShapedArray(a.shape, dtype) for a in arrays])
     check(prog, arrays, dtype == DType.Float16, chained=False)
+
+
+@pytest.mark.parametrize("cols", [2, 37, 257, 1024, 4097])
+@pytest.mark.parametrize("op", ["max", "min"])
+def test_largest_and_smallest_of_rows_with_values_that_are_no_ordinary_numbers(op, cols):
+    """A NaN at any place is the result, infinities are values, and -0 is below +0: bit for bit, on every lane of the row."""
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((9, cols)).astype(np.float32)
+    x[0, 0] = x[1, -1] = x[2, cols // 2] = np.nan
+    x[3, cols // 3], x[4, cols // 3] = np.inf, -np.inf
+    x[5], x[6] = np.copysign(0.0, -1), 0.0
+    x[7], x[7, -1], x[8], x[8, 0] = np.copysign(0.0, -1), 0.0, -np.inf, np.nan
+
+    def f(v):
+        m = getattr(v, op)(-1, keepdims=True)
+        return [m.reshape([9]), v.sub(m)]
+    prog = J.jit(f, [ShapedArray(x.shape, DType.Float32)])
+    assert [type(u.source) for u in plan_units(prog)] == [RowChain]
+    if WARM_ONLY:
+        check(prog, [x], False)
+    m, y = run_program(backend(), prog, [x])
+    m = np.asarray(m).reshape(9)
+    # the order of the operation: -0 below +0, anything below a NaN
+    key = lambda v: (1, 0.0, 0) if np.isnan(v) else (0, float(v), 0 if np.signbit(v) else 1)  # noqa: E731
+    low = lambda v: (0, 0.0, 0) if np.isnan(v) else (1, float(v), 0 if np.signbit(v) else 1)  # noqa: E731
+    want = np.array([max(r, key=key) if op == "max" else min(r, key=low) for r in x], np.float32)
+    np.testing.assert_array_equal(m, want)
+    np.testing.assert_array_equal(np.signbit(m[5:8]), np.signbit(want[5:8]))
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(np.asarray(y).reshape(x.shape), x - want[:, None])
