@@ -73,8 +73,23 @@ def _shape(g: dict, o: dict) -> Optional[dict]:
             work = max(1.0, count / tuner.CU_COUNT) * cycles / 2400
             again = row_tiles * o["w_bytes"] / 10e6 if o["w_bytes"] > 4 << 20 else 0.0
             if row_tiles <= 65535 and (best is None or 2.6 + work + again < best["us"]):
-                best = dict(us=2.6 + work + again, work=work, MT=MT, VN=VN, waves=waves)
+                best = dict(us=2.6 + work + again, work=work, count=count, MT=MT, VN=VN, waves=waves)
     return best
+
+
+def _slices(steps: int, count: int) -> int:
+    """Workgroups that share the k steps of each of `count` tiles (folded inside the launch by the last of them).
+
+    A long k axis in a few workgroups is bound by what one CU can have in flight and by its matrix instructions, and the fold
+    costs about 1.3 us, so the axis is cut where a slice keeps 24 steps of 64 bytes (64 in two slices, 32 in eight) and every
+    slice's workgroup still has a CU to itself.  microseconds with the weights in the L2 / from beyond it: float16 8 x 768 x
+    3072 4.8 / 7.5 whole, 4.4 / 5.1 in four slices, 24 x 512 x 4096 7.1 / 10.7 and 5.1 / 6.2; float32 8 x 512 x 2048 7.1 / 8.3
+    and 4.6 / 5.1, 64 x 128 x 4096 14.8 / 15.1 and in eight 5.9 / 5.8, 64 x 512 x 4096 (128 tiles) 15.4 / 15.9 and in two
+    10.3 / 10.8.  Shorter axes lose from the L2 what they win from memory (float16 2 x 1024 x 2048 3.3 / 6.0 and 4.1 / 5.1)."""
+    for slices, least in ((8, 256), (4, 96), (2, 128)):
+        if steps >= least and count * slices <= tuner.CU_COUNT:
+            return slices
+    return 1
 
 
 def _tile_launch(g: dict, o: dict, tile: dict) -> dict:
@@ -133,9 +148,11 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
             return None
     # Steps in equal shares for the waves, in equal batches of what the registers of a full workgroup hold in flight.
     MT, VN, steps = best["MT"], best["VN"], max(1, o["K"] // (64 // o["eb"]))
-    share = -(-steps // best["waves"])
+    slices = _slices(steps, best["count"])
+    waves = min(best["waves"], -(-steps // slices))
+    share = -(-steps // (waves * slices))
     most = max(1, (104 - 4 * MT * VN) // (4 * (MT + VN)))
-    return dict(R=o["R"], MT=MT, C=o["C"], short=o["short"], wide=o["wide"], along_k=o["along_k"], VN=VN, waves=-(-steps // share),
+    return dict(R=o["R"], MT=MT, C=o["C"], short=o["short"], wide=o["wide"], along_k=o["along_k"], VN=VN, waves=-(-steps // (share * slices)), slices=slices,
                 batch=-(-share // -(-share // most)), nbatch=o["nbatch"], row=o["row"])
 
 
@@ -144,7 +161,7 @@ def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_ar
     s, w = p["short"], p["wide"]
     text = fill(template("gemm_few.hip.inc"), dict(
         F32=1 if g["dtype"] == DType.Float32 else 0, R=p["R"], MT=p["MT"], C=p["C"], K=g["K"], WK=1 if p["along_k"] else 0, VN=p["VN"],
-        WAVES=p["waves"], BATCH=p["batch"], EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
+        WAVES=p["waves"], BATCH=p["batch"], SLICES=p["slices"], EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
         X_ROW=g[p["row"][s]], W_ROW=g[p["row"][w]], W_K=g[w + "_sk"], ROW="rr" if s == "a" else "c", COL="c" if s == "a" else "rr", C_SM=g["c_sm"], C_SN=g["c_sn"],
         EPILOGUE_ARGS=epi_args))
-    return text, (-(-p["C"] // (16 * p["VN"])), p["nbatch"], -(-p["R"] // (16 * p["MT"]))), (64 * p["waves"], 1, 1)
+    return text, (-(-p["C"] // (16 * p["VN"])) * p["slices"], p["nbatch"], -(-p["R"] // (16 * p["MT"]))), (64 * p["waves"], 1, 1)

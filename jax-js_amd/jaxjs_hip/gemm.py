@@ -652,14 +652,19 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
             lines.append(f"    jh_b{k} = rem % {size}; rem /= {size};")
             lines.append(f"    a_base += (long long)jh_b{k} * {sa}ll; b_base += (long long)jh_b{k} * {sb}ll; c_base += (long long)jh_b{k} * {sc}ll;")
         lines.append("  }")
+        if few["slices"] > 1:
+            params += ", float* __restrict__ jh_part, unsigned* __restrict__ jh_count"
         text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "")
         need = _min_bytes(t.epilogue)
         for tg in ("a", "b"):
             need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * byteWidth(g["dtype"]))
-        step = LaunchStep(name, grid, block, 0, [("in", i) for i in range(kernel.nargs)] + [("out", 0)])
-        return KernelSource([src_options + _prelude(numerics) + text], [step], [], "gemm", need,
-                            dict(few=True, direct_lds=False, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0], waves=few["waves"], columns=16 * few["VN"],
-                                 along_k=few["along_k"], splitk=1))
+        args, scratch = [("in", i) for i in range(kernel.nargs)] + [("out", 0)], []
+        if few["slices"] > 1:  # the slices' sums, and a counter for each tile
+            args += [("scratch", 0), ("scratch", 1)]
+            scratch = [math.prod(grid) * 256 * few["MT"] * few["VN"] * 4, math.prod(grid) // few["slices"] * 4]
+        return KernelSource([src_options + _prelude(numerics) + text], [LaunchStep(name, grid, block, 0, args)], scratch, "gemm", need,
+                            dict(few=True, direct_lds=False, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0] // few["slices"], waves=few["waves"],
+                                 columns=16 * few["VN"], along_k=few["along_k"], splitk=few["slices"]), zeroed_scratch=[1] if scratch else [])
 
     # Element loaders for gather operands: the operand's lowered expression (masked load through its view
     # chain) with the flat output index rebuilt from (tile row, batch coordinates) and ridx = k.

@@ -461,6 +461,26 @@ def test_gemm_too_small_for_tiles(dt, M, N, K, bt):
     np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), want, err_msg=str(ks.info))
 
 
+@pytest.mark.parametrize("dt,M,N,K,bt,slices", [
+    (DType.Float16, 8, 768, 3072, False, 4), (DType.Float16, 3, 130, 3075, False, 4), (DType.Float16, 16, 513, 4100, False, 4), (DType.Float16, 24, 1024, 4096, True, 2),
+    (DType.Float16, 24, 130, 8200, False, 8), (DType.Float16, 70, 64, 3100, True, 4), (DType.Float16, 8, 1024, 3040, False, 1),
+    (DType.Float32, 8, 512, 2049, False, 4), (DType.Float32, 64, 128, 4096, False, 8), (DType.Float32, 33, 300, 2049, True, 4), (DType.Float32, 64, 500, 2060, True, 2),
+], ids=lambda v: v.value if isinstance(v, DType) else str(v))
+def test_gemm_too_small_for_tiles_with_its_k_axis_in_slices(dt, M, N, K, bt, slices):
+    """Slices of unequal numbers of steps, the ragged step in one of them, ragged tiles; launches behind one another find
+    the counters as they need them."""
+    npdt = np.float16 if dt == DType.Float16 else np.float32
+    A, B = RNG.integers(-2, 3, (M, K)).astype(npdt), RNG.integers(-2, 3, (K, N)).astype(npdt)
+    A[:, RNG.random(K) < 0.8] = 0  # keep every sum an exact float16
+    k, arrays = matmulKernel(M, N, K, dt, b_transposed=bt), [A, np.ascontiguousarray(B.T) if bt else B]
+    want = A.astype(np.float32) @ B.astype(np.float32)
+    assert np.abs(want).max() <= 2048
+    for _ in range(3):
+        got, ks = device_run(k, arrays)
+        assert ks.info.get("few") and ks.info["splitk"] == slices, ks.info
+        np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), want, err_msg=str(ks.info))
+
+
 def test_single_rows_and_small_operands_stay_with_the_reduction_classes():
     from jaxjs_hip.tuner import tuneHip
     for M, N, K in ((1, 14336, 4096), (14336, 1, 4096), (5, 300, 700), (16, 64, 64), (8, 100, 2048)):
