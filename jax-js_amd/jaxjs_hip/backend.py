@@ -34,7 +34,7 @@ from .alu import Kernel, byteWidth
 from .errors import HipRuntimeError, SlotError, UnsupportedRoutineError
 from .kernelgen import NUMERICS, KernelSource, generate
 from .routine import Routine
-from .rowchain import RowChain, gen_rows
+from .composite import Composite
 from .runtime import Device, check, compile_source, pack_args
 from .schedule import Schedule
 
@@ -404,13 +404,13 @@ class HipBackend:
         return await self._prepare_async(key, routine, lambda: generateRoutine(routine, self.numerics))
 
     def prepareSync(self, source, **tune_opts) -> Executable:
-        """`prepareKernelSync` / `prepareRoutineSync` / a chain of Kernels over the same rows, by the source's type."""
+        """`prepareKernelSync` / `prepareRoutineSync` / a source of several dispatches in one launch, by the source's type."""
         if isinstance(source, Kernel):
             return self.prepareKernelSync(source, **tune_opts)
         if isinstance(source, Routine):
             return self.prepareRoutineSync(source)
         key = (source.key(), self.numerics)
-        return self._cached(key) or self._remember(key, self._build(source, gen_rows(source, self.numerics)))
+        return self._cached(key) or self._remember(key, self._build(source, source.generate(self.numerics)))
 
     def scheduleProgram(self, prog) -> Schedule:
         """The schedule of a jit program, cached by the program's structure like the executables it consists of."""
@@ -424,18 +424,19 @@ class HipBackend:
             self._programs.popitem(last=False)
         return found
 
-    def _dispatch_chain(self, exe: Executable, ins, outs) -> None:
-        chain, prep = exe.source, exe.data
+    def _dispatch_composite(self, exe: Executable, ins, outs) -> None:
+        source, prep = exe.source, exe.data
+        sizes = source.output_bytes()
         if prep.released:
             raise ValueError("executable was released (evicted from the backend's cache): prepare it again")
-        if len(ins) != len(chain.inputs) or len(outs) != len(chain.outputs):
-            raise ValueError(f"the chain takes {len(chain.inputs)} inputs and {len(chain.outputs)} outputs")
+        if len(ins) != len(source.inputs) or len(outs) != len(sizes):
+            raise ValueError(f"the launch takes {len(source.inputs)} inputs and {len(sizes)} outputs")
         for gid, need in prep.ks.min_input_bytes.items():
             if ins[gid]["size"] < need:
-                raise ValueError(f"input {gid} holds {ins[gid]['size']} bytes, the chain addresses {need}")
-        for s, j in zip(outs, chain.outputs):
-            if s["size"] < chain.stages[j].kernel.bytes:
-                raise ValueError(f"output slot holds {s['size']} bytes, the chain writes {chain.stages[j].kernel.bytes}")
+                raise ValueError(f"input {gid} holds {ins[gid]['size']} bytes, the launch addresses {need}")
+        for s, size in zip(outs, sizes):
+            if s["size"] < size:
+                raise ValueError(f"output slot holds {s['size']} bytes, the launch writes {size}")
         self._launch_steps(prep, ins, outs)
 
     def _launch_steps(self, prep: _Prepared, ins, outs) -> None:
@@ -527,8 +528,8 @@ class HipBackend:
         if isinstance(exe.source, Routine):
             self._dispatch_routine(exe, ins, outs)
             return
-        if isinstance(exe.source, RowChain):
-            self._dispatch_chain(exe, ins, outs)
+        if isinstance(exe.source, Composite):
+            self._dispatch_composite(exe, ins, outs)
             return
 
         kernel: Kernel = exe.source

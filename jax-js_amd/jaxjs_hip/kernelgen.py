@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import os
 from dataclasses import dataclass, field
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, Optional, Sequence, Tuple
 
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
 from .codegen import CTYPE, SOURCE_OPTION, STORAGE_CTYPE, HipExpCodegen, const_literal, strip_parens
@@ -275,24 +275,57 @@ def generate(kernel: Kernel, numerics: str = "wasm", tune: Optional[TuneResult] 
     raise ValueError(f"unknown kernel class {t.klass}")
 
 
-def _gen_map(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelSource:
-    V, block, grid = t.params["V"], t.params["block"], t.params["grid"]
-    used = _used_args(kernel.nargs, t.exp)
+def _map_body(kernel: Kernel, t: TuneResult, numerics: str, space: str) -> str:
+    """`jh_map` of one elementwise Kernel, in a namespace of its own."""
     out_t = STORAGE_CTYPE[kernel.dtype]
+    used = _used_args(kernel.nargs, t.exp)
     params, args = _params(used, out_t)
-    body = _Body(t.exp, args, IDENT, "gidx", "g0", V, t.vector_loads, numerics, "  ")
+    body = _Body(t.exp, args, IDENT, "gidx", "g0", t.params["V"], t.vector_loads, numerics, "  ")
     load_fields, hoisted, loads = body.batched()
     body.indent = "        "
     lane_body, lane_value = body.lanes(loads)
     scalar_body, scalar_value = body.scalar("    ")
-    src = _compile_options_of(kernel, t) + _prelude(numerics) + fill(template("map.hip.inc"), dict(
-        SIZE=kernel.size, V=V, BLOCK=block, UNROLL=t.params.get("unroll", 1), NT_STORE=t.params.get("nt_store", 0), NAME=name, PARAMS=params, OUT_T=out_t,
-        LOAD_FIELDS=load_fields, LOAD_PARAMS=_in_params(used)[0], LOAD_ARGS=_in_params(used)[1],
+    return fill(template("map.hip.inc"), dict(
+        SPACE=space, SIZE=kernel.size, V=t.params["V"], BLOCK=t.params["block"], UNROLL=t.params.get("unroll", 1), NT_STORE=t.params.get("nt_store", 0),
+        PARAMS=params, OUT_T=out_t, LOAD_FIELDS=load_fields, LOAD_PARAMS=_in_params(used)[0], LOAD_ARGS=_in_params(used)[1],
         VECTOR_LOADS=hoisted, LANE_BODY=lane_body, LANE_VALUE=lane_value,
         SCALAR_BODY=scalar_body, SCALAR_VALUE=scalar_value))
-    step = LaunchStep(name, (grid, 1, 1), (block, 1, 1), 0,
+
+
+def _gen_map(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelSource:
+    params, names = _params(_used_args(kernel.nargs, t.exp), STORAGE_CTYPE[kernel.dtype])
+    src = _compile_options_of(kernel, t) + _prelude(numerics) + _map_body(kernel, t, numerics, "jh_0") + (
+        f"extern \"C\" __global__ __launch_bounds__({t.params['block']}) void {name}({params}) {{\n"
+        f"  jh_0::jh_map({', '.join(names + ['out'])}, (int)blockIdx.x, (int)gridDim.x);\n}}\n")
+    step = LaunchStep(name, (t.params["grid"], 1, 1), (t.params["block"], 1, 1), 0,
                       [("in", i) for i in range(kernel.nargs)] + [("out", 0)])
     return KernelSource([src], [step], [], "map", _min_bytes(t.exp), dict(t.params))
+
+
+def gen_maps(kernels: Sequence[Kernel], numerics: str, name: str = "jh_maps") -> KernelSource:
+    """Elementwise Kernels (of class "map") side by side in one launch: the first one's workgroups, then the next one's.
+    Inputs are numbered through, each Kernel has an output."""
+    tuned = [tuneHip(k) for k in kernels]
+    options, bodies, params, args, need = "", [], [], [], {}
+    calls, first, n_in = [], 0, 0
+    for k, (kernel, t) in enumerate(zip(kernels, tuned)):
+        options = _compile_options_of(kernel, t) or options
+        bodies.append(_map_body(kernel, t, numerics, f"jh_{k}"))
+        used = _used_args(kernel.nargs, t.exp)
+        names = [f"in{n_in + i}" for i in range(kernel.nargs)]
+        params += [f"const {STORAGE_CTYPE[d or DType.Float32]}* __restrict__ {n}" for d, n in zip(used, names)] + [f"{STORAGE_CTYPE[kernel.dtype]}* __restrict__ out{k}"]
+        args += [("in", n_in + i) for i in range(kernel.nargs)] + [("out", k)]
+        need.update({n_in + i: b for i, b in _min_bytes(t.exp).items()})
+        grid = t.params["grid"]
+        call = f"jh_{k}::jh_map({', '.join(names + [f'out{k}'])}, block{f' - {first}' if first else ''}, {grid});"
+        calls.append(f"  {'else ' if k else ''}{f'if (block < {first + grid}) ' if k + 1 < len(kernels) else ''}{call}")
+        first, n_in = first + grid, n_in + kernel.nargs
+    block = max(t.params["block"] for t in tuned)
+    assert all(t.klass == "map" and t.params["block"] == block for t in tuned)
+    src = options + _prelude(numerics) + "".join(bodies) + (
+        f"extern \"C\" __global__ __launch_bounds__({block}) void {name}({', '.join(params)}) {{\n"
+        "  const int block = (int)blockIdx.x;\n" + "\n".join(calls) + "\n}\n")
+    return KernelSource([src], [LaunchStep(name, (first, 1, 1), (block, 1, 1), 0, args)], [], "maps", need, dict(kernels=len(kernels), grid=first))
 
 
 def _gen_map_transposed(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelSource:

@@ -14,6 +14,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 from .alu import AluExp, AluOp, DType, Kernel, byteWidth
 from .codegen import CTYPE, SOURCE_OPTION, STORAGE_CTYPE, _fits_i32, const_literal
+from .composite import Composite
 from .kernelgen import IDENT, KernelSource, LaunchStep, _Body, _lane_accumulate, _prelude, _reduce_text, fill, template
 from . import tuner
 
@@ -102,7 +103,7 @@ class Stage:
 
 
 @dataclass
-class RowChain:
+class RowChain(Composite):
     R: int
     C: int
     stages: List[Stage]
@@ -112,6 +113,18 @@ class RowChain:
 
     def key(self) -> tuple:
         return ("rows", self.R, self.C, tuple((s.kernel.key(), tuple(s.refs)) for s in self.stages), tuple(self.outputs))
+
+    def output_bytes(self) -> List[int]:
+        return [self.stages[j].kernel.bytes for j in self.outputs]
+
+    def generate(self, numerics: str) -> KernelSource:
+        return gen_rows(self, numerics)
+
+    def extents(self) -> List[int]:
+        return [self.R, self.C]
+
+    def label(self):
+        return "Rows", [("kernels", str(len(self.stages))), ("size", str(self.R * self.C))]
 
 
 def lower_stage(kernel: Kernel, R: int, C: int) -> Optional[Stage]:

@@ -16,6 +16,7 @@ from typing import Any, Dict, List, Optional, Sequence
 
 from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
+from .composite import MAPS_MOST, Maps, joins_maps
 from .errors import SlotError
 from .kernelgen import generate
 from .routine import Routine
@@ -136,6 +137,20 @@ def plan_dispatches(prog) -> List[_Dispatch]:
     return out
 
 
+def adjacent_maps(steps: Sequence[_Dispatch], k: int, view) -> int:
+    """How many dispatches from `k` on are elementwise Kernels that run side by side in one launch (see `Maps`)."""
+    n, written = 0, set()
+    while n < MAPS_MOST and k + n < len(steps):
+        d = steps[k + n]
+        if d.kernel is None or not joins_maps(d.kernel) or written & set(d.inputs):
+            break
+        if n and collect_chain(view, k + n, lambda o, last: True) is not None:
+            break  # the first of Kernels over the same rows
+        written.add(d.output)
+        n += 1
+    return n
+
+
 def plan_units(prog) -> List[Unit]:
     """The program's dispatches with runs of Kernels over the same rows joined."""
     steps = plan_dispatches(prog)
@@ -154,6 +169,13 @@ def plan_units(prog) -> List[Unit]:
             chain, n = found
             units.append(Unit(chain, chain.inputs, [steps[k + j].output for j in chain.outputs]))
             k += n
+            continue
+        together = adjacent_maps(steps, k, view)
+        if together > 1:
+            run = steps[k:k + together]
+            ids = [i for d in run for i in d.inputs]
+            units.append(Unit(Maps([d.kernel for d in run], ids), ids, [d.output for d in run]))
+            k += together
             continue
         options = dict(filter_bands=True) if s.routine is None and is_filter_cotangent(s.kernel) else {}
         units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))

@@ -14,7 +14,7 @@ from dataclasses import dataclass, field
 from typing import Callable, List, Optional, Tuple
 
 from .alu import Kernel
-from .rowchain import RowChain
+from .composite import Composite
 
 _enabled = False
 _flush: List[Callable[[], None]] = []
@@ -78,10 +78,11 @@ def traceSourceInfo(source) -> TraceInfo:
         else:
             color = "secondary"
             props.append(("reduction", f"{source.reduction.op}:{source.reduction.size}"))
-    elif isinstance(source, RowChain):
+    elif isinstance(source, Composite):
         color = "secondary"
-        label = f"Rows[{humanSize(source.R)}x{humanSize(source.C)}]"
-        props += [("kernels", str(len(source.stages))), ("size", str(source.R * source.C))]
+        name, more = source.label()
+        props += more
+        label = f"{name}[{'x'.join(humanSize(n) for n in source.extents())}]"
     else:
         color = "tertiary"
         label = str(source.name)

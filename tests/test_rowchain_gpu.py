@@ -106,3 +106,18 @@ def test_largest_and_smallest_of_rows_with_values_that_are_no_ordinary_numbers(o
     np.testing.assert_array_equal(np.signbit(m[5:8]), np.signbit(want[5:8]))
     with np.errstate(invalid="ignore"):
         np.testing.assert_array_equal(np.asarray(y).reshape(x.shape), x - want[:, None])
+
+
+@pytest.mark.parametrize("count", [2, 8, 11])
+@pytest.mark.parametrize("size", [1, 7, 1000, 262145])
+def test_elementwise_kernels_side_by_side(count, size):
+    """Sizes off the vector width, several types, more Kernels than one launch takes; a masked read; one operand for all."""
+    rng = np.random.default_rng(size)
+    arrays = [rng.standard_normal(size).astype(np.float16 if i % 3 == 2 else np.float32) for i in range(count)]
+    arrays.append(rng.integers(-9, 9, size).astype(np.int32))
+
+    def f(*a):
+        return [x.mul(float(i + 1)).add(x) if i % 2 else L.concatenate([x, x], 0) for i, x in enumerate(a[:-1])] + [a[-1].add(3)]
+    prog = J.jit(f, [ShapedArray(x.shape, {"f": DType.Float32, "e": DType.Float16, "i": DType.Int32}[x.dtype.char]) for x in arrays])
+    assert [len(u.outputs) for u in plan_units(prog)] == {2: [3], 8: [8, 1], 11: [8, 4]}[count]
+    check(prog, arrays, True, chained=False)

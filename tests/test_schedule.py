@@ -342,3 +342,26 @@ def test_a_call_that_runs_out_of_memory_gives_back_what_it_took(room):
     with pytest.raises(MemoryError):
         schedule.run([1, 2, 3])
     assert list(be._slots) == [1, 2, 3] and sum(len(free) for free in be._pool.values()) == room
+
+
+def test_elementwise_kernels_share_a_launch_until_one_reads_another():
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.composite import Maps
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import plan_units
+
+    def f(a, b, c):
+        p, q = a.mul(2.0), b.add(1.0)        # two results that the program returns
+        m = L.matmul(p, q)
+        r, t = m.sub(c), c.mul(3.0)
+        return [p, q, m, r, t, J.exp(r.mul(t))]
+    prog = J.jit(f, [ShapedArray((48, 48), DType.Float32)] * 3)
+    units = plan_units(prog)
+    groups = [len(u.outputs) for u in units if isinstance(u.source, Maps)]
+    assert groups and groups[0] == 2
+    for u in units:
+        if isinstance(u.source, Maps):
+            assert not set(u.inputs) & set(u.outputs) and len(u.inputs) == sum(k.nargs for k in u.source.kernels)
+    made = [o for u in units for o in u.outputs]
+    assert len(made) == len(set(made)) and set(prog.outputs) <= set(made)
