@@ -156,12 +156,21 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
                 batch=-(-share // -(-share // most)), nbatch=o["nbatch"], row=o["row"])
 
 
-def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_args: str, decode: str):
-    """(source text behind the prelude, grid, block)."""
+def chain_pitch(K: int, dtype: DType) -> int:
+    """Elements from row to row of a short operand in LDS: whole 16-byte groups, and rows start four banks apart."""
+    group = 8 if dtype == DType.Float16 else 4
+    return -(-K // group) * group + group
+
+
+def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_args: str, decode: str, rows=None):
+    """(source text behind the prelude, grid, block).  `rows`: the short operand's rows as a `RowText` with outputs of its own
+    name, made in LDS."""
     s, w = p["short"], p["wide"]
-    text = fill(template("gemm_few.hip.inc"), dict(
+    text = (rows.machinery if rows else "") + fill(template("gemm_few.hip.inc"), dict(
         F32=1 if g["dtype"] == DType.Float32 else 0, R=p["R"], MT=p["MT"], C=p["C"], K=g["K"], WK=1 if p["along_k"] else 0, VN=p["VN"],
-        WAVES=p["waves"], BATCH=p["batch"], SLICES=p["slices"], EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
+        WAVES=p["waves"], BATCH=p["batch"], SLICES=p["slices"], CHAIN=1 if rows else 0, PITCH=chain_pitch(g["K"], g["dtype"]),
+        X_NONE=f"  const jh_val* const {names[g['gid_' + s]]} = nullptr;  // (the epilogue's parameters name every operand)" if rows else "",
+        CHAIN_LOADS=rows.loads if rows else "", CHAIN_STAGES=rows.stages if rows else "", EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
         X_ROW=g[p["row"][s]], W_ROW=g[p["row"][w]], W_K=g[w + "_sk"], ROW="rr" if s == "a" else "c", COL="c" if s == "a" else "rr", C_SM=g["c_sm"], C_SN=g["c_sn"],
         EPILOGUE_ARGS=epi_args))
     return text, (-(-p["C"] // (16 * p["VN"])) * p["slices"], p["nbatch"], -(-p["R"] // (16 * p["MT"]))), (64 * p["waves"], 1, 1)

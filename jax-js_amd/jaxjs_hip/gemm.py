@@ -9,10 +9,10 @@ from __future__ import annotations
 
 import math
 
-from typing import Dict, List
+from typing import Dict, List, Optional
 
 from .alu import AluExp, AluOp, DType, Kernel, byteWidth
-from .codegen import CTYPE, STORAGE_CTYPE, HipExpCodegen, strip_parens
+from .codegen import CTYPE, SOURCE_OPTION, STORAGE_CTYPE, HipExpCodegen, strip_parens
 from .kernelgen import KernelSource, LaunchStep, _Body, _min_bytes, _prelude, _used_args, epilogue_compile_options, fill, template
 from . import tuner
 from .fewgen import gen_few, plan_few
@@ -542,12 +542,22 @@ def tap_major_form(oexp: AluExp, K: int):
     return None
 
 
-def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelSource:
+def few_plan(t: TuneResult) -> Optional[dict]:
+    """The plan of the contraction `t` where the kernel for few rows or tiles takes it."""
+    g = t.gemm
+    if g is None or t.params.get("gemm_tile") or _repack_operand(g) is not None:
+        return None
+    return plan_few(g, lambda: choose_tile(g))
+
+
+def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None) -> KernelSource:
+    """`rows`: the rows of the short operand of a contraction that `few_plan` takes, made in the same launch (a `RowText` whose
+    inputs come behind the kernel's)."""
     g = t.gemm
     re = kernel.reduction
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
-    few = plan_few(g, lambda: choose_tile(g)) if not override and _repack_operand(g) is None else None
+    few = few_plan(t)
     tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g)
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
@@ -652,19 +662,28 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str) -> KernelS
             lines.append(f"    jh_b{k} = rem % {size}; rem /= {size};")
             lines.append(f"    a_base += (long long)jh_b{k} * {sa}ll; b_base += (long long)jh_b{k} * {sb}ll; c_base += (long long)jh_b{k} * {sc}ll;")
         lines.append("  }")
+        gids = list(range(kernel.nargs))
+        if rows:
+            gids.remove(g["gid_" + few["short"]])
+            params = ", ".join([f"const {STORAGE_CTYPE[used[i] or DType.Float32]}* __restrict__ {names[i]}" for i in gids] + rows.params + [f"{out_t}* __restrict__ out"])
         if few["slices"] > 1:
             params += ", float* __restrict__ jh_part, unsigned* __restrict__ jh_count"
-        text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "")
+        text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "", rows)
         need = _min_bytes(t.epilogue)
         for tg in ("a", "b"):
             need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * byteWidth(g["dtype"]))
-        args, scratch = [("in", i) for i in range(kernel.nargs)] + [("out", 0)], []
+        if rows:
+            src_options = src_options or (SOURCE_OPTION + "-fno-slp-vectorize\n" if rows.halves else "")
+            need = {k: need[i] for k, i in enumerate(gids) if i in need}
+            need.update({len(gids) + k: b for k, b in rows.need.items()})
+            gids = list(range(len(gids) + len(rows.params)))
+        args, scratch = [("in", i) for i in gids] + [("out", 0)], []
         if few["slices"] > 1:  # the slices' sums, and a counter for each tile
             args += [("scratch", 0), ("scratch", 1)]
             scratch = [math.prod(grid) * 256 * few["MT"] * few["VN"] * 4, math.prod(grid) // few["slices"] * 4]
         return KernelSource([src_options + _prelude(numerics) + text], [LaunchStep(name, grid, block, 0, args)], scratch, "gemm", need,
                             dict(few=True, direct_lds=False, M=g["M"], N=g["N"], K=K_full, nbatch=few["nbatch"], tiles=grid[0] // few["slices"], waves=few["waves"],
-                                 columns=16 * few["VN"], along_k=few["along_k"], splitk=few["slices"]), zeroed_scratch=[1] if scratch else [])
+                                 columns=16 * few["VN"], along_k=few["along_k"], splitk=few["slices"], rows=bool(rows)), zeroed_scratch=[1] if scratch else [])
 
     # Element loaders for gather operands: the operand's lowered expression (masked load through its view
     # chain) with the flat output index rebuilt from (tile row, batch coordinates) and ridx = k.

@@ -309,16 +309,29 @@ def _fold_text(op: AluOp, dtype: DType, halves: bool) -> str:
     return _reduce_text(op, dtype)
 
 
-def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSource:
-    p = plan_rows(chain)
+@dataclass
+class RowText:
+    """A chain as source text: `machinery` in front of the kernel, `loads` of the rows and `stages` inside it.  They use the names t
+    (lane of the row), gidx (row), live (whether it is stored), at (its first element) and put (its first element in the
+    outputs); inputs are in_name{i}, outputs out{stage}."""
+    machinery: str
+    loads: str
+    stages: str
+    params: List[str]
+    need: Dict[int, int]
+    halves: bool
+
+
+def row_text(chain: RowChain, p: dict, numerics: str, in_name: str = "in") -> RowText:
+    """The chain as text under plan `p` (vector width V, lanes T, iterations)."""
     V, T = p["V"], p["T"]
     types = _types(chain)
     rows, _ = _rows_held(chain)
-    params = [f"const {STORAGE_CTYPE[d or DType.Float32]}* __restrict__ in{k}" for k, d in enumerate(types)]
+    params = [f"const {STORAGE_CTYPE[d or DType.Float32]}* __restrict__ {in_name}{k}" for k, d in enumerate(types)]
     params += [f"{STORAGE_CTYPE[chain.stages[j].kernel.dtype]}* __restrict__ out{j}" for j in chain.outputs]
     halves = any(d == DType.Float16 for d in types) or any(
         e is not None and e.collect(lambda n: n.dtype == DType.Float16) for s in chain.stages for e in (s.exp, s.epilogue))
-    loop = ["#pragma unroll", "  for (int i = 0; i < JH_ITER; ++i) {", "    const int c0 = (i * JH_T + t) * JH_V;", "    if (i < JH_FULL || c0 < JH_C) {"]
+    loop = ["#pragma unroll", "  for (int i = 0; i < JH_ITER; ++i) {", "    const int c0 = (i * JH_T + t) * JH_V;", "    if (i < JH_FULL || c0 < JH_WIDTH) {"]
     end = ["    }", "  }"]
     loads: List[str] = []
     for k in rows:
@@ -330,13 +343,13 @@ def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSou
             ct = STORAGE_CTYPE[types[k]]
             # rows that this launch reads once and that are many: past the caches (see jh_vload_nt)
             kind = "jh_vload_nt" if chain.R * chain.C >= (1 << 22) else "jh_vload"
-            loads.append(f"      x{k}[i] = {kind}<{ct}, JH_V>(in{k} + at + c0);")
+            loads.append(f"      x{k}[i] = {kind}<{ct}, JH_V>({in_name}{k} + at + c0);")
         loads += end
     text: List[str] = []
     folds: Dict[tuple, str] = {}   # a fold that an earlier stage has done already
     n_folds = 0
     for j, st in enumerate(chain.stages):
-        args = [f"in{k}" if kind == "in" else "nullptr" for kind, k in st.refs]
+        args = [f"{in_name}{k}" if kind == "in" else "nullptr" for kind, k in st.refs]
         over: Dict[int, str] = {}
         for n in _loads(st):
             kind, k = st.refs[n.arg[0]]
@@ -358,7 +371,7 @@ def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSou
             text += loop + [hoisted, "#pragma unroll", "      for (int lane = 0; lane < JH_V; ++lane) {", "        const int ridx = c0 + lane;", "        (void)ridx;",
                             lane_body, f"        y{j}[i].v[lane] = ({out_t})({value});", "      }"]
             if stored:
-                text.append(f"      if (live) jh_vstore<{out_t}, JH_V>(out{j} + at + c0, y{j}[i]);")
+                text.append(f"      if (live) jh_vstore<{out_t}, JH_V>(out{j} + put + c0, y{j}[i]);")
             text += end
             continue
         if st.kind == "reduce":
@@ -383,14 +396,20 @@ def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSou
         text += [scalar_body, f"  const {out_t} y{j} = ({out_t})({value});"]
         if stored:
             text.append(f"  if (live && t == 0) out{j}[gidx] = y{j};")
-    src = (SOURCE_OPTION + "-fno-slp-vectorize\n" if halves else "") + _prelude(numerics) + fill(template("rows.hip.inc"), dict(
-        R=chain.R, C=chain.C, V=V, T=T, ITER=p["iters"], FULL=p["full"], BLOCK=p["block"], REDUCTIONS=n_folds, NAME=name, PARAMS=", ".join(params),
-        LOADS="\n".join(loads), STAGES="\n".join(x for x in text if x)))
+    machinery = fill(template("row_fold.hip.inc"), dict(C=chain.C, V=V, T=T, ITER=p["iters"], FULL=p["full"], REDUCTIONS=n_folds))
     need: Dict[int, int] = {}
     for st in chain.stages:
         for n in _loads(st):
             kind, k = st.refs[n.arg[0]]
             if kind == "in":
                 need[k] = max(need.get(k, 0), n.arg[1] * byteWidth(n.dtype))
-    step = LaunchStep(name, (p["grid"], 1, 1), (p["block"], 1, 1), 0, [("in", k) for k in range(len(types))] + [("out", i) for i in range(len(chain.outputs))])
-    return KernelSource([src], [step], [], "rows", need, dict(p, R=chain.R, C=chain.C, kernels=len(chain.stages)))
+    return RowText(machinery, "\n".join(loads), "\n".join(x for x in text if x), params, need, halves)
+
+
+def gen_rows(chain: RowChain, numerics: str, name: str = "jh_rows") -> KernelSource:
+    p = plan_rows(chain)
+    r = row_text(chain, p, numerics)
+    src = (SOURCE_OPTION + "-fno-slp-vectorize\n" if r.halves else "") + _prelude(numerics) + r.machinery + fill(template("rows.hip.inc"), dict(
+        R=chain.R, BLOCK=p["block"], NAME=name, PARAMS=", ".join(r.params), LOADS=r.loads, STAGES=r.stages))
+    step = LaunchStep(name, (p["grid"], 1, 1), (p["block"], 1, 1), 0, [("in", k) for k in range(len(_types(chain)))] + [("out", i) for i in range(len(chain.outputs))])
+    return KernelSource([src], [step], [], "rows", r.need, dict(p, R=chain.R, C=chain.C, kernels=len(chain.stages)))

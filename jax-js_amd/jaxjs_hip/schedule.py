@@ -20,7 +20,8 @@ from .composite import MAPS_MOST, Maps, joins_maps
 from .errors import SlotError
 from .kernelgen import generate
 from .routine import Routine
-from .rowchain import _tidy, collect_chain, index_form
+from .rowchain import RowChain, _tidy, collect_chain, index_form
+from .rowproduct import join_rows
 from .runtime import LaunchRef, LaunchStepC, check
 from .shape import prod, unravelAlu
 from .tuner import match_gemm
@@ -176,6 +177,15 @@ def plan_units(prog) -> List[Unit]:
             ids = [i for d in run for i in d.inputs]
             units.append(Unit(Maps([d.kernel for d in run], ids), ids, [d.output for d in run]))
             k += together
+            continue
+        product = None
+        if s.routine is None and units and isinstance(units[-1].source, RowChain) and len(units[-1].outputs) == 1:
+            rows = units[-1].outputs[0]
+            if rows in s.inputs and rows not in kept and last_read[rows] == k:
+                product = join_rows(units[-1].source, rows, s.kernel, s.inputs)
+        if product is not None:
+            units[-1] = Unit(product, product.inputs, [s.output])
+            k += 1
             continue
         options = dict(filter_bands=True) if s.routine is None and is_filter_cotangent(s.kernel) else {}
         units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))

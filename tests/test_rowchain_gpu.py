@@ -10,6 +10,7 @@ from jaxjs_hip import library as L
 from jaxjs_hip import workloads as W
 from jaxjs_hip.jit import ShapedArray
 from jaxjs_hip.rowchain import RowChain, gen_rows
+from jaxjs_hip.rowproduct import RowProduct
 from jaxjs_hip.schedule import plan_units
 from jit_util import run_program
 from oracle.backend import OracleBackend
@@ -20,7 +21,10 @@ OPS = {"softmax": lambda x: L.softmax(x, -1), "logsoftmax": lambda x: L.logSoftm
 SHAPES = [(1, 2), (3, 7), (64, 10), (5, 64), (300, 66), (2, 33, 257), (1100, 1024), (7, 4097), (3, 50257)]
 
 
-def check(prog, arrays, f16, chained=True):
+def check(prog, arrays, f16, chained=True, terms=0):
+    """`terms` of a product behind the chain: each of as many additions rounds a partial sum of up to 4 by 2^-23 at most, on either
+    side and in an order of its own, so the two differ by a random walk of 2 sqrt(terms) such steps and a few times that.  In float16 the product and the two sums
+    behind it are rounded, values of up to 4 (2^-9 apart below) that may cancel in the result: an ulp for each."""
     chains = [u.source for u in plan_units(prog) if isinstance(u.source, RowChain)]
     assert len(chains) == 1 or not chained, [type(u.source).__name__ for u in plan_units(prog)]
     if WARM_ONLY:
@@ -36,7 +40,7 @@ def check(prog, arrays, f16, chained=True):
         if g.dtype.kind in "iu":
             np.testing.assert_array_equal(g, w)
         else:
-            np.testing.assert_allclose(g.astype(np.float64), w.astype(np.float64), rtol=1e-2 if f16 else 2e-5, atol=2e-3 if f16 else 2e-6)
+            np.testing.assert_allclose(g.astype(np.float64), w.astype(np.float64), rtol=1e-2 if f16 else 2e-5, atol=2e-3 + (3 * 2.0 ** -9 if terms else 0) if f16 else 2e-6 + 8 * terms ** 0.5 * 2.0 ** -23)
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=str)
@@ -121,3 +125,35 @@ def test_elementwise_kernels_side_by_side(count, size):
     prog = J.jit(f, [ShapedArray(x.shape, {"f": DType.Float32, "e": DType.Float16, "i": DType.Int32}[x.dtype.char]) for x in arrays])
     assert [len(u.outputs) for u in plan_units(prog)] == {2: [3], 8: [8, 1], 11: [8, 4]}[count]
     check(prog, arrays, True, chained=False)
+
+
+@pytest.mark.parametrize("rows,k,n", [(2, 256, 130), (16, 100, 200), (5, 100, 333), (8, 768, 2304), (13, 333, 777), (33, 256, 260), (64, 512, 1000), (8, 2048, 512)], ids=str)
+@pytest.mark.parametrize("dtype", [DType.Float32, DType.Float16], ids=lambda d: d.value)
+@pytest.mark.parametrize("transposed", [False, True])
+def test_rows_made_in_the_launch_of_their_product(transposed, dtype, rows, k, n):
+    """Rows and columns off the tile and the vector width, more rows than a workgroup makes at once, a k axis in slices."""
+    rng, t = np.random.default_rng(k), np.float16 if dtype == DType.Float16 else np.float32
+    arrays = [rng.standard_normal((rows, k)).astype(t), (1 + 0.1 * rng.standard_normal(k)).astype(t), (0.1 * rng.standard_normal(k)).astype(t),
+              (rng.standard_normal((n, k) if transposed else (k, n)) * k ** -0.5).astype(t), rng.standard_normal(n).astype(t), rng.standard_normal((rows, n)).astype(t)]
+
+    def f(x, g, b, w, c, r):
+        return r.add(L.matmul(L.standardize(x).mul(g).add(b), L.swapaxes(w, 0, 1) if transposed else w).add(c))
+    prog = J.jit(f, [ShapedArray(a.shape, dtype) for a in arrays])
+    few = any(isinstance(u.source, RowProduct) for u in plan_units(prog))
+    assert few or transposed and k < 512, [type(u.source).__name__ for u in plan_units(prog)]  # (short rows of such weights are dot products)
+    check(prog, arrays, dtype == DType.Float16, chained=False, terms=k)
+
+
+def test_rows_that_something_else_reads_stay_a_launch_of_their_own():
+    def f(x, w, v):
+        h = L.standardize(x)
+        return [L.matmul(h, w), L.matmul(h, v)]
+    def g(x, w):
+        h = L.standardize(x)
+        return [h, L.matmul(h, w)]
+    rng = np.random.default_rng(0)
+    x, w, v = (rng.standard_normal(s).astype(np.float32) for s in ((8, 256), (256, 96), (256, 64)))
+    for fn, arrays in ((f, [x, w, v]), (g, [x, w])):
+        prog = J.jit(fn, [ShapedArray(a.shape, DType.Float32) for a in arrays])
+        assert not any(isinstance(u.source, RowProduct) for u in plan_units(prog))
+        check(prog, arrays, False, chained=False, terms=256)
