@@ -367,24 +367,54 @@ FFT_PASS_RADIX_MAX = 13       # larger prime factors: one thread per output of a
 FFT_PASS_POINTS = 8192        # points a workgroup keeps in LDS, twice (128 KiB as float pairs)
 
 
-FFT_NESTED = {6: 2, 8: 2, 9: 3, 10: 2, 12: 3, 14: 2, 15: 3, 16: 4}  # butterflies made of two smaller ones: points of the outer
+FFT_NESTED = {6: 2, 8: 2, 9: 3, 10: 2, 12: 3, 16: 4}  # butterflies made of two smaller ones: points of the outer
 
 
-def _fft_radices(L: int, double: bool = False) -> Optional[list]:
-    """L as a product of butterfly sizes up to 16, as few as possible (a stage is a round trip through LDS and a wait for
-    its twiddles), then the smallest largest and the smallest sum; None when a prime factor is too large.  In float64, where
-    a stage's results are not rounded in between, the nested butterflies of odd sizes only add roundings (10^6 points: 5.7 and
-    6.3e-16; in float32 7.2 and 6.2e-8)."""
-    sizes = [r for r in (2, 3, 4, 5, 7, 11, 13, *FFT_NESTED) if not double or r in (8, 16) or r not in FFT_NESTED]
+def _fft_radices(L: int) -> Optional[list]:
+    """L as a product of butterfly sizes, powers of two in eights and sixteens; None when a prime factor is too large."""
+    out, two = [], 0
+    while L % 2 == 0:
+        L, two = L // 2, two + 1
+    while two:  # 2^4k and 2^3k first choice; 2, 4 only for what is left
+        step = 3 if two in (3, 6, 9) else 4 if two >= 4 else two
+        out.append(1 << step)
+        two -= step
+    for p in (3, 5, 7, 11, 13):
+        while L % p == 0:
+            out.append(p)
+            L //= p
+    return out if L == 1 else None
+
+
+def _fft_fewest(L: int) -> list:
+    """L as a product of as few butterfly sizes as possible, then the smallest largest and the smallest sum."""
     best = {1: (0, 0, 0, [])}
     for n in (d for d in range(2, L + 1) if L % d == 0):
-        for r in sizes:
+        for r in (2, 3, 4, 5, 7, 11, 13, *FFT_NESTED):
             rest = best.get(n // r) if n % r == 0 else None
             if rest is not None:
                 option = (rest[0] + 1, max(rest[1], r), rest[2] + r, sorted(rest[3] + [r], reverse=True))
                 if n not in best or option < best[n]:
                     best[n] = option
-    return best[L][3] if L in best else None
+    return best[L][3]
+
+
+def _fft_threads(L: int, cols: int, radices: list) -> int:
+    return _round64(max(L // r for r in radices) * cols, 512 if max(radices) > 10 else 1024)
+
+
+def _fft_stages(L: int, cols: int, blocks: int, double: bool) -> list:
+    """The butterfly sizes of a pass.  A stage less is a round trip through LDS and a wait for twiddles less, but larger
+    butterflies are fewer threads: two stages less pay always (7776: 11.6 -> 9.3 us, 531441 16.9 -> 15.3, 2250 4.9 -> 4.2),
+    one where the workgroups fill the chip and have more than a wave for every SIMD (10^6 21.3 -> 20.3, 500 rows of 1500 6.5 ->
+    6.1; one row of 3000 4.7 -> 4.9, 512 of 1000 in workgroups of four waves 4.6 -> 4.7).  In float64, where a stage's results are not rounded in
+    between, the larger butterflies only add roundings (10^6 points: 5.7 and 6.3e-16; in float32 7.2 and 6.2e-8)."""
+    plain = _fft_radices(L) or [1]
+    if double or L < 2:
+        return plain
+    fewest = _fft_fewest(L)
+    less = len(plain) - len(fewest)
+    return fewest if less >= 2 or (less == 1 and blocks >= 128 and _fft_threads(L, cols, fewest) > 256) else plain
 
 
 def _fft_lengths(n: int, limit: int) -> Optional[list]:
@@ -431,6 +461,15 @@ def _fft_butterfly(R: int, sign: float) -> str:
                   f"  const jh_c e = jh_c{{{'-' if sign > 0 else ''}d.im, {s}d.re}};",  # d times +-i
                   "  v[0] = jh_c{a.re + c.re, a.im + c.im}; v[1] = jh_c{b.re + e.re, b.im + e.im};",
                   "  v[2] = jh_c{a.re - c.re, a.im - c.im}; v[3] = jh_c{b.re - e.re, b.im - e.im};"]
+    elif R in FFT_NESTED and math.gcd(FFT_NESTED[R], R // FFT_NESTED[R]) == 1:
+        # coprime sizes (Good 1958): points at B a + A b, results at the k with k = i (mod A), k = j (mod B), no twiddles
+        A, B = FFT_NESTED[R], R // FFT_NESTED[R]
+        lines.append(f"  jh_c t[{A}][{B}];")
+        for a in range(A):
+            lines.append(f"  {{ jh_c x[{B}] = {{{', '.join(f'v[{(B * a + A * b) % R}]' for b in range(B))}}}; jh_dft(x); " + " ".join(f"t[{a}][{j}] = x[{j}];" for j in range(B)) + " }")
+        for j in range(B):
+            at = [next(k for k in range(R) if k % A == i and k % B == j) for i in range(A)]
+            lines.append(f"  {{ jh_c x[{A}] = {{{', '.join(f't[{a}][{j}]' for a in range(A))}}}; jh_dft(x); " + " ".join(f"v[{at[i]}] = x[{i}];" for i in range(A)) + " }")
     elif R in FFT_NESTED:
         A, B = FFT_NESTED[R], R // FFT_NESTED[R]  # v[a + A*b]: transforms over b, twiddles, transforms over a
         lines.append(f"  jh_c t[{A}][{B}];")
@@ -493,8 +532,8 @@ def _fft_passes(n: int, rows: int, ctype: str, eb: int, inverse: bool, numerics:
         alone = len(lengths) == 1
         total = rows * S * D
         cols = _fft_columns(Ln, total, points, alone)
-        radices = _fft_radices(Ln, ctype == "double") or [1]
-        threads = _round64(max(Ln // r for r in radices) * cols, 512 if max(radices) > 10 else 1024)
+        radices = _fft_stages(Ln, cols, -(-total // cols), ctype == "double")
+        threads = _fft_threads(Ln, cols, radices)
         low_bits = max(1, (Ln * D - 1).bit_length() // 2)
         kinds = sorted({k for r in radices for k in ((r, FFT_NESTED[r], r // FFT_NESTED[r]) if r in FFT_NESTED else (r,))})
         blocks = -(-total // cols)
@@ -502,18 +541,13 @@ def _fft_passes(n: int, rows: int, ctype: str, eb: int, inverse: bool, numerics:
         # to the eight XCDs in turn), whose L2 then serves the second of them.
         grid = blocks if alone else -(-blocks // 8) * 8
         tile = "JH_DEV int jh_tile() { return " + ("(int)blockIdx.x" if alone else f"(int)(blockIdx.x % 8) * {grid // 8} + (int)(blockIdx.x / 8)") + "; }"
-        calls, ahead, shapes, NS = [], [], [], 1
+        calls, NS = [], 1
         for s, r in enumerate(radices):
             src, dst = (s + 1) & 1, s & 1
-            kind = f"{r}, {NS}, {'true' if s == 0 else 'false'}, {'true' if s == len(radices) - 1 else 'false'}"
-            ahead.append(f"  const jh_ahead ahead{s} = jh_look_up<{kind}>((int)threadIdx.x < JH_L / {r} * JH_COLS ? (int)threadIdx.x : 0);")
-            calls.append(f"  jh_stage<{kind}>(in_re, in_im, out_re, out_im, re[{src}], im[{src}], re[{dst}], im[{dst}], ahead{s});")
+            calls.append(f"  jh_stage<{r}, {NS}, {'true' if s == 0 else 'false'}, {'true' if s == len(radices) - 1 else 'false'}>(in_re, in_im, out_re, out_im, re[{src}], im[{src}], re[{dst}], im[{dst}]);")
             if s < len(radices) - 1:
                 calls.append("  __syncthreads();")
-            shapes.append((NS, "true" if s == len(radices) - 1 else "false"))
             NS *= r
-        arrived = [f"  jh_arrived<{NS}, {last}>(ahead{s});" for s, (NS, last) in enumerate(shapes)]
-        calls = ahead + calls[:1] + arrived + calls[1:]
         sources.append(_prelude(numerics) + fill(template("fft_pass.hip.inc"), dict(
             N=n, L=Ln, COLS=cols, THREADS=threads, S=S, D=D, TOTAL=total, GUARD=1 if grid * cols != total else 0, L1=lengths[0], L2=lengths[1] if len(lengths) == 3 else 1,
             POINTS_FIRST=1 if final else 0, POINTS_LAST=1 if alone else 0, SCALE=repr(1.0 / n) if inverse and final else "1.0", LOW_BITS=low_bits,

@@ -244,11 +244,12 @@ def test_fft_in_passes(shape, dt):
         assert "passes" in ks.info and err < {"float32": 5e-7, "float64": 1e-14, "float16": 2e-3}[np.dtype(dt).name], (ks.info, err)
 
 
-@pytest.mark.parametrize("shape", [(1, 6), (3, 9), (2, 10), (5, 12), (1, 14), (7, 15), (2, 90), (3, 140 * 15), (1, 10 * 12 * 14 * 15), (2, 9 ** 5)], ids=str)
-def test_fft_butterflies_made_of_two_smaller_ones(shape):
-    """Every such size first, last and alone; more butterflies than threads, with twiddles read ahead for the first of them."""
-    from jaxjs_hip.routinegen import FFT_NESTED, _fft_radices
-    assert any(r in FFT_NESTED for r in _fft_radices(shape[-1]) or ()) or shape[-1] > 8192
+@pytest.mark.parametrize("shape", [(1, 6), (3, 9), (2, 10), (5, 12), (1, 14), (7, 15), (2, 90), (3, 140 * 15), (2, 120), (3, 12 * 12 * 9), (2, 8000), (1, 10 * 12 * 14 * 15), (2, 9 ** 5)], ids=str)
+def test_fft_butterflies_made_of_two_smaller_ones(monkeypatch, shape):
+    """Every such size first, last and alone, and more butterflies than threads, also where a length of so few rows keeps to
+    the smaller ones by itself."""
+    from jaxjs_hip import routinegen
+    monkeypatch.setattr(routinegen, "_fft_stages", lambda L, *rest: routinegen._fft_fewest(L) if L > 1 else [1])
     re, im = RNG.standard_normal(shape).astype(F32), RNG.standard_normal(shape).astype(F32)
     for inverse in (False, True):
         got, ks = R.run_gpu(R.fft(re, im, inverse), [re, im])
