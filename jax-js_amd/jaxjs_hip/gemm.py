@@ -20,6 +20,33 @@ from .tuner import TuneResult, classify_loads
 from .wgradgen import gen_wgrad
 
 
+def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool):
+    """(rate relative to 256x256 tiles on a long axis, plan) of a tile on the direct-to-LDS path where the k axis is so short
+    that a workgroup's prologue and its stores of C weigh as much as its matrix instructions; None: as on a long axis.
+
+    What helps is a second wave on every SIMD, in the same workgroup or in another one of the CU, whose phases overlap the
+    first one's: 256x256 in eight waves (8192 x 1536 x 768 25.9 -> 24.1 us, 4096 x 4096 x 1024 36.7 -> 34.7, 2048 x 5632 x
+    2048 51.2 -> 48.6, the same at 4096^3); 128x256 and 128x192 in two shallow stages, three workgroups to a CU (8192 x 3072
+    x 768 43.4 -> 40.7).  128x192 tiles deal a width of 768 or 2304 out evenly: 8192 x 768 x 768 15.1 -> 13.4 us on 256
+    workgroups instead of 192, 8192 x 2304 x 768 37.6 -> 34.1, 3072 x 3072 x 768 24.2 -> 20.8.  Operands that both run along k
+    take deeper slabs in eight waves (6144 x 6144 x 512 54.9 -> 49.3, 8192 x 2304 x 768 42.6 -> 37.8).  On longer axes 128x192
+    tiles are still the faster ones at such widths (8192 x 768 x 3072 40.6 and 38.2), but the plan of that product is a
+    settled one."""
+    if g["K"] > 2048 or g["K"] % 64:
+        return None
+    if (bm, bn) == (256, 256):
+        return 1.06, dict(WM=2, WN=4)
+    if (bm, bn) == (128, 192):
+        if per_cu == 1:
+            return 0.70 if both_k else 0.68, dict(BK=64, STAGES=4)
+        return (0.83, dict(WM=4, WN=2, BK=64, STAGES=3)) if both_k else (0.87, dict(BK=32, STAGES=2, PIPE=0))
+    if (bm, bn) == (256, 128) and both_k:
+        return 0.85 if per_cu == 1 else 0.95, dict(WM=4, WN=2)
+    if (bm, bn) == (128, 256) and not both_k and per_cu > 1 and g["K"] <= 1024:
+        return 0.97, dict(WM=1, WN=4, BK=32, STAGES=2, PIPE=0)
+    return None
+
+
 def choose_tile(g: dict) -> Dict[str, int]:
     """Block tile (and wave arrangement) for one GEMM: f16 by a small cost model, f32 128x128 down to 64x64."""
     nb = 1
@@ -147,14 +174,6 @@ def choose_tile(g: dict) -> Dict[str, int]:
         # Ragged lengths take it through clamped edge loads (scores of 128 heads over 577 positions: 48.9 us on the
         # 128x256 tiles the estimate below picked, 26.1 us here; 384 heads over 197: 17.2 -> 15.1 us).
         return dict(BM=128, BN=128, BK=32, STAGES=2, PIPE=0)
-    if (g["K"] <= 1024 and g["K"] % 32 == 0 and plain_k and g["M"] % 128 == 0 and g["N"] % 256 == 0 and tiles(128, 256) >= 2 * CU
-            and not loose_ops and repack is None and not (g["a_sk"] == 1 and g["b_sk"] == 1)):
-        # A short k axis under many tiles (the projections of a transformer block: 8192 x 2304 x 768, 8192 x 3072 x 768):
-        # a workgroup's prologue and its C stores weigh as much as its MFMAs.  128x256 tiles in two shallow stages
-        # (48 KiB, 164 registers) put three workgroups on a CU, whose phases overlap: 39.5 -> 36.3 us and 43.4 -> 40.7 us;
-        # the same as the deep pipeline at 4096 x 4096 x 1024 and 2048 x 8192 x 512; slower from k = 3072 (65.9 against
-        # 41.9 us) and with fewer than two tiles per CU (8192 x 768 x 768: 17.0 against 14.9 us).
-        return dict(BM=128, BN=256, WM=1, WN=4, BK=32, STAGES=2, PIPE=0)
     if not plain_k and cut_k and g["K"] >= 8192 and tiles(128, 128) * 8 <= CU:
         # A handful of tiles over a very long k axis read through gather loaders (the filter cotangent of a convolution:
         # 9 taps x 64 x 64 or 128 x 128 outputs, k = batch x positions): 64x64 tiles waste no half-empty MFMA tile and
@@ -174,9 +193,10 @@ def choose_tile(g: dict) -> Dict[str, int]:
         # [1,512,1500] * [512,512,3]: 48 tiles, 40.5 us; 192 of 64x64, 33.5 us.  [1,384,3000] stride 2: 36 tiles, 46.5 us;
         # 144 of 64x64, 24.3 us.  [1,256,8000] * [256,256,7]: 126 tiles, 50.5 us; 250 of 128x64, 42.3 us (64x64: 49.6).
         return dict(BM=64, BN=64) if tiles(128, 128) * 4 <= 1.5 * CU else dict(BM=128, BN=64)
+    both_k = g["a_sk"] == 1 and g["b_sk"] == 1
     best = None
     for bm, bn, eff, extra in ((256, 256, 1.00, dict()), (128, 256, 0.84, dict(WM=1, WN=4)), (256, 128, 0.79, dict()),
-                                (128, 128, 0.62, dict())):
+                                (128, 128, 0.62, dict()), (128, 192, 0.68, dict())):
         if (bm > 128 and g["M"] < bm) or (bn > 128 and g["N"] < bn):
             continue
         per_cu = -(-tiles(bm, bn) // tuner.CU_COUNT)
@@ -187,17 +207,25 @@ def choose_tile(g: dict) -> Dict[str, int]:
             # A ragged k axis, operands off the 16-byte grid or an edge the direct loads cannot clamp run the general
             # template, whose small tiles lose more
             # (8000^3: 838 / 597 / 691 / 512 TFLOP/s for the four shapes, against 1340 for whole 256x256 tiles).
-            eff = {(256, 256): 0.63, (128, 256): 0.45, (256, 128): 0.52, (128, 128): 0.38}[(bm, bn)]
+            eff = {(256, 256): 0.63, (128, 256): 0.45, (256, 128): 0.52, (128, 128): 0.38}.get((bm, bn), eff)
+        short = _short_axis_tile(g, bm, bn, per_cu, both_k) if whole and repack is None else None
+        if short is not None:
+            eff, extra = short
+        elif bn == 192:
+            continue
         cost = per_cu * bm * bn * (g["K"] + 100) / eff
         if best is None or cost < best[0]:
             best = (cost, dict(BM=bm, BN=bn, **extra), per_cu)
     tile, per_cu = dict(best[1]), best[2]
-    both_k = g["a_sk"] == 1 and g["b_sk"] == 1
     if (tile["BM"], tile["BN"]) == (128, 128) and per_cu == 1 and plain_k and g["K"] % 64 == 0:
         # One 128x128 workgroup per CU (or fewer): nothing shares the CU's LDS, so the slabs can be 64 deep in four
         # stages (128 KiB: twice the bytes in flight per workgroup; 2048^3 20.7 -> 19.6 us, 128x14336x4096 35.2 -> 27.4 us).
         if not both_k:
             tile.update(BK=64, STAGES=4)
+        # Eight waves where the k axis is short: a second one on each SIMD covers the first one's prologue and stores (8192 x
+        # 512 x 512 7.7 -> 7.3 us, 1600 x 512 x 512 7.3 -> 6.2, 4096 x 768 x 768 8.6 -> 7.9; from k = 1024 on no gain).
+        if g["K"] < 1024 and not loose_ops and repack is None and edge_ok(128, 128):
+            tile.update(BK=64, STAGES=4, WM=4, WN=2)
         # Half the CUs or fewer would get a workgroup: cut the k axis in two, four when a quarter or fewer would, the
         # slices folded inside the launch by the last one to arrive (128x14336x4096: 27.4 -> 26.0 us with a fold
         # launch, 24.7 folded in the launch; 128x4096x4096: 16.1 us in two slices, 13.9 in four; with 112 tiles four
