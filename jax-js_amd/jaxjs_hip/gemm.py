@@ -20,7 +20,7 @@ from .tuner import TuneResult, classify_loads
 from .wgradgen import gen_wgrad
 
 
-def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool):
+def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool, reads: bool):
     """(rate relative to 256x256 tiles on a long axis, plan) of a tile on the direct-to-LDS path where the k axis is so short
     that a workgroup's prologue and its stores of C weigh as much as its matrix instructions; None: as on a long axis.
 
@@ -29,10 +29,10 @@ def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool):
     2048 51.2 -> 48.6, the same at 4096^3); 128x256 and 128x192 in two shallow stages, three workgroups to a CU (8192 x 3072
     x 768 43.4 -> 40.7).  128x192 tiles deal a width of 768 or 2304 out evenly: 8192 x 768 x 768 15.1 -> 13.4 us on 256
     workgroups instead of 192, 8192 x 2304 x 768 37.6 -> 34.1, 3072 x 3072 x 768 24.2 -> 20.8.  Operands that both run along k
-    take deeper slabs in eight waves (6144 x 6144 x 512 54.9 -> 49.3, 8192 x 2304 x 768 42.6 -> 37.8).  On longer axes 128x192
-    tiles are still the faster ones at such widths (8192 x 768 x 3072 40.6 and 38.2), but the plan of that product is a
-    settled one."""
-    if g["K"] > 2048 or g["K"] % 64:
+    take deeper slabs in eight waves (6144 x 6144 x 512 54.9 -> 49.3, 8192 x 2304 x 768 42.6 -> 37.8).  Up to 4096 the 128x192
+    tiles, one to a CU, stand behind an epilogue that `reads` buffers, whose loads add to the stores (8192 x 768 x 3072 with
+    bias and residual 44.3 -> 41.2; the bare product, 40.6 and 38.2, keeps the plan it had)."""
+    if g["K"] > (4096 if reads and (bm, bn) == (128, 192) and per_cu == 1 else 2048) or g["K"] % 64:
         return None
     if (bm, bn) == (256, 256):
         return 1.06, dict(WM=2, WN=4)
@@ -47,8 +47,9 @@ def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool):
     return None
 
 
-def choose_tile(g: dict) -> Dict[str, int]:
-    """Block tile (and wave arrangement) for one GEMM: f16 by a small cost model, f32 128x128 down to 64x64."""
+def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
+    """Block tile (and wave arrangement) for one GEMM: f16 by a small cost model, f32 128x128 down to 64x64.  `reads`: whether
+    the epilogue reads buffers."""
     nb = 1
     for b in g["batch"]:
         nb *= b[0]
@@ -208,7 +209,7 @@ def choose_tile(g: dict) -> Dict[str, int]:
             # template, whose small tiles lose more
             # (8000^3: 838 / 597 / 691 / 512 TFLOP/s for the four shapes, against 1340 for whole 256x256 tiles).
             eff = {(256, 256): 0.63, (128, 256): 0.45, (256, 128): 0.52, (128, 128): 0.38}.get((bm, bn), eff)
-        short = _short_axis_tile(g, bm, bn, per_cu, both_k) if whole and repack is None else None
+        short = _short_axis_tile(g, bm, bn, per_cu, both_k, reads) if whole and repack is None else None
         if short is not None:
             eff, extra = short
         elif bn == 192:
@@ -586,7 +587,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None)
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
     few = few_plan(t)
-    tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g)
+    tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g, bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex)))
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
         raise ValueError("a tile override must give both BM and BN")
