@@ -123,6 +123,37 @@ def _tiles_stand(o: dict, t: dict) -> bool:
     return t["count"] >= many and o["R"] > FEW_ROWS or t["count"] >= FEW_WORKGROUPS and o["w_bytes"] > 96 << 20 and not o["loose"]
 
 
+def _in_steps(best: dict, o: dict, slices: int) -> dict:
+    """The plan of a shape: steps in equal shares for the waves, in equal batches of what the registers of a full workgroup hold
+    in flight."""
+    MT, VN, steps = best["MT"], best["VN"], max(1, o["K"] // (64 // o["eb"]))
+    waves = min(best["waves"], -(-steps // slices))
+    share = -(-steps // (waves * slices))
+    most = max(1, (104 - 4 * MT * VN) // (4 * (MT + VN)))
+    return dict(R=o["R"], MT=MT, C=o["C"], short=o["short"], wide=o["wide"], along_k=o["along_k"], VN=VN, waves=-(-steps // (share * slices)), slices=slices,
+                batch=-(-share // -(-share // most)), nbatch=o["nbatch"], row=o["row"])
+
+
+def plan_whole_rows(g: dict) -> Optional[dict]:
+    """The plan of `g` in tiles that hold whole rows of the result, or None; with the launch's estimated microseconds."""
+    o = _operands(g)
+    if o is None or g["batch"]:
+        return None
+    f32, step = o["eb"] == 4, 64 // o["eb"]
+    best = None
+    for MT in (1, 2, 4):
+        for VN in ((1, 2, 4) if f32 or o["along_k"] else (2, 4, 8)):
+            across, down = (16 * VN, 16 * MT) if o["short"] == "a" else (16 * MT, 16 * VN)
+            if MT * VN > 16 or across < g["N"] or (not o["along_k"] and o["C"] < VN):
+                continue
+            waves = max(1, min(16, o["K"] // step or 1, FEW_LDS // (MT * 16 * (16 * VN + 1) * 4)))
+            cycles = -(-o["K"] // step) * (28 * (MT * _loads(g, o["short"], True) + VN * _loads(g, o["wide"], o["along_k"])) + MT * VN * (32 if f32 else 4)) + waves * MT * VN * 16
+            us = 2.6 + max(1.0, -(-g["M"] // down) / tuner.CU_COUNT) * cycles / 2400
+            if best is None or us < best["us"]:
+                best = dict(us=us, MT=MT, VN=VN, waves=waves)
+    return dict(_in_steps(best, o, 1), us=best["us"]) if best is not None else None
+
+
 def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
     """Workgroup shape for `g` (see tuner.match_gemm) if one operand runs along k, the other along either axis, and this
     kernel is expected to beat the LDS tiles, else None.  `tiles_of()` gives the tile plan to compare with.
@@ -146,14 +177,7 @@ def plan_few(g: dict, tiles_of=None) -> Optional[dict]:
         stream = o["w_bytes"] / 4.5e6  # the weights from memory, which either waits for
         if _tiles_stand(o, t) or max(us, stream) >= 0.95 * max(t["us"], stream):
             return None
-    # Steps in equal shares for the waves, in equal batches of what the registers of a full workgroup hold in flight.
-    MT, VN, steps = best["MT"], best["VN"], max(1, o["K"] // (64 // o["eb"]))
-    slices = _slices(steps, best["count"])
-    waves = min(best["waves"], -(-steps // slices))
-    share = -(-steps // (waves * slices))
-    most = max(1, (104 - 4 * MT * VN) // (4 * (MT + VN)))
-    return dict(R=o["R"], MT=MT, C=o["C"], short=o["short"], wide=o["wide"], along_k=o["along_k"], VN=VN, waves=-(-steps // (share * slices)), slices=slices,
-                batch=-(-share // -(-share // most)), nbatch=o["nbatch"], row=o["row"])
+    return _in_steps(best, o, _slices(max(1, o["K"] // (64 // o["eb"])), best["count"]))
 
 
 def chain_pitch(K: int, dtype: DType) -> int:
@@ -162,15 +186,17 @@ def chain_pitch(K: int, dtype: DType) -> int:
     return -(-K // group) * group + group
 
 
-def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_args: str, decode: str, rows=None):
+def gen_few(g: dict, p: dict, name: str, params: str, names, epi_fn: str, epi_args: str, decode: str, rows=None, behind=None, made_t: str = "float"):
     """(source text behind the prelude, grid, block).  `rows`: the short operand's rows as a `RowText` with outputs of its own
-    name, made in LDS."""
+    name, made in LDS.  `behind`: what happens to the rows of the result (of type `made_t`), as a `RowText` that reads them from
+    LDS; a workgroup's tile has to hold them whole."""
     s, w = p["short"], p["wide"]
-    text = (rows.machinery if rows else "") + fill(template("gemm_few.hip.inc"), dict(
+    text = ((rows or behind).machinery if rows or behind else "") + fill(template("gemm_few.hip.inc"), dict(
         F32=1 if g["dtype"] == DType.Float32 else 0, R=p["R"], MT=p["MT"], C=p["C"], K=g["K"], WK=1 if p["along_k"] else 0, VN=p["VN"],
         WAVES=p["waves"], BATCH=p["batch"], SLICES=p["slices"], CHAIN=1 if rows else 0, PITCH=chain_pitch(g["K"], g["dtype"]),
         X_NONE=f"  const jh_val* const {names[g['gid_' + s]]} = nullptr;  // (the epilogue's parameters name every operand)" if rows else "",
-        CHAIN_LOADS=rows.loads if rows else "", CHAIN_STAGES=rows.stages if rows else "", EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
+        CHAIN_LOADS=(rows or behind).loads if rows or behind else "", CHAIN_STAGES=(rows or behind).stages if rows or behind else "",
+        BEHIND=1 if behind else 0, HEIGHT=g["M"], MADE_ROWS=16 * (p["MT"] if s == "a" else p["VN"]), FIRST_ROW="r0" if s == "a" else "c0", MADE_T=made_t, EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, A_OFF=g["a_off"], B_OFF=g["b_off"], BATCH_DECODE=decode, X_PTR=names[g["gid_" + s]], W_PTR=names[g["gid_" + w]], X_BASE=s + "_base", W_BASE=w + "_base",
         X_ROW=g[p["row"][s]], W_ROW=g[p["row"][w]], W_K=g[w + "_sk"], ROW="rr" if s == "a" else "c", COL="c" if s == "a" else "rr", C_SM=g["c_sm"], C_SN=g["c_sn"],
         EPILOGUE_ARGS=epi_args))
     return text, (-(-p["C"] // (16 * p["VN"])) * p["slices"], p["nbatch"], -(-p["R"] // (16 * p["MT"]))), (64 * p["waves"], 1, 1)

@@ -579,14 +579,15 @@ def few_plan(t: TuneResult) -> Optional[dict]:
     return plan_few(g, lambda: choose_tile(g))
 
 
-def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None) -> KernelSource:
+def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None, behind=None, few=None) -> KernelSource:
     """`rows`: the rows of the short operand of a contraction that `few_plan` takes, made in the same launch (a `RowText` whose
-    inputs come behind the kernel's)."""
+    inputs come behind the kernel's).  `behind`: what happens to the result's rows in the same launch, under the plan `few` (a
+    `RowText`; its inputs come behind the kernel's and its outputs are the launch's)."""
     g = t.gemm
     re = kernel.reduction
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
-    few = few_plan(t)
+    few = few or few_plan(t)
     tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g, bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex)))
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
@@ -695,9 +696,11 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None)
         if rows:
             gids.remove(g["gid_" + few["short"]])
             params = ", ".join([f"const {STORAGE_CTYPE[used[i] or DType.Float32]}* __restrict__ {names[i]}" for i in gids] + rows.params + [f"{out_t}* __restrict__ out"])
+        if behind:
+            params = ", ".join(f"const {STORAGE_CTYPE[used[i] or DType.Float32]}* __restrict__ {names[i]}" for i in gids) + ", " + ", ".join(behind.params)
         if few["slices"] > 1:
             params += ", float* __restrict__ jh_part, unsigned* __restrict__ jh_count"
-        text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "", rows)
+        text, grid, block = gen_few(g, few, name, params, names, epi_fn, epi_args, "\n".join(lines) if g["batch"] else "", rows, behind, out_t)
         need = _min_bytes(t.epilogue)
         for tg in ("a", "b"):
             need[g["gid_" + tg]] = max(need.get(g["gid_" + tg], 0), g[tg + "_len"] * byteWidth(g["dtype"]))
@@ -706,7 +709,13 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None)
             need = {k: need[i] for k, i in enumerate(gids) if i in need}
             need.update({len(gids) + k: b for k, b in rows.need.items()})
             gids = list(range(len(gids) + len(rows.params)))
-        args, scratch = [("in", i) for i in gids] + [("out", 0)], []
+        outs = 1
+        if behind:
+            src_options = src_options or (SOURCE_OPTION + "-fno-slp-vectorize\n" if behind.halves else "")
+            outs = sum(" __restrict__ out" in q for q in behind.params)
+            need.update({len(gids) + k: b for k, b in behind.need.items()})
+            gids = list(range(len(gids) + len(behind.params) - outs))
+        args, scratch = [("in", i) for i in gids] + [("out", i) for i in range(outs)], []
         if few["slices"] > 1:  # the slices' sums, and a counter for each tile
             args += [("scratch", 0), ("scratch", 1)]
             scratch = [math.prod(grid) * 256 * few["MT"] * few["VN"] * 4, math.prod(grid) // few["slices"] * 4]

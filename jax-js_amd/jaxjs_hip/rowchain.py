@@ -322,12 +322,13 @@ class RowText:
     halves: bool
 
 
-def row_text(chain: RowChain, p: dict, numerics: str, in_name: str = "in") -> RowText:
-    """The chain as text under plan `p` (vector width V, lanes T, iterations)."""
+def row_text(chain: RowChain, p: dict, numerics: str, in_name: str = "in", local: Optional[int] = None) -> RowText:
+    """The chain as text under plan `p` (vector width V, lanes T, iterations).  Input `local`, read as rows only, is no
+    parameter: its row starts at the pointer `jh_row`."""
     V, T = p["V"], p["T"]
     types = _types(chain)
     rows, _ = _rows_held(chain)
-    params = [f"const {STORAGE_CTYPE[d or DType.Float32]}* __restrict__ {in_name}{k}" for k, d in enumerate(types)]
+    params = [f"const {STORAGE_CTYPE[d or DType.Float32]}* __restrict__ {in_name}{k}" for k, d in enumerate(types) if k != local]
     params += [f"{STORAGE_CTYPE[chain.stages[j].kernel.dtype]}* __restrict__ out{j}" for j in chain.outputs]
     halves = any(d == DType.Float16 for d in types) or any(
         e is not None and e.collect(lambda n: n.dtype == DType.Float16) for s in chain.stages for e in (s.exp, s.epilogue))
@@ -343,7 +344,8 @@ def row_text(chain: RowChain, p: dict, numerics: str, in_name: str = "in") -> Ro
             ct = STORAGE_CTYPE[types[k]]
             # rows that this launch reads once and that are many: past the caches (see jh_vload_nt)
             kind = "jh_vload_nt" if chain.R * chain.C >= (1 << 22) else "jh_vload"
-            loads.append(f"      x{k}[i] = {kind}<{ct}, JH_V>({in_name}{k} + at + c0);")
+            base = f"{in_name}{k} + at" if k != local else "jh_row"
+            loads.append(f"      x{k}[i] = {kind}<{ct}, JH_V>({base} + c0);")
         loads += end
     text: List[str] = []
     folds: Dict[tuple, str] = {}   # a fold that an earlier stage has done already
@@ -401,7 +403,7 @@ def row_text(chain: RowChain, p: dict, numerics: str, in_name: str = "in") -> Ro
     for st in chain.stages:
         for n in _loads(st):
             kind, k = st.refs[n.arg[0]]
-            if kind == "in":
+            if kind == "in" and k != local:
                 need[k] = max(need.get(k, 0), n.arg[1] * byteWidth(n.dtype))
     return RowText(machinery, "\n".join(loads), "\n".join(x for x in text if x), params, need, halves)
 

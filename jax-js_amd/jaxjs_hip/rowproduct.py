@@ -1,4 +1,4 @@
-"""A chain of Kernels over rows and the product of those rows with a matrix, in one launch (`gemm_few.hip.inc`).
+"""A chain of Kernels over rows and a product of those rows, or whose result they are, in one launch (`gemm_few.hip.inc`).
 
 A layer normalisation in front of a linear layer on a few tokens is a launch of a few microseconds whose result the
 product's workgroups read at once.  Here each of them makes the rows it needs in LDS, while its first share of the matrix
@@ -6,6 +6,9 @@ is on its way: the same work many times over, but beside a wait that is there an
 and a linear layer, microseconds in two launches -> in one: float16 8 x 768 x 2304 5.4 -> 4.0, 8 x 768 x 3072 6.7 -> 4.1, 64 x
 512 x 1536 5.2 -> 3.6, 16 x 2048 x 2048 7.5 -> 5.6; float32 8 x 768 x 3072 6.6 -> 4.2, 64 x 1024 x 1000 8.2 -> 6.1, 8 x 2048 x
 2048 9.3 -> 8.5; a decode step of a transformer block 38.0 -> 35.1.
+
+`ProductRows` is the other way round: a softmax behind a narrow output layer works on the rows of a result of which a
+workgroup holds whole rows, before they are stored.
 """
 
 from __future__ import annotations
@@ -18,7 +21,7 @@ from .composite import Composite
 from .gemm import few_plan, gen_gemm
 from .kernelgen import KernelSource
 from .rowchain import RowChain, plan_rows, row_text
-from .fewgen import chain_pitch
+from .fewgen import chain_pitch, plan_whole_rows
 
 ROWS_MOST = 64             # rows of the product: every 16 of them are made by all of its column tiles
 ROWS_BYTES = 96 * 1024     # of a workgroup's rows: 12 x 2048 float32 9.5 -> 9.1 us, 16 x 2048 9.9 -> 10.0
@@ -56,12 +59,74 @@ class RowProduct(Composite):
         return gen_gemm(self.kernel, t, numerics, "jh_row_product", rows=text)
 
 
-def lane_plan(chain: RowChain, waves: int, rows: int) -> dict:
+class ProductRows(Composite):
+    """`kernel` and `chain`, whose input `local` is the kernel's result and nothing else's."""
+
+    def __init__(self, kernel: Kernel, inputs: Sequence[int], chain: RowChain, local: int, few: dict):
+        self.kernel, self.chain, self.local, self.few = kernel, chain, local, few
+        self.inputs = list(inputs[:kernel.nargs]) + [b for k, b in enumerate(chain.inputs) if k != local]
+
+    def key(self) -> tuple:
+        return ("product rows", self.kernel.key(), self.chain.key(), self.local)
+
+    def output_bytes(self) -> List[int]:
+        return self.chain.output_bytes()
+
+    def extents(self) -> List[int]:
+        return [self.kernel.size, self.kernel.reduction.size]
+
+    def label(self):
+        return "ProductRows", [("kernels", str(len(self.chain.stages) + 1)), ("size", str(self.kernel.size))]
+
+    def generate(self, numerics: str) -> KernelSource:
+        t = tuner.tuneNullopt(self.kernel)
+        t.klass, t.gemm = "gemm", tuner.match_gemm(self.kernel)
+        p = self.few
+        plan = lane_plan(self.chain, p["waves"], 16 * (p["MT"] if p["short"] == "a" else p["VN"]), 2)
+        text = row_text(self.chain, plan, numerics, "row", self.local)
+        # inputs of the chain are numbered through without the local one
+        text.need = {k - (k > self.local): b for k, b in text.need.items()}
+        return gen_gemm(self.kernel, t, numerics, "jh_product_rows", behind=text, few=p)
+
+
+# Whole rows in a workgroup are few, wide tiles: taken up to this estimate, or where they come in rounds anyway.  softmax behind a
+# linear layer, microseconds in two launches -> in one: float32 16 x 2 x 64 5.8 -> 3.4, 64 x 10 x 256 5.5 -> 3.8, 64 x 10 x 1024 5.9 ->
+# 4.3, 1024 x 46 x 256 5.4 -> 4.0, 8192 x 64 x 1024 23.3 -> 19.5; float16 1024 x 64 x 256 5.6 -> 4.0, 8192 x 10 x 1024 7.1 -> 5.4.  Past
+# the line 64 x 46 x 1024 6.4 -> 8.6, float16 64 x 64 x 1024 5.6 -> 7.3.
+BEHIND_US = 5.0
+
+
+def join_behind(kernel: Kernel, inputs: Sequence[int], buffer: int, chain: RowChain) -> Optional[ProductRows]:
+    """`kernel`, which writes `buffer`, in one launch with `chain`, the only reader of that result; or None."""
+    if kernel.reduction is None or buffer not in chain.inputs or kernel.size != chain.R * chain.C:
+        return None
+    local = chain.inputs.index(buffer)
+    for st in chain.stages:
+        for n in st.exp.collect(lambda n: n.op == AluOp.GlobalIndex) + (st.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex) if st.epilogue is not None else []):
+            if st.refs[n.arg[0]] == ("in", local) and (id(n) not in st.full or n.dtype != kernel.dtype):
+                return None
+    g = tuner.match_gemm(kernel)
+    if g is None or g["M"] != chain.R or g["N"] != chain.C or g["c_sn"] != 1 or g["c_sm"] != chain.C or g["gid_a"] == g["gid_b"]:
+        return None
+    p = plan_whole_rows(g)
+    if p is None:
+        return None
+    rows = 16 * (p["MT"] if p["short"] == "a" else p["VN"])
+    if p["us"] > BEHIND_US and chain.R < 2 * tuner.CU_COUNT * rows:
+        return None
+    lanes = lane_plan(chain, p["waves"], rows, 2)
+    sums = p["waves"] * 16 * p["MT"] * (16 * p["VN"] + 1) * 4
+    if lanes["iters"] * lanes["V"] > LANE_ELEMENTS or sums + rows * (chain.C + 16) * byteWidth(kernel.dtype) > LDS_BYTES:
+        return None
+    return ProductRows(kernel, inputs, chain, local, p)
+
+
+def lane_plan(chain: RowChain, waves: int, rows: int, least: int = 16) -> dict:
     """Lanes of a row inside one wave, as many as let the workgroup make all its rows at once."""
     p = dict(plan_rows(chain))
     V, groups = p["V"], chain.C // p["V"]
     T = 64
-    while T > 16 and (waves * 64 // T < rows or T >= 2 * groups):
+    while T > least and (waves * 64 // T < rows or T >= 2 * groups):
         T //= 2
     iters = -(-groups // T)
     p.update(T=T, iters=iters, full=sum(1 for i in range(iters) if (i + 1) * T * V <= chain.C))

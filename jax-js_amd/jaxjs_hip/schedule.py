@@ -21,7 +21,7 @@ from .errors import SlotError
 from .kernelgen import generate
 from .routine import Routine
 from .rowchain import RowChain, _tidy, collect_chain, index_form
-from .rowproduct import join_rows
+from .rowproduct import join_behind, join_rows
 from .runtime import LaunchRef, LaunchStepC, check
 from .shape import prod, unravelAlu
 from .tuner import match_gemm
@@ -168,6 +168,13 @@ def plan_units(prog) -> List[Unit]:
         found = collect_chain(view, k, lambda o, last: o in kept or last_read.get(o, -1) > last)
         if found is not None:
             chain, n = found
+            before = steps[k - 1] if units and units[-1].outputs == [steps[k - 1].output] and isinstance(units[-1].source, Kernel) else None
+            if before is not None and before.output not in kept and last_read.get(before.output, -1) < k + n:
+                joined = join_behind(before.kernel, before.inputs, before.output, chain)
+                if joined is not None:
+                    units[-1] = Unit(joined, joined.inputs, [steps[k + j].output for j in chain.outputs])
+                    k += n
+                    continue
             units.append(Unit(chain, chain.inputs, [steps[k + j].output for j in chain.outputs]))
             k += n
             continue

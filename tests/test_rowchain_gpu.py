@@ -10,7 +10,7 @@ from jaxjs_hip import library as L
 from jaxjs_hip import workloads as W
 from jaxjs_hip.jit import ShapedArray
 from jaxjs_hip.rowchain import RowChain, gen_rows
-from jaxjs_hip.rowproduct import RowProduct
+from jaxjs_hip.rowproduct import ProductRows, RowProduct
 from jaxjs_hip.schedule import plan_units
 from jit_util import run_program
 from oracle.backend import OracleBackend
@@ -157,3 +157,24 @@ def test_rows_that_something_else_reads_stay_a_launch_of_their_own():
         prog = J.jit(fn, [ShapedArray(a.shape, DType.Float32) for a in arrays])
         assert not any(isinstance(u.source, RowProduct) for u in plan_units(prog))
         check(prog, arrays, False, chained=False, terms=256)
+
+
+@pytest.mark.parametrize("rows,k,n", [(3, 40, 2), (64, 256, 10), (33, 64, 10), (17, 100, 33), (200, 96, 64), (1024, 512, 16), (8200, 64, 46)], ids=str)
+@pytest.mark.parametrize("order", ["kn", "nk", "first along rows"])
+@pytest.mark.parametrize("dtype", [DType.Float32, DType.Float16], ids=lambda d: d.value)
+@pytest.mark.parametrize("op", ["softmax", "argmax"])
+def test_rows_of_a_narrow_product_in_its_launch(op, dtype, order, rows, k, n):
+    """Rows off the tile, columns off the vector width and up to the widest tile, operands in all orders the kernel reads;
+    the result alone, and an argmax (whose ties and order are exact)."""
+    rng, t = np.random.default_rng(k), np.float16 if dtype == DType.Float16 else np.float32
+    x, w = rng.standard_normal((rows, k)).astype(t), (rng.standard_normal((k, n)) * k ** -0.5).astype(t)
+    if op == "argmax":  # small integers: the same sums in any order
+        x, w = rng.integers(-2, 3, (rows, k)).astype(t), rng.integers(-1, 2, (k, n)).astype(t)
+    arrays = [np.ascontiguousarray(x.T) if order == "first along rows" else x, np.ascontiguousarray(w.T) if order != "kn" else w, np.zeros(n, t)]
+
+    def f(a, b, c):
+        a = L.swapaxes(a, 0, 1) if order == "first along rows" else a
+        return OPS[op](L.matmul(a, L.swapaxes(b, 0, 1) if order != "kn" else b).add(c))
+    prog = J.jit(f, [ShapedArray(a.shape, dtype) for a in arrays])
+    assert any(isinstance(u.source, ProductRows) for u in plan_units(prog)), [type(u.source).__name__ for u in plan_units(prog)]
+    check(prog, arrays, dtype == DType.Float16, chained=False, terms=k)
