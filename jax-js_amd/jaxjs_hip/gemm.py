@@ -47,6 +47,43 @@ def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool, reads
     return None
 
 
+def _f32_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
+    """Tile and slices of a float32 product of whole 16-byte groups with a single-stride k axis and enough tiles to fill the
+    chip.  128-row tiles take eight waves, two on a SIMD (2048 x 2048 x 1024 84.3 -> 81.0 us, 4032 x 4032 x 2368 657 -> 632, 1024 x
+    1024 x 1024 29.3 -> 28.5).
+
+    With two workgroups for every CU in some shape: the area of the tiles a CU gets, at the shape's rate (2048 x 3072 x 768 111
+    -> 106 us in 128x64, 3224 x 1388 x 2964 320 in 64x64 and 354 in 128x64).  With fewer, by an estimate in microseconds: 3.7;
+    that area times the depth of a slice, a CU that has one workgroup alone a fifth or a sixth slower; for the fold of slices
+    inside the launch 0.65 a slice and 0.61 for every 10^6 partial sums; and a thirtieth for every halving of the axis, since
+    workgroups that share a CU even their numbers out (128 x 14336 x 4096 178 in two slices, 190 in eight).  It is a fit to 11 products in both orders of B
+    and all plans, within half a per cent of the fastest one in the mean and a third faster than a rule of 1.5 workgroups of
+    128x64 a CU: 1280 x 640 x 320 19.3 -> 11.8 in 200 tiles instead of 100, 640 x 896 x 3136 84 -> 54 in eight slices, 192 x
+    2112 x 1408 35 -> 22, 1536 x 768 x 768 36.6 -> 28.2, 768 x 1152 x 704 25.4 -> 21.4."""
+    CU, best = tuner.CU_COUNT, None
+
+    def plan(bm, bn, split=1):
+        return dict(BM=bm, BN=bn, BK=32, WM=4 if bm == 128 else 2, WN=2, **(dict(SPLITK=split, FUSEK=1) if split > 1 else {}))
+    for bm, bn, rate in ((128, 128, 266e3), (128, 64, 248.5e3), (64, 64, 230e3)):
+        if g["M"] >= bm and g["N"] >= bn and tiles(bm, bn) >= 2 * CU:
+            cost = -(-tiles(bm, bn) // CU) * bm * bn / rate
+            if best is None or cost < best[0]:
+                best = (cost, plan(bm, bn))
+    if best is not None:
+        return best[1]
+    for bm, bn, rate, alone in ((64, 64, 185.5e3, 0.79), (128, 64, 222.0e3, 0.83)):
+        for split in (1, 2, 4, 8):
+            if split > 1 and (nb > 1 or g["K"] % (4 * split) or g["K"] // split < 128):
+                continue
+            per_cu = -(-tiles(bm, bn) * split // CU)
+            us = 3.66 + per_cu * bm * bn * (g["K"] / split + 2.7) / (rate * (alone if per_cu == 1 else 1.0))
+            if split > 1:
+                us = (us + 0.645 * split + 0.611e-6 * split * g["M"] * g["N"]) * 1.035 ** (split.bit_length() - 1)
+            if best is None or us < best[0]:
+                best = (us, plan(bm, bn, split))
+    return best[1]
+
+
 def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
     """Block tile (and wave arrangement) for one GEMM: f16 by a small cost model, f32 128x128 down to 64x64.  `reads`: whether
     the epilogue reads buffers."""
@@ -93,6 +130,8 @@ def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
         # second one hides the first one's staging latency).  Slabs are 32 deep (measured 3-6 % over 16 on
         # 2048^3 and 4096^3: half the barriers); gather operands keep the 16-deep slabs they were tuned with.
         bk = 32 if plain_k else 16
+        if plain_k and not loose_ops and g["M"] >= 128 and g["N"] >= 64 and tiles(128, 64) * 4 > CU:
+            return _f32_tile(g, tiles, nb)
         # Among the shapes that do, the cheapest by (rounds of two workgroups per CU) x (tile area) / (rate of the
         # shape relative to 128x128: 0.97, 0.80): a last round that is nearly empty costs a whole one (products of
         # attention weights and values over 577 positions, 640 tiles of 128x64: 85.1 us, 66.1 us in 1280 of 64x64; the
@@ -1004,6 +1043,8 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
 
     tmpl = "gemm_f16.hip.inc" if g["dtype"] == DType.Float16 else "gemm_f32.hip.inc"
     fBK = int(tile.get("BK", 16)) if g["dtype"] == DType.Float32 else 0  # slab depth of the f32 template
+    if g["dtype"] == DType.Float32 and fBK in (16, 32, 64) and (BM * fBK // 4 % nthreads or BN * fBK // 4 % nthreads):
+        raise ValueError(f"{nthreads} threads do not share out a {BM}- or {BN}-row slab {fBK} deep in whole groups")
     if g["dtype"] == DType.Float32 and (fBK not in (16, 32, 64) or 2 * (BM + BN) * (fBK + 4) * 4 > 160 * 1024):
         raise ValueError(f"f32 slab depth {fBK} is not 16, 32 or 64, or two {BM}+{BN}-row slabs of it do not fit the LDS")
     # Fast path: direct global->LDS loads need whole tiles (no bounds predicates) and 32-deep slabs.
