@@ -677,7 +677,39 @@ def test_gemm_f16_direct_lds_edge_tiles(M, N, K, layout, tile, bias):
     assert np.all(err <= bound), f"max excess {np.max(err - bound)} with {ks.info}"
 
 
+@pytest.mark.parametrize("tile", [
+    dict(BM=128, BN=192, BK=32, STAGES=2, PIPE=0), dict(BM=128, BN=192, BK=32), dict(BM=128, BN=192, BK=64, STAGES=4), dict(BM=128, BN=192, BK=64, STAGES=3, WM=4),
+    dict(BM=256, BN=256, WM=2, WN=4), dict(BM=256, BN=128, WM=4, WN=2), dict(BM=128, BN=128, BK=64, STAGES=4, WM=4, WN=2),
+], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()))
+@pytest.mark.parametrize("M,N,K,layout,bias", [(300, 392, 128, "NN", True), (136, 200, 64, "NN", False), (304, 584, 320, "TN", True), (130, 193, 192, "NT", False), (520, 776, 2048, "NT", True)])
+def test_gemm_f16_tiles_of_short_k_axes(M, N, K, layout, bias, tile):
+    """192 columns (rows of 384 bytes in LDS, loads dealt unevenly to the phases, 12 groups of a row in the epilogue) and
+    eight waves: one slab and many, edges in both directions, both orders of both operands."""
+    test_gemm_f16_direct_lds_edge_tiles(M, N, K, layout, tile, bias)
+
+
 F32_SHAPES = [(64, 64, 64), (128, 128, 64), (200, 264, 136), (1024, 1024, 1024), (96, 1028, 72), (512, 384, 100)]
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1280, 640, 320, dict(BM=64, splitk=1)), (640, 896, 3136, dict(BM=64, splitk=8)), (196, 2112, 1424, dict(BM=64, splitk=4)), (1100, 1100, 516, dict(BM=64, splitk=1)),
+    (1020, 1020, 1040, dict(BM=128, BN=64, splitk=4)), (2044, 2044, 100, dict(BM=128, BN=64, splitk=1)), (4092, 4092, 36, dict(BM=128, BN=128, splitk=1)),
+], ids=str)
+@pytest.mark.parametrize("transposed", [False, True])
+def test_gemm_f32_tiles_and_slices(transposed, M, N, K, tile):
+    """Eight waves, edge tiles in both directions, slices that end inside a slab; small integers, exact sums, twice over."""
+    A, B = RNG.integers(-8, 9, (M, K)).astype(np.float32), RNG.integers(-8, 9, (K, N)).astype(np.float32)
+    k, bufs = matmulKernel(M, N, K, DType.Float32, b_transposed=transposed), [A, np.ascontiguousarray(B.T) if transposed else B]
+    for _ in range(2):
+        got, ks = device_run(k, bufs)
+        assert all(ks.info.get(key) == v for key, v in tile.items()), ks.info
+        np.testing.assert_array_equal(got.reshape(M, N), A @ B, err_msg=str(ks.info))
+
+
+def test_gemm_f32_threads_that_do_not_share_out_a_slab():
+    from jaxjs_hip.kernelgen import generate
+    with pytest.raises(ValueError):
+        generate(matmulKernel(512, 512, 512, DType.Float32), gemm_tile=(("BK", 16), ("BM", 128), ("BN", 64), ("WM", 4), ("WN", 2)))
 
 
 @pytest.mark.parametrize("M,N,K", F32_SHAPES, ids=lambda v: str(v))
