@@ -236,6 +236,12 @@ def find_wgrad(kernel, t, g: dict) -> Optional[dict]:
     return None if p is None else dict(m, **p)
 
 
+def _fold_waves(slices: int) -> int:
+    """Waves of the fold that share the slices of 64 pieces: about four loads each, all in flight at once (56 slices of [64, 64, 3,
+    3]: 6.1 -> 4.6 us with 14 waves instead of four)."""
+    return max(4, min(16, slices // 4))
+
+
 def is_filter_cotangent(kernel) -> bool:
     """Whether `kernel` is better prepared with the option `filter_bands`."""
     if kernel.reduction is None or kernel.size == 0:
@@ -254,7 +260,7 @@ def gen_wgrad(kernel, g: dict, w: dict, numerics: str, name: str, params: str, n
     c_row = f"c * {w['T']} + tap" if w["joined"] else "c"
     src = src_options + _prelude(numerics) + fill(template("wgrad_f16.hip.inc"), dict(
         {k: w[k] for k in ("C", "O", "W", "H", "OW", "OH", "KW", "KY", "GROUPS", "PH", "PW", "SC", "SB", "CTO", "CTB", "R", "NB", "IC", "PI", "PC", "IMG_OFF", "CT_OFF")},
-        SLICES=w["slices"], ALIGN=16 if aligned else 2, EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, IMG_PTR=names[g["gid_" + w["img"]]],
+        SLICES=w["slices"], PARTS=_fold_waves(w["slices"]), ALIGN=16 if aligned else 2, EPILOGUE_FN=epi_fn, NAME=name, PARAMS=params, IMG_PTR=names[g["gid_" + w["img"]]],
         CT_PTR=names[g["gid_" + w["ct"]]], ROW=c_row if image_rows else "o", COL="o" if image_rows else c_row,
         C_SM=g["c_sm"], C_SN=g["c_sn"], C_ST=0 if w["joined"] else g["batch"][0][3], B0="0" if w["joined"] else "tap", OUT_T=out_t, EPILOGUE_PARAMS=epi_params, EPILOGUE_ARGS=epi_args))
     args = [("in", i) for i in range(kernel.nargs)] + [("out", 0)]
@@ -263,7 +269,7 @@ def gen_wgrad(kernel, g: dict, w: dict, numerics: str, name: str, params: str, n
     if w["slices"] > 1:
         scratch = [w["slices"] * pieces * 16]
         steps = [LaunchStep(name, (w["tiles"] * w["slices"], 1, 1), (256, 1, 1), 0, args + [("scratch", 0)]),
-                 LaunchStep(name + "_fold", (pieces // 64, 1, 1), (256, 1, 1), 0, args + [("scratch", 0)])]
+                 LaunchStep(name + "_fold", (pieces // 64, 1, 1), (64 * _fold_waves(w["slices"]), 1, 1), 0, args + [("scratch", 0)])]
     need = dict(need)
     for tag, end in ((w["img"], w["IMG_OFF"] + (w["NB"] - 1) * w["SB"] + (w["C"] - 1) * w["SC"] + w["H"] * w["W"]),
                      (w["ct"], w["CT_OFF"] + (w["NB"] - 1) * w["CTB"] + (w["O"] - 1) * w["CTO"] + w["OH"] * w["OW"])):
