@@ -182,7 +182,7 @@ def gen_conv(kernel, g: dict, oexp: AluExp, numerics: str, name: str, params: st
              need: dict, tile: dict, a_gather_fns: Optional[str] = None):
     """KernelSource of the patch-in-LDS convolution for a GEMM whose B operand `oexp` is a stride-1 window walk, or None
     when the shape is outside what the template covers (it then stays on the generic gather loaders)."""
-    from .kernelgen import KernelSource, LaunchStep, _prelude, fill, template
+    from .kernelgen import Early, KernelSource, LaunchStep, _prelude, fill, template
 
     if g.get("b_k0") != g["K"] or (a_gather_fns is None and g["a_k0"] != g["K"]) or len(g["batch"]) > 1:
         return None
@@ -237,28 +237,30 @@ def gen_conv(kernel, g: dict, oexp: AluExp, numerics: str, name: str, params: st
     if not CS or C % CS or cv["KW"] * CS * P * 2 > 160 * 1024:
         return None
     sb_c = g["batch"][0][3] if g["batch"] else 0
+    # the filter through its view, or through its element loader (the flipped, transposed filter of a cotangent), which takes
+    # every buffer of the kernel and reads this one
+    if a_gather_fns is None:
+        value = f"w[{g['a_off']}ll + (long long)o * {g['a_sm']}ll + (long long)(c * {cv['T']} + tap) * {g['a_sk']}ll]"
+    else:
+        value = f"jh_gather_a(o, c * {cv['T']} + tap, 0, 0, 0{''.join(', w' if i == g['gid_a'] else ', nullptr' for i in range(kernel.nargs))})"
+    weights = fill(template("conv_weights.hip.inc"), dict(GATHER_FNS=a_gather_fns or "", W_T="jh_f16", T=cv["T"], O=O, C=C, VALUE=value, SPACE="jh_0"))
     src = _prelude(numerics) + fill(template("conv_f16.hip.inc"), dict(
         OW=OW, OWP=OWP, OH=cv["OH"], W=cv["W"], H=cv["H"], KH=cv["KH"], KW=cv["KW"], PH=cv["PH"], PW=cv["PW"], C=C, O=O,
         SC=cv["SC"], SB=cv["SB"], NB=cv["NB"], BM=BM, BN=BN, WM=WM, WN=WN, CS=CS, R=R, P=P, G=G, SMAX=smax,
         SX=SX, SY=SY, RP=RP, QMIN=qmin, XCH=int(xch),
         EPILOGUE_FN=epi_fn, EPILOGUE_ARGS=epi_args, NAME=name, PARAMS=params, IMG_PTR=names[cv["gid"]],
-        A_GATHER=0 if a_gather_fns is None else 1, A_GATHER_FNS=a_gather_fns or "",
-        A_OFF=g["a_off"], A_SM=g["a_sm"], A_SK=g["a_sk"], C_SM=g["c_sm"], C_SN=g["c_sn"], C_SB=sb_c))
+        WEIGHTS=weights, C_SM=g["c_sm"], C_SN=g["c_sn"], C_SB=sb_c))
     T = cv["T"]
     total_w = T * O * C
     nargs = kernel.nargs
-    if a_gather_fns is None:
-        prep_args = [("in", g["gid_a"]), ("scratch", 0)]
-    else:  # the element loader of a gathered filter takes every buffer of the kernel
-        prep_args = [("in", i) for i in range(nargs)] + [("out", 0), ("scratch", 0)]
-    prep = LaunchStep(name + "_wprep", (-(-total_w // 256), 1, 1), (256, 1, 1), 0, prep_args)
+    prep = LaunchStep(name + "_wprep", (-(-total_w // 256), 1, 1), (256, 1, 1), 0, [("in", g["gid_a"]), ("scratch", 0)])
     tiles = n_tiles * (O // BM) * cv["NB"]
     main = LaunchStep(name, (tiles, 1, 1), (64 * WM * WN, 1, 1), 0,
                       [("in", i) for i in range(nargs)] + [("out", 0), ("scratch", 0)])
     need = dict(need)
-    if a_gather_fns is None:
+    if a_gather_fns is None:  # (the element loader's extents are in already)
         need[g["gid_a"]] = max(need.get(g["gid_a"], 0), g["a_len"] * 2)
     need[cv["gid"]] = max(need.get(cv["gid"], 0), ((cv["NB"] - 1) * cv["SB"] + (C - 1) * cv["SC"] + cv["H"] * cv["W"]) * 2)
     info = dict(BM=BM, BN=BN, WM=WM, WN=WN, BK=16, direct_lds=False, tiles=tiles, M=O, N=g["N"], K=g["K"], nbatch=cv["NB"], splitk=1,
                 conv=dict(cv, CS=CS, R=R, P=P, G=G, OWP=OWP, exchange=bool(xch)), gather=dict(a="none" if a_gather_fns is None else "element (pre-pass)", b="patch"))
-    return KernelSource([src], [prep, main], [total_w * 2], "gemm", need, info)
+    return KernelSource([src], [prep, main], [total_w * 2], "gemm", need, info, early=Early(weights, g["gid_a"], -(-total_w // 256), total_w * 2))

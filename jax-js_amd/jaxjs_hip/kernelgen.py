@@ -52,6 +52,16 @@ class LaunchStep:
 
 
 @dataclass
+class Early:
+    """A first step that only lays an input out in scratch buffer 0: `jh_weights` in the namespace jh_0 of `text`, over workgroups
+    of 256.  Several such steps can share a launch (`composite.Weights`)."""
+    text: str
+    gid: int
+    blocks: int
+    bytes: int
+
+
+@dataclass
 class KernelSource:
     sources: List[str]
     steps: List[LaunchStep]
@@ -62,6 +72,7 @@ class KernelSource:
     info: Dict[str, object] = field(default_factory=dict)
     # Scratch buffers (indices) that must hold zeros before the executable's first launch; the kernels leave them zeroed.
     zeroed_scratch: List[int] = field(default_factory=list)
+    early: Optional[Early] = None
 
 
 def _used_args(nargs: int, *exps: Optional[AluExp]) -> List[Optional[DType]]:

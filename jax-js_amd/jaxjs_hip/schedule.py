@@ -16,7 +16,7 @@ from typing import Any, Dict, List, Optional, Sequence
 
 from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
-from .composite import MAPS_MOST, Maps, joins_maps
+from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
 from .kernelgen import generate
 from .routine import Routine
@@ -35,6 +35,7 @@ class Unit:
     def __init__(self, source, inputs: Sequence[int], outputs: Sequence[int], **options):
         self.source, self.inputs, self.outputs, self.options = source, list(inputs), list(outputs), options
         self.exe = None
+        self.early: Optional[int] = None  # the buffer that holds what this unit's first step would make (see `Weights`)
 
 
 _LONG_OPS = (AluOp.Erf, AluOp.Erfc, AluOp.Sin, AluOp.Cos, AluOp.Asin, AluOp.Atan)  # dozens of instructions each
@@ -212,7 +213,7 @@ def place_intermediates(units: Sequence[Unit], sizes: Dict[int, int], keep) -> D
         for b in u.outputs:
             first.setdefault(b, k)
             last[b] = k
-        for b in u.inputs:
+        for b in u.inputs + ([u.early] if u.early is not None else []):
             if b in first:
                 last[b] = k
     placed: Dict[int, int] = {-1: 0}
@@ -246,7 +247,6 @@ class Schedule:
         self._sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
         self._made = list(dict.fromkeys(o for o in prog.outputs if o >= prog.nargs))
         self._increfs = [s.output for s in prog.steps if s.kind == "incref"]
-        self._work = place_intermediates(self.units, self._sizes, set(self._made))
         self._lock = threading.Lock()
         pinned = []
         try:  # a unit that is prepared here must not push out one that was prepared before it
@@ -254,10 +254,33 @@ class Schedule:
                 u.exe = backend.prepareSync(u.source, **u.options)
                 backend.pin(u.exe)
                 pinned.append(u.exe)
+            for u in self._weights():
+                u.exe = backend.prepareSync(u.source)
+                backend.pin(u.exe)
+                pinned.append(u.exe)
+                self.units.insert(0, u)
+            self._work = place_intermediates(self.units, self._sizes, set(self._made))
             self._bind()
         finally:
             for exe in pinned:
                 backend.unpin(exe)
+
+    def _weights(self) -> List[Unit]:
+        """Launches that lay out the weights of several units, which read them from the program's inputs, into buffers of the call."""
+        found = [u for u in self.units if isinstance(u.source, Kernel) and u.source.size and u.exe.data.ks.early is not None
+                 and u.inputs[u.exe.data.ks.early.gid] < self.prog.nargs]
+        out = []
+        for at in range(0, len(found), WEIGHTS_MOST):
+            group = found[at:at + WEIGHTS_MOST]
+            if len(group) < 2:
+                continue
+            sources = [u.exe.data.ks for u in group]
+            for u, ks in zip(group, sources):
+                u.early = max([*self._sizes, self.prog.nargs - 1, *(i for v in self.units for i in v.inputs + v.outputs)]) + 1
+                self._sizes[u.early] = ks.early.bytes
+            ids = [u.inputs[ks.early.gid] for u, ks in zip(group, sources)]
+            out.append(Unit(Weights([u.source for u in group], sources, ids), ids, [u.early for u in group]))
+        return out
 
     def _bind(self) -> None:
         """The native launch list.  Buffer table: inputs, outputs made here, workspace."""
@@ -284,12 +307,14 @@ class Schedule:
                     self._need[b] = max(self._need.get(b, 0), need)
                 elif self._sizes[b] < need:
                     raise ValueError(f"buffer {b} holds {self._sizes[b]} bytes, its reader addresses {need}")
-            for step, fn in zip(prep.ks.steps, prep.functions):
+            for k, (step, fn) in enumerate(zip(prep.ks.steps, prep.functions)):
+                if k == 0 and u.early is not None:
+                    continue
                 c = LaunchStepC(fn, (ctypes.c_uint32 * 3)(*step.grid), (ctypes.c_uint32 * 3)(*step.block), step.shared, len(step.args))
                 steps.append(c)
                 for kind, i in step.args:
-                    if kind in ("in", "out"):
-                        b = (u.inputs if kind == "in" else u.outputs)[i]
+                    if kind in ("in", "out") or (kind, i) == ("scratch", 0) and u.early is not None:
+                        b = u.inputs[i] if kind == "in" else u.outputs[i] if kind == "out" else u.early
                         refs.append(LaunchRef(0, table[b]) if b in table else LaunchRef(self._work[b], self._workspace))
                     else:
                         refs.append(LaunchRef(prep.scratch[i] if kind == "scratch" else int(i), -1))

@@ -141,3 +141,37 @@ def test_infinities_and_nans_reach_the_taps_that_see_them(size):
     want, _ = reference(x, ct, 3, 3, SAME(3))
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
     np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)].astype(np.float16).astype(np.float64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(2, 64, 64, 12, 3), (3, 128, 64, 10, 3)], ids=str)
+def test_weights_of_several_convolutions_are_laid_out_by_one_launch(shape):
+    """Two convolutions of the same Kernel over different filters, one behind them, a cotangent that reads its filter flipped, and
+    one whose filter the program computes (it keeps its own pre-pass); small integers, twice over with the filters exchanged."""
+    from jaxjs_hip.composite import Weights
+    from jaxjs_hip.schedule import Schedule
+    from jit_util import run_program
+    from oracle.backend import OracleBackend
+    B, C, O, S, K = shape
+    p, q = ConvParams(0, [1, 1], [(K // 2, K // 2)] * 2, [1, 1], [1, 1]), ConvParams(0, [1, 1], [(0, 0)] * 2, [1, 1], [1, 1])
+    rng = np.random.default_rng(C)
+    x = rng.integers(-1, 2, (B, C, S, S)).astype(np.float16)
+    w1, w2 = (((rng.random((O, C, K, K)) < 0.2) * rng.integers(-1, 2, (O, C, K, K))).astype(np.float16) for _ in range(2))
+    w3 = ((rng.random((64, O, 1, 1)) < 0.1) * rng.integers(-1, 2, (64, O, 1, 1))).astype(np.float16)
+
+    def f(x, w1, w2, w3):
+        a, b = J.conv(x, w1, p), J.conv(x, w2, p)
+        return [a, b, J.conv(a, w3, q), J.convTransposeLhs(b, w2, [B, C, S, S], p), J.conv(x, w1.mul(2.0).add(w2), p)]
+    prog = J.jit(f, [ShapedArray(v.shape, DType.Float16) for v in (x, w1, w2, w3)])
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    sch = Schedule(backend(), prog)
+    assert isinstance(sch.units[0].source, Weights) and len(sch.units[0].outputs) == 3 and sum(isinstance(u.source, Weights) for u in sch.units) == 1
+    assert len({u.early for u in sch.units if u.early is not None}) == len(sch.units[0].outputs)
+    before = backend().live_slots()
+    for arrays in ([x, w1, w2, w3], [x, w2, w1, w3]):
+        got, want = run_program(backend(), prog, arrays), run_program(OracleBackend(), prog, arrays)
+        for a, b in zip(got, want):
+            assert np.abs(b.astype(np.float32)).max() <= 2048
+            np.testing.assert_array_equal(a, b)
+    assert backend().live_slots() == before
