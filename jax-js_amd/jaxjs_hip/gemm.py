@@ -618,6 +618,19 @@ def few_plan(t: TuneResult) -> Optional[dict]:
     return plan_few(g, lambda: choose_tile(g))
 
 
+def _flipped_filter(g: dict) -> bool:
+    """Whether a product of two gather operands whose k axis would be cut is left whole where it is the cotangent of a
+    convolution towards its image, so that the patch template takes it and reads the flipped filter through its pre-pass.  The
+    slices read both operands element by element; the template's time is its walk over k, whatever the tiles (9 us per 1000 of
+    k up to one tile a CU).  Of 119 shapes ([2..32, 64..512, 7..56 square], windows of 3 and 5) all 93 with k <= 4096 gain,
+    1.16 to 4.6 times ([32,256,14,14] 3x3 93.5 -> 30.9 us, [16,64,28,28] 5x5 50.1 -> 22.7); behind a longer axis few tiles
+    lose (2 x [512,7,7] 41.6 against 53.5 us in 16 tiles, 52.2 against 54.3 in 64) and from 100 tiles on it gains
+    (65.6 -> 55.1 in 128).  Same error against double sums."""
+    if g["dtype"] != DType.Float16 or not (g.get("a_gather") and g.get("b_gather")) or len(g["batch"]) != 1:
+        return False
+    return g["K"] <= 4096 or -(-g["M"] // 64) * -(-g["N"] // 128) * g["batch"][0][0] >= 96
+
+
 def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None, behind=None, few=None) -> KernelSource:
     """`rows`: the rows of the short operand of a contraction that `few_plan` takes, made in the same launch (a `RowText` whose
     inputs come behind the kernel's).  `behind`: what happens to the result's rows in the same launch, under the plan `few` (a
@@ -652,6 +665,14 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
         if (K_full % split or (K_full // split) % vec_k
                 or any(g[t + "_k0"] != K_full and (K_full // split) % g[t + "_k0"] and g[t + "_k0"] % (K_full // split) for t in ("a", "b"))):
             split = 1
+    if split > 1 and not override and not wgrad and _flipped_filter(g):
+        import copy
+
+        t2 = copy.copy(t)
+        t2.params = dict(t.params, gemm_tile=(("BM", 128), ("BN", 128), ("SPLITK", 1)))
+        whole = gen_gemm(kernel, t2, numerics, name)
+        if whole.info.get("conv"):
+            return whole
     # ... or, with FUSEK (f32 template), folded inside the same launch by the slice that arrives last at the tile's
     # counter: one launch instead of two.
     fusek = 0

@@ -181,3 +181,31 @@ def test_weights_of_several_convolutions_are_laid_out_by_one_launch(shape):
             assert np.abs(v).max() <= 2048
             np.testing.assert_array_equal(u.astype(np.float32), v.reshape(u.shape))
     assert backend().live_slots() == before
+
+
+def image_cotangent(B, C, O, S, K):
+    p = ConvParams(0, [1, 1], [(K // 2, K // 2)] * 2, [1, 1], [1, 1])
+    rng = np.random.default_rng(B * C + S)
+    ct, w = (rng.integers(-3, 4, s).astype(np.float16) for s in ((B, O, S, S), (O, C, K, K)))
+    prog = J.jit(lambda ct, w: [J.convTransposeLhs(ct, w, [B, C, S, S], p)], [ShapedArray(v.shape, DType.Float16) for v in (ct, w)])
+    return next(s.kernel for s in prog.steps if s.kind == "execute"), ct, w
+
+
+@pytest.mark.parametrize("shape,patch", [((2, 128, 128, 14, 3), True), ((3, 64, 64, 13, 5), True), ((2, 64, 256, 10, 3), True), ((4, 64, 192, 14, 5), False), ((24, 64, 192, 14, 5), False),
+                                         ((48, 64, 192, 14, 5), True)], ids=str)
+def test_the_cotangent_towards_the_image_is_left_whole(shape, patch):
+    """Both sides of the rule: up to k = 4096, and behind it by the number of tiles."""
+    kernel, *_ = image_cotangent(*shape)
+    assert (generate(kernel, "fast").info.get("conv") is not None) == patch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(2, 128, 128, 14, 3), (3, 64, 64, 13, 5), (2, 64, 256, 10, 3), (2, 64, 128, 7, 3)], ids=str)
+def test_the_cotangent_towards_the_image_by_patches(shape):
+    """Small integers: every sum is exact up to its rounding to float16."""
+    B, C, O, S, K = shape
+    kernel, ct, w = image_cotangent(*shape)
+    got = device_run(kernel, [v.reshape(-1) for v in (ct, w)])[0].reshape(B, C, S, S)
+    windows = np.lib.stride_tricks.sliding_window_view(np.pad(ct.astype(np.float32), [(0, 0)] * 2 + [(K // 2,) * 2] * 2), (K, K), (2, 3))
+    want = np.tensordot(windows, w.astype(np.float32).transpose(1, 0, 2, 3)[:, :, ::-1, ::-1], ([1, 4, 5], [1, 2, 3])).transpose(0, 3, 1, 2)
+    np.testing.assert_array_equal(got, want.astype(np.float16))
