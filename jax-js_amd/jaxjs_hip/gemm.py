@@ -622,7 +622,7 @@ def _flipped_filter(g: dict) -> bool:
     """Whether a product of two gather operands whose k axis would be cut is left whole where it is the cotangent of a
     convolution towards its image, so that the patch template takes it and reads the flipped filter through its pre-pass.  The
     slices read both operands element by element; the template's time is its walk over k, whatever the tiles (9 us per 1000 of
-    k up to one tile a CU).  Of 119 shapes ([2..32, 64..512, 7..56 square], windows of 3 and 5) all 93 with k <= 4096 gain,
+    k up to one tile a CU).  Of 120 shapes ([2..32, 64..512, 7..56 square], windows of 3 and 5) all 90 with k <= 4096 gain,
     1.16 to 4.6 times ([32,256,14,14] 3x3 93.5 -> 30.9 us, [16,64,28,28] 5x5 50.1 -> 22.7); behind a longer axis few tiles
     lose (2 x [512,7,7] 41.6 against 53.5 us in 16 tiles, 52.2 against 54.3 in 64) and from 100 tiles on it gains
     (65.6 -> 55.1 in 128).  Same error against double sums."""
