@@ -6,6 +6,9 @@ accumulation onto repeated destinations (atomic adds in any order: compared with
 its sines and cosines from the device math library, whose last-place differences from the host's can decide a
 float32 rounding tie in a butterfly (seen for radix-3 stages behind an even stride; power-of-two and prime sizes come
 out bit-identical): compared within 1e-5 of the row's largest magnitude."""
+import itertools
+import math
+
 import numpy as np
 import pytest
 
@@ -84,6 +87,42 @@ def test_cholesky_pivots_that_are_no_ordinary_numbers(n, dt):
     a = np.stack(mats)
     got, want, _ = both(R.cholesky(a), [a])
     assert_bits(got, want, f"cholesky {n} {np.dtype(dt).name}")
+
+
+def _squares(total, bits):
+    """Whole numbers of at most `bits` bits whose squares add up to `total`, the larger ones first."""
+    parts = []
+    while total > 4000:
+        m = math.isqrt(total)
+        low = max(0, m.bit_length() - bits)
+        parts.append(m >> low << low)
+        total -= parts[-1] ** 2
+    for a, b, c in itertools.product(range(math.isqrt(total) + 1), repeat=3):
+        d = total - a * a - b * b - c * c
+        if d >= 0 and math.isqrt(d) ** 2 == d:
+            return parts + [a, b, c, math.isqrt(d)]
+
+
+@pytest.mark.parametrize("dt,bits", [(F32, 24), (np.float16, 11)], ids=["float32", "float16"])
+@pytest.mark.parametrize("before", [0, 5, 26, 40])
+def test_cholesky_pivots_whose_root_is_subnormal(before, dt, bits):
+    """A pivot that products cancel down to a few units of the product of two smallest numbers: its rounded root is far from the
+    root itself (1 for 1.41), and the quotients below are by the rounded one.  Inside a panel, across two and in the second."""
+    unit = 2.0 ** -149 if dt == F32 else 2.0 ** -24  # smallest number of the type
+    mats, pivots = [], []
+    for left in (1, 2, 3, 5, 6, 7, 30, 200, 2000):  # what is left of the pivot, in units squared
+        parts = _squares(int(1 / unit) - left, bits)
+        p = before + len(parts)
+        a = np.eye(before + 48)
+        a[p, before:p] = np.array(parts, dtype=np.float64) * unit
+        a[p, p] = unit
+        a[p + 1:, before] = -unit * np.arange(1, len(a) - p)
+        mats.append(a.astype(dt))
+        pivots.append((p, dt(math.sqrt(left) * unit)))
+    a = np.stack(mats)
+    got, want, _ = both(R.cholesky(a), [a])
+    assert np.isfinite(want[0]).all() and [w[p, p] for w, (p, _) in zip(want[0], pivots)] == [v for _, v in pivots]
+    assert_bits(got, want, f"cholesky {a.shape} {np.dtype(dt).name}")
 
 
 def test_cholesky_not_positive_definite_and_empty():
