@@ -212,6 +212,17 @@ def test_jacobi_eigh_by_blocks_at_ragged_orders(n):
     assert_bits(got, want, f"jacobi_eigh {n} {ks.info}")
 
 
+@pytest.mark.parametrize("dt", [np.float16, F32, np.float64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("n", [16, 31, 35, 61, 64, 65])
+def test_jacobi_eigh_by_blocks_around_half_a_wave_per_block(n, dt):
+    """Fewer rows above a block than half a wave has lanes, as many, more; a partial last block; the order behind."""
+    a = RNG.standard_normal((2, n, n))
+    sym = (a + np.swapaxes(a, -1, -2)).astype(dt)
+    got, want, ks = both(R.jacobi_eigh(sym, 2, 0.0), [sym])
+    assert ks.info["block"] == 4
+    assert_bits(got, want, f"jacobi_eigh {n} {np.dtype(dt).name}")
+
+
 @pytest.mark.parametrize("scale", [1e-44, 1e-30, 1e30, 1e38])
 @pytest.mark.parametrize("n", [14, 65])
 def test_jacobi_eigh_at_the_ends_of_the_element_range(n, scale):
