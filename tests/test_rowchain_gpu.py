@@ -43,6 +43,16 @@ def check(prog, arrays, f16, chained=True, terms=0):
             np.testing.assert_allclose(g.astype(np.float64), w.astype(np.float64), rtol=1e-2 if f16 else 2e-5, atol=2e-3 + (3 * 2.0 ** -9 if terms else 0) if f16 else 2e-6 + 8 * terms ** 0.5 * 2.0 ** -23)
 
 
+class OneByOne:
+    """A program whose Kernels are dispatched one after the other, each in a launch of its own."""
+
+    def __init__(self, prog):
+        self.consts, self.steps, self.outputs, self.prog = prog.consts, prog.steps, prog.outputs, prog
+
+    def execute(self, be, slots):
+        return self.prog.execute(be, slots, {k: be.prepareKernelSync(s.kernel) for k, s in enumerate(self.steps) if s.kind == "execute"})
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=str)
 @pytest.mark.parametrize("dtype", [DType.Float32, DType.Float16], ids=lambda d: d.value)
 @pytest.mark.parametrize("op", list(OPS))
@@ -115,7 +125,8 @@ def test_largest_and_smallest_of_rows_with_values_that_are_no_ordinary_numbers(o
 @pytest.mark.parametrize("count", [2, 8, 11])
 @pytest.mark.parametrize("size", [1, 7, 1000, 262145])
 def test_elementwise_kernels_side_by_side(count, size):
-    """Sizes off the vector width, several types, more Kernels than one launch takes; a masked read; one operand for all."""
+    """Sizes off the vector width, several types, more Kernels than one launch takes; a masked read; one operand for all.  The
+    same bits as from the Kernels dispatched one by one."""
     rng = np.random.default_rng(size)
     arrays = [rng.standard_normal(size).astype(np.float16 if i % 3 == 2 else np.float32) for i in range(count)]
     arrays.append(rng.integers(-9, 9, size).astype(np.int32))
@@ -125,6 +136,8 @@ def test_elementwise_kernels_side_by_side(count, size):
     prog = J.jit(f, [ShapedArray(x.shape, {"f": DType.Float32, "e": DType.Float16, "i": DType.Int32}[x.dtype.char]) for x in arrays])
     assert [len(u.outputs) for u in plan_units(prog)] == {2: [3], 8: [8, 1], 11: [8, 4]}[count]
     check(prog, arrays, True, chained=False)
+    for i, (together, apart) in enumerate(zip(run_program(backend(), prog, arrays), run_program(backend(), OneByOne(prog), arrays))):
+        assert together.dtype == apart.dtype and together.tobytes() == apart.tobytes(), i
 
 
 @pytest.mark.parametrize("rows,k,n", [(2, 256, 130), (16, 100, 200), (5, 100, 333), (8, 768, 2304), (13, 333, 777), (33, 256, 260), (64, 512, 1000), (8, 2048, 512)], ids=str)
