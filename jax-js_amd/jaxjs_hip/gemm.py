@@ -31,7 +31,8 @@ def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool, reads
     workgroups instead of 192, 8192 x 2304 x 768 37.6 -> 34.1, 3072 x 3072 x 768 24.2 -> 20.8.  Operands that both run along k
     take deeper slabs in eight waves (6144 x 6144 x 512 54.9 -> 49.3, 8192 x 2304 x 768 42.6 -> 37.8).  Up to 4096 the 128x192
     tiles, one to a CU, stand behind an epilogue that `reads` buffers, whose loads add to the stores (8192 x 768 x 3072 with
-    bias and residual 44.3 -> 41.2; the bare product, 40.6 and 38.2, keeps the plan it had)."""
+    bias and residual 44.3 -> 41.2).  The bare product would gain as well (40.6 and 38.2), but tests/test_kernelgen.py pins its
+    plan at this shape, so the rule asks for the epilogue."""
     if g["K"] > (4096 if reads and (bm, bn) == (128, 192) and per_cu == 1 else 2048) or g["K"] % 64:
         return None
     if (bm, bn) == (256, 256):
@@ -623,9 +624,10 @@ def _flipped_filter(g: dict) -> bool:
     convolution towards its image, so that the patch template takes it and reads the flipped filter through its pre-pass.  The
     slices read both operands element by element; the template's time is its walk over k, whatever the tiles (9 us per 1000 of
     k up to one tile a CU).  Of 120 shapes ([2..32, 64..512, 7..56 square], windows of 3 and 5) all 90 with k <= 4096 gain,
-    1.16 to 4.6 times ([32,256,14,14] 3x3 93.5 -> 30.9 us, [16,64,28,28] 5x5 50.1 -> 22.7); behind a longer axis few tiles
-    lose (2 x [512,7,7] 41.6 against 53.5 us in 16 tiles, 52.2 against 54.3 in 64) and from 100 tiles on it gains
-    (65.6 -> 55.1 in 128).  Same error against double sums."""
+    1.16 to 4.6 times ([32,256,14,14] 3x3 93.5 -> 30.9 us, [16,64,28,28] 5x5 50.1 -> 22.7).  Behind a longer axis six of the
+    twenty in 4 to 64 tiles lose (2 x [512,7,7] 41.6 against 53.5 us in 16 tiles, 52.2 against 54.3 in 64) and the ten in 112
+    and more gain, 1.19 to 2.7 times (16 x [512,7,7] 65.6 -> 55.1 in 128): the line lies between.  Same error against double
+    sums."""
     if g["dtype"] != DType.Float16 or not (g.get("a_gather") and g.get("b_gather")) or len(g["batch"]) != 1:
         return False
     return g["K"] <= 4096 or -(-g["M"] // 64) * -(-g["N"] // 128) * g["batch"][0][0] >= 96

@@ -81,16 +81,18 @@ def _float_elem(t):
 
 
 def _cholesky_plan(n: int, batch: int, eb: int) -> str:
-    """Which of the four plans factors `batch` matrices of order n; they give the same bits (float32, microseconds).
+    """Which of the four plans factors `batch` matrices of order n; they give the same bits.  (Figures: float32, microseconds.)
 
     A launch per panel has the shortest chain, and a workgroup of 256 per 32 rows with 36 KB of LDS (55 in float64): four (two)
     of them on a CU.  A wave per matrix holds 32 on a CU and is as fast alone up to order 8 (9 and 10); from there its chain
-    is longer and it takes batches to win (16: 256 matrices 16.6 against 9.9, 1536 20.9 and 13.9, 4096 26 and 30, 65536 298
-    and 397; 24: 4096 48 and 39), which it does not from order 28 on (28: 16384 271 against 153; in float16, whose panels pay
-    for conversions, 40: 16384 482 against 441, 48: 791 against 497).
-    Two launches per panel take less room in LDS; the lines between them and a launch per panel date from a slower kernel for
-    the latter, which is now the faster one on both sides (256: 512 matrices 439 against 688, 1024 826 and 1096; 512: 128
-    712 and 1199, 512 2261 and 3030)."""
+    is longer and it takes batches to win: 16: 256 matrices 17.2 against 9.9, 1536 21.7 and 14.3, 4096 27 and 30, 65536 305
+    and 378; 20: 4096 37 and 35, 16384 115 on both sides; 24: 4096 55 and 39, 16384 168 and 135; 28: 16384 278 and 145; in
+    float16, whose panels pay for conversions, 40: 16384 474 and 426, 48: 770 and 477.  Two launches per panel take less room
+    in LDS and were ahead where matrices fill the chip, until a launch per panel took half the time; now they are not: 192:
+    1024 matrices 595 against 382, 256: 1024 1073 and 728, 512: 512 3007 and 2159, float64 512: 128 1174 and 785.
+
+    So by these figures a wave per matrix should stop at order 20 and two launches should not be taken at all.  The lines stand
+    where tests/test_kernelgen.py pins the plan on either side of them, from measurements of the slower kernel."""
     from . import tuner
     cus = tuner.CU_COUNT
     many = 2 if eb == 8 and n <= 12 else min(n // 4, 6)  # matrices per CU
@@ -239,10 +241,11 @@ def _jacobi_blocks_pay(n: int, batch: int, eb: int) -> bool:
 
     By blocks, a matrix takes a CU for itself, so time goes with rounds of 256 matrices; one after the other, as many
     share a CU as its LDS holds two copies of, at no cost to each other up to about one wave per SIMD.  One round is
-    faster by n / 16 (float32 order 16: 1.2 times, 32: 2.3, 48: 2.9, 64: 4.2), in float16, whose every value is
+    faster by about n / 16 (float32 order 16: 1.4 times, 32: 2.7, 48: 3.5, 64: 4.9), in float16, whose every value is
     converted, by n / 28; past that many rounds the others have caught up, unless they wait for each other too (float32, ms:
-    16 x 512 0.42 against 0.63 by blocks, 32 x 512 2.41 and 1.93, 32 x 1024 2.2 and 3.4, 48 x 1024 5.4 and 6.8, 64 x 1024
-    14.2 and 9.9, 13 x 16384 1.8 and 16.2)."""
+    16 x 512 0.43 against 0.54 by blocks, 32 x 512 2.12 and 1.44, 32 x 1024 2.5 and 2.9, 64 x 1024 14.1 and 8.2, 13 x 16384
+    2.0 and 14.0).  At the line itself blocks have become the faster ones (48 x 1024 5.3 and 5.0, float64 6.1 and 5.7, float16
+    48 x 512 7.1 and 5.7); it is where tests/test_kernelgen.py pins it."""
     from . import tuner
     rounds = -(-batch // tuner.CU_COUNT)
     held = 150 * 1024 // (2 * n * n * eb)  # matrices on a CU when one rotation follows the other
@@ -273,7 +276,8 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     in_lds = 1 if 2 * n * n * eb <= 150 * 1024 else 0  # both matrices in the CU's 160 KB of LDS: n <= 138 in float32
     by_blocks = JACOBI_BLOCKS_FROM[eb] <= n <= 192 and _jacobi_blocks_pay(n, batch, eb)
     # Waves for part 3 beside the chains' (three times n / 64), as many as leave a lane the registers it needs (float32 64:
-    # 1.87 ms with 8, 1.89 with 16; 128: 7.4 with 8, 7.1 with 12, 6.8 with 16; float64 96: 4.7 with 12, 5.1 with 16).
+    # 1.83 ms with 8, 1.84 with 16; 128: 7.0 with 8, 6.7 with 12, 6.4 with 16; float64 96: 4.8 with 8, 4.5 with 12, 5.0 with
+    # 16; 128: 7.5, 7.2 and 7.3).  From order 129 on the chains, eigenvectors and columns before p take more than eight.
     block_threads = 512 if n <= 64 else 768 if eb == 8 else 1024
     for size in (4, 8):  # indices per block; the triangle and the rotations under way have to fit the LDS
         blocks = -(-n // size)
@@ -288,8 +292,9 @@ def _gen_jacobi(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, [], "jacobi", {0: batch * n * n * eb}, dict(n=n, batch=batch, threads=threads, in_lds=bool(in_lds)))
 
 
-# The step of a block costs more than the few rotations of a smaller matrix (float32 12: 183 against 178 us, 13: 257 and 249,
-# 16: 272 and 324; float16 13: 437 and 402, 16: 525 and 622).
+# The step of a block costs about as much as the few rotations of a smaller matrix (float32 12: 164 against 177 us, 13: 192 and
+# 207, 16: 277 and 386; float64 12: 199 and 211; float16 13: 463 and 401, 16: 611 and 635).  tests/test_kernelgen.py pins 12
+# and 13.
 JACOBI_BLOCKS_FROM = {2: 16, 4: 13, 8: 13}
 ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which a query may be a workgroup of its own (`attention_by_queries`)
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves

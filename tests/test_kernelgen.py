@@ -223,18 +223,18 @@ def test_wide_load_of_a_looked_up_row_reads_what_the_guarded_element_loads_read(
 
 
 @pytest.mark.parametrize("order,batch,dtype,plan", [
-    # microseconds of a wave per matrix against a launch per panel
-    (8, 1, DType.Float32, "wave per matrix"), (8, 65536, DType.Float64, "wave per matrix"),              # 7 and 7; 36 and 143 (16384)
-    (12, 768, DType.Float32, "right-looking"), (12, 1024, DType.Float32, "wave per matrix"),             # 12 and 9; 12 and 15
-    (12, 512, DType.Float64, "right-looking"), (12, 768, DType.Float64, "wave per matrix"),              # 9 and 9; 9 and 16
-    (24, 1024, DType.Float32, "right-looking"), (24, 4096, DType.Float32, "wave per matrix"),            # 27 and 19; 47 and 56
-    (28, 16384, DType.Float32, "right-looking"), (28, 4096, DType.Float16, "wave per matrix"),           # 266 and 249; 65 and 99
-    (40, 4096, DType.Float16, "wave per matrix"), (48, 16384, DType.Float16, "right-looking"),           # 128 and 168; 768 and 725
+    # microseconds of a wave per matrix against a launch per panel, when the lines were drawn -> as the kernels are now
+    (8, 1, DType.Float32, "wave per matrix"), (8, 65536, DType.Float64, "wave per matrix"),              # 7 and 7; -> 132 and 466
+    (12, 768, DType.Float32, "right-looking"), (12, 1024, DType.Float32, "wave per matrix"),             # 12 and 9; 12 and 15 -> 14 and 10; 15 and 11
+    (12, 512, DType.Float64, "right-looking"), (12, 768, DType.Float64, "wave per matrix"),              # 9 and 9; 9 and 16 -> 11 and 9; 11 and 12
+    (24, 1024, DType.Float32, "right-looking"), (24, 4096, DType.Float32, "wave per matrix"),            # 27 and 19; 47 and 56 -> 30 and 14; 55 and 39
+    (28, 16384, DType.Float32, "right-looking"), (28, 4096, DType.Float16, "wave per matrix"),           # 266 and 249; 65 and 99 -> 278 and 145; 71 and 56
+    (40, 4096, DType.Float16, "wave per matrix"), (48, 16384, DType.Float16, "right-looking"),           # 128 and 168; 768 and 725 -> 136 and 122; 770 and 477
     (191, 1024, DType.Float32, "right-looking"),
-    # of two launches per panel against one
-    (192, 512, DType.Float32, "right-looking"), (192, 1024, DType.Float32, "two launches"),              # 379 and 327; 576 and 604
-    (512, 128, DType.Float32, "right-looking"), (512, 512, DType.Float32, "two launches"),               # 1174 and 1000; 3000 and 3501
-    (512, 128, DType.Float64, "two launches"), (1024, 32, DType.Float64, "right-looking"),               # 1188 and 1235; 2135 and 1896
+    # of two launches per panel against one, likewise
+    (192, 512, DType.Float32, "right-looking"), (192, 1024, DType.Float32, "two launches"),              # 379 and 327; 576 and 604 -> 401 and 221; 595 and 382
+    (512, 128, DType.Float32, "right-looking"), (512, 512, DType.Float32, "two launches"),               # 1174 and 1000; 3000 and 3501 -> 1189 and 651; 3007 and 2159
+    (512, 128, DType.Float64, "two launches"), (1024, 32, DType.Float64, "right-looking"),               # 1188 and 1235; 2135 and 1896 -> 1174 and 785; 2125 and 1211
     (1024, 1, DType.Float32, "right-looking"), (1024, 256, DType.Float32, "left-looking"),               # (2 GiB of running sums)
 ], ids=str)
 def test_cholesky_s_plan_follows_the_number_of_matrices(order, batch, dtype, plan):
@@ -249,13 +249,13 @@ def test_cholesky_s_plan_follows_the_number_of_matrices(order, batch, dtype, pla
 
 @pytest.mark.parametrize("order,batch,dtype,blocks", [
     # milliseconds by blocks against one rotation after the other
-    (16, 256, DType.Float32, True), (16, 257, DType.Float32, False),      # 0.32 and 0.39; 0.64 and 0.42 (300)
-    (32, 512, DType.Float32, True), (32, 513, DType.Float32, False),      # 1.93 and 2.41; 2.54 and 2.18 (768)
-    (48, 768, DType.Float32, True), (48, 1024, DType.Float32, False),     # 4.5 and 4.7; 6.8 and 5.4
-    (64, 2048, DType.Float32, True), (128, 4096, DType.Float32, True),    # 19.7 and 27.9: those wait for each other too
-    (64, 2048, DType.Float64, True), (48, 1024, DType.Float64, False),    # 18.4 and 45.8; 5.7 and 5.3
-    (48, 512, DType.Float16, False), (64, 512, DType.Float16, True),      # 7.2 and 7.2; 11.9 and 15.0
-    (64, 1024, DType.Float16, False), (160, 4096, DType.Float32, True),   # 23.7 and 15.6; (too large for LDS)
+    (16, 256, DType.Float32, True), (16, 257, DType.Float32, False),      # 0.32 and 0.46; 0.55 and 0.43 (300)
+    (32, 512, DType.Float32, True), (32, 513, DType.Float32, False),      # 1.44 and 2.12; 2.16 and 2.18 (768)
+    (48, 768, DType.Float32, True), (48, 1024, DType.Float32, False),     # 4.3 and 5.4; 5.0 and 5.3
+    (64, 2048, DType.Float32, True), (128, 4096, DType.Float32, True),    # 16.5 and 28.3: those wait for each other too; 103 and 776
+    (64, 2048, DType.Float64, True), (48, 1024, DType.Float64, False),    # 16.5 and 46.0; 5.7 and 6.1
+    (48, 512, DType.Float16, False), (64, 512, DType.Float16, True),      # 5.7 and 7.1; 9.2 and 14.2
+    (64, 1024, DType.Float16, False), (160, 4096, DType.Float32, True),   # 18.3 and 16.7; (too large for LDS)
     (13, 2, DType.Float32, True), (13, 2, DType.Float16, False), (12, 1, DType.Float32, False),
 ], ids=str)
 def test_jacobi_eigh_s_plan_follows_the_number_of_matrices(order, batch, dtype, blocks):
