@@ -155,8 +155,9 @@ int jh_launch_repeat(jh_function fn, uint32_t grid_x, uint32_t grid_y, uint32_t 
  * src/frontend/jit.ts:111-162) in one call, without host work of the caller's language between the launches.  The
  * arguments of all steps lie one after the other in `args`: an argument is the 64-bit `value` itself, or, when `buffer`
  * is not negative, the address `value` bytes behind `buffers[buffer]`.  Empty grids are skipped.  Stops at the first
- * launch that fails.  At most 128 arguments per step.
+ * launch that fails.  At most JH_LAUNCH_ARGS arguments per step.
  */
+#define JH_LAUNCH_ARGS 128
 typedef struct {
   jh_function fn;
   uint32_t grid[3], block[3];

@@ -401,7 +401,7 @@ int jh_launch_repeat(jh_function fn, uint32_t gx, uint32_t gy, uint32_t gz, uint
 int jh_launch_list(const jh_step *steps, uint32_t num_steps, const jh_arg *args, const uint64_t *buffers) {
   JH_NEED_INIT();
   if (num_steps && (!steps || !args || !buffers)) return fail(-5, "null launch list");
-  constexpr uint32_t kMaxArgs = 128;
+  constexpr uint32_t kMaxArgs = JH_LAUNCH_ARGS;
   uint64_t cells[kMaxArgs];
   void *argv[kMaxArgs];
   for (uint32_t i = 0; i < kMaxArgs; ++i) argv[i] = &cells[i];

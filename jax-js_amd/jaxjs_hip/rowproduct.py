@@ -21,6 +21,7 @@ from .composite import Composite
 from .gemm import few_plan, gen_gemm
 from .kernelgen import KernelSource
 from .rowchain import RowChain, plan_rows, row_text
+from .runtime import LAUNCH_ARGS
 from .fewgen import chain_pitch, plan_whole_rows
 
 ROWS_MOST = 64             # rows of the product: every 16 of them are made by all of its column tiles
@@ -118,7 +119,8 @@ def join_behind(kernel: Kernel, inputs: Sequence[int], buffer: int, chain: RowCh
     sums = p["waves"] * 16 * p["MT"] * (16 * p["VN"] + 1) * 4
     if lanes["iters"] * lanes["V"] > LANE_ELEMENTS or sums + rows * (chain.C + 16) * byteWidth(kernel.dtype) > LDS_BYTES:
         return None
-    return ProductRows(kernel, inputs, chain, local, p)
+    joined = ProductRows(kernel, inputs, chain, local, p)
+    return joined if len(joined.inputs) + len(chain.outputs) <= LAUNCH_ARGS else None
 
 
 def lane_plan(chain: RowChain, waves: int, rows: int, least: int = 16) -> dict:
@@ -155,4 +157,5 @@ def join_rows(chain: RowChain, buffer: int, kernel: Kernel, inputs: Sequence[int
         return None
     if dtype != g["dtype"] or (p["R"], g["K"]) != (chain.R, chain.C) or g["batch"] or g[s + "_off"] or g[p["row"][s]] != chain.C:
         return None
-    return RowProduct(chain, kernel, gid, inputs)
+    joined = RowProduct(chain, kernel, gid, inputs)
+    return joined if len(joined.inputs) + (3 if p["slices"] > 1 else 1) <= LAUNCH_ARGS else None  # (slices have sums and counters)

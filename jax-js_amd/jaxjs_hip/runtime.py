@@ -47,6 +47,9 @@ class DeviceInfo(ctypes.Structure):
     ]
 
 
+LAUNCH_ARGS = 128  # `JH_LAUNCH_ARGS`: arguments of one step of a launch list
+
+
 class LaunchStepC(ctypes.Structure):
     """`jh_step`: one launch of a list."""
     _fields_ = [("fn", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3), ("block", ctypes.c_uint32 * 3), ("shared_bytes", ctypes.c_uint32),

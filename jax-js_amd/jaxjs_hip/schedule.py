@@ -22,7 +22,7 @@ from .kernelgen import generate
 from .routine import Routine
 from .rowchain import RowChain, _tidy, collect_chain, index_form
 from .rowproduct import join_behind, join_rows
-from .runtime import LaunchRef, LaunchStepC, check
+from .runtime import LAUNCH_ARGS, LaunchRef, LaunchStepC, check
 from .shape import prod, unravelAlu
 from .tuner import match_gemm
 from .wgradgen import is_filter_cotangent
@@ -140,15 +140,17 @@ def plan_dispatches(prog) -> List[_Dispatch]:
 
 
 def adjacent_maps(steps: Sequence[_Dispatch], k: int, view) -> int:
-    """How many dispatches from `k` on are elementwise Kernels that run side by side in one launch (see `Maps`)."""
-    n, written = 0, set()
+    """How many dispatches from `k` on are elementwise Kernels that run side by side in one launch (see `Maps`), whose arguments
+    a step of a launch list takes."""
+    n, args, written = 0, 0, set()
     while n < MAPS_MOST and k + n < len(steps):
         d = steps[k + n]
-        if d.kernel is None or not joins_maps(d.kernel) or written & set(d.inputs):
+        if d.kernel is None or not joins_maps(d.kernel) or written & set(d.inputs) or args + d.kernel.nargs + 1 > LAUNCH_ARGS:
             break
         if n and collect_chain(view, k + n, lambda o, last: True) is not None:
             break  # the first of Kernels over the same rows
         written.add(d.output)
+        args += d.kernel.nargs + 1
         n += 1
     return n
 

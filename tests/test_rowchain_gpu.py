@@ -14,6 +14,7 @@ from jaxjs_hip.rowproduct import ProductRows, RowProduct
 from jaxjs_hip.schedule import plan_units
 from jit_util import run_program
 from oracle.backend import OracleBackend
+from test_schedule import WIDE, wide_programs
 
 pytestmark = pytest.mark.gpu
 OPS = {"softmax": lambda x: L.softmax(x, -1), "logsoftmax": lambda x: L.logSoftmax(x, -1), "standardize": lambda x: L.standardize(x, -1),
@@ -138,6 +139,18 @@ def test_elementwise_kernels_side_by_side(count, size):
     check(prog, arrays, True, chained=False)
     for i, (together, apart) in enumerate(zip(run_program(backend(), prog, arrays), run_program(backend(), OneByOne(prog), arrays))):
         assert together.dtype == apart.dtype and together.tobytes() == apart.tobytes(), i
+
+
+@pytest.mark.parametrize("name", WIDE)
+def test_launches_of_as_many_arguments_as_a_launch_list_takes(name):
+    """Small whole numbers: every sum is exact."""
+    prog, _ = wide_programs()[name]
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    rng = np.random.default_rng(len(name))
+    arrays = [rng.integers(-2, 3, v.aval.shape).astype(np.float32) for v in prog.jaxpr.inBinders]
+    for got, want in zip(run_program(backend(), prog, arrays), run_program(OracleBackend(), prog, arrays)):
+        np.testing.assert_array_equal(got, want)
 
 
 @pytest.mark.parametrize("rows,k,n", [(2, 256, 130), (16, 100, 200), (5, 100, 333), (8, 768, 2304), (13, 333, 777), (33, 256, 260), (64, 512, 1000), (8, 2048, 512)], ids=str)

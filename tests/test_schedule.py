@@ -365,3 +365,51 @@ def test_elementwise_kernels_share_a_launch_until_one_reads_another():
             assert not set(u.inputs) & set(u.outputs) and len(u.inputs) == sum(k.nargs for k in u.source.kernels)
     made = [o for u in units for o in u.outputs]
     assert len(made) == len(set(made)) and set(prog.outputs) <= set(made)
+
+
+def wide_programs():
+    """Programs whose Kernels, joined, would read more buffers than a step of a launch list takes, by name; and the
+    arguments of the launches each keeps."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+
+    def total(xs):
+        return xs[0] if len(xs) == 1 else total(xs[1:]).add(xs[0])
+
+    def maps(kernels):
+        return lambda *xs: [total(xs).mul(float(k + 1)) for k in range(kernels)]
+
+    def product_behind_rows(first, along, behind):
+        def f(w, x, *v):
+            h = x.add(total(v[:first]))
+            return L.matmul(h.sub(h.max(-1, keepdims=True)).add(total(v[first:first + along])), w).add(total(v[first + along:]))
+        return J.jit(f, [f32(256, 128), f32(8, 256)] + [f32(256)] * (first + along) + [f32(128)] * behind)
+
+    def rows_behind_product(before, top, along):
+        def f(a, w, *v):
+            h = L.matmul(a, w).add(total(v[:before]))
+            return h.sub(h.add(total(v[before:before + top])).max(-1, keepdims=True)).add(total(v[before + top:]))
+        return J.jit(f, [f32(64, 64), f32(64, 16)] + [f32(16)] * (before + top + along))
+    f32 = lambda *shape: ShapedArray(shape, DType.Float32)  # noqa: E731
+    return {"8 maps of 15": (J.jit(maps(8), [f32(1000)] * 15), [128]), "8 maps of 16": (J.jit(maps(8), [f32(1000)] * 16), [119, 17]),
+            "8 maps of 20": (J.jit(maps(8), [f32(1000)] * 20), [126, 42]), "3 maps of 60": (J.jit(maps(3), [f32(1000)] * 60), [122, 61]),
+            "product behind rows, 128": (product_behind_rows(5, 60, 60), [128]), "product behind rows, 143": (product_behind_rows(20, 60, 60), [82, 63]),
+            "rows behind a product, 128": (rows_behind_product(60, 4, 61), [128]), "rows behind a product, 129": (rows_behind_product(60, 5, 61), [63, 68])}
+
+
+WIDE = ["8 maps of 15", "8 maps of 16", "8 maps of 20", "3 maps of 60", "product behind rows, 128", "product behind rows, 143", "rows behind a product, 128",
+        "rows behind a product, 129"]
+
+
+@pytest.mark.parametrize("name", WIDE)
+def test_no_launch_takes_more_arguments_than_a_launch_list(name):
+    import os
+    import re
+    from jaxjs_hip.runtime import LAUNCH_ARGS
+    from jaxjs_hip.schedule import Schedule
+    header = open(os.path.join(os.path.dirname(os.path.dirname(__file__)), "include", "jaxhip.h")).read()
+    assert int(re.search(r"#define JH_LAUNCH_ARGS (\d+)", header).group(1)) == LAUNCH_ARGS
+    prog, args = wide_programs()[name]
+    s = Schedule(_stand_in(), prog)
+    assert [c.num_args for c in s._steps[:s._n_steps]] == args, [type(u.source).__name__ for u in s.units]
