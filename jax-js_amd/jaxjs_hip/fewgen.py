@@ -144,7 +144,7 @@ def plan_whole_rows(g: dict) -> Optional[dict]:
     for MT in (1, 2, 4):
         for VN in ((1, 2, 4) if f32 or o["along_k"] else (2, 4, 8)):
             across, down = (16 * VN, 16 * MT) if o["short"] == "a" else (16 * MT, 16 * VN)
-            if MT * VN > 16 or across < g["N"] or (not o["along_k"] and o["C"] < VN):
+            if MT * VN > 16 or across < g["N"] or (not o["along_k"] and o["C"] < VN) or -(-o["R"] // (16 * MT)) > 65535:  # (gridDim.z)
                 continue
             waves = max(1, min(16, o["K"] // step or 1, FEW_LDS // (MT * 16 * (16 * VN + 1) * 4)))
             cycles = -(-o["K"] // step) * (28 * (MT * _loads(g, o["short"], True) + VN * _loads(g, o["wide"], o["along_k"])) + MT * VN * (32 if f32 else 4)) + waves * MT * VN * 16

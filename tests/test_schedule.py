@@ -413,3 +413,18 @@ def test_no_launch_takes_more_arguments_than_a_launch_list(name):
     prog, args = wide_programs()[name]
     s = Schedule(_stand_in(), prog)
     assert [c.num_args for c in s._steps[:s._n_steps]] == args, [type(u.source).__name__ for u in s.units]
+
+
+@pytest.mark.parametrize("rows,columns_first,joined", [(4194240, False, True), (4194241, False, False), (5000000, False, False), (5000000, True, True)])
+def test_rows_behind_a_product_stay_within_the_grid(rows, columns_first, joined):
+    """65535 tiles of 64 rows where the rows are the short operand's (the third dimension of the grid); along the first there is room."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rowproduct import ProductRows
+    from jaxjs_hip.schedule import Schedule
+    prog = J.jit(lambda x, w: L.softmax(L.matmul(x, L.swapaxes(w, 0, 1) if columns_first else w), -1),
+                 [ShapedArray((rows, 32), DType.Float32), ShapedArray((10, 32) if columns_first else (32, 10), DType.Float32)])
+    s = Schedule(_stand_in(), prog)
+    assert any(isinstance(u.source, ProductRows) for u in s.units) == joined, [type(u.source).__name__ for u in s.units]
+    assert all(c.grid[1] <= 65535 and c.grid[2] <= 65535 for c in s._steps[:s._n_steps])
