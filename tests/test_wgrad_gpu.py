@@ -56,17 +56,32 @@ def test_plan_covers_the_case(case):
     assert joined["wgrad"] == info["wgrad"]
 
 
-def test_an_exchange_that_is_more_than_one_stays_a_launch():
-    """What reads the cotangent besides its own transpose, or reads it at other positions, is not joined."""
-    case = CASES[0]
-    _, cts = cotangent_program(*case)
+# What is done with a cotangent: (from the cotangent, the same in numpy, the Kernels of the schedule: buffers they read and write).
+# Buffer 2 is the product in its own order, where that is a result of its own.
+READERS = {
+    "returned": (lambda c: [c()], lambda c: [c], [([0, 1], 3)]),
+    "squared": (lambda c: [(lambda v: v.mul(v))(c())], lambda c: [c * c], [([0, 1], 3)]),
+    "exchanged again": (lambda c: (lambda v: [v, J.transpose(v, [1, 0, 2, 3]).mul(2.0)])(c()), lambda c: [c, 2 * c.transpose(1, 0, 2, 3)], [([0, 1], 3), ([3], 4)]),
+    "flipped": (lambda c: [J.flip(c(), [2])], lambda c: [c[:, :, ::-1]], [([0, 1], 2), ([2], 3)]),
+    "read at two places": (lambda c: (lambda v: [v.add(J.flip(v, [3]))])(c()), lambda c: [c + c[..., ::-1]], [([0, 1], 2), ([2], 3)]),
+    "two of them": (lambda c: [c().mul(c())], lambda c: [c * c], [([0, 1], 2), ([0, 1], 3), ([2, 3], 4)]),
+}
+
+
+def reader_program(name, case):
     p = ConvParams(0, [1, 1], list(case[7]), [1, 1], [1, 1])
-    avals = [ShapedArray((case[0], case[1], case[3], case[4]), DType.Float16), ShapedArray(cts, DType.Float16)]
+    _, cts = cotangent_program(*case)
     ws = [case[2], case[1], case[5], case[6]]
-    flipped = J.jit(lambda x, ct: J.flip(J.convTransposeRhs(x, ct, ws, p), [2]), avals)
-    assert len(plan_units(flipped)) == 2
-    scaled = J.jit(lambda x, ct: J.convTransposeRhs(x, ct, ws, p).mul(J.convTransposeRhs(x, ct, ws, p)), avals)
-    assert all(u.options == dict(filter_bands=True) or u.options == {} for u in plan_units(scaled))
+    avals = [ShapedArray((case[0], case[1], case[3], case[4]), DType.Float16), ShapedArray(cts, DType.Float16)]
+    return J.jit(lambda x, ct: READERS[name][0](lambda: J.convTransposeRhs(x, ct, ws, p)), avals)
+
+
+@pytest.mark.parametrize("name", list(READERS))
+def test_an_exchange_that_is_more_than_one_stays_a_launch(name):
+    """What reads the cotangent besides its own transpose, or reads it at other positions, is not joined."""
+    units = plan_units(reader_program(name, CASES[0]))
+    assert [(u.inputs, u.outputs[0]) for u in units] == READERS[name][2]
+    assert [u.options == dict(filter_bands=True) for u in units] == [u.inputs == [0, 1] for u in units]
 
 
 @pytest.mark.parametrize("kw", [dict(stride=2), dict(dilation=2), dict(dtype=DType.Float32), dict(w=7), dict(kh=1), dict(batch=1, cin=16, cout=16)], ids=str)
@@ -91,6 +106,60 @@ def reference(x, ct, kh, kw, pad):
     return want, scale
 
 
+def sparse_integers(shape, rng):
+    """Mostly zeros, the rest 1 or -1: sums of products that float16 holds, to which every term left out or taken twice shows."""
+    return ((rng.random(shape) < 0.25) * rng.choice([-1, 1], shape)).astype(np.float16)
+
+
+def run(prog, arrays):
+    """The program's results, in their own types."""
+    be = backend()
+    slots = [be.malloc(v.nbytes, np.ascontiguousarray(v).tobytes()) for v in arrays]
+    outs = prog.execute(be, slots, prog.prepare(be))
+    got = [np.frombuffer(be.readSync(o), np.float16) for o in outs]
+    for s in slots + outs:
+        be.decRef(s)
+    return got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_sums_of_whole_numbers_are_exact(case):
+    """By the Kernel itself, and in the filter's own order by its program."""
+    batch, cin, cout, h, w, kh, kw, pad = case
+    kernel, cts = cotangent_kernel(*case)
+    rng = np.random.default_rng(batch * h + kw)
+    x, ct = sparse_integers((batch, cin, h, w), rng), sparse_integers(cts, rng)
+    want, scale = reference(x, ct, kh, kw, pad)
+    assert scale.max() <= 2048
+    got = device_run(kernel, [x.reshape(-1), ct.reshape(-1)], filter_bands=True)[0].reshape(cin, cout, kh, kw)
+    np.testing.assert_array_equal(got.astype(np.float64), want)
+    own, = run(cotangent_program(*case)[0], [x, ct])
+    np.testing.assert_array_equal(own.reshape(cout, cin, kh, kw).astype(np.float64), want.transpose(1, 0, 2, 3))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(READERS))
+def test_what_reads_the_cotangent_gets_it(name):
+    batch, cin, cout, h, w, kh, kw, pad = case = CASES[0]
+    rng = np.random.default_rng(len(name))
+    cts = cotangent_program(*case)[1]
+    x, ct = sparse_integers((batch, cin, h, w), rng), sparse_integers(cts, rng)
+    want = READERS[name][1](reference(x, ct, kh, kw, pad)[0].transpose(1, 0, 2, 3))
+    assert max(np.abs(v).max() for v in want) <= 2048
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    for got, w in zip(run(reader_program(name, case), [x, ct]), want):
+        np.testing.assert_array_equal(got.reshape(w.shape).astype(np.float64), w)
+
+
+def rounding_bound(want, n):
+    """Float32 sums of n exact products of standard normals: partial sums of up to 5 sqrt(n), each addition off by at most
+    2^-24 of that and by 3^-1/2 of it in the mean square, n of them at random: four deviations are 12 n 2^-24.  (A row or a column of an
+    image left out changes a sum by its square root and more.)  Then one rounding to float16."""
+    return np.abs(want) * 2.0 ** -11 + 12 * n * 2.0 ** -24 + 2.0 ** -25
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_sums_against_the_definition(case):
@@ -99,11 +168,8 @@ def test_sums_against_the_definition(case):
     x = RNG.standard_normal((batch, cin, h, w)).astype(np.float16)
     ct = RNG.standard_normal(cts).astype(np.float16)
     got = device_run(kernel, [x.reshape(-1), ct.reshape(-1)], filter_bands=True)[0].reshape(cin, cout, kh, kw).astype(np.float64)
-    want, scale = reference(x, ct, kh, kw, pad)
-    # float32 sums of exact products (n terms: at most n half-ulps of the running sum), one rounding to float16
-    n = batch * cts[2] * cts[3]
-    bound = np.abs(want) * 2.0 ** -11 + scale * n * 2.0 ** -24 + 2.0 ** -25
-    assert np.all(np.abs(got - want) <= bound)
+    want, _ = reference(x, ct, kh, kw, pad)
+    assert np.all(np.abs(got - want) <= rounding_bound(want, batch * cts[2] * cts[3]))
 
 
 @pytest.mark.gpu
@@ -115,14 +181,9 @@ def test_a_program_gets_the_filters_own_order(case):
     ct = RNG.standard_normal(cts).astype(np.float16)
     if WARM_ONLY:
         pytest.skip("warm-up run")
-    be = backend()
-    slots = [be.malloc(v.nbytes, np.ascontiguousarray(v).tobytes()) for v in (x, ct)]
-    outs = prog.execute(be, slots, prog.prepare(be))
-    got = np.frombuffer(be.readSync(outs[0]), np.float16).reshape(cout, cin, kh, kw).astype(np.float64)
-    for s in slots + outs:
-        be.decRef(s)
-    want, scale = (v.transpose(1, 0, 2, 3) for v in reference(x, ct, kh, kw, pad))
-    assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + scale * batch * cts[2] * cts[3] * 2.0 ** -24 + 2.0 ** -25)
+    got = run(prog, [x, ct])[0].reshape(cout, cin, kh, kw).astype(np.float64)
+    want = reference(x, ct, kh, kw, pad)[0].transpose(1, 0, 2, 3)
+    assert np.all(np.abs(got - want) <= rounding_bound(want, batch * cts[2] * cts[3]))
 
 
 @pytest.mark.gpu
