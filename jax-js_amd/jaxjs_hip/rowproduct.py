@@ -90,11 +90,31 @@ class ProductRows(Composite):
         return gen_gemm(self.kernel, t, numerics, "jh_product_rows", behind=text, few=p)
 
 
-# Whole rows in a workgroup are few, wide tiles: taken up to this estimate, or where they come in rounds anyway.  softmax behind a
-# linear layer, microseconds in two launches -> in one: float32 16 x 2 x 64 5.8 -> 3.4, 64 x 10 x 256 5.5 -> 3.8, 64 x 10 x 1024 5.9 ->
-# 4.3, 1024 x 46 x 256 5.4 -> 4.0, 8192 x 64 x 1024 23.3 -> 19.5; float16 1024 x 64 x 256 5.6 -> 4.0, 8192 x 10 x 1024 7.1 -> 5.4.  Past
-# the line 64 x 46 x 1024 6.4 -> 8.6, float16 64 x 64 x 1024 5.6 -> 7.3.
+# Whole rows in a workgroup are few, wide tiles: taken up to this estimate, and where they come in rounds anyway by what they
+# replace (`_rounds_pay`).  softmax behind a linear layer, rows x columns x k, microseconds in two launches -> in one: float32 16 x
+# 2 x 64 5.8 -> 3.4, 64 x 10 x 256 5.5 -> 3.8, 64 x 10 x 1024 5.9 -> 4.3, 1024 x 46 x 256 5.4 -> 4.0; float16 1024 x 64 x 256 5.6 ->
+# 4.0, 8192 x 10 x 1024 7.1 -> 5.4.  Past the line 64 x 46 x 1024 6.4 -> 8.6, float16 64 x 64 x 1024 5.6 -> 7.3.
 BEHIND_US = 5.0
+
+
+def _rounds_pay(kernel: Kernel, g: dict, p: dict, rows: int) -> bool:
+    """Whether whole rows in two rounds of workgroups and more beat the product's own launch and the rows' behind it: always where
+    the product alone is a dot product per element, and else by the tiles it would take, which read the operands once for all
+    columns and are the better the fuller they are.
+
+    Of 440 products of up to 360000 rows, 4 to 64 columns and k from 32 to 4096, time in one launch over time in two: dot products 0.03
+    to 0.63; float32 up to 32 columns 0.06 to 1.0 (one 1.12; 70000 x 10 x 512 64 -> 27 us, 116672 x 32 x 416 77 -> 62), more columns 1.0
+    to 1.64 (100000 x 64 x 1024 164 -> 207); float16 with a wide operand off the 16-byte grid, which tiles load element by element,
+    0.4 to 1.04 (50000 x 33 x 2048 108 -> 65) unless the other one is off the 4-byte grid too (0.6 to 1.5), with the rows along memory
+    and up to 24 columns 0.75 to 1.05, and otherwise 0.56 to 2.2 and 1.17 in the mean (95323 x 33 x 1727 95 -> 208)."""
+    if kernel.size // g["N"] < 2 * tuner.CU_COUNT * rows:
+        return False
+    if not tuner.tuneHip(kernel).klass.startswith("gemm"):
+        return True
+    if byteWidth(g["dtype"]) == 4:
+        return g["N"] <= 32
+    s, w = p["short"], p["wide"]
+    return not p["along_k"] and (g[w + "_sk"] % 8 != 0 and g[p["row"][s]] % 2 == 0 or s == "b" and g["N"] <= 24)
 
 
 def join_behind(kernel: Kernel, inputs: Sequence[int], buffer: int, chain: RowChain) -> Optional[ProductRows]:
@@ -113,7 +133,7 @@ def join_behind(kernel: Kernel, inputs: Sequence[int], buffer: int, chain: RowCh
     if p is None:
         return None
     rows = 16 * (p["MT"] if p["short"] == "a" else p["VN"])
-    if p["us"] > BEHIND_US and chain.R < 2 * tuner.CU_COUNT * rows:
+    if p["us"] > BEHIND_US and not _rounds_pay(kernel, g, p, rows):
         return None
     lanes = lane_plan(chain, p["waves"], rows, 2)
     sums = p["waves"] * 16 * p["MT"] * (16 * p["VN"] + 1) * 4

@@ -428,3 +428,24 @@ def test_rows_behind_a_product_stay_within_the_grid(rows, columns_first, joined)
     s = Schedule(_stand_in(), prog)
     assert any(isinstance(u.source, ProductRows) for u in s.units) == joined, [type(u.source).__name__ for u in s.units]
     assert all(c.grid[1] <= 65535 and c.grid[2] <= 65535 for c in s._steps[:s._n_steps])
+
+
+@pytest.mark.parametrize("dtype,order,rows,cols,k,joined", [
+    (DType.Float32, "kn", 100000, 32, 512, True), (DType.Float32, "kn", 100000, 33, 512, False), (DType.Float32, "nk", 200000, 48, 1024, False),
+    (DType.Float32, "first along rows", 60000, 32, 864, True), (DType.Float32, "first along rows", 60000, 33, 864, False),
+    (DType.Float16, "nk", 90000, 33, 2048, False), (DType.Float16, "nk", 90000, 16, 512, False), (DType.Float16, "kn", 90000, 64, 256, False),
+    (DType.Float16, "kn", 60000, 33, 1260, True), (DType.Float16, "kn", 60000, 33, 1261, False), (DType.Float16, "kn", 60000, 40, 1260, False),
+    (DType.Float16, "first along rows", 94000, 24, 1024, True), (DType.Float16, "first along rows", 94000, 25, 1024, False),
+    (DType.Float16, "first along rows", 94001, 40, 512, True), (DType.Float16, "nk", 1024, 64, 256, True), (DType.Float32, "kn", 1000000, 10, 64, True)], ids=str)
+def test_which_rows_behind_a_product_of_many_join(dtype, order, rows, cols, k, joined):
+    """Both sides of the rule for products that come in rounds of workgroups, and below its estimate."""
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rowproduct import ProductRows
+    from jaxjs_hip.schedule import plan_units
+    t = lambda x, yes: L.swapaxes(x, 0, 1) if yes else x  # noqa: E731
+    prog = J.jit(lambda a, b: L.softmax(L.matmul(t(a, order == "first along rows"), t(b, order != "kn")), -1),
+                 [ShapedArray((k, rows) if order == "first along rows" else (rows, k), dtype), ShapedArray((k, cols) if order == "kn" else (cols, k), dtype)])
+    units = plan_units(prog)
+    assert any(isinstance(u.source, ProductRows) for u in units) == joined, [type(u.source).__name__ for u in units]
