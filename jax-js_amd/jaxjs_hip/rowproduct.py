@@ -166,8 +166,13 @@ def join_rows(chain: RowChain, buffer: int, kernel: Kernel, inputs: Sequence[int
         return None
     rows, eb = min(chain.R, 16 * p["MT"]), byteWidth(g["dtype"])
     lanes = lane_plan(chain, p["waves"], rows)
-    sums = p["waves"] * 16 * p["MT"] * (16 * p["VN"] + 1) * 4
-    if rows * chain.C * eb > ROWS_BYTES or lanes["iters"] * lanes["V"] > LANE_ELEMENTS or sums + 16 * p["MT"] * chain_pitch(g["K"], g["dtype"]) * eb > LDS_BYTES:
+    lds = p["waves"] * 16 * p["MT"] * (16 * p["VN"] + 1) * 4 + 16 * p["MT"] * chain_pitch(g["K"], g["dtype"]) * eb
+    if rows * chain.C * eb > ROWS_BYTES or lanes["iters"] * lanes["V"] > LANE_ELEMENTS or lds > LDS_BYTES:
+        return None
+    # Workgroups that wait for a place make their rows beside no other's wait: float32 2 x 1856 x 5739 16.7 -> 20.0 us, 8 x 1423 x 9152
+    # 25.6 -> 29.3, float16 8 x 1728 x 9088 17.5 -> 18.8, all with one to a CU; where a CU holds two, 3 x 1664 x 11328 12.5 -> 11.8.
+    count = -(-p["C"] // (16 * p["VN"])) * p["slices"] * -(-chain.R // (16 * p["MT"]))
+    if count > tuner.CU_COUNT * min(LDS_BYTES // lds, 32 // p["waves"]):
         return None
     s = p["short"]
     gid = g["gid_" + s]

@@ -449,3 +449,19 @@ def test_which_rows_behind_a_product_of_many_join(dtype, order, rows, cols, k, j
                  [ShapedArray((k, rows) if order == "first along rows" else (rows, k), dtype), ShapedArray((k, cols) if order == "kn" else (cols, k), dtype)])
     units = plan_units(prog)
     assert any(isinstance(u.source, ProductRows) for u in units) == joined, [type(u.source).__name__ for u in units]
+
+
+@pytest.mark.parametrize("dtype,rows,k,cols,order,joined", [
+    (DType.Float32, 2, 1216, 4096, "kn", True), (DType.Float32, 2, 1856, 4096, "nk", True), (DType.Float32, 2, 1856, 4097, "nk", False),
+    (DType.Float32, 8, 1423, 8192, "kn", True), (DType.Float32, 8, 1423, 9152, "kn", False), (DType.Float16, 8, 1728, 9088, "kn", False),
+    (DType.Float16, 3, 1664, 11328, "nk", True), (DType.Float16, 8, 768, 3072, "kn", True)], ids=str)
+def test_rows_are_made_in_workgroups_that_all_have_a_place(dtype, rows, k, cols, order, joined):
+    from jaxjs_hip import jit as J
+    from jaxjs_hip import library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.rowproduct import RowProduct
+    from jaxjs_hip.schedule import plan_units
+    prog = J.jit(lambda x, g, w: L.matmul(L.standardize(x).mul(g), L.swapaxes(w, 0, 1) if order == "nk" else w),
+                 [ShapedArray((rows, k), dtype), ShapedArray((k,), dtype), ShapedArray((cols, k) if order == "nk" else (k, cols), dtype)])
+    units = plan_units(prog)
+    assert any(isinstance(u.source, RowProduct) for u in units) == joined, [type(u.source).__name__ for u in units]
