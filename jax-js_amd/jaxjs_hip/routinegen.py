@@ -34,6 +34,7 @@ SORT_FEW, SORT_FEW_WAVES = 16, 256
 # 1 x 20000: 58 us with tiles of 16384, 36 of 8192, 33 of 4096, 37 of 2048; 100 x 16384 stays at 16384, 42.5 against 45.6).
 SORT_SMALL_TILE, SORT_FEW_TILES = 4096, 64
 SORT_LOCAL, SORT_TILES = 16, 1024  # words of a lane in a tile's register runs, from 1024 tiles on
+SORT_HELD = 8     # pieces of 16 bytes that a lane hands to others at a time: whole lines of 128 bytes (float32 32768 x 1024: 70.6 us, 83 with 4)
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
 CHOLESKY_PANEL_FROM = 192  # matrix order from which many matrices may take two launches a panel, and a plan counts its panels
 CHOLESKY_WAVE_BELOW = {2: 44, 4: 28, 8: 28}  # matrix order, by bytes per element, below which many matrices take a wave each
@@ -656,17 +657,18 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
     values = dict(N=n, P=P, ROWS=rows, ARGSORT=1 if argsort else 0, KIND=kind, T=ctype, GROUP=SORT_GROUP if P > 256 else 4)
     need = {0: rows * n * byteWidth(dtype)}
     outs = [("out", 0), ("out", 1)] if argsort else [("out", 0), ("out", 0)]
-    if P <= (64 if word == 4 and not argsort else 32 if short else 16) * most:
+    if P <= (64 if word == 4 else 16) * most:
         # 16 lanes per row pair most words inside a lane and reach every other one by DPP; with few rows up to 64, since the
         # launch then waits for one wave's chain.  Sorts gain from registers up to 64 lanes (8000 x 4000 float32: 118 us
-        # against 134 through LDS); wider words pay for every lane exchange twice and argsort gathers its values (argsort
-        # float32 4000 x 2000: 95 us in 64 lanes, 54 through LDS; 30000 x 1000: 206 in 32, 154; float16 8000 x 4000: 183 and 144).
+        # against 134 through LDS), and so does float16 Argsort, whose words are as wide (8000 x 4000: 104 us, 141 through LDS;
+        # 1000 x 3000: 21.5 and 28.2); words of 8 bytes pay for every lane exchange twice (argsort float32 30000 x 1000: 158 us in
+        # 32 lanes, 148 through LDS; 3000 x 1000: 23.9 and 21.0).
         E = min(max(2, P // 16), most)
         while E > max(2, P // 64) and rows * (P // E) < SORT_WAVES * 64:
             E //= 2
         E = max(E, P // 64, 1)
         if E <= SORT_FEW or rows * (P // E) >= SORT_FEW_WAVES * 64:
-            src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=0, TILE=P, THREADS=256, E=E, W=P))
+            src = _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=0, TILE=P, THREADS=256, E=E, W=P, HELD=SORT_HELD))
             steps = [LaunchStep("jh_sort_rows", (-(-rows * (P // E) // 256), 1, 1), (256, 1, 1), 0, [("in", 0)] + outs)]
             return KernelSource([src], steps, [], "sort", need, dict(n=n, rows=rows, P=P, tile=P, argsort=argsort, launches=1))
     tile = min(P, SORT_TILE * 8 // word)
@@ -680,7 +682,7 @@ def _gen_sort(routine: Routine, numerics: str) -> Optional[KernelSource]:
     # loses by them, 30000 x 1000 in 32 lanes: 206 -> 243).
     doubles = argsort and dtype in (DType.Float32, DType.Int32, DType.Uint32, DType.Bool) and n <= 1 << 20
     opening = SOURCE_OPTION + "-ffinite-math-only\n" if doubles else ""
-    src = opening + _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=1 if doubles else 0, TILE=tile, THREADS=threads, E=E, W=64 * E))
+    src = opening + _prelude(numerics) + fill(template("sort.hip.inc"), dict(values, DOUBLES=1 if doubles else 0, TILE=tile, THREADS=threads, E=E, W=64 * E, HELD=1))
     tiles = rows * (P // tile)
     steps = [LaunchStep("jh_sort_local", (tiles, 1, 1), (threads, 1, 1), 0, [("in", 0), ("scratch", 0)] + outs)]
     k = tile * 2

@@ -124,10 +124,10 @@ def test_argsort_matches_host_routine(shape, dtype):
 
 # Edges of the register network: lanes 1 to 64 per row and 2 to 64 words per lane (row lengths around powers of two, few and
 # many rows), rows past the last whole workgroup, runs of a tile in LDS, tiles chosen for few and for many rows, fused
-# strides over memory, and the longest float16 row whose key and position share a word.
+# strides over memory, pieces of a lane that other lanes store (2 to 16 of them, rows off the 16-byte grid), and the longest float16 row whose key and position share a word.
 @pytest.mark.parametrize("shape,dtype", [((70, 16), DType.Float32), ((33, 17), DType.Float16), ((1000, 33), DType.Int32), ((3, 129), DType.Float32),
                                          ((2100, 1024), DType.Float32), ((300, 1000), DType.Float64), ((9000, 130), DType.Float32), ((260, 4095), DType.Float32),
-                                         ((3, 4096), DType.Float32), ((70, 8192), DType.Int32), ((1030, 16384), DType.Float32), ((2, 40000), DType.Float32),
+                                         ((3, 4096), DType.Float32), ((2101, 1023), DType.Float16), ((301, 4001), DType.Float16), ((5001, 100), DType.Float64), ((70, 8192), DType.Int32), ((1030, 16384), DType.Float32), ((2, 40000), DType.Float32),
                                          ((1, 140000), DType.Float16), ((1, 1 << 20), DType.Int32), ((1, (1 << 20) + 1), DType.Float32), ((1, 65536), DType.Float16), ((1, 65537), DType.Float16)],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v.value)
 @pytest.mark.parametrize("name", [Routines.Sort, Routines.Argsort], ids=lambda n: n.value)
