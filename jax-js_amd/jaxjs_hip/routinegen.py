@@ -13,7 +13,7 @@ time, which is what the Backend interface prescribes for a routine a backend lac
 
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Tuple
 
 from .alu import DType, byteWidth
 from .codegen import SOURCE_OPTION
@@ -65,7 +65,7 @@ def _round64(n: int, cap: int = 1024) -> int:
     return max(64, min(cap, (n + 63) // 64 * 64))
 
 
-_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1,
+_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1, RHS=1,
                         ELEM="float", CMP="float")
 # Element types of the dense routines: C type, the type magnitudes are compared in, bytes per element.
 _FLOAT_ELEMS = {DType.Float32: ("float", "float", 4), DType.Float64: ("double", "double", 8), DType.Float16: ("jh_f16", "float", 2)}
@@ -164,6 +164,18 @@ def _gen_cholesky(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, scratch, "cholesky", need, dict(n=n, batch=batch, launches=len(steps), **info))
 
 
+def _trisolve_few(n: int, total: int) -> Optional[Tuple[int, int]]:
+    """Right-hand sides of a workgroup and rows of a staged block where `total` right-hand sides of order n are few enough to
+    keep theirs and the solved entries in LDS, a workgroup to a CU; None where they are not."""
+    from . import tuner
+    width = -(-n // 8) * 8
+    for rhs in (8, 16, 32, 64):
+        rb = min(32, n, (160 * 1024 - 64 - 8 * width * rhs) // (16 * width + 16))
+        if rb >= 1 and total <= rhs * tuner.CU_COUNT:
+            return rhs, rb
+    return None
+
+
 def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
     t = routine.type
     a_shape, b_shape = list(t.inputShapes[0]), list(t.inputShapes[1])
@@ -185,6 +197,12 @@ def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
         return _empty("trisolve", n=n, m=m, batch=mats)
     unit = 1 if (routine.params or {}).get("unitDiagonal", False) else 0
     need = {0: mats * n * n * eb, 1: mats * m * n * eb}
+    few = _trisolve_few(n, mats * m)
+    if few is not None:
+        rhs, rb = few
+        src = _linalg_source(numerics, ROUTINE=1, N=n, M=m, THREADS=256, UNIT=unit, STAGED=2, RB=rb, RHS=rhs, ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_trisolve_few", (mats * -(-m // rhs), 1, 1), (256, 1, 1), 0, [("in", 0), ("in", 1), ("out", 0)])]
+        return KernelSource([src], steps, [], "trisolve", need, dict(n=n, m=m, batch=mats, threads=256, staged=n >= TRISOLVE_STAGED_FROM, rows_per_block=rb))
     if TRISOLVE_STAGED_FROM <= n <= TRISOLVE_STAGED_MAX_N:
         # one wave of 64 right-hand sides + three waves staging blocks of rows in LDS as doubles (two buffers <= 128 KB)
         rb = max(1, min(8, TRISOLVE_STAGED_MAX_N // n))

@@ -533,3 +533,19 @@ def test_jacobi_eigh_of_many_small_matrices(n, batch):
     got, want, ks = both(R.jacobi_eigh(sym), [sym])
     assert ("block" in ks.info) == (batch <= 256)
     assert_bits(got, want, f"jacobi_eigh {batch} x {n}")
+
+
+@pytest.mark.parametrize("n,m,mats,dt", [(1, 1, 1, F32), (7, 8, 1, F32), (8, 9, 3, F32), (9, 1, 2, F32), (17, 2049, 1, F32), (25, 4100, 1, F32), (40, 8200, 1, F32), (127, 17, 1, F32),
+                                         (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16)],
+                         ids=lambda v: np.dtype(v).name if isinstance(v, type) else str(v))
+def test_triangular_solve_of_few_right_hand_sides(n, m, mats, dt):
+    """Groups of eight entries and rows of a staged block that are not whole, 8 to 64 right-hand sides a workgroup, lanes without one; a zero, an infinite and
+    a subnormal pivot, right-hand sides of infinities and NaN, which have no part in rows that they do not belong to."""
+    a = (np.triu(RNG.standard_normal((mats, n, n))) + np.sqrt(n) * np.eye(n)).astype(dt) if n > 1 else np.full((mats, 1, 1), 3, dt)
+    b = RNG.standard_normal((mats, m, n)).astype(dt)
+    if n > 4:
+        a[0, 1, 1], a[0, 2, 2], a[0, 3, 3] = 0.0, np.inf, np.finfo(dt).smallest_subnormal
+        b[0, 0, 0], b[0, m - 1, n // 2] = np.inf, np.nan
+        a += np.tril(np.full((n, n), np.nan), -1).astype(dt)  # the strictly lower part must not matter
+    got, want, ks = both(R.triangular_solve(a, b), [a, b])
+    assert_bits(got, want, f"triangular_solve {mats} x {n} x {m} {np.dtype(dt).name} {ks.info}")
