@@ -65,7 +65,7 @@ def _round64(n: int, cap: int = 1024) -> int:
     return max(64, min(cap, (n + 63) // 64 * 64))
 
 
-_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1, RHS=1,
+_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1, RHS=1, ELEM_BYTES=4,
                         ELEM="float", CMP="float")
 # Element types of the dense routines: C type, the type magnitudes are compared in, bytes per element.
 _FLOAT_ELEMS = {DType.Float32: ("float", "float", 4), DType.Float64: ("double", "double", 8), DType.Float16: ("jh_f16", "float", 2)}
@@ -232,6 +232,20 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     batch = prod(shape[:-2])
     if batch == 0 or m == 0:
         return _empty("lu", m=m, n=n, batch=batch)
+    if m <= 4096:
+        rows = -(-m // 1024)  # of a thread of the panel's workgroup, in registers with as many columns as fit
+        width = min(32, 1 << (64 // (rows * (2 if eb == 8 else 1))).bit_length() - 1, max(8, 1 << (min(m, n) - 1).bit_length()))
+        src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb)
+        steps = []
+        for j in range(0, max(min(m, n), 1), width):
+            steps.append(LaunchStep("jh_lu_panel", (batch, 1, 1), (_round64(m - j), 1, 1), 0,
+                                    [("in", 0), ("out", 0), ("out", 1), ("out", 2), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j)]))
+            strips = -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
+            if strips:
+                steps.append(LaunchStep("jh_lu_strip", (batch * strips, 1, 1), (512, 1, 1), 0,
+                                        [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j)]))
+        return KernelSource([src], steps, [batch * width * m * 8, batch * m * 4, max(batch * 4, 16)], "lu", {0: batch * m * n * eb},
+                            dict(m=m, n=n, batch=batch, launches=len(steps), **({"variant": "by columns"} if min(m, n) >= LU_BY_COLUMNS_FROM else {})))
     if min(m, n) >= LU_BY_COLUMNS_FROM and batch * m * n < (1 << 31):
         # Large matrices: two launches per column, the rank-1 update of the trailing block over the whole chip; the same
         # operations per element as the single-workgroup kernel (bit-identical).
@@ -247,12 +261,7 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
                                         [("out", 0), ("scratch", 0), ("scratch", 1), ("const", j)]))
         return KernelSource([src], steps, [batch * m * 8, max(batch * 4, 16)], "lu", {0: batch * m * n * eb},
                             dict(m=m, n=n, batch=batch, launches=len(steps), variant="by columns"))
-    if m > 4096:  # single workgroup: the multipliers of one column live in LDS as doubles
-        return None
-    threads = _round64(max(m, n))
-    src = _linalg_source(numerics, ROUTINE=2, N=n, M=m, THREADS=threads, ELEM=ctype, CMP=cmp_t)
-    steps = [LaunchStep("jh_lu", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("out", 2)])]
-    return KernelSource([src], steps, [], "lu", {0: batch * m * n * eb}, dict(m=m, n=n, batch=batch, threads=threads))
+    return None
 
 
 def _jacobi_blocks_pay(n: int, batch: int, eb: int) -> bool:

@@ -535,6 +535,20 @@ def test_jacobi_eigh_of_many_small_matrices(n, batch):
     assert_bits(got, want, f"jacobi_eigh {batch} x {n}")
 
 
+@pytest.mark.parametrize("shape,dt", [((33, 31), F32), ((64, 40), F32), ((3, 32, 65), F32), ((40, 7), np.float64), ((9, 2500), F32), ((1024, 33), F32), ((1025, 40), F32),
+                                      ((2049, 20), F32), ((3073, 17), np.float16), ((4096, 9), F32), ((1030, 34), np.float64), ((2200, 12), np.float64), ((3, 1), F32),
+                                      ((0, 5, 5), F32), ((300, 8, 8), F32)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else np.dtype(v).name)
+def test_lu_panels_at_their_edges(shape, dt):
+    """Panels that are not whole, one to four rows a thread and the widths that go with them, columns behind the last panel.  Elements of few values: equal
+    magnitudes in many waves, of which the first row has to win, and zero columns."""
+    a = RNG.integers(-2, 3, shape).astype(dt)
+    if a.ndim == 2 and min(shape) > 4:
+        a[shape[0] // 2:, :] *= 0.5
+        a[:, 2] = a[:, 1]  # cancels: a zero pivot column
+    got, want, ks = both(R.lu(a), [a])
+    assert_bits(got, want, f"lu {shape} {np.dtype(dt).name} {ks.info}")
+
+
 @pytest.mark.parametrize("n,m,mats,dt", [(1, 1, 1, F32), (7, 8, 1, F32), (8, 9, 3, F32), (9, 1, 2, F32), (17, 2049, 1, F32), (25, 4100, 1, F32), (40, 8200, 1, F32), (127, 17, 1, F32),
                                          (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16)],
                          ids=lambda v: np.dtype(v).name if isinstance(v, type) else str(v))
