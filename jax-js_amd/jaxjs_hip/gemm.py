@@ -48,7 +48,7 @@ def _short_axis_tile(g: dict, bm: int, bn: int, per_cu: int, both_k: bool, reads
     return None
 
 
-def _f32_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
+def _f32_staged_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
     """Tile and slices of a float32 product of whole 16-byte groups with a single-stride k axis and enough tiles to fill the
     chip.  128-row tiles take eight waves, two on a SIMD (2048 x 2048 x 1024 84.3 -> 81.0 us, 4032 x 4032 x 2368 657 -> 632, 1024 x
     1024 x 1024 29.3 -> 28.5).
@@ -83,6 +83,60 @@ def _f32_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
             if best is None or us < best[0]:
                 best = (us, plan(bm, bn, split))
     return best[1]
+
+
+# Plans of float32 products by direct loads: tile and waves, stages of a 32-deep slab (64 to 72 KB: two workgroups to a CU), and
+# what `_f32_tile` estimates with, in microseconds: a launch; k steps that filling and emptying the pipeline costs; elements of
+# C and k a microsecond, for a CU, alone as a part of that; folding a slice, and 10^6 of its partial sums.
+_F32_PLANS = ((dict(BM=64, BN=64, WM=2, WN=2, WK=2, STAGES=4), 2.18, 71.0, 274.5e3, 0.948, 0.455, 0.873),
+              (dict(BM=64, BN=64, WM=2, WN=2, WK=1, STAGES=4), 1.70, 62.5, 269.0e3, 0.927, 0.710, 0.391),
+              (dict(BM=128, BN=64, WM=4, WN=2, WK=1, STAGES=3), 1.98, 35.0, 277.5e3, 0.959, 0.831, 0.714),
+              (dict(BM=128, BN=128, WM=4, WN=2, WK=1, STAGES=2), 3.10, 12.2, 281.9e3, 0.988, 1.130, 0.993))
+
+
+def _f32_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
+    """Plan of a float32 product whose slabs go to LDS by direct loads (`_f32_direct`), by an estimate: a launch, the tiles of the
+    CU that gets most of them at the plan's rate, and the fold of slices of the k axis inside the launch.  It is a fit to 132
+    products of 64 to 8192 rows, columns and k in both orders of B under all plans, within 1.7 per cent of the fastest one in
+    the mean, 26 at worst (128 x 2144 x 216).  Against staging slabs in registers: 1024 x 1024 x 1024 25.9 -> 19.8 us, 2048
+    150 -> 124, 4096 1080 -> 946 (145 TFLOP/s), 8192 8596 -> 7565, 3632 x 3088 x 144 49.6 -> 37.0, 1280 x 640 x 320 10.5 -> 7.6, 960 x 384 x
+    3696 95.9 -> 41.5, 3672 x 768 x 1408 86.9 -> 69.4."""
+    best = None
+    for plan, launch, fill, rate, alone, fold, sums in _F32_PLANS:
+        count = tiles(plan["BM"], plan["BN"])
+        for split in (1, 2, 4, 8):
+            if split > 1 and (nb > 1 or g["K"] % (4 * split) or g["K"] // split < 64):
+                continue
+            per_cu = -(-count * split // tuner.CU_COUNT)
+            us = launch + per_cu * plan["BM"] * plan["BN"] * (g["K"] / split + fill) / (rate * (alone if per_cu == 1 else 1.0))
+            if split > 1:
+                us += fold * split + sums * 1e-6 * split * g["M"] * g["N"]
+            if best is None or us < best[0]:
+                best = (us, dict(plan, BK=32, DLDS=1, **(dict(SPLITK=split, FUSEK=1) if split > 1 else {})))
+    return best[1]
+
+
+def is_direct_product(kernel: Kernel) -> bool:
+    """Whether `kernel` is better prepared with the option `direct_f32`: a float32 product that no other kernel takes.  (Why it is an
+    option, which programs' schedules set, and not the plan of every such Kernel: the plans of smaller products, slabs staged in registers,
+    are pinned by tests/test_kernelgen.py.)"""
+    if kernel.reduction is None or kernel.size == 0:
+        return False
+    t = tuner.tuneHip(kernel)
+    return t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and few_plan(t) is None
+
+
+def _f32_direct(g: dict) -> bool:
+    """Whether float32 operands can go to LDS by direct loads: plain ones of whole 16-byte groups, one stride along k, and offsets
+    inside a slab that unsigned 32-bit byte counts hold."""
+    return (not any(g.get(tag + w) for tag in "ab" for w in ("_gather", "_loose")) and g["a_k0"] == g["K"] and g["b_k0"] == g["K"] and g["K"] % 4 == 0
+            and _f32_direct_span(g, 128, 128, 64))
+
+
+def _f32_direct_span(g: dict, bm: int, bn: int, bk: int) -> bool:
+    """Whether the lanes' offsets inside a slab of a tile are unsigned 32-bit byte counts."""
+    strides = [(bm, g["a_sm"]), (bk, g["a_sk"]), (bn, g["b_sn"]), (bk, g["b_sk"])]
+    return min(s for _, s in strides) >= 0 and max(bm * g["a_sm"] + bk * g["a_sk"], bn * g["b_sn"] + bk * g["b_sk"]) < 1 << 29
 
 
 def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
@@ -131,8 +185,12 @@ def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
         # second one hides the first one's staging latency).  Slabs are 32 deep (measured 3-6 % over 16 on
         # 2048^3 and 4096^3: half the barriers); gather operands keep the 16-deep slabs they were tuned with.
         bk = 32 if plain_k else 16
-        if plain_k and not loose_ops and g["M"] >= 128 and g["N"] >= 64 and tiles(128, 64) * 4 > CU:
+        # Direct loads where a schedule asks for them, and for any Kernel of at least two 128x128 tiles per CU, whose plans nothing pins
+        # (8192^3 8596 -> 7565 us; 4096^3 1080 -> 946).
+        if _f32_direct(g) and (g.get("direct") or tiles(128, 128) >= 2 * CU):
             return _f32_tile(g, tiles, nb)
+        if plain_k and not loose_ops and g["M"] >= 128 and g["N"] >= 64 and tiles(128, 64) * 4 > CU:
+            return _f32_staged_tile(g, tiles, nb)
         # Among the shapes that do, the cheapest by (rounds of two workgroups per CU) x (tile area) / (rate of the
         # shape relative to 128x128: 0.97, 0.80): a last round that is nearly empty costs a whole one (products of
         # attention weights and values over 577 positions, 640 tiles of 128x64: 85.1 us, 66.1 us in 1280 of 64x64; the
@@ -614,7 +672,7 @@ def tap_major_form(oexp: AluExp, K: int):
 def few_plan(t: TuneResult) -> Optional[dict]:
     """The plan of the contraction `t` where the kernel for few rows or tiles takes it."""
     g = t.gemm
-    if g is None or t.params.get("gemm_tile") or _repack_operand(g) is not None:
+    if g is None or g.get("direct") or t.params.get("gemm_tile") or _repack_operand(g) is not None:
         return None
     return plan_few(g, lambda: choose_tile(g))
 
@@ -650,7 +708,10 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
     WM, WN = tile.get("WM", 2), tile.get("WN", 2)
     if BM % (32 * WM) or BN % (32 * WN):
         raise ValueError(f"tile {BM}x{BN} does not divide into {WM}x{WN} waves of 32x32 MFMA tiles")
-    nthreads = 64 * WM * WN
+    # float32 with direct loads: WK waves share out the k of a slab
+    direct32 = int(tile.get("DLDS", 0)) if g["dtype"] == DType.Float32 and not few else 0
+    WK = tile.get("WK", 1) if direct32 else 1
+    nthreads = 64 * WM * WN * WK
     out_t = STORAGE_CTYPE[kernel.dtype]
     in_t = STORAGE_CTYPE[g["dtype"]]
 
@@ -1066,9 +1127,17 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
 
     tmpl = "gemm_f16.hip.inc" if g["dtype"] == DType.Float16 else "gemm_f32.hip.inc"
     fBK = int(tile.get("BK", 16)) if g["dtype"] == DType.Float32 else 0  # slab depth of the f32 template
-    if g["dtype"] == DType.Float32 and fBK in (16, 32, 64) and (BM * fBK // 4 % nthreads or BN * fBK // 4 % nthreads):
+    if direct32:
+        stages = int(tile.get("STAGES", 4))
+        if not _f32_direct(g):
+            raise ValueError("direct loads of float32 operands need plain ones of whole 16-byte groups, with one stride along k")
+        if fBK not in (32, 64) or BM * fBK * 4 % (16 * nthreads) or BN * fBK * 4 % (16 * nthreads) or fBK % (8 * WK):
+            raise ValueError(f"{nthreads} threads in {WK} parts of k do not share out a {BM}- or {BN}-row slab {fBK} deep")
+        if stages < 2 or max(stages * (BM + BN) * fBK * 4, (WK - 1) * BM * BN * 4) > 160 * 1024:
+            raise ValueError(f"{stages} stages of {BM}+{BN} rows {fBK} deep do not fit the LDS")
+    elif g["dtype"] == DType.Float32 and fBK in (16, 32, 64) and (BM * fBK // 4 % nthreads or BN * fBK // 4 % nthreads):
         raise ValueError(f"{nthreads} threads do not share out a {BM}- or {BN}-row slab {fBK} deep in whole groups")
-    if g["dtype"] == DType.Float32 and (fBK not in (16, 32, 64) or 2 * (BM + BN) * (fBK + 4) * 4 > 160 * 1024):
+    if not direct32 and g["dtype"] == DType.Float32 and (fBK not in (16, 32, 64) or 2 * (BM + BN) * (fBK + 4) * 4 > 160 * 1024):
         raise ValueError(f"f32 slab depth {fBK} is not 16, 32 or 64, or two {BM}+{BN}-row slabs of it do not fit the LDS")
     # Fast path: direct global->LDS loads need whole tiles (no bounds predicates) and 32-deep slabs.
     # Slab depth.  When both operands run along k in memory, 64-deep slabs make every row of a slab one whole
@@ -1131,6 +1200,9 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
         sched = dict(COMMIT_A=tile.get("CA", 2), COMMIT_B=tile.get("CB", 3), FETCH_A=tile.get("FA", 0),
                      FETCH_B=tile.get("FB", 1), IGLP=tile.get("IGLP", -1), SCHED_FENCE=tile.get("FENCE", 0),
                      A_LOOSE=loose["a"], B_LOOSE=loose["b"])
+    elif direct32:
+        tmpl = "gemm_f32_dlds.hip.inc"
+        sched = dict(BK=fBK, STAGES=stages, WK=WK, FUSEK=fusek)
     else:
         sched = dict(BK=fBK, FRAG_FENCE=int(tile.get("FENCE", 1)), FUSEK=fusek, A_LOOSE=loose["a"], B_LOOSE=loose["b"])
     if not dlds:

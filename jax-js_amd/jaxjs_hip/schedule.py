@@ -18,6 +18,7 @@ from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
 from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
+from .gemm import is_direct_product
 from .kernelgen import generate
 from .routine import Routine
 from .rowchain import RowChain, _tidy, collect_chain, index_form
@@ -197,7 +198,7 @@ def plan_units(prog) -> List[Unit]:
             units[-1] = Unit(product, product.inputs, [s.output])
             k += 1
             continue
-        options = dict(filter_bands=True) if s.routine is None and is_filter_cotangent(s.kernel) else {}
+        options = {} if s.routine is not None else dict(filter_bands=True) if is_filter_cotangent(s.kernel) else dict(direct_f32=True) if is_direct_product(s.kernel) else {}
         units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))
         k += 1
     return units

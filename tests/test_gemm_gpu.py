@@ -688,6 +688,32 @@ def test_gemm_f16_tiles_of_short_k_axes(M, N, K, layout, bias, tile):
     test_gemm_f16_direct_lds_edge_tiles(M, N, K, layout, tile, bias)
 
 
+# Slabs of float32 operands by direct loads, under every plan: edge tiles in both directions, k axes of one slab, of whole slabs and of a
+# few floats more, fewer slabs than stages, slices that end inside a slab.
+@pytest.mark.parametrize("M,N,K,split", [(64, 64, 32, 1), (260, 124, 36, 1), (132, 196, 60, 1), (192, 128, 64, 1), (200, 264, 1000, 1), (68, 60, 528, 4), (516, 384, 1056, 8)], ids=str)
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("plan", [dict(BM=64, BN=64, WM=2, WN=2, WK=2, STAGES=4), dict(BM=64, BN=64, WM=2, WN=2, WK=1, STAGES=4), dict(BM=128, BN=64, WM=4, WN=2, WK=1, STAGES=3),
+                                  dict(BM=128, BN=128, WM=4, WN=2, WK=1, STAGES=2)], ids=lambda p: "x".join(map(str, p.values())))
+def test_gemm_f32_direct_loads(plan, layout, M, N, K, split):
+    full = [M, N, K]
+    a, b = ([K, M], [1, 0]) if layout == "TN" else ([M, K], [0, 1]), ([N, K], [0, 1]) if layout == "NT" else ([K, N], [1, 0])
+    stA = ShapeTracker.fromShape(a[0]).permute(a[1]).reshape([M, 1, K]).expand(full)
+    stB = ShapeTracker.fromShape(b[0]).permute(b[1]).reshape([1, N, K]).expand(full)
+    k = reduceKernel(full, [(DType.Float32, stA), (DType.Float32, stB)], lambda x, y: AluExp.mul(x, y), AluOp.Add)
+    A, B = RNG.uniform(-1, 1, (M, K)).astype(np.float32), RNG.uniform(-1, 1, (K, N)).astype(np.float32)
+    bufs = [np.ascontiguousarray(A.T) if layout == "TN" else A, np.ascontiguousarray(B.T) if layout == "NT" else B]
+    tile = dict(plan, BK=32, DLDS=1, **(dict(SPLITK=split, FUSEK=1) if split > 1 else {}))
+    got, ks = device_run(k, bufs, gemm_tile=tuple(sorted(tile.items())))
+    assert "global_load_lds_dwordx4" in ks.sources[0], ks.info
+    _check(got, A, B, K, out_f16=False)
+    if (plan["WK"], split) == (2, 4):  # infinities and NaN stay in their rows and columns: what stands in for k behind the axis is zero in both operands
+        bufs[0] = bufs[0].copy()
+        bufs[0][(K - 1, M - 1) if layout == "TN" else (M - 1, K - 1)] = np.inf
+        got, _ = device_run(k, bufs, gemm_tile=tuple(sorted(tile.items())))
+        got = got.reshape(M, N)
+        assert np.all(np.isinf(got[-1])) and np.all(np.isfinite(got[:-1]))
+
+
 F32_SHAPES = [(64, 64, 64), (128, 128, 64), (200, 264, 136), (1024, 1024, 1024), (96, 1028, 72), (512, 384, 100)]
 
 

@@ -465,3 +465,18 @@ def test_rows_are_made_in_workgroups_that_all_have_a_place(dtype, rows, k, cols,
                  [ShapedArray((rows, k), dtype), ShapedArray((k,), dtype), ShapedArray((cols, k) if order == "nk" else (k, cols), dtype)])
     units = plan_units(prog)
     assert any(isinstance(u.source, RowProduct) for u in units) == joined, [type(u.source).__name__ for u in units]
+
+
+def test_schedules_ask_for_direct_loads_of_float32_products():
+    from jaxjs_hip import DType, jit as J, library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.kernelgen import generate
+    from jaxjs_hip.schedule import plan_units
+
+    def units(dtype, m, n, k):
+        return plan_units(J.jit(lambda a, b: L.matmul(a, b), [ShapedArray((m, k), dtype), ShapedArray((k, n), dtype)]))
+    for shape, takes in (((512, 512, 512), True), ((1032, 1028, 100), True), ((1032, 1028, 101), False), ((1032, 1027, 100), False), ((132, 196, 60), False)):
+        unit, = units(DType.Float32, *shape)
+        assert unit.options == (dict(direct_f32=True) if takes else {})
+        assert ("global_load_lds_dwordx4" in generate(unit.source, **unit.options).sources[0]) == takes
+    assert units(DType.Float16, 512, 512, 512)[0].options == {}
