@@ -15,6 +15,7 @@ from __future__ import annotations
 
 from typing import Optional, Tuple
 
+from . import tuner
 from .alu import DType, byteWidth
 from .codegen import SOURCE_OPTION
 from .kernelgen import KernelSource, LaunchStep, _prelude, fill, template
@@ -738,9 +739,21 @@ def attention_by_queries(heads: int, queries: int, size: int) -> bool:
     return queries <= ATTENTION_FEW_QUERIES and heads <= 128
 
 
-def _gen_attention(routine: Routine, numerics: str) -> Optional[KernelSource]:
+def attention_copiers(heads: int, keys: int, size: int, threads: int) -> int:
+    """Workgroups that write an extended cache beside those that attend to it, which otherwise each write their head's part on the way.
+
+    A workgroup writes at 100 GB/s, and few of them leave the chip idle: a decoding step of 12 heads over 1024 keys of 64 28.4 us apart, 27.5
+    on the way, 25.6 beside; over 4096 42.2, 47.5, 38.1; 48 heads over 1024 29.7, 27.8, 26.2, over 2048 37.1, 34.0, 32.3.  With more of them
+    the second reading costs more than it hides: 96 heads over 1024 34.1, 29.5, 30.6, over 2048 45.0, 36.8, 41.2; 192 over 1024 44.2, 34.6, 41.1."""
+    if heads > tuner.CU_COUNT // 4:
+        return 0
+    return min(tuner.CU_COUNT - heads, -(-2 * heads * keys * (size // 8) // threads))
+
+
+def _gen_attention(routine: Routine, numerics: str, appended=None) -> Optional[KernelSource]:
     """Fused attention over [B, L, N, H] / [B, S, N, H] float16 operands with H = 32, 64 or 128 and any L and S >= 1
-    (contiguous, or strided views with unit stride along the head dimension)."""
+    (contiguous, or strided views with unit stride along the head dimension).  `appended`: the parts that keys and values are put
+    together of (`attentioncache.Appended`); inputs are then q, the parts of k, the parts of v, and outputs the result, k and v."""
     import math
 
     t = routine.type
@@ -781,10 +794,16 @@ def _gen_attention(routine: Routine, numerics: str) -> Optional[KernelSource]:
             threads *= 2
         passes = -(-S // (threads // lanes))
         rounds = -(-passes // 10)  # ten keys and values of 16 bytes each in flight per thread
+        copiers = 0 if appended is None else attention_copiers(B * N, S, H, threads)
         src = _prelude(numerics) + fill(template("attention_few.hip.inc"), dict(
-            NH=N, L=L, S=S, H=H, CAUSAL=1 if params.get("isCausal") else 0, SCALE_LOG2E=repr(scale * math.log2(math.e)), THREADS=threads,
-            PASSES=-(-passes // rounds), ROUNDS=rounds, QB=qb, QL=ql, QN=qn, QOFF=qo, KB=kb, KS=ksp, KN=kn, KOFF=ko, VB=vb, VS=vsp, VN=vn, VOFF=vo,
-            OB=L * N * H, OL=N * H, ON=H))
+            NH=N, HEADS=B * N, COPIERS=copiers, L=L, S=S, H=H, CAUSAL=1 if params.get("isCausal") else 0, SCALE_LOG2E=repr(scale * math.log2(math.e)), THREADS=threads,
+            PASSES=-(-passes // rounds), ROUNDS=rounds, QB=qb, QL=ql, QN=qn, QOFF=qo, OB=L * N * H, OL=N * H, ON=H,
+            **(dict(APPENDED=0, KB=kb, KS=ksp, KN=kn, KOFF=ko, VB=vb, VS=vsp, VN=vn, VOFF=vo, **{f"{o}1{x}": 0 for o in "KV" for x in ("B", "S", "N", "OFF")})
+               if appended is None else dict(APPENDED=appended[0].first, **{k: v for o, a in zip("KV", appended) for k, v in a.fields(o).items()}))))
+        if appended is not None:
+            need = {0: need[0], 1: appended[0].need[0], 3: appended[0].need[1], 2: appended[1].need[0], 4: appended[1].need[1]}
+            args = [("in", i) for i in range(5)] + [("out", 1), ("out", 2), ("out", 0)]
+            return KernelSource([src], [LaunchStep("jh_attention_few", (B * N + copiers, 1, 1), (threads, 1, 1), 0, args)], [], "attention", need, dict(B=B, L=L, S=S, N=N, H=H, blocks=B * N, threads=threads))
         steps = [LaunchStep("jh_attention_few", (B * L * N, 1, 1), (threads, 1, 1), 0, [("in", 0), ("in", 1), ("in", 2), ("out", 0)])]
         return KernelSource([src], steps, [], "attention", need, dict(B=B, L=L, S=S, N=N, H=H, causal=bool(params.get("isCausal")), blocks=B * L * N, threads=threads))
     src = _prelude(numerics) + fill(template("attention.hip.inc"), dict(

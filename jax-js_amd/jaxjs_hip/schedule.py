@@ -16,6 +16,7 @@ from typing import Any, Dict, List, Optional, Sequence
 
 from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
+from .attentioncache import join_cache
 from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
 from .gemm import is_direct_product
@@ -188,6 +189,18 @@ def plan_units(prog) -> List[Unit]:
             ids = [i for d in run for i in d.inputs]
             units.append(Unit(Maps([d.kernel for d in run], ids), ids, [d.output for d in run]))
             k += together
+            continue
+        cached = join_cache(units[-1].source, units[-1].outputs, s.routine, s.inputs) if s.routine is not None and units and isinstance(units[-1].source, Maps) else None
+        if cached is not None:
+            joined, at = cached
+            maps, made = units[-1].source.kernels, units.pop().outputs
+            rest = [i for i in range(len(maps)) if i not in at]
+            before = steps[k - len(maps):k]
+            if rest:
+                ids = [i for r in rest for i in before[r].inputs]
+                units.append(Unit(maps[rest[0]] if len(rest) == 1 else Maps([maps[r] for r in rest], ids), ids, [made[r] for r in rest]))
+            units.append(Unit(joined, joined.inputs, s.outputs + [made[i] for i in at]))
+            k += 1
             continue
         product = None
         if s.routine is None and units and isinstance(units[-1].source, RowChain) and len(units[-1].outputs) == 1:

@@ -282,3 +282,36 @@ def test_sums_along_the_columns_are_not_taken_for_a_softmax():
     want = run_program(OracleBackend(), column, arrays)[0].astype(np.float64)
     np.testing.assert_allclose(got[1], want, rtol=1e-2, atol=3e-3 * np.abs(want).max())
     assert np.abs(got[0] - got[1]).max() > 0.1
+
+
+# Caches extended in the launch that attends to them: heads that write their own part (more than a quarter of the CUs) and copiers beside them, a cache
+# of one row, several new rows, new rows in front, key counts around the passes and several rounds, every head size; B, S, new, N, H, in front.
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, 64, False), (2, 127, 1, 3, 64, False), (1, 128, 3, 5, 32, True), (3, 700, 1, 2, 128, False), (8, 1024, 1, 12, 64, False), (13, 129, 2, 5, 128, True),
+                                  (1, 2600, 1, 2, 64, False), (10, 1400, 1, 7, 32, False)], ids=str)
+def test_attention_over_caches_that_the_program_extends(case):
+    if WARM_ONLY:
+        pytest.skip("warm-up run")
+    from jaxjs_hip import jit as J, library as L
+    from jaxjs_hip.attentioncache import CachedAttention
+    from jaxjs_hip.jit import ShapedArray
+    B, S, T, N, H, front = case
+
+    def f(q, keys, values, qkv):
+        k, v = (J.shrink(qkv, [(0, B), (0, T), (i * N * H, (i + 1) * N * H)]).reshape([B, T, N, H]) for i in (0, 1))
+        keys, values = (L.concatenate([n, o] if front else [o, n], 1) for o, n in ((keys, k), (values, v)))
+        return [L.dotProductAttention(q, keys, values), keys, values]
+    shapes = [(B, 1, N, H), (B, S, N, H), (B, S, N, H), (B, T, 2 * N * H)]
+    prog = J.jit(f, [ShapedArray(s, F16) for s in shapes])
+    rng = np.random.default_rng(S)
+    q, keys, values, qkv = [rng.standard_normal(s).astype(np.float16) for s in shapes]
+    keys[0, 0, 0, :8] = -0.0  # the sum of both padded parts makes these positive
+    be = backend()
+    assert any(isinstance(u.source, CachedAttention) for u in be.scheduleProgram(prog).units)
+    k, v = (qkv[:, :, i * N * H:(i + 1) * N * H].reshape(B, T, N, H) for i in (0, 1))
+    k, v = (np.concatenate([n, o] if front else [o, n], 1) + np.float16(0) for o, n in ((keys, k), (values, v)))
+    for _ in range(2):
+        got = run_program(be, prog, [q, keys, values, qkv])
+        np.testing.assert_array_equal(got[1].view(np.uint16), k.reshape(-1).view(np.uint16))
+        np.testing.assert_array_equal(got[2].view(np.uint16), v.reshape(-1).view(np.uint16))
+        want = R.run_oracle(attention_routine(B, 1, S + T, N, False, H=H), [q, k, v])[0]
+        np.testing.assert_allclose(got[0].astype(np.float64).reshape(want.shape), want.astype(np.float64), rtol=2e-3, atol=1e-3)

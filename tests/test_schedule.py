@@ -480,3 +480,23 @@ def test_schedules_ask_for_direct_loads_of_float32_products():
         assert unit.options == (dict(direct_f32=True) if takes else {})
         assert ("global_load_lds_dwordx4" in generate(unit.source, **unit.options).sources[0]) == takes
     assert units(DType.Float16, 512, 512, 512)[0].options == {}
+
+
+def test_an_attention_is_joined_with_the_copies_that_extend_its_caches():
+    from jaxjs_hip import DType, jit as J, library as L
+    from jaxjs_hip.jit import ShapedArray, jitCompile
+    from jaxjs_hip.rewrite import fuse_attention
+    from jaxjs_hip.schedule import plan_units
+
+    def kinds(queries, times=1, third=False):
+        def f(q, keys, values, k, v, x):
+            keys, values = L.concatenate([keys] + [k] * times, 1), L.concatenate([values] + [v] * times, 1)
+            out = [L.dotProductAttention(q, keys, values), keys, values]
+            return out + [x.mul(2)] if third else out
+        prog = J.jit(f, [ShapedArray((2, n, 4, 64), DType.Float16) for n in (queries, 300, 300, 1, 1, 1)])
+        prog = jitCompile(fuse_attention(prog.jaxpr, prog.consts), prog.consts, 30)
+        return [(type(u.source).__name__, len(u.outputs)) for u in plan_units(prog)]
+    assert kinds(1) == [("CachedAttention", 3)]
+    assert ("CachedAttention", 3) in kinds(1, third=True)  # beside another elementwise Kernel
+    assert kinds(2) == [("Maps", 2), ("Routine", 1)]       # two workgroups read a head's keys
+    assert kinds(1, times=2)[-1] == ("Routine", 1)         # three parts
