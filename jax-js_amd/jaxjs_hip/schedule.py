@@ -21,7 +21,7 @@ from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
 from .gemm import is_direct_product
 from .kernelgen import generate
-from .routine import Routine
+from .routine import Routine, Routines
 from .rowchain import RowChain, _tidy, collect_chain, index_form
 from .rowproduct import join_behind, join_rows
 from .runtime import LAUNCH_ARGS, LaunchRef, LaunchStepC, check
@@ -157,9 +157,22 @@ def adjacent_maps(steps: Sequence[_Dispatch], k: int, view) -> int:
     return n
 
 
+def before_rotations(steps: Sequence[_Dispatch]) -> set:
+    """The buffers that a JacobiEigh's matrix is made from.  Which sign and place an eigenvector gets from the rotations hangs on the
+    last bits of the matrix, so the products in front keep the order of sums that their Kernels have one by one (an SVD of
+    1024 x 128 returned negated vectors where its Gram matrix had another)."""
+    found: set = set()
+    for s in reversed(steps):
+        written = [s.output] if s.routine is None else s.outputs
+        if (s.routine is not None and s.routine.name == Routines.JacobiEigh) or any(o in found for o in written):
+            found.update(s.inputs)
+    return found
+
+
 def plan_units(prog) -> List[Unit]:
     """The program's dispatches with runs of Kernels over the same rows joined."""
     steps = plan_dispatches(prog)
+    rotated = before_rotations(steps)
     last_read: Dict[int, int] = {}
     for k, s in enumerate(steps):
         for i in s.inputs:
@@ -211,7 +224,8 @@ def plan_units(prog) -> List[Unit]:
             units[-1] = Unit(product, product.inputs, [s.output])
             k += 1
             continue
-        options = {} if s.routine is not None else dict(filter_bands=True) if is_filter_cotangent(s.kernel) else dict(direct_f32=True) if is_direct_product(s.kernel) else {}
+        options = {} if s.routine is not None else dict(filter_bands=True) if is_filter_cotangent(s.kernel) \
+            else dict(direct_f32=True) if s.output not in rotated and is_direct_product(s.kernel) else {}
         units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))
         k += 1
     return units

@@ -500,3 +500,20 @@ def test_an_attention_is_joined_with_the_copies_that_extend_its_caches():
     assert ("CachedAttention", 3) in kinds(1, third=True)  # beside another elementwise Kernel
     assert kinds(2) == [("Maps", 2), ("Routine", 1)]       # two workgroups read a head's keys
     assert kinds(1, times=2)[-1] == ("Routine", 1)         # three parts
+
+
+def test_products_in_front_of_rotations_keep_their_order_of_sums():
+    """The Gram matrix of an SVD, also by way of other Kernels: an eigenvector's sign hangs on its last bits.  The product behind
+    the rotations is as any other."""
+    from jaxjs_hip import DType, jit as J, library as L
+    from jaxjs_hip.gemm import is_direct_product
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.routine import Routines
+    from jaxjs_hip.schedule import plan_units
+
+    x = ShapedArray((1024, 128), DType.Float32)
+    for f in (lambda a: list(L.svd(a)), lambda a: list(L.eigh(J.sin(L.matmul(L.swapaxes(a, 0, 1), a))))):
+        units = plan_units(J.jit(f, [x]))
+        at = next(i for i, u in enumerate(units) if getattr(u.source, "name", None) == Routines.JacobiEigh)
+        assert is_direct_product(units[0].source) and not any(u.options for u in units[:at])
+    assert plan_units(J.jit(lambda a: L.matmul(L.swapaxes(a, 0, 1), a), [x]))[0].options == dict(direct_f32=True)
