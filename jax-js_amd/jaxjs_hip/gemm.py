@@ -380,6 +380,45 @@ def _repack_operand(g: dict):
     return tags
 
 
+def is_sliced_product(kernel: Kernel) -> bool:
+    """Whether `kernel` is better prepared with the option `sliced_f16`.  (An option for the reason that `direct_f32` is one.)
+
+    Slices of the k axis that need not be equal, of operands that a pre-pass may have to copy first, where the tile plan cuts in
+    halves and cuts no copies: 343 x 896 x 7104 40.2 -> 18.5 us, 448 x 395 x 3264 18.8 -> 10.9, 1125 x 768 x 4800 28.7 -> 18.4, 2176 x
+    265 x 3843 (weights along k) 68.7 -> 24.1, 4070 x 448 x 5184 31.9 -> 29.0.  In one slice, copies of both operands in one launch
+    instead of two (1984 x 1543 x 1281 26.4 -> 23.1), and behind fewer than 512 rows, where the general template's element loads cost
+    18 ns per k (379 x 5964 x 6175 111 -> 66), from k = 1024 on (3520 x 355 x 666 12.8 against 15.2).  Of 60 shapes drawn, 27 take it, none
+    slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4)."""
+    if kernel.reduction is None or kernel.size == 0:
+        return False
+    t = tuner.tuneHip(kernel)
+    if t.klass != "gemm" or t.gemm["dtype"] != DType.Float16 or few_plan(t) is not None:
+        return False
+    p = sliced_plan(t.gemm)
+    return p is not None and (p["slices"] > 1 or (p["repack"] == "ab" and (t.gemm["K"] >= 1024 or _repack_operand(t.gemm) is not None)))
+
+
+def sliced_plan(g: dict) -> Optional[dict]:
+    """Copies (`repack`, see `_repack_operand`, or ""), padded k axis, slab depth and slices of the k axis for a float16 product of up to
+    one 128x128 tile per CU; None where the tile plan stands.  Slice z walks the slabs from z * slabs / slices on.  The number of
+    slices is the cheapest by 6 ns per element of k, and 2 us and the partial sums at 5 TB/s for the fold's launch."""
+    if g["dtype"] != DType.Float16 or g["batch"] or g.get("a_gather") or g.get("b_gather") or g["a_k0"] != g["K"] or g["b_k0"] != g["K"]:
+        return None
+    M, N, K = g["M"], g["N"], g["K"]
+    count = -(-M // 128) * -(-N // 128)
+    if min(M, N) < 128 or K < 256 or count > tuner.CU_COUNT or any(g[s] != 1 and g[k] != 1 for s, k in (("a_sm", "a_sk"), ("b_sn", "b_sk"))):
+        return None
+    tags = "".join(t for t, rows in (("a", M), ("b", N))
+                   if g.get(t + "_loose") or K % 32 or not _edge_ok(rows, 128, g[t + "_sk"] == 1))
+    deep = 64 if K % 64 == 0 or K % 32 else 32
+    slabs = -(-K // deep)
+    if sum(M if t == "a" else N for t in tags) * slabs * deep * 2 > (1 << 30):
+        return None
+    most = max(1, min(slabs // 4, tuner.CU_COUNT // count))
+    us = [-(-slabs // n) * deep * 0.006 + (2.0 + n * M * N * 8 / 5e6 if n > 1 else 0.0) for n in range(1, most + 1)]
+    return dict(slices=us.index(min(us)) + 1, repack=tags, deep=deep, k=slabs * deep)
+
+
 def _edge_ok(extent: int, tile: int, k_contiguous: bool) -> bool:
     """Whether the direct-to-LDS template can take an operand whose row count is `extent` in tiles of `tile` rows: whole
     tiles, or an edge tile whose loads can be clamped -- to the last row when the operand runs along k in memory, to
@@ -672,7 +711,7 @@ def tap_major_form(oexp: AluExp, K: int):
 def few_plan(t: TuneResult) -> Optional[dict]:
     """The plan of the contraction `t` where the kernel for few rows or tiles takes it."""
     g = t.gemm
-    if g is None or g.get("direct") or t.params.get("gemm_tile") or _repack_operand(g) is not None:
+    if g is None or g.get("direct") or g.get("sliced") or t.params.get("gemm_tile") or _repack_operand(g) is not None:
         return None
     return plan_few(g, lambda: choose_tile(g))
 
@@ -700,7 +739,10 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
     assert g is not None and re is not None and t.epilogue is not None
     override = dict(t.params.get("gemm_tile") or {})
     few = few or few_plan(t)
-    tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few else choose_tile(g, bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex)))
+    sliced = sliced_plan(g) if g.get("sliced") and not few and not override else None
+    tile = dict() if ("BM" in override or "BN" in override) else dict(BM=128, BN=128) if few \
+        else dict(BM=128, BN=128, BK=sliced["deep"], STAGES=4, SPLITK=sliced["slices"]) if sliced \
+        else choose_tile(g, bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex)))
     tile.update(override)
     if "BM" not in tile or "BN" not in tile:
         raise ValueError("a tile override must give both BM and BN")
@@ -722,13 +764,13 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
     split = 1 if wgrad else int(tile.get("SPLITK", 1))
     K_full = g["K"]
     two_stride = dict(a=g["a_k0"] != K_full, b=g["b_k0"] != K_full)  # of the whole k axis, before any slicing
-    if split > 1:
+    if split > 1 and not sliced:
         vec_k = 8 if g["dtype"] == DType.Float16 else 4
         # a two-stride k axis is cut into whole runs, or a run into whole slices
         if (K_full % split or (K_full // split) % vec_k
                 or any(g[t + "_k0"] != K_full and (K_full // split) % g[t + "_k0"] and g[t + "_k0"] % (K_full // split) for t in ("a", "b"))):
             split = 1
-    if split > 1 and not override and not wgrad and _flipped_filter(g):
+    if split > 1 and not override and not wgrad and not sliced and _flipped_filter(g):
         import copy
 
         t2 = copy.copy(t)
@@ -736,26 +778,13 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
         whole = gen_gemm(kernel, t2, numerics, name)
         if whole.info.get("conv"):
             return whole
-    # ... or, with FUSEK (f32 template), folded inside the same launch by the slice that arrives last at the tile's
-    # counter: one launch instead of two.
-    fusek = 0
-    if split > 1:
-        KS = K_full // split
-        run_full = dict(a=g["a_k0"], b=g["b_k0"])
-        # (a slice inside one run has a single stride, like a slice of a single-stride axis)
-        g = dict(g, K=KS, a_k0=KS if g["a_k0"] == K_full or g["a_k0"] > KS else g["a_k0"],
-                 b_k0=KS if g["b_k0"] == K_full or g["b_k0"] > KS else g["b_k0"])
-        fusek = split if tile.get("FUSEK", 0) else 0
-        if not fusek:
-            out_t = "float"
-
     # An operand off the 16-byte grid that a pre-pass copies into scratch (see `_repack_operand`): from here on it is a
     # dense [K][rows_pad] operand named `jh_repack`.
-    repack = _repack_operand(g) if split == 1 and tile.get("REPACK", 1) and not few and not wgrad else None
+    repack = sliced["repack"] if sliced else _repack_operand(g) if split == 1 and tile.get("REPACK", 1) and not few and not wgrad else None
     load_rows = dict(a=g["M"], b=g["N"])
     repack_src = {}
     if repack:
-        k_pad = -(-g["K"] // 32) * 32
+        k_pad = sliced["k"] if sliced else -(-g["K"] // 32) * 32
         for tg in repack:
             rows = load_rows[tg]
             srow = g["a_sm"] if tg == "a" else g["b_sn"]
@@ -767,6 +796,19 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
             load_rows[tg] = rows_pad
             g = dict(g, **{tg + "_off": 0, tg + "_sk": 1 if kc else rows_pad, rkey: k_pad if kc else 1, tg + "_loose": False})
         g = dict(g, K=k_pad, a_k0=k_pad, b_k0=k_pad)
+
+    # ... or, with FUSEK (f32 template), folded inside the same launch by the slice that arrives last at the tile's
+    # counter: one launch instead of two.
+    fusek = 0
+    if split > 1 and not sliced:
+        KS = K_full // split
+        run_full = dict(a=g["a_k0"], b=g["b_k0"])
+        # (a slice inside one run has a single stride, like a slice of a single-stride axis)
+        g = dict(g, K=KS, a_k0=KS if g["a_k0"] == K_full or g["a_k0"] > KS else g["a_k0"],
+                 b_k0=KS if g["b_k0"] == K_full or g["b_k0"] > KS else g["b_k0"])
+        fusek = split if tile.get("FUSEK", 0) else 0
+    if split > 1 and not fusek:
+        out_t = "float"
 
     used = _used_args(kernel.nargs, t.epilogue)
     used[g["gid_a"]] = g["dtype"]
@@ -1106,7 +1148,11 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
     for b in g["batch"]:
         nbatch *= b[0]
     pitch = -(-kernel.size // 8) * 8  # elements between two slices' partial outputs
-    if split > 1:
+    if sliced and split > 1:
+        lines.append(f"  const int jh_first = (int)blockIdx.y * {g['K'] // sliced['deep']} / {split};  // slab")
+        lines.append(f"  a_base += (long long)jh_first * {sliced['deep'] * g['a_sk']}ll; b_base += (long long)jh_first * {sliced['deep'] * g['b_sk']}ll;"
+                     f" c_base += (long long)blockIdx.y * {pitch}ll;")
+    elif split > 1:
         # a slice starts K elements further along k: K * sk for one stride, (K / k0) runs of sk1 for two
         # (whether the axis has two strides is the whole axis's property: a slice of exactly one run has k0 == K too)
         # and for runs cut into r slices each, slice z is piece z % r of run z / r
@@ -1154,6 +1200,8 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
     any_gather = bool(g.get("a_gather") or g.get("b_gather"))
     loose = {tag: 1 if g.get(tag + "_loose") and not g.get(tag + "_gather") else 0 for tag in ("a", "b")}
     dlds = g["dtype"] == DType.Float16 and full and tile.get("DLDS", 1) and not any_gather and not (loose["a"] or loose["b"])
+    if sliced and not dlds:
+        raise ValueError("uneven slices of the k axis need the direct-to-LDS template")
     if repack and not dlds:  # the copy only serves the direct loads: plan again without it
         import copy
 
@@ -1171,6 +1219,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
         # Scalar-base addressing needs every lane offset inside one slab of a tile to fit 32 bits.
         span = 2 * max((BM - 1) * abs(g["a_sm"]) + dBK * abs(g["a_sk"]), (BN - 1) * abs(g["b_sn"]) + dBK * abs(g["b_sk"]))
         sched["SADDR"] = 1 if tile.get("SADDR", 1) and span < 2 ** 31 and g["a_sm"] >= 0 and g["a_sk"] >= 0 and g["b_sn"] >= 0 and g["b_sk"] >= 0 else 0
+        sched.update(SLICES=split if sliced else 1)
         sched.update(PIN=tile.get("PIN", 1), BAR_AT=tile.get("BAR_AT", 2), READ_AHEAD=tile.get("RA", 1), LOADS_LATE=tile.get("LATE", 1))
         # Tile walk: groups of 4 tile rows (8192^3: 865 -> 853 us against groups of 8, 873 with 16; one group spanning
         # all rows loses a third).  Nontemporal C stores only for the f32 partials of a k split, where a wave's store
@@ -1240,13 +1289,14 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
                                 4: "tap-major strided" if tap_major is not None else f"k{gather_group.get(tag, 8)}", 5: "rows4", 6: "k4", 7: f"k{gather_group.get(tag, 8)}"}[gather_flags[tag]] for tag in ("a", "b")}
         if tap_major is not None:
             info["tap_major"] = tap_major
+    scratch, copies, preps = [], [], []
     if repack:
         src += "\nstruct __attribute__((packed, aligned(2))) jh_half8_u { jh_half8 v; };\n"
-        preps, scratch = [], []
-        for si, tg in enumerate(repack):
+        calls = []
+        for tg in repack:
             rs = repack_src[tg]
             if rs["kc"]:
-                groups, outer, total = rs["k_pad"] // 8, rs["rows"], rs["rows"] * (rs["k_pad"] // 8)
+                groups, total = rs["k_pad"] // 8, rs["rows"] * (rs["k_pad"] // 8)
                 body = (f"  const int r = (int)(i / {groups}), k0 = (int)(i % {groups}) * 8;\n"
                         f"  const jh_f16* __restrict__ p = src + {rs['off']}ll + (long long)r * {rs['srow']}ll + k0;\n"
                         f"  const int valid = {rs['k']} - k0;\n"
@@ -1262,8 +1312,7 @@ def gen_gemm(kernel: Kernel, t: TuneResult, numerics: str, name: str, rows=None,
             src += (f"""
 // Operand {tg.upper()} {what}, first element {rs['off']}: eight elements per thread, one under-aligned 16-byte load and one
 // aligned store; what lies past the operand's extents is zeros.
-extern "C" __global__ __launch_bounds__(256) void {name}_repack_{tg}(const jh_f16* __restrict__ src, jh_f16* __restrict__ dst) {{
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+static __device__ __forceinline__ void jh_repack_of_{tg}(const jh_f16* __restrict__ src, jh_f16* __restrict__ dst, const long long i) {{
   if (i >= {total}ll) return;
 {body}  jh_half8 v;
   if (valid >= 8) {{
@@ -1275,13 +1324,24 @@ extern "C" __global__ __launch_bounds__(256) void {name}_repack_{tg}(const jh_f1
   *reinterpret_cast<jh_half8*>(q) = v;
 }}
 """)
-            preps.append(LaunchStep(f"{name}_repack_{tg}", (-(-total // 256), 1, 1), (256, 1, 1), 0, [("in", rs["gid"]), ("scratch", si)]))
-            step.args.append(("scratch", si))
+            calls.append((tg, -(-total // 256)))
+            copies.append(("scratch", len(scratch) + (split > 1)))  # (the buffer of a split's partial sums is the first)
             scratch.append(rs["k_pad"] * rs["rows_pad"] * 2)
+        step.args += copies
+        for group in ([calls] if sliced else [[c] for c in calls]):  # one launch for both, but where tests pin single Kernels' launches
+            jump, first = "", 0
+            for tg, blocks in group:
+                jump += (f"  if (blockIdx.x >= {first}u && blockIdx.x < {first + blocks}u)"
+                         f" jh_repack_of_{tg}(src_{tg}, dst_{tg}, (long long)(blockIdx.x - {first}u) * 256 + threadIdx.x);\n")
+                first += blocks
+            tags = "".join(tg for tg, _ in group)
+            src += (f'\nextern "C" __global__ __launch_bounds__(256) void {name}_repack_{tags}('
+                    + ", ".join(f"const jh_f16* __restrict__ src_{tg}, jh_f16* __restrict__ dst_{tg}" for tg in tags) + f") {{\n{jump}}}\n")
+            preps.append(LaunchStep(f"{name}_repack_{tags}", (first, 1, 1), (256, 1, 1), 0,
+                                    [a for tg in tags for a in (("in", repack_src[tg]["gid"]), copies[repack.index(tg)])]))
         info["repack"] = repack
-        return KernelSource([src], preps + [step], scratch, "gemm", need, info)
     if split == 1:
-        return KernelSource([src], [step], [], "gemm", need, info)
+        return KernelSource([src], preps + [step], scratch, "gemm", need, info)
     if fusek:
         info["fused_fold"] = True
         return KernelSource([src], [step], [split * tiles * BM * BN * 4, tiles * 4], "gemm", need, info, zeroed_scratch=[1])
@@ -1290,4 +1350,4 @@ extern "C" __global__ __launch_bounds__(256) void {name}_repack_{tg}(const jh_f1
     ks2, steps2, partial_len = fold_stage(kernel, numerics, name, split, pitch, slice_major=True)
     info["stage2"] = ks2.info
     need.update({gid_: b_ for gid_, b_ in ks2.min_input_bytes.items() if gid_ != kernel.nargs})
-    return KernelSource([src] + ks2.sources, [step] + steps2, [partial_len * 4], "gemm+fold", need, info)
+    return KernelSource([src] + ks2.sources, preps + [step] + steps2, [partial_len * 4] + scratch, "gemm+fold", need, info)

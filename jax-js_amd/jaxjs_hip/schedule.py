@@ -19,7 +19,7 @@ from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
 from .attentioncache import join_cache
 from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
-from .gemm import is_direct_product
+from .gemm import is_direct_product, is_sliced_product
 from .kernelgen import generate
 from .routine import Routine, Routines
 from .rowchain import RowChain, _tidy, collect_chain, index_form
@@ -225,7 +225,8 @@ def plan_units(prog) -> List[Unit]:
             k += 1
             continue
         options = {} if s.routine is not None else dict(filter_bands=True) if is_filter_cotangent(s.kernel) \
-            else dict(direct_f32=True) if s.output not in rotated and is_direct_product(s.kernel) else {}
+            else dict(direct_f32=True) if s.output not in rotated and is_direct_product(s.kernel) \
+            else dict(sliced_f16=True) if is_sliced_product(s.kernel) else {}
         units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))
         k += 1
     return units

@@ -490,9 +490,10 @@ def match_transposed_map(kernel: Kernel) -> Optional[dict]:
 def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True,
             gemm_tile: Optional[tuple] = None, col_strip: Optional[tuple] = None,
             row_lanes: Optional[int] = None, row_unroll: Optional[int] = None, row_nt: Optional[int] = None, col_nt: Optional[int] = None,
-            map_unroll: Optional[int] = None, map_nt: Optional[int] = None, filter_bands: bool = False, direct_f32: bool = False) -> TuneResult:
+            map_unroll: Optional[int] = None, map_nt: Optional[int] = None, filter_bands: bool = False, direct_f32: bool = False, sliced_f16: bool = False) -> TuneResult:
     """Pick the kernel class and its parameters for one Kernel on MI355X.  `filter_bands`: a convolution's filter cotangent
-    takes the kernel of `wgradgen.py` where that covers it.  `direct_f32`: a float32 product of any size has its slabs by direct loads."""
+    takes the kernel of `wgradgen.py` where that covers it.  `direct_f32`: a float32 product of any size has its slabs by direct loads.
+    `sliced_f16`: a float16 product follows `sliced_plan`."""
     t = tuneNullopt(kernel)
     re = kernel.reduction
     size = kernel.size
@@ -539,7 +540,7 @@ def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True
                 t.params["wgrad"] = find_wgrad(kernel, t, g)
             if t.params.get("wgrad") or _gemm_worthwhile(g):
                 t.klass = "gemm"
-                t.gemm = dict(g, direct=True) if direct_f32 else g
+                t.gemm = dict(g, direct=True) if direct_f32 else dict(g, sliced=True) if sliced_f16 else g
                 if gemm_tile:
                     t.params["gemm_tile"] = dict(gemm_tile)
                 return t

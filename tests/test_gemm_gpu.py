@@ -688,6 +688,24 @@ def test_gemm_f16_tiles_of_short_k_axes(M, N, K, layout, bias, tile):
     test_gemm_f16_direct_lds_edge_tiles(M, N, K, layout, tile, bias)
 
 
+# float16 products in uneven slices: a slab more or less in a slice, slabs of 32 and of 64, operands copied for their rows' start, their ragged
+# k axis or edges that cannot be clamped; one slice of copies; twice over, small integers, exact sums.
+@pytest.mark.parametrize("M,N,K", [(128, 128, 256), (129, 136, 1120), (300, 257, 2051), (131, 391, 1056), (384, 520, 4800), (515, 260, 1090)], ids=str)
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+def test_gemm_f16_uneven_slices(layout, M, N, K):
+    full = [M, N, K]
+    a, b = ([K, M], [1, 0]) if layout == "TN" else ([M, K], [0, 1]), ([N, K], [0, 1]) if layout == "NT" else ([K, N], [1, 0])
+    stA = ShapeTracker.fromShape(a[0]).permute(a[1]).reshape([M, 1, K]).expand(full)
+    stB = ShapeTracker.fromShape(b[0]).permute(b[1]).reshape([1, N, K]).expand(full)
+    k = reduceKernel(full, [(DType.Float16, stA), (DType.Float16, stB)], lambda x, y: AluExp.mul(x, y), AluOp.Add)
+    A, B = RNG.integers(-2, 3, (M, K)).astype(np.float16), RNG.integers(-1, 2, (K, N)).astype(np.float16)  # |sums| <= 4 sqrt(K) or so: exact in float16
+    bufs = [np.ascontiguousarray(A.T) if layout == "TN" else A, np.ascontiguousarray(B.T) if layout == "NT" else B]
+    for _ in range(2):
+        got, ks = device_run(k, bufs, sliced_f16=True)
+        assert ks.info["direct_lds"] and (K < 1024 or ks.info["splitk"] > 1), ks.info
+        np.testing.assert_array_equal(got.reshape(M, N).astype(np.float32), A.astype(np.float32) @ B.astype(np.float32), err_msg=str(ks.info))
+
+
 # Slabs of float32 operands by direct loads, under every plan: edge tiles in both directions, k axes of one slab, of whole slabs and of a
 # few floats more, fewer slabs than stages, slices that end inside a slab.
 @pytest.mark.parametrize("M,N,K,split", [(64, 64, 32, 1), (260, 124, 36, 1), (132, 196, 60, 1), (192, 128, 64, 1), (200, 264, 1000, 1), (68, 60, 528, 4), (516, 384, 1056, 8)], ids=str)

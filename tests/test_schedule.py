@@ -517,3 +517,15 @@ def test_products_in_front_of_rotations_keep_their_order_of_sums():
         at = next(i for i, u in enumerate(units) if getattr(u.source, "name", None) == Routines.JacobiEigh)
         assert is_direct_product(units[0].source) and not any(u.options for u in units[:at])
     assert plan_units(J.jit(lambda a: L.matmul(L.swapaxes(a, 0, 1), a), [x]))[0].options == dict(direct_f32=True)
+
+
+def test_schedules_ask_for_uneven_slices_of_float16_products():
+    from jaxjs_hip import DType, jit as J, library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import plan_units
+
+    for (m, n, k, t), takes in (((448, 395, 3264, True), True), ((2176, 265, 3843, True), True), ((1984, 1543, 1281, True), True), ((3520, 355, 666, True), False),
+                                ((704, 320, 3600, False), False), ((2048, 2048, 2048, False), False), ((8192, 8192, 8192, False), False)):
+        shapes = [ShapedArray((m, k), DType.Float16), ShapedArray((n, k) if t else (k, n), DType.Float16)]
+        unit, = plan_units(J.jit(lambda a, b: L.matmul(a, L.swapaxes(b, 0, 1) if t else b), shapes))
+        assert unit.options == (dict(sliced_f16=True) if takes else {}), (m, n, k)
