@@ -34,10 +34,9 @@ class GraphedProgram:
         for u in units:
             backend.pin(u.exe)
             self._exes.append(u.exe)
-        sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
         for u in units:
             for o in u.outputs:
-                slot = backend.malloc(sizes[o])
+                slot = backend.malloc(schedule.size_of(o))
                 self._slots[o] = slot
                 self._owned.append(slot)
 

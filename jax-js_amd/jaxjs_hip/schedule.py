@@ -356,6 +356,10 @@ class Schedule:
         self._inputs = [(i, self._need.get(i, 0)) for i in range(n)]
         self._zeroed = any(u.exe.data.ks.zeroed_scratch for u in self.units)
 
+    def size_of(self, buffer: int) -> int:
+        """Bytes of a buffer that a unit writes, of the program's or of the schedule's own."""
+        return self._sizes[buffer]
+
     def live(self) -> bool:
         """False once an executable of the schedule was released (evicted from the backend's cache)."""
         if self._releases != self.backend._releases:

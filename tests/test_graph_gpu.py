@@ -123,3 +123,20 @@ def test_graph_replay_of_a_k_split_folded_inside_the_launch():
         rng = np.random.default_rng(300 + r)
         return [rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)]
     _check_program(prog, operands)
+
+
+def test_graph_replay_of_convolutions_whose_weights_share_a_launch():
+    """The layouts' launch at the program's front writes buffers that are the schedule's and not the program's."""
+    from jaxjs_hip import DType
+    from jaxjs_hip import jit as J
+    from jaxjs_hip.composite import Weights
+    from jaxjs_hip.convolution import ConvParams
+    from jaxjs_hip.jit import ShapedArray
+
+    p = ConvParams(0, [1, 1], [(1, 1), (1, 1)], [1, 1], [1, 1])
+    shapes = [(2, 64, 14, 14), (64, 64, 3, 3), (64, 64, 3, 3)]
+    prog = J.jit(lambda x, a, b: [J.conv(J.conv(x, a, p), b, p)], [ShapedArray(s, DType.Float16) for s in shapes])
+    if WARM_ONLY:
+        pytest.skip("kernels are compiled by the convolution tests")
+    assert any(isinstance(u.source, Weights) for u in backend().scheduleProgram(prog).units)
+    _check_program(prog, lambda r: [(np.random.default_rng(10 * r + i).standard_normal(s) * 0.1).astype(np.float16) for i, s in enumerate(shapes)])
