@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
-from typing import Any, Dict, List, Optional, Sequence
+from typing import Any, Dict, List, Optional, Sequence, Tuple
 
 from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
@@ -21,6 +21,7 @@ from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
 from .errors import SlotError
 from .gemm import is_direct_product, is_sliced_product
 from .kernelgen import generate
+from .patches import Layouts, Packed, packs
 from .routine import Routine, Routines
 from .rowchain import RowChain, _tidy, collect_chain, index_form
 from .rowproduct import join_behind, join_rows
@@ -38,6 +39,7 @@ class Unit:
         self.source, self.inputs, self.outputs, self.options = source, list(inputs), list(outputs), options
         self.exe = None
         self.early: Optional[int] = None  # the buffer that holds what this unit's first step would make (see `Weights`)
+        self.sizes: Dict[int, int] = {}   # bytes of the outputs that are buffers of the schedule and not of the program
 
 
 _LONG_OPS = (AluOp.Erf, AluOp.Erfc, AluOp.Sin, AluOp.Cos, AluOp.Asin, AluOp.Atan)  # dozens of instructions each
@@ -76,48 +78,58 @@ def join_epilogue(product: Kernel, buffer: int, following: Kernel, inputs: Seque
     return Kernel(product.nargs, product.size, product.exp_raw, Reduction(re.dtype, re.op, re.size, exp))
 
 
-def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int]) -> Optional[Kernel]:
+def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int]) -> Tuple[Optional[Kernel], Optional[Packed]]:
     """The filter cotangent `product`, which writes `buffer`, with its outputs in the order in which the elementwise `following`
-    (reading `inputs`) reads them, and that Kernel as the rest of its epilogue; or None.
+    (reading `inputs`) reads them, and that Kernel as the rest of its epilogue, where a kernel of its own takes it then or its operands
+    are laid out (which comes with it); or None twice.
 
     The transpose rule of a convolution leaves the filter's cotangent with its channels exchanged, and puts them right by a
     copy ([64, 64, 3, 3]: a launch of 4.7 us; the product's last launch writes one order as fast as the other)."""
     re = product.reduction
     if re is None or following.reduction is not None or following.size != product.size or product.size == 0:
-        return None
+        return None, None
     reads = following.exp.collect(lambda n: n.op == AluOp.GlobalView)
     if not reads or any(inputs[n.arg[0]] != buffer or n.dtype != re.epilogue.dtype or n.arg[1] is not reads[0].arg[1] for n in reads):
-        return None
+        return None, None
     inside = set(id(n) for r in reads for s in r.src for n in s.collect(lambda n: n.op == AluOp.Special))
     if following.exp.collect(lambda n: n.op == AluOp.GlobalIndex or (n.op == AluOp.Special and id(n) not in inside)) \
             or re.epilogue.collect(lambda n: n.op in (AluOp.GlobalIndex, AluOp.GlobalView) or (n.op == AluOp.Special and n.arg[0] == "gidx")):
-        return None
+        return None, None
     views = product.exp.collect(lambda n: n.op == AluOp.GlobalView)
     st = reads[0].arg[1]
     shape = list(views[0].arg[1].shape[:-1]) if views else []
     if len(st.views) != 1 or st.views[0].mask is not None or st.views[0].offset != 0 or any(list(v.arg[1].shape[:-1]) != shape for v in views) \
             or sorted(st.shape) != sorted(shape) or prod(shape) != product.size:
-        return None
-    # axis k of the result is the product's axis with that stride; the walks of both Kernels have to be the plain ones
+        return None, None
+    # axis k of the result is the product's axis with that stride (any that is left, of length one); the walks of both Kernels have to be the plain ones
     strides = [prod(shape[i + 1:]) for i in range(len(shape))]
-    order = [next((i for i, (n, s) in enumerate(zip(shape, strides)) if (n, s) == want), -1) for want in zip(st.shape, st.views[0].strides)]
-    if sorted(order) != list(range(len(shape))):
-        return None
+    order: List[int] = []
+    for n, s in zip(st.shape, st.views[0].strides):
+        order.append(next((i for i, m in enumerate(shape) if i not in order and m == n and (n == 1 or strides[i] == s)), -1))
+    if -1 in order:
+        return None, None
     walk = lambda dims: [u.simplify() for u in unravelAlu(dims, AluVar.gidx)]  # noqa: E731
     if any(list(r.src) != walk(st.shape) for r in reads) or any(list(v.src) != walk(shape) + [AluVar.ridx] for v in views):
-        return None
+        return None, None
     exp = product.exp.rewrite(lambda n: AluExp.globalView(n.dtype, n.arg[0], n.arg[1].permute(order + [len(order)]), walk(st.shape) + [AluVar.ridx])
                               if n.op == AluOp.GlobalView else None)
     epilogue = following.exp.rewrite(lambda n: re.epilogue if n.op == AluOp.GlobalView else None)
     joined = Kernel(product.nargs, product.size, exp, Reduction(re.dtype, re.op, re.size, epilogue))
-    return joined if is_filter_cotangent(joined) else None
+    if is_filter_cotangent(joined):
+        return joined, None
+    packed = packs(joined, COPY_US)
+    return (joined, packed) if packed is not None else (None, None)
 
 
 class _Dispatch:
     """One dispatch of a program: `kernel` or `routine`, and buffer ids."""
 
-    def __init__(self, kernel, routine, inputs, output, outputs):
+    def __init__(self, kernel, routine, inputs, output, outputs, packed=None):
         self.kernel, self.routine, self.inputs, self.output, self.outputs = kernel, routine, inputs, output, outputs
+        self.packed = packed  # `kernel` with its operands laid out, where that is why it was made of two
+
+
+COPY_US = 3.0  # the copy that `join_transposed` spares
 
 
 def plan_dispatches(prog) -> List[_Dispatch]:
@@ -133,9 +145,13 @@ def plan_dispatches(prog) -> List[_Dispatch]:
         before = out[-1] if out else None
         if before is not None and before.kernel is not None and d.kernel is not None and before.output in d.inputs \
                 and reads[before.output] == 1 and before.output not in kept:
-            joined = join_epilogue(before.kernel, before.output, d.kernel, d.inputs) or join_transposed(before.kernel, before.output, d.kernel, d.inputs)
+            joined, packed = join_epilogue(before.kernel, before.output, d.kernel, d.inputs), None
             if joined is not None:
-                out[-1] = _Dispatch(joined, None, before.inputs, d.output, d.outputs)
+                packed = packs(joined, COPY_US) if before.packed is not None else None
+            else:
+                joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs)
+            if joined is not None:
+                out[-1] = _Dispatch(joined, None, before.inputs, d.output, d.outputs, packed)
                 continue
         out.append(d)
     return out
@@ -180,6 +196,7 @@ def plan_units(prog) -> List[Unit]:
     kept = set(prog.outputs)
     view = [(s.kernel, s.inputs, s.output) if s.routine is None else (None, s.inputs, -1) for s in steps]
     units: List[Unit] = []
+    fresh = max([prog.nargs - 1, *(i for s in prog.steps if s.kind == "malloc" for i in [s.output]), *(i for s in steps for i in s.inputs)]) + 1
     k = 0
     while k < len(steps):
         s = steps[k]
@@ -224,10 +241,25 @@ def plan_units(prog) -> List[Unit]:
             units[-1] = Unit(product, product.inputs, [s.output])
             k += 1
             continue
-        options = {} if s.routine is not None else dict(filter_bands=True) if is_filter_cotangent(s.kernel) \
-            else dict(direct_f32=True) if s.output not in rotated and is_direct_product(s.kernel) \
-            else dict(sliced_f16=True) if is_sliced_product(s.kernel) else {}
-        units.append(Unit(s.kernel if s.routine is None else s.routine, s.inputs, [s.output] if s.routine is None else s.outputs, **options))
+        if s.routine is not None:
+            units.append(Unit(s.routine, s.inputs, s.outputs))
+        elif is_filter_cotangent(s.kernel):
+            units.append(Unit(s.kernel, s.inputs, [s.output], filter_bands=True))
+        else:
+            kernel, inputs = s.kernel, list(s.inputs)
+            packed = (s.packed or packs(kernel)) if s.output not in rotated else None
+            if packed is not None:
+                kernel, made = packed.product, []
+                reads = [inputs[gid] for _layout, gid, _to in packed.layouts]
+                inputs += [-1] * (kernel.nargs - len(inputs))
+                for layout, _gid, to in packed.layouts:
+                    inputs[to] = fresh
+                    made.append(fresh)
+                    fresh += 1
+                units.append(Unit(Layouts([layout for layout, _gid, _to in packed.layouts], reads), reads, made))
+                units[-1].sizes = {to: layout.bytes for to, (layout, _gid, _to) in zip(made, packed.layouts)}
+            options = dict(direct_f32=True) if s.output not in rotated and is_direct_product(kernel) else dict(sliced_f16=True) if is_sliced_product(kernel) else {}
+            units.append(Unit(kernel, inputs, [s.output], **options))
         k += 1
     return units
 
@@ -276,6 +308,8 @@ class Schedule:
         self.backend, self.prog = backend, prog
         self.units = plan_units(prog)
         self._sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
+        for u in self.units:
+            self._sizes.update(u.sizes)
         self._made = list(dict.fromkeys(o for o in prog.outputs if o >= prog.nargs))
         self._increfs = [s.output for s in prog.steps if s.kind == "incref"]
         self._lock = threading.Lock()

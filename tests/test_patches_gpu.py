@@ -1,0 +1,178 @@
+"""Convolutions and their cotangents whose operands are laid out in front of the product, against float64 on the CPU.
+
+Sizes are at the edges of the layouts: k axes that end inside a 16-byte group, a slab and a slice, rows that do not divide over
+a workgroup's lanes, more groups of k than a workgroup has lanes, windows that hang over all sides, strides and dilations,
+channels below and above the matrix tiles, operands that are read twice or by the epilogue too."""
+import numpy as np
+import pytest
+import torch
+
+from jaxjs_hip import DType
+from jaxjs_hip import jit as J
+from jaxjs_hip.convolution import ConvParams
+from jaxjs_hip.jit import ShapedArray
+from jaxjs_hip.patches import Layouts
+from jaxjs_hip.schedule import plan_units
+
+from gpu_util import backend
+
+CASES = [  # dtype, batch, channels in and out, size, window, stride, padding, dilation
+    ("f32", 2, 41, 50, 16, 3, 1, 1, 1),
+    ("f32", 3, 20, 33, 21, 5, 2, 2, 1),
+    ("f32", 1, 37, 64, 19, 3, 1, 2, 2),
+    ("f32", 4, 130, 35, 9, 3, 1, 1, 1),
+    ("f32", 5, 35, 64, 25, 1, 1, 0, 1),
+    ("f32", 2, 17, 23, 30, 3, 1, 1, 1),
+    ("f16", 2, 172, 56, 20, 3, 2, 1, 1),
+    ("f16", 3, 41, 129, 13, 5, 2, 2, 1),
+    ("f16", 1, 90, 40, 17, 5, 1, 2, 1),
+    ("f16", 6, 45, 70, 11, 1, 1, 0, 1),
+    ("f16", 2, 26, 44, 21, 3, 1, 1, 1),
+]
+NP = dict(f32=np.float32, f16=np.float16)
+
+
+def programs(dtype, B, C, O, S, W, stride, pad, dilation):
+    p = ConvParams(0, [stride] * 2, [(pad, pad)] * 2, [1, 1], [dilation] * 2)
+    xs, ws = (B, C, S, S), (O, C, W, W)
+    out = (S + 2 * pad - dilation * (W - 1) - 1) // stride + 1
+    d = dict(f32=DType.Float32, f16=DType.Float16)[dtype]
+    x, w, ct = ShapedArray(xs, d), ShapedArray(ws, d), ShapedArray((B, O, out, out), d)
+    return dict(forward=(J.jit(lambda x, w: J.conv(x, w, p), [x, w]), (xs, ws)),
+                image=(J.jit(lambda ct, w: J.convTransposeLhs(ct, w, list(xs), p), [ct, w]), ((B, O, out, out), ws)),
+                filter=(J.jit(lambda x, ct: J.convTransposeRhs(x, ct, list(ws), p), [x, ct]), (xs, (B, O, out, out)))), (xs, ws, (B, O, out, out))
+
+
+def expected(which, args, shapes, stride, pad, dilation):
+    xs, ws, _ = shapes
+    t = [torch.from_numpy(a.astype(np.float64)) for a in args]
+    kw = dict(stride=stride, padding=pad, dilation=dilation)
+    if which == "forward":
+        return torch.nn.functional.conv2d(t[0], t[1], **kw).numpy()
+    if which == "image":
+        return torch.nn.grad.conv2d_input(list(xs), t[1], t[0], **kw).numpy()
+    return torch.nn.grad.conv2d_weight(t[0], list(ws), t[1], **kw).numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_laid_out_operands_give_the_convolution(case):
+    dtype, stride, pad, dilation = case[0], *case[6:]
+    be = backend()
+    rng = np.random.default_rng(len(str(case)))
+    made, shapes = programs(*case)
+    packed = 0
+    for which, (prog, operands) in made.items():
+        args = [rng.standard_normal(s).astype(NP[dtype]) for s in operands]
+        packed += any(isinstance(u.source, Layouts) for u in plan_units(prog))
+        prepared = prog.prepare(be)
+        slots = [be.malloc(a.nbytes, a) for a in args]
+        want = expected(which, args, shapes, stride, pad, dilation)
+        for _ in range(2):
+            out, = prog.execute(be, slots, prepared)
+            got = np.frombuffer(bytes(be.readSync(out)), NP[dtype]).reshape(want.shape).astype(np.float64)
+            be.decRef(out)
+            # float32 sums of n products of unit variance: each of up to n roundings is half a unit in the last place of a partial sum of
+            # at most a few sqrt(n); float16 results round once more, to 2^-11 of themselves
+            n = dict(forward=shapes[1][1] * case[5] ** 2, image=shapes[1][0] * case[5] ** 2, filter=shapes[2][0] * shapes[2][2] ** 2)[which]
+            bound = n * 2.0 ** -24 * 4 * np.sqrt(n) + (2.0 ** -11 * np.abs(want) + 2.0 ** -24 if dtype == "f16" else 0.0)
+            assert np.all(np.abs(got - want) <= bound), (which, float(np.max(np.abs(got - want) / bound)))
+        for s in slots:
+            be.decRef(s)
+    assert packed
+
+
+@pytest.mark.gpu
+def test_an_operand_that_the_epilogue_reads_too():
+    """The image joins the result behind the convolution: it is laid out beside its own buffer, which the epilogue reads."""
+    be = backend()
+    p = ConvParams(0, [1, 1], [(1, 1), (1, 1)], [1, 1], [1, 1])
+    x, w = ShapedArray((3, 41, 19, 19), DType.Float32), ShapedArray((41, 41, 3, 3), DType.Float32)
+    prog = J.jit(lambda x, w: J.conv(x, w, p).add(x), [x, w])
+    assert any(isinstance(u.source, Layouts) for u in plan_units(prog))
+    rng = np.random.default_rng(5)
+    args = [rng.standard_normal(a.shape).astype(np.float32) for a in (x, w)]
+    slots = [be.malloc(a.nbytes, a) for a in args]
+    out, = prog.execute(be, slots, prog.prepare(be))
+    got = np.frombuffer(bytes(be.readSync(out)), np.float32).reshape(args[0].shape)
+    want = expected("forward", args, (x.shape, w.shape, None), 1, 1, 1) + args[0]
+    n = 41 * 9
+    assert np.max(np.abs(got - want)) <= (n + 1) * 2.0 ** -24 * 4 * np.sqrt(n)
+    for s in slots + [out]:
+        be.decRef(s)
+
+
+def evaluate(e, env):
+    """An index or mask expression with C's division, which a masked element may come to with a negative operand."""
+    from jaxjs_hip.alu import AluOp
+
+    if e.op == AluOp.Const:
+        return np.int64(int(e.arg))
+    if e.op == AluOp.Special:
+        return env[e.arg[0]]
+    a = [np.asarray(evaluate(x, env)).astype(np.int64) for x in e.src]
+    if e.op in (AluOp.Idiv, AluOp.Mod):
+        q = np.abs(a[0]) // a[1] * np.sign(a[0])
+        return q if e.op == AluOp.Idiv else a[0] - q * a[1]
+    r = {AluOp.Add: lambda: a[0] + a[1], AluOp.Sub: lambda: a[0] - a[1], AluOp.Mul: lambda: a[0] * a[1], AluOp.Cmplt: lambda: a[0] < a[1],
+         AluOp.Cmpne: lambda: a[0] != a[1], AluOp.Cast: lambda: a[0], AluOp.Where: lambda: np.where(a[0] != 0, a[1], a[2])}[e.op]()
+    return r != 0 if e.dtype == DType.Bool else r
+
+
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_layouts_hold_the_elements_of_their_views(case):
+    """Every element of a layout by its (row, k) expression against the Kernel's own index expression, and zeros behind the axis."""
+    from jaxjs_hip.alu import AluExp
+    from jaxjs_hip.patches import pack
+
+    for prog, _operands in programs(*case)[0].values():
+        for u in prog.steps:
+            if u.kind != "execute" or u.kernel is None or (found := pack(u.kernel)) is None:
+                continue
+            for x, _gid, _to in found.layouts:
+                rows = int(np.prod(x.rows))
+                r, k = np.arange(0, rows, max(1, rows // 61), dtype=np.int64)[:, None], np.arange(x.st.shape[-1], dtype=np.int64)[None, :]
+                cond, load = x.place()
+                names = dict(row=r, k=k)
+                index = np.broadcast_to(evaluate(load.src[0], names), (r.shape[0], k.shape[1]))
+                inside = np.ones(index.shape, bool) if cond is None else np.broadcast_to(evaluate(cond, names), index.shape)
+                at, rest = [], r
+                for n in reversed(x.rows):
+                    at.insert(0, rest % n)
+                    rest = rest // n
+                axes = [AluExp.special(DType.Int32, f"x{i}", n) for i, n in enumerate(x.st.shape)]
+                ref, valid = x.st.toAluExp(axes)
+                env = {f"x{i}": v for i, v in enumerate(at + [k])}
+                ok = np.broadcast_to(evaluate(valid, env), index.shape)
+                assert np.array_equal(inside, ok)
+                assert np.array_equal(index[ok], np.broadcast_to(evaluate(ref, env), index.shape)[ok])
+                assert not ok.any() or (index[ok].min() >= 0 and index[ok].max() < load.arg[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[0], CASES[6]], ids=str)
+def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
+    """Replays of a graph with other values in between, and the dispatches of a traced run, against the launch list."""
+    from jaxjs_hip.graph import GraphedProgram
+
+    be = backend()
+    for prog, operands in programs(*case)[0].values():
+        prepared = prog.prepare(be)
+        if not any(isinstance(u.source, Layouts) for u in prepared.schedule.units):
+            continue
+        rng = np.random.default_rng(3)
+        slots = [be.malloc(a.nbytes, a) for a in (rng.standard_normal(s).astype(NP[case[0]]) for s in operands)]
+        graph = GraphedProgram(be, prog, slots)
+        for _ in range(3):
+            for s, shape in zip(slots, operands):
+                be.dev.h2d(be.slotPointer(s), rng.standard_normal(shape).astype(NP[case[0]]).tobytes())
+            out, = prog.execute(be, slots, prepared)
+            apart, = prepared.schedule._run_by_unit(slots)
+            graph.launch()
+            want = bytes(be.readSync(out))
+            assert bytes(be.readSync(apart)) == want and bytes(be.readSync(graph.outputs[0])) == want
+            be.decRef(out)
+            be.decRef(apart)
+        graph.close()
+        for s in slots:
+            be.decRef(s)
