@@ -110,6 +110,8 @@ class Packed:
 
     def __init__(self, layouts: List[Tuple[Layout, int, int]], product: Kernel):
         self.layouts, self.product = layouts, product
+        self.options = {}  # that the product is prepared with, beside its own
+        self.instead: Optional[Kernel] = None  # the contraction that would run otherwise
 
 
 def _operands(kernel: Kernel):
@@ -203,8 +205,8 @@ def _us_gathered(kernel: Kernel) -> float:
         loads = tuner._load_nodes(t.exp)
         half = byteWidth(loads[0].dtype) == 2
         vectors = all(str((t.vector_loads or {}).get(id(n), "")).startswith("vector") for n in loads)
-        runs = all(tuner._flatten_k_split(v.arg[1]) is not None for v in _operands(kernel)[0])
-        rate = 8e6 if vectors else 4e6 if K <= 64 else 2.5e6 if runs else 0.5e6 if half else 1.0e6  # products a microsecond
+        runs = all(w.mask is None for v in _operands(kernel)[0] for w in v.arg[1].views) and all(v.arg[1].views[0].strides[-1] == 1 for v in _operands(kernel)[0])
+        rate = 8e6 if vectors else 4e6 if K <= 64 else 2.5e6 if runs or K <= 128 else 0.65e6 if half else 1.0e6  # products a microsecond
         return 3.0 + kernel.size * K / rate
     g = t.gemm
     if not (g.get("a_gather") or g.get("b_gather")):
@@ -214,31 +216,60 @@ def _us_gathered(kernel: Kernel) -> float:
         return 0.0
     half = g["dtype"] == DType.Float16
     split = int(info.get("splitk", 1))
-    rounds = max(1.0, info["tiles"] * split / tuner.CU_COUNT) ** 0.7  # workgroups that share a CU hide each other's loads
+    rounds = max(1.0, info["tiles"] * split / tuner.CU_COUNT) ** 0.5  # workgroups that share a CU hide each other's loads
     single = sum(x == "element" for x in info.get("gather", {}).values())  # operands without vector loads
     per_k = (0.045 + 0.0275 * single + (0.03 if g.get("a_loose") or g.get("b_loose") else 0.0)) if half else 0.05 + 0.01 * single
     return max(3.0, per_k * K / split * rounds - 1.0) + (2.0 if split > 1 else 0.0)
 
 
-def _us_packed(packed: Packed) -> float:
-    """Estimated time of the layouts' launch and the product, in microseconds, fitted to the same Kernels: two launches, 0.6 million
-    elements laid out a microsecond (1.2 TB/s in float16, 2.4 in float32), and the product's walk over k."""
+def _us_packed(packed: Packed, sums_stay: bool) -> float:
+    """Estimated time of the layouts' launch and the product, in microseconds, fitted to the same Kernels: two launches, 0.5 to 0.6
+    million elements laid out a microsecond (1.2 TB/s in float16, 2 in float32), and the product's walk over k.  `sums_stay`: a
+    float32 contraction that a reduction by rows or columns computes stays with one, whose many short sums lose less than
+    the one of a matrix instruction's accumulator (relative error against 64 bits 1.4e-7 and 5.5e-7 over k = 30250).  Vectors of four make
+    a lane's sum four times as long, so a row gets up to four times as many lanes (9 x [28, 18, 18] by 25 x 5 x 5, stride 2, 1.32e-7
+    as it stands, 1.32e-7 laid out, 0.96e-7 with the lanes; 26, 10.4 and 11 us), and one that has them all and a longer axis is left as it is.
+
+    Other products of 2 to 31 rows or columns, which go to the reductions by rows as a rule, go to the matrix cores where that is estimated to
+    be faster: the reductions read the other operand once for each of those rows.  float16 16 x [64, 38, 38] to 24 channels, 3 x 3,
+    108 us there and 32 in tiles, 22 x [18, 26, 26] to 28, stride 2, 96 and 27, 25 x [64, 17, 17] to 27, stride 2, 84 and 33; but 3 x [59, 11, 11] to
+    23 8.9 and 9.9."""
     product = packed.product
     t, K = tuner.tuneHip(product), product.reduction.size
     half = packed.layouts[0][0].dtype == DType.Float16
-    us = 6.5 + sum(x.bytes // byteWidth(x.dtype) for x, _gid, _to in packed.layouts) / 6e5
-    if t.klass != "gemm":
-        return us + product.size * K / (5e6 if half else 3e6)
-    if few_plan(t) is not None:
-        return us + K * (0.005 if half else 0.008)
+    us = 7.0 + sum(x.bytes // byteWidth(x.dtype) for x, _gid, _to in packed.layouts) / (6e5 if half else 5e5)
+    if sums_stay:
+        packed.options = dict(allow_gemm=False)
+        s = tuner.tuneHip(product, allow_gemm=False)
+        if s.klass != "reduce_row":
+            return float("inf")
+        lanes = s.params["T"]
+        if lanes < 256 and K >= 8 * lanes:
+            lanes = packed.options["row_lanes"] = min(256, 4 * lanes)
+        if K > 32 * lanes:
+            return float("inf")
+        return us + product.size * K / 3e6
+    sums = product.size * K / (5e6 if half else 3e6) if t.klass != "gemm" else None
+    if sums is not None:
+        t = tuner.tuneHip(product, thin_rows=True)
+        if t.klass != "gemm":
+            return us + sums
     g, side = t.gemm, 128 if half else 64
-    tiles = -(-g["M"] // side) * -(-g["N"] // side) * prod([b[0] for b in g["batch"]])
-    slices = max(1, min(8, tuner.CU_COUNT // tiles, K // 512)) if half or not g["batch"] else 1
-    return us + K / slices * (0.0065 if half else 0.0165) * max(1.0, tiles / tuner.CU_COUNT) + (3.0 if slices > 1 else 0.0)
+    if few_plan(t) is not None:
+        walk = K * (0.005 if half else 0.008)
+    else:
+        tiles = -(-g["M"] // side) * -(-g["N"] // side) * prod([b[0] for b in g["batch"]])
+        slices = max(1, min(8, tuner.CU_COUNT // tiles, K // 512)) if half or not g["batch"] else 1
+        walk = K / slices * (0.0065 if half else 0.0165) * max(1.0, tiles / tuner.CU_COUNT) + (3.0 if slices > 1 else 0.0)
+    if sums is not None and sums <= walk:
+        return us + sums
+    packed.options = dict(thin_rows=True) if sums is not None else {}
+    return us + walk
 
 
-def packs(kernel: Kernel, spared: float = 0.0) -> Optional[Packed]:
-    """As `pack`, where that is estimated to be the faster side by a tenth; `spared`: microseconds of another launch that goes with it.
+def packs(kernel: Kernel, spared: float = 0.0, instead: Optional[Kernel] = None) -> Optional[Packed]:
+    """As `pack`, where that is estimated to be the faster side by a tenth; `instead`: the contraction that would run otherwise, if
+    that is another one, and `spared`: microseconds of a launch that comes with it.
 
     The tenth keeps what is about the same where it was.  Convolutions with a patch template or bands of their own stay with them
     (8 x [192, 45, 45] by 128 x 3 x 3 float16: 31 us there, 74 laid out), and so do short k axes (float16 [59, 45, 45] by 36 x 1 x 1,
@@ -246,5 +277,7 @@ def packs(kernel: Kernel, spared: float = 0.0) -> Optional[Packed]:
     found = pack(kernel)
     if found is None:
         return None
-    before = _us_gathered(kernel)
-    return found if before and _us_packed(found) < 0.9 * (before + spared) else None
+    found.instead = instead = instead or kernel
+    before = _us_gathered(instead)
+    sums_stay = instead.reduction.size > 64 and found.layouts[0][0].dtype == DType.Float32 and tuner.tuneHip(instead).klass != "gemm"
+    return found if before and _us_packed(found, sums_stay) < 0.9 * (before + spared) else None

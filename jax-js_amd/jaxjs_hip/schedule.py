@@ -117,7 +117,7 @@ def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Seq
     joined = Kernel(product.nargs, product.size, exp, Reduction(re.dtype, re.op, re.size, epilogue))
     if is_filter_cotangent(joined):
         return joined, None
-    packed = packs(joined, COPY_US)
+    packed = packs(joined, COPY_US, product)
     return (joined, packed) if packed is not None else (None, None)
 
 
@@ -147,7 +147,7 @@ def plan_dispatches(prog) -> List[_Dispatch]:
                 and reads[before.output] == 1 and before.output not in kept:
             joined, packed = join_epilogue(before.kernel, before.output, d.kernel, d.inputs), None
             if joined is not None:
-                packed = packs(joined, COPY_US) if before.packed is not None else None
+                packed = packs(joined, COPY_US, before.packed.instead) if before.packed is not None else None
             else:
                 joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs)
             if joined is not None:
@@ -258,7 +258,7 @@ def plan_units(prog) -> List[Unit]:
                     fresh += 1
                 units.append(Unit(Layouts([layout for layout, _gid, _to in packed.layouts], reads), reads, made))
                 units[-1].sizes = {to: layout.bytes for to, (layout, _gid, _to) in zip(made, packed.layouts)}
-            options = dict(direct_f32=True) if s.output not in rotated and is_direct_product(kernel) else dict(sliced_f16=True) if is_sliced_product(kernel) else {}
+            options = packed.options if packed is not None and packed.options else dict(direct_f32=True) if s.output not in rotated and is_direct_product(kernel) else dict(sliced_f16=True) if is_sliced_product(kernel) else {}
             units.append(Unit(kernel, inputs, [s.output], **options))
         k += 1
     return units

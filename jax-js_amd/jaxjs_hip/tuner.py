@@ -490,10 +490,10 @@ def match_transposed_map(kernel: Kernel) -> Optional[dict]:
 def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True,
             gemm_tile: Optional[tuple] = None, col_strip: Optional[tuple] = None,
             row_lanes: Optional[int] = None, row_unroll: Optional[int] = None, row_nt: Optional[int] = None, col_nt: Optional[int] = None,
-            map_unroll: Optional[int] = None, map_nt: Optional[int] = None, filter_bands: bool = False, direct_f32: bool = False, sliced_f16: bool = False) -> TuneResult:
+            map_unroll: Optional[int] = None, map_nt: Optional[int] = None, filter_bands: bool = False, direct_f32: bool = False, sliced_f16: bool = False, thin_rows: bool = False) -> TuneResult:
     """Pick the kernel class and its parameters for one Kernel on MI355X.  `filter_bands`: a convolution's filter cotangent
     takes the kernel of `wgradgen.py` where that covers it.  `direct_f32`: a float32 product of any size has its slabs by direct loads.
-    `sliced_f16`: a float16 product follows `sliced_plan`."""
+    `sliced_f16`: a float16 product follows `sliced_plan`.  `thin_rows`: a product of few rows or columns goes to the matrix cores all the same."""
     t = tuneNullopt(kernel)
     re = kernel.reduction
     size = kernel.size
@@ -538,7 +538,7 @@ def tuneHip(kernel: Kernel, *, allow_gemm: bool = True, allow_split: bool = True
                 from .wgradgen import find_wgrad
 
                 t.params["wgrad"] = find_wgrad(kernel, t, g)
-            if t.params.get("wgrad") or _gemm_worthwhile(g):
+            if t.params.get("wgrad") or _gemm_worthwhile(g, thin_rows):
                 t.klass = "gemm"
                 t.gemm = dict(g, direct=True) if direct_f32 else dict(g, sliced=True) if sliced_f16 else g
                 if gemm_tile:
@@ -688,7 +688,7 @@ GEMM_MIN_K = 32     # a shorter reduce axis than this: the reduction classes
 GEMM_MIN_ROWS = 32  # fewer rows (or columns) than this only against a large operand (see _gemm_worthwhile)
 
 
-def _gemm_worthwhile(g: dict) -> bool:
+def _gemm_worthwhile(g: dict, thin_rows: bool = False) -> bool:
     """MFMA tiles only pay off for a real dense contraction; thin shapes stream better through the
     row-reduce template (matvec and friends).  The tile loaders move 128-bit vectors along an operand's unit-stride
     axis (k or the row axis); the direct-to-LDS template needs every such vector whole and on the 16-byte grid, the
@@ -701,7 +701,7 @@ def _gemm_worthwhile(g: dict) -> bool:
     wide = max(g["M"], g["N"])
     # one row or column is a matvec: the reduction classes stream a large operand at the HBM rate
     reduces = thin < 2 or (thin < GEMM_MIN_ROWS and (wide < 128 or g["K"] < 256 or wide * g["K"] < (1 << 20)))
-    if reduces:
+    if reduces and not (thin_rows and thin >= 2):
         # ... but an operand that runs along the outputs is walked there one output a lane, or cut over k with a second launch
         # for the fold, where the kernel for few rows takes one launch: float16 1 x 768 x 768 6.3 -> 3.1 us, 8 x 512 x 512
         # 5.7 -> 2.7, 1 x 4096 x 2048 8.4 -> 4.2, 12 x 54 x 576 5.6 -> 2.7; float32 22 x 407 x 329 5.6 -> 2.8,

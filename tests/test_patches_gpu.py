@@ -176,3 +176,16 @@ def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
         graph.close()
         for s in slots:
             be.decRef(s)
+
+
+@pytest.mark.parametrize("case,options", [(("f16", 16, 24, 64, 38, 3, 1, 1, 1), dict(thin_rows=True)), (("f16", 2, 61, 21, 21, 3, 1, 1, 1), {}),
+                                          (("f32", 9, 28, 25, 18, 5, 2, 2, 1), dict(allow_gemm=False, row_lanes=64)), (("f32", 10, 67, 21, 55, 3, 1, 1, 1), None)], ids=str)
+def test_few_rows_behind_a_layout(case, options):
+    """Products of few rows: tiles, and a float32 sum by lanes that stays one, or stays where it was (`options` None), for the cotangent
+    towards the image (of the first), the forward direction (of the second and third) and the filter's (of the last)."""
+    made, _ = programs(*case)
+    prog = made["image" if case[1] == 16 else "filter" if options is None else "forward"][0]
+    units = plan_units(prog)
+    assert any(isinstance(u.source, Layouts) for u in units) == (options is not None)
+    if options is not None:
+        assert {k: v for k, v in units[-1].options.items()} == options
