@@ -258,7 +258,9 @@ def plan_units(prog) -> List[Unit]:
                     fresh += 1
                 units.append(Unit(Layouts([layout for layout, _gid, _to in packed.layouts], reads), reads, made))
                 units[-1].sizes = {to: layout.bytes for to, (layout, _gid, _to) in zip(made, packed.layouts)}
-            options = packed.options if packed is not None and packed.options else dict(direct_f32=True) if s.output not in rotated and is_direct_product(kernel) else dict(sliced_f16=True) if is_sliced_product(kernel) else {}
+            options = packed.options if packed is not None else {}
+            if not options and s.output not in rotated:
+                options = dict(direct_f32=True) if is_direct_product(kernel) else dict(sliced_f16=True) if is_sliced_product(kernel) else {}
             units.append(Unit(kernel, inputs, [s.output], **options))
         k += 1
     return units

@@ -519,6 +519,21 @@ def test_products_in_front_of_rotations_keep_their_order_of_sums():
     assert plan_units(J.jit(lambda a: L.matmul(L.swapaxes(a, 0, 1), a), [x]))[0].options == dict(direct_f32=True)
 
 
+@pytest.mark.parametrize("m,n", [(1024, 128), (2048, 256), (4096, 136), (3264, 400)], ids=str)
+def test_float16_products_in_front_of_rotations_keep_their_order_of_sums(m, n):
+    from jaxjs_hip import DType, jit as J, library as L
+    from jaxjs_hip.gemm import is_sliced_product
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.routine import Routines
+    from jaxjs_hip.schedule import plan_units
+
+    x = ShapedArray((m, n), DType.Float16)
+    for f in (lambda a: list(L.svd(a)), lambda a: list(L.eigh(L.matmul(L.swapaxes(a, 0, 1), a)))):
+        units = plan_units(J.jit(f, [x]))
+        at = next(i for i, u in enumerate(units) if getattr(u.source, "name", None) == Routines.JacobiEigh)
+        assert is_sliced_product(units[0].source) and not any(u.options for u in units[:at])
+
+
 def test_schedules_ask_for_uneven_slices_of_float16_products():
     from jaxjs_hip import DType, jit as J, library as L
     from jaxjs_hip.jit import ShapedArray
