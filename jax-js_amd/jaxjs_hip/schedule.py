@@ -78,10 +78,10 @@ def join_epilogue(product: Kernel, buffer: int, following: Kernel, inputs: Seque
     return Kernel(product.nargs, product.size, product.exp_raw, Reduction(re.dtype, re.op, re.size, exp))
 
 
-def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int]) -> Tuple[Optional[Kernel], Optional[Packed]]:
+def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Sequence[int], layouts: bool) -> Tuple[Optional[Kernel], Optional[Packed]]:
     """The filter cotangent `product`, which writes `buffer`, with its outputs in the order in which the elementwise `following`
-    (reading `inputs`) reads them, and that Kernel as the rest of its epilogue, where a kernel of its own takes it then or its operands
-    are laid out (which comes with it); or None twice.
+    (reading `inputs`) reads them, and that Kernel as the rest of its epilogue, where a kernel of its own takes it then or, with
+    `layouts`, its operands are laid out (which comes with it); or None twice.
 
     The transpose rule of a convolution leaves the filter's cotangent with its channels exchanged, and puts them right by a
     copy ([64, 64, 3, 3]: a launch of 4.7 us; the product's last launch writes one order as fast as the other)."""
@@ -117,7 +117,7 @@ def join_transposed(product: Kernel, buffer: int, following: Kernel, inputs: Seq
     joined = Kernel(product.nargs, product.size, exp, Reduction(re.dtype, re.op, re.size, epilogue))
     if is_filter_cotangent(joined):
         return joined, None
-    packed = packs(joined, COPY_US, product)
+    packed = packs(joined, COPY_US, product) if layouts else None
     return (joined, packed) if packed is not None else (None, None)
 
 
@@ -140,6 +140,7 @@ def plan_dispatches(prog) -> List[_Dispatch]:
         for i in set(d.inputs):
             reads[i] = reads.get(i, 0) + 1
     kept = set(prog.outputs)
+    rotated = before_rotations(made)
     out: List[_Dispatch] = []
     for d in made:
         before = out[-1] if out else None
@@ -149,7 +150,7 @@ def plan_dispatches(prog) -> List[_Dispatch]:
             if joined is not None:
                 packed = packs(joined, COPY_US, before.packed.instead) if before.packed is not None else None
             else:
-                joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs)
+                joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs, d.output not in rotated)
             if joined is not None:
                 out[-1] = _Dispatch(joined, None, before.inputs, d.output, d.outputs, packed)
                 continue

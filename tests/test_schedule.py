@@ -519,6 +519,32 @@ def test_products_in_front_of_rotations_keep_their_order_of_sums():
     assert plan_units(J.jit(lambda a: L.matmul(L.swapaxes(a, 0, 1), a), [x]))[0].options == dict(direct_f32=True)
 
 
+def _filter_cotangent_program(behind):
+    """A convolution's filter cotangent whose operands are laid out, the copy that exchanges its channels joined, and what is behind."""
+    from jaxjs_hip import DType, jit as J
+    from jaxjs_hip.convolution import ConvParams
+    from jaxjs_hip.jit import ShapedArray
+
+    p = ConvParams(0, [1, 1], [(2, 2), (2, 2)], [1, 1], [1, 1])
+    return J.jit(lambda x, ct: behind(J.convTransposeRhs(x, ct, [54, 43, 5, 5], p)), [ShapedArray((9, 43, 37, 37), DType.Float32), ShapedArray((9, 54, 37, 37), DType.Float32)])
+
+
+def test_a_copy_is_not_joined_for_layouts_that_are_held_back(monkeypatch):
+    """In front of rotations no operands are laid out, and nothing is joined because they would be."""
+    from jaxjs_hip import jit as J, library as L, schedule
+    from jaxjs_hip.patches import Layouts
+
+    assert [type(u.source) for u in schedule.plan_units(_filter_cotangent_program(lambda w: w))][0] is Layouts
+
+    def gram(w):
+        m = w.reshape([54, 43 * 25])
+        return [w] + list(L.eigh(L.matmul(m, L.swapaxes(m, 0, 1))))
+    prog = _filter_cotangent_program(gram)
+    units = [(u.source.key() if hasattr(u.source, "reduction") else type(u.source), u.options) for u in schedule.plan_units(prog)]
+    monkeypatch.setattr(schedule, "packs", lambda *a: None)
+    assert units == [(u.source.key() if hasattr(u.source, "reduction") else type(u.source), u.options) for u in schedule.plan_units(prog)]
+
+
 @pytest.mark.parametrize("m,n", [(1024, 128), (2048, 256), (4096, 136), (3264, 400)], ids=str)
 def test_float16_products_in_front_of_rotations_keep_their_order_of_sums(m, n):
     from jaxjs_hip import DType, jit as J, library as L
