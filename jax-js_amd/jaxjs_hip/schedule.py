@@ -147,10 +147,11 @@ def plan_dispatches(prog) -> List[_Dispatch]:
         if before is not None and before.kernel is not None and d.kernel is not None and before.output in d.inputs \
                 and reads[before.output] == 1 and before.output not in kept:
             joined, packed = join_epilogue(before.kernel, before.output, d.kernel, d.inputs), None
-            if joined is not None:
-                packed = packs(joined, COPY_US, before.packed.instead) if before.packed is not None else None
-            else:
+            if joined is None:
                 joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs, d.output not in rotated)
+            elif before.packed is not None:  # two joined for the sake of layouts: a third only if they stay
+                packed = packs(joined, COPY_US, before.packed.instead)
+                joined = joined if packed is not None else None
             if joined is not None:
                 out[-1] = _Dispatch(joined, None, before.inputs, d.output, d.outputs, packed)
                 continue

@@ -2,9 +2,10 @@
 import numpy as np
 import pytest
 
-from jaxjs_hip.alu import AluExp, DType
+from jaxjs_hip.alu import AluExp, AluVar, DType
 from jaxjs_hip.rowchain import index_form
 from jaxjs_hip.schedule import Unit, place_intermediates
+from jaxjs_hip.shape import ShapeTracker
 
 
 @pytest.mark.parametrize("seed", range(40))
@@ -543,6 +544,30 @@ def test_a_copy_is_not_joined_for_layouts_that_are_held_back(monkeypatch):
     units = [(u.source.key() if hasattr(u.source, "reduction") else type(u.source), u.options) for u in schedule.plan_units(prog)]
     monkeypatch.setattr(schedule, "packs", lambda *a: None)
     assert units == [(u.source.key() if hasattr(u.source, "reduction") else type(u.source), u.options) for u in schedule.plan_units(prog)]
+
+
+def test_an_epilogue_that_ends_the_layouts_stays_a_launch_of_its_own(monkeypatch):
+    from types import SimpleNamespace
+
+    from jaxjs_hip import schedule
+    from jaxjs_hip.alu import Kernel
+    from jaxjs_hip.patches import Layouts, packs
+
+    made = _filter_cotangent_program(lambda w: w)
+    last = [s for s in made.steps if s.kind == "execute"][-1]
+    n = last.kernel.size
+    twice = Kernel(1, n, AluExp.mul(AluExp.globalView(DType.Float32, 0, ShapeTracker.fromShape([n]), [AluVar.gidx]), AluExp.const(DType.Float32, 2.0)))
+    step = SimpleNamespace(kind="execute", kernel=twice, routine=None, inputs=[last.output], output=last.output + 1, outputs=[], size=0)
+    prog = SimpleNamespace(steps=made.steps + [step], outputs=[step.output], nargs=made.nargs)
+    assert [type(u.source) is Layouts for u in schedule.plan_units(prog)] == [True, False]  # the product with the copy and the factor
+    calls = []
+
+    def once(*a):
+        calls.append(a)
+        return packs(*a) if len(calls) == 1 else None
+    monkeypatch.setattr(schedule, "packs", once)
+    units = schedule.plan_units(prog)
+    assert len(calls) == 2 and [type(u.source) is Layouts for u in units] == [True, False, False]
 
 
 @pytest.mark.parametrize("m,n", [(1024, 128), (2048, 256), (4096, 136), (3264, 400)], ids=str)
