@@ -37,14 +37,15 @@ class Layout:
         return prod(self.rows) * self.K * byteWidth(self.dtype)
 
     def place(self):
-        """(mask or None, load) of element (row, k), or None where its expression has another form."""
+        """(mask or None, load) of element (row, k), or None where its expression has another form or is not a 32-bit number (a plain
+        operand may lie anywhere in its buffer: the templates find its rows by 64-bit strides)."""
         row = AluExp.special(DType.Int32, "row", max(prod(self.rows), 1))
         at = [u.simplify() for u in unravelAlu(self.rows, row)] + [AluExp.special(DType.Int32, "k", self.st.shape[-1])]
         e = AluExp.globalView(self.dtype, 0, self.st, at).rewriteGlobalViews().reduceExactIndex().simplify()
         cond = None
         if e.op == AluOp.Where and e.src[2].op == AluOp.Const and float(e.src[2].arg) == 0.0:
             cond, e = e.src[0], e.src[1]
-        return (cond, e) if e.op == AluOp.GlobalIndex else None
+        return (cond, e) if e.op == AluOp.GlobalIndex and e.src[0].min >= -(1 << 31) and e.src[0].max < 1 << 31 else None
 
 
 class Layouts(Composite):

@@ -149,6 +149,21 @@ def test_layouts_hold_the_elements_of_their_views(case):
                 assert not ok.any() or (index[ok].min() >= 0 and index[ok].max() < load.arg[1])
 
 
+@pytest.mark.parametrize("stride,taken", [(1 << 10, True), ((1 << 31) // 32, True), (1 << 27, False)], ids=str)
+def test_operands_past_32_bit_indices_are_not_laid_out(stride, taken):
+    """A plain operand whose rows lie far apart, beside a gathered one: element 2^31 of its buffer has no 32-bit index."""
+    from jaxjs_hip.alu import AluExp, AluOp
+    from jaxjs_hip.lowering import reduceKernel
+    from jaxjs_hip.patches import pack
+    from jaxjs_hip.shape import ShapeTracker, View
+
+    M, N, K = 256, 32, 70
+    a = ShapeTracker.fromShape([M, K - 2]).pad([(0, 0), (1, 1)]).reshape([M, 1, K]).expand([M, N, K])
+    b = ShapeTracker([View.create([N, K], [stride, 1], 0, None)]).reshape([1, N, K]).expand([M, N, K])
+    found = pack(reduceKernel([M, N, K], [(DType.Float16, a), (DType.Float16, b)], AluExp.mul, AluOp.Add))
+    assert (found is not None) == taken
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", [CASES[0], CASES[6]], ids=str)
 def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
