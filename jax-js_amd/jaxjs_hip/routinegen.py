@@ -37,6 +37,7 @@ SORT_SMALL_TILE, SORT_FEW_TILES = 4096, 64
 SORT_LOCAL, SORT_TILES = 16, 1024  # words of a lane in a tile's register runs, from 1024 tiles on
 SORT_HELD = 8     # pieces of 16 bytes that a lane hands to others at a time: whole lines of 128 bytes (float32 32768 x 1024: 70.6 us, 83 with 4)
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
+LAUNCH_THREADS = (1 << 32) - 1  # of a launch, along one axis
 CHOLESKY_PANEL_FROM = 192  # matrix order from which many matrices may take two launches a panel, and a plan counts its panels
 CHOLESKY_WAVE_BELOW = {2: 44, 4: 28, 8: 28}  # matrix order, by bytes per element, below which many matrices take a wave each
 
@@ -66,7 +67,7 @@ def _round64(n: int, cap: int = 1024) -> int:
     return max(64, min(cap, (n + 63) // 64 * 64))
 
 
-_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1, RHS=1, ELEM_BYTES=4,
+_LINALG_DEFAULTS = dict(N=1, M=1, THREADS=64, UNIT=0, IN_LDS=0, MAX_SWEEPS=0, TOL="0.0", BATCH=1, AHEAD=16, STAGED=0, RB=1, RHS=1, ELEM_BYTES=4, BLOCK="unsigned",
                         ELEM="float", CMP="float")
 # Element types of the dense routines: C type, the type magnitudes are compared in, bytes per element.
 _FLOAT_ELEMS = {DType.Float32: ("float", "float", 4), DType.Float64: ("double", "double", 8), DType.Float16: ("jh_f16", "float", 2)}
@@ -236,15 +237,15 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     if m <= 4096:
         rows = -(-m // 1024)  # of a thread of the panel's workgroup, in registers with as many columns as fit
         width = min(32, 1 << (64 // (rows * (2 if eb == 8 else 1))).bit_length() - 1, max(8, 1 << (min(m, n) - 1).bit_length()))
-        src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb)
+        src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb, BLOCK="unsigned" if batch * -(-n // 8) + batch < 1 << 32 else "unsigned long long")
         steps = []
         for j in range(0, max(min(m, n), 1), width):
             steps.append(LaunchStep("jh_lu_panel", (batch, 1, 1), (_round64(m - j), 1, 1), 0,
                                     [("in", 0), ("out", 0), ("out", 1), ("out", 2), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j)]))
             strips = -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
-            if strips:
-                steps.append(LaunchStep("jh_lu_strip", (batch * strips, 1, 1), (512, 1, 1), 0,
-                                        [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j)]))
+            for first in range(0, batch * strips, LAUNCH_THREADS // 512):
+                steps.append(LaunchStep("jh_lu_strip", (min(batch * strips - first, LAUNCH_THREADS // 512), 1, 1), (512, 1, 1), 0,
+                                        [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j), ("const", first)]))
         return KernelSource([src], steps, [batch * width * m * 8, batch * m * 4, max(batch * 4, 16)], "lu", {0: batch * m * n * eb},
                             dict(m=m, n=n, batch=batch, launches=len(steps), **({"variant": "by columns"} if min(m, n) >= LU_BY_COLUMNS_FROM else {})))
     if min(m, n) >= LU_BY_COLUMNS_FROM and batch * m * n < (1 << 31):

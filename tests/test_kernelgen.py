@@ -315,3 +315,24 @@ def test_attention_takes_a_workgroup_per_query_only_for_few_queries_of_few_heads
     shapes = [[B, t, N, size] for t in (queries, 2048, 2048)]
     ks = generateRoutine(Routine(Routines.Attention, RoutineType(shapes, [DType.Float16] * 3, [shapes[0]], [DType.Float16]), dict(scale=0.125)))
     assert [s.name for s in ks.steps] == ["jh_attention_few" if by_queries else "jh_attention"]
+
+
+@pytest.mark.parametrize("shape", [(140000, 8, 512), (3, 8, 100_000_000), (9_000_000, 8, 16), (2_000_000, 70, 33), (1 << 25, 1, 1200)], ids=str)
+def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
+    """Every strip of every matrix once, in launches of the size that the device takes."""
+    from jaxjs_hip.routine import Routine, Routines, RoutineType
+    from jaxjs_hip.routinegen import generateRoutine
+
+    batch, m, n = shape
+    ks = generateRoutine(Routine(Routines.LU, RoutineType([shape], [DType.Float32], [shape, (batch, min(m, n)), (batch, m)], [DType.Float32, DType.Int32, DType.Int32])))
+    assert all(s.grid[0] * s.block[0] < 1 << 32 for s in ks.steps)
+    done = {}
+    for s in ks.steps:
+        if s.name == "jh_lu_strip":
+            j, first = s.args[-2][1], s.args[-1][1]
+            assert first == done.get(j, 0)
+            done[j] = first + s.grid[0]
+    width = max(8, min(32, 1 << (min(m, n) - 1).bit_length()))
+    for j, blocks in done.items():
+        assert blocks == batch * (-(-j // 8) + -(-(n - min(j + width, m, n)) // 8))
+    assert ("(unsigned long long)first + blockIdx.x" in ks.sources[0]) == (max(done.values(), default=0) >= 1 << 32)

@@ -549,6 +549,17 @@ def test_lu_panels_at_their_edges(shape, dt):
     assert_bits(got, want, f"lu {shape} {np.dtype(dt).name} {ks.info}")
 
 
+@pytest.mark.parametrize("shape", [(5, 40, 70), (23, 9, 11)], ids=str)
+def test_lu_strips_in_several_launches(shape, monkeypatch):
+    """More strips than a launch holds, with the bound lowered to seven of them: launches that begin and end inside a matrix."""
+    from jaxjs_hip import routinegen
+    monkeypatch.setattr(routinegen, "LAUNCH_THREADS", 7 * 512 + 511)
+    a = RNG.uniform(-1, 1, shape).astype(F32)
+    got, want, ks = both(R.lu(a), [a])
+    assert max(s.grid[0] for s in ks.steps if s.name == "jh_lu_strip") == 7
+    assert_bits(got, want, f"lu {shape} {ks.info}")
+
+
 @pytest.mark.parametrize("n,m,mats,dt", [(1, 1, 1, F32), (7, 8, 1, F32), (8, 9, 3, F32), (9, 1, 2, F32), (17, 2049, 1, F32), (25, 4100, 1, F32), (40, 8200, 1, F32), (127, 17, 1, F32),
                                          (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16)],
                          ids=lambda v: np.dtype(v).name if isinstance(v, type) else str(v))
