@@ -31,7 +31,7 @@ from typing import Dict, List, Optional, Sequence
 
 from . import tracing
 from .alu import Kernel, byteWidth
-from .errors import HipRuntimeError, SlotError, UnsupportedRoutineError
+from .errors import DeviceMemoryError, HipRuntimeError, SlotError, UnsupportedRoutineError
 from .kernelgen import NUMERICS, KernelSource, generate
 from .routine import Routine
 from .composite import Composite
@@ -298,7 +298,16 @@ class HipBackend:
             blobs = [compile_source(src, f"{ks.klass}.hip") for src in ks.sources]
         modules = [self.dev.load_module(b) for b in blobs]
         functions = [self.dev.function(modules[s.module], s.name) for s in ks.steps]
-        scratch = [self.dev.malloc(self._rounded(b)) for b in ks.scratch_bytes]
+        scratch = []
+        try:
+            for b in ks.scratch_bytes:
+                scratch.append(self.dev.malloc(self._rounded(b)))
+        except DeviceMemoryError:
+            for ptr in scratch:
+                self.dev.free(ptr)
+            for m in modules:
+                self.dev.unload_module(m)
+            raise
         for i in ks.zeroed_scratch:
             self.dev.h2d(scratch[i], bytes(ks.scratch_bytes[i]))
         return Executable(source, _Prepared(ks, functions, scratch, modules))

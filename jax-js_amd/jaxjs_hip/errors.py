@@ -32,3 +32,7 @@ class UnsupportedRoutineError(Exception):
 
 class HipRuntimeError(RuntimeError):
     """A failure reported by the native runtime (compile error, launch failure, missing library)."""
+
+
+class DeviceMemoryError(HipRuntimeError):
+    """The device has no room for an allocation."""

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 from typing import Dict, List, Sequence
 
+from .errors import DeviceMemoryError
 from .jit import JitProgram
 
 
@@ -21,12 +22,19 @@ class GraphedProgram:
         self.backend, self.prog = backend, prog
         self._slots: Dict[int, int] = {i: s for i, s in enumerate(inputs)}
         self._owned: List[int] = []
-        for s in inputs:
-            backend.incRef(s)
-            self._owned.append(s)
         # The units of the program's schedule, compiled and loaded before any capture; a routine is several launches and
         # outputs, recorded the same way.
         schedule = backend.scheduleProgram(prog)
+        try:
+            self._make_room(schedule)
+        except DeviceMemoryError:
+            if not schedule.laid_out:
+                raise
+            schedule = schedule.without_layouts()
+            self._make_room(schedule)
+        for s in inputs:
+            backend.incRef(s)
+            self._owned.append(s)
         prog, units = schedule.prog, schedule.units
         # The graph launches these executables' code objects and writes their scratch buffers without going through
         # dispatch: pin them so that neither cache eviction nor clearCache() can release them under a replay.
@@ -34,11 +42,6 @@ class GraphedProgram:
         for u in units:
             backend.pin(u.exe)
             self._exes.append(u.exe)
-        for u in units:
-            for o in u.outputs:
-                slot = backend.malloc(schedule.size_of(o))
-                self._slots[o] = slot
-                self._owned.append(slot)
 
         def issue():
             for u in units:
@@ -59,6 +62,20 @@ class GraphedProgram:
             backend.trace, backend.capturing = trace, False
         self.outputs = [self._slots[o] for o in prog.outputs]
         self.kernels = len(units)
+
+    def _make_room(self, schedule) -> None:
+        """A slot for every buffer that the schedule's units write."""
+        made: Dict[int, int] = {}
+        try:
+            for u in schedule.units:
+                for o in u.outputs:
+                    made[o] = self.backend.malloc(schedule.size_of(o))
+        except BaseException:
+            for s in made.values():
+                self.backend.decRef(s)
+            raise
+        self._slots.update(made)
+        self._owned.extend(made.values())
 
     def launch(self) -> None:
         """Queue one replay of the whole program (asynchronous, in order with everything else)."""

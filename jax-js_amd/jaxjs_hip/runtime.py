@@ -15,7 +15,7 @@ import numpy as np
 from typing import List, Optional, Sequence, Tuple
 
 from .codegen import SOURCE_OPTION, SOURCE_OPTIONS_ALLOWED
-from .errors import HipRuntimeError
+from .errors import DeviceMemoryError, HipRuntimeError
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG, "csrc", "libjaxhip.so")
@@ -130,10 +130,13 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
-def check(rc: int, what: str) -> None:
+OUT_OF_MEMORY = 2  # hipErrorOutOfMemory
+
+
+def check(rc: int, what: str, error=HipRuntimeError) -> None:
     if rc != 0:
         msg = load_library().jh_last_error().decode(errors="replace")
-        raise HipRuntimeError(f"{what} failed (status {rc}): {msg}")
+        raise error(f"{what} failed (status {rc}): {msg}")
 
 
 _toolchain: Optional[str] = None
@@ -222,7 +225,8 @@ class Device:
     # -- memory ---------------------------------------------------------------------------------
     def malloc(self, nbytes: int) -> int:
         p = ctypes.c_void_p()
-        check(self.lib.jh_malloc(nbytes, ctypes.byref(p)), f"jh_malloc({nbytes})")
+        rc = self.lib.jh_malloc(nbytes, ctypes.byref(p))
+        check(rc, f"jh_malloc({nbytes})", DeviceMemoryError if rc == OUT_OF_MEMORY else HipRuntimeError)
         return p.value or 0
 
     def free(self, ptr: int) -> None:

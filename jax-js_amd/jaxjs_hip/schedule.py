@@ -18,7 +18,7 @@ from . import tracing
 from .alu import AluExp, AluOp, AluVar, DType, Kernel, Reduction, byteWidth
 from .attentioncache import join_cache
 from .composite import MAPS_MOST, WEIGHTS_MOST, Maps, Weights, joins_maps
-from .errors import SlotError
+from .errors import DeviceMemoryError, SlotError
 from .gemm import is_direct_product, is_sliced_product
 from .kernelgen import generate
 from .patches import Layouts, Packed, packs
@@ -132,7 +132,7 @@ class _Dispatch:
 COPY_US = 3.0  # the copy that `join_transposed` spares
 
 
-def plan_dispatches(prog) -> List[_Dispatch]:
+def plan_dispatches(prog, layouts: bool = True) -> List[_Dispatch]:
     """The program's dispatches, elementwise Kernels behind a contraction joined to it where nothing else reads its result."""
     made = [_Dispatch(s.kernel, s.routine, s.inputs, s.output, s.outputs) for s in prog.steps if s.kind == "execute"]
     reads: Dict[int, int] = {}
@@ -148,7 +148,7 @@ def plan_dispatches(prog) -> List[_Dispatch]:
                 and reads[before.output] == 1 and before.output not in kept:
             joined, packed = join_epilogue(before.kernel, before.output, d.kernel, d.inputs), None
             if joined is None:
-                joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs, d.output not in rotated)
+                joined, packed = join_transposed(before.kernel, before.output, d.kernel, d.inputs, layouts and d.output not in rotated)
             elif before.packed is not None:  # two joined for the sake of layouts: a third only if they stay
                 packed = packs(joined, COPY_US, before.packed.instead)
                 joined = joined if packed is not None else None
@@ -187,9 +187,9 @@ def before_rotations(steps: Sequence[_Dispatch]) -> set:
     return found
 
 
-def plan_units(prog) -> List[Unit]:
-    """The program's dispatches with runs of Kernels over the same rows joined."""
-    steps = plan_dispatches(prog)
+def plan_units(prog, layouts: bool = True) -> List[Unit]:
+    """The program's dispatches with runs of Kernels over the same rows joined.  `layouts`: operands may be laid out as matrices."""
+    steps = plan_dispatches(prog, layouts)
     rotated = before_rotations(steps)
     last_read: Dict[int, int] = {}
     for k, s in enumerate(steps):
@@ -249,7 +249,7 @@ def plan_units(prog) -> List[Unit]:
             units.append(Unit(s.kernel, s.inputs, [s.output], filter_bands=True))
         else:
             kernel, inputs = s.kernel, list(s.inputs)
-            packed = (s.packed or packs(kernel)) if s.output not in rotated else None
+            packed = (s.packed or packs(kernel)) if layouts and s.output not in rotated else None
             if packed is not None:
                 kernel, made = packed.product, []
                 reads = [inputs[gid] for _layout, gid, _to in packed.layouts]
@@ -299,9 +299,12 @@ def place_intermediates(units: Sequence[Unit], sizes: Dict[int, int], keep) -> D
 
 
 class Schedule:
-    """A jit program prepared for one backend."""
+    """A jit program prepared for one backend.
 
-    def __init__(self, backend, prog):
+    Operands that are laid out as matrices are memory that a program does without as well (up to 1 GiB a contraction): a call for which
+    the device has no room runs by a second schedule that lays out none, and so do later ones."""
+
+    def __init__(self, backend, prog, layouts: bool = True):
         from .jit import jitCompile
         from .rewrite import fuse_attention
 
@@ -310,7 +313,10 @@ class Schedule:
         if fused is not None:
             prog = jitCompile(fused, prog.consts, backend.maxArgs)
         self.backend, self.prog = backend, prog
-        self.units = plan_units(prog)
+        self.units = plan_units(prog, layouts)
+        self.laid_out = any(isinstance(u.source, Layouts) for u in self.units)
+        self._lean: Optional[Schedule] = None
+        self._no_room = False  # for its layouts, in an earlier call
         self._sizes = {s.output: s.size for s in prog.steps if s.kind == "malloc"}
         for u in self.units:
             self._sizes.update(u.sizes)
@@ -320,7 +326,13 @@ class Schedule:
         pinned = []
         try:  # a unit that is prepared here must not push out one that was prepared before it
             for u in self.units:
-                u.exe = backend.prepareSync(u.source, **u.options)
+                try:
+                    u.exe = backend.prepareSync(u.source, **u.options)
+                except DeviceMemoryError:  # of the executable's own workspace
+                    if not u.options:
+                        raise
+                    u.options = {}
+                    u.exe = backend.prepareSync(u.source)
                 backend.pin(u.exe)
                 pinned.append(u.exe)
             for u in self._weights():
@@ -406,7 +418,22 @@ class Schedule:
             self._releases = self.backend._releases
         return True
 
+    def without_layouts(self) -> "Schedule":
+        if self._lean is None or not self._lean.live():
+            self._lean = Schedule(self.backend, self.source, layouts=False)
+        return self._lean
+
     def run(self, inputs: Sequence[int]) -> List[int]:
+        if not self._no_room:
+            try:
+                return self._run(inputs)
+            except DeviceMemoryError:
+                if not self.laid_out:
+                    raise
+                self._no_room = True
+        return self.without_layouts().run(inputs)
+
+    def _run(self, inputs: Sequence[int]) -> List[int]:
         be, prog = self.backend, self.prog
         if len(inputs) != prog.nargs:
             raise ValueError(f"jit program takes {prog.nargs} inputs, got {len(inputs)}")
@@ -454,15 +481,19 @@ class Schedule:
         """The same dispatches one at a time, for per-dispatch timestamps."""
         be, prog = self.backend, self.prog
         scope = dict(enumerate(inputs))
-        owned = []
-        for u in self.units:
-            for o in u.outputs:
-                scope[o] = be.malloc(self._sizes[o])
-                if o not in self._made:
-                    owned.append(scope[o])
-            be.dispatch(u.exe, [scope[i] for i in u.inputs], [scope[o] for o in u.outputs])
-        for s in owned:
-            be.decRef(s)
+        made: Dict[int, int] = {}
+        try:
+            for u in self.units:
+                for o in u.outputs:
+                    scope[o] = made[o] = be.malloc(self._sizes[o])
+                be.dispatch(u.exe, [scope[i] for i in u.inputs], [scope[o] for o in u.outputs])
+        except BaseException:
+            for s in made.values():
+                be.decRef(s)
+            raise
+        for o, s in made.items():
+            if o not in self._made:
+                be.decRef(s)
         for o in self._increfs:
             be.incRef(scope[o])
         return [scope[o] for o in prog.outputs]

@@ -193,6 +193,45 @@ def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
             be.decRef(s)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[0], CASES[6]], ids=str)
+def test_programs_without_room_for_layouts(case, monkeypatch):
+    """Executed, under capture and one dispatch at a time: the bits of the schedule that lays out nothing."""
+    from jaxjs_hip.errors import DeviceMemoryError
+    from jaxjs_hip.graph import GraphedProgram
+    from jaxjs_hip.schedule import Schedule
+
+    be = backend()
+    made, shapes = programs(*case)
+    prog, operands = made["forward"]
+    rng = np.random.default_rng(11)
+    slots = [be.malloc(a.nbytes, a) for a in (rng.standard_normal(s).astype(NP[case[0]]) for s in operands)]
+    want, = Schedule(be, prog, layouts=False).run(slots)
+    size, plain = int(np.prod(shapes[2])) * np.dtype(NP[case[0]]).itemsize, be._alloc
+
+    def small(n):
+        if n > size:
+            raise DeviceMemoryError(f"no room for {n} bytes")
+        return plain(n)
+    before = be.live_slots()
+    monkeypatch.setattr(be, "_alloc", small)
+    schedule = Schedule(be, prog)
+    monkeypatch.setattr(be, "scheduleProgram", lambda p: Schedule(be, p))
+    assert schedule.laid_out
+    outs = schedule.run(slots) + schedule.run(slots)
+    graph = GraphedProgram(be, prog, slots)
+    for _ in range(2):
+        graph.launch()
+        for o in outs + graph.outputs:
+            assert bytes(be.readSync(o)) == bytes(be.readSync(want))
+    graph.close()
+    for o in outs:
+        be.decRef(o)
+    assert be.live_slots() == before
+    for s in slots + [want]:
+        be.decRef(s)
+
+
 @pytest.mark.parametrize("case,options", [(("f16", 16, 24, 64, 38, 3, 1, 1, 1), dict(thin_rows=True)), (("f16", 2, 61, 21, 21, 3, 1, 1, 1), {}),
                                           (("f32", 9, 28, 25, 18, 5, 2, 2, 1), dict(allow_gemm=False, row_lanes=64)), (("f32", 10, 67, 21, 55, 3, 1, 1, 1), None)], ids=str)
 def test_few_rows_behind_a_layout(case, options):

@@ -570,6 +570,45 @@ def test_an_epilogue_that_ends_the_layouts_stays_a_launch_of_its_own(monkeypatch
     assert [type(u.source) is Layouts for u in units] == [True, False, False]
 
 
+def test_a_program_without_room_for_layouts_runs_without_them():
+    from types import SimpleNamespace
+
+    from jaxjs_hip.errors import DeviceMemoryError
+    from jaxjs_hip.graph import GraphedProgram
+    from jaxjs_hip.schedule import Schedule
+
+    prog = _filter_cotangent_program(lambda w: w)
+    size = 9 * 54 * 37 * 37 * 4  # of the larger input
+
+    def device(most):
+        be, launched = _stand_in(), []
+
+        def alloc(n):
+            if n > most:
+                raise DeviceMemoryError(f"no room for {n} bytes")
+            return 64
+        be._alloc, be._release = alloc, lambda ptr, n: None
+        be.dev.lib = SimpleNamespace(jh_launch_list=lambda steps, n, refs, buf: launched.append(n) or 0)
+        return be, launched, [be.malloc(size) for _ in range(2)]
+    be, launched, inputs = device(1 << 40)
+    schedule = Schedule(be, prog)
+    assert schedule.laid_out and len(schedule.run(inputs)) == 1
+    be, launched, inputs = device(size)
+    schedule = Schedule(be, prog)
+    for n in (1, 2):
+        assert len(schedule.run(inputs)) == 1 and len(launched) == n
+        assert be.live_slots() == 2 + n  # what the attempt with layouts made was given back
+    lean = schedule.without_layouts()
+    assert not lean.laid_out and launched == [lean._n_steps] * 2
+    graph = GraphedProgram.__new__(GraphedProgram)
+    graph.backend, graph._slots, graph._owned = be, {}, []
+    with pytest.raises(DeviceMemoryError):
+        graph._make_room(schedule)
+    assert be.live_slots() == 4 and not graph._owned
+    graph._make_room(lean)
+    assert be.live_slots() == 4 + len(graph._owned)
+
+
 @pytest.mark.parametrize("m,n", [(1024, 128), (2048, 256), (4096, 136), (3264, 400)], ids=str)
 def test_float16_products_in_front_of_rotations_keep_their_order_of_sums(m, n):
     from jaxjs_hip import DType, jit as J, library as L
