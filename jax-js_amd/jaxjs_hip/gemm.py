@@ -94,18 +94,20 @@ _F32_PLANS = ((dict(BM=64, BN=64, WM=2, WN=2, WK=2, STAGES=4), 2.18, 71.0, 274.5
               (dict(BM=128, BN=128, WM=4, WN=2, WK=1, STAGES=2), 3.10, 12.2, 281.9e3, 0.988, 1.130, 0.993))
 
 
-def _f32_tile(g: dict, tiles, nb: int) -> Dict[str, int]:
+def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Dict[str, int]:
     """Plan of a float32 product whose slabs go to LDS by direct loads (`_f32_direct`), by an estimate: a launch, the tiles of the
     CU that gets most of them at the plan's rate, and the fold of slices of the k axis inside the launch.  It is a fit to 132
     products of 64 to 8192 rows, columns and k in both orders of B under all plans, within 1.7 per cent of the fastest one in
     the mean, 26 at worst (128 x 2144 x 216).  Against staging slabs in registers: 1024 x 1024 x 1024 25.9 -> 19.8 us, 2048
     150 -> 124, 4096 1080 -> 946 (145 TFLOP/s), 8192 8596 -> 7565, 3632 x 3088 x 144 49.6 -> 37.0, 1280 x 640 x 320 10.5 -> 7.6, 960 x 384 x
-    3696 95.9 -> 41.5, 3672 x 768 x 1408 86.9 -> 69.4."""
+    3696 95.9 -> 41.5, 3672 x 768 x 1408 86.9 -> 69.4.
+    `parts`: slices of the k axis that staging in registers takes, each a chain of roundings as long as itself.  Here a chain is half
+    of what a wave has of a slice, and only plans that make it no longer are taken.  The others grew the error of four in 400 drawn products."""
     best = None
     for plan, launch, fill, rate, alone, fold, sums in _F32_PLANS:
         count = tiles(plan["BM"], plan["BN"])
         for split in (1, 2, 4, 8):
-            if split > 1 and (nb > 1 or g["K"] % (4 * split) or g["K"] // split < 64):
+            if 2 * plan["WK"] * split < parts or (split > 1 and (nb > 1 or g["K"] % (4 * split) or g["K"] // split < 64)):
                 continue
             per_cu = -(-count * split // tuner.CU_COUNT)
             us = launch + per_cu * plan["BM"] * plan["BN"] * (g["K"] / split + fill) / (rate * (alone if per_cu == 1 else 1.0))
@@ -188,7 +190,7 @@ def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
         # Direct loads where a schedule asks for them, and for any Kernel of at least two 128x128 tiles per CU, whose plans nothing pins
         # (8192^3 8596 -> 7565 us; 4096^3 1080 -> 946).
         if _f32_direct(g) and (g.get("direct") or tiles(128, 128) >= 2 * CU):
-            return _f32_tile(g, tiles, nb)
+            return _f32_tile(g, tiles, nb, 1 if tiles(128, 128) >= 2 * CU else choose_tile(dict(g, direct=False)).get("SPLITK", 1))
         if plain_k and not loose_ops and g["M"] >= 128 and g["N"] >= 64 and tiles(128, 64) * 4 > CU:
             return _f32_staged_tile(g, tiles, nb)
         # Among the shapes that do, the cheapest by (rounds of two workgroups per CU) x (tile area) / (rate of the

@@ -336,3 +336,18 @@ def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
     for j, blocks in done.items():
         assert blocks == batch * (-(-j // 8) + -(-(n - min(j + width, m, n)) // 8))
     assert ("(unsigned long long)first + blockIdx.x" in ks.sources[0]) == (max(done.values(), default=0) >= 1 << 32)
+
+
+@pytest.mark.parametrize("m,n,k", [(652, 896, 704), (512, 1408, 768), (192, 3904, 832), (448, 1536, 576), (2072, 256, 640), (608, 832, 576), (1080, 512, 640), (1024, 1024, 1024),
+                                   (960, 384, 3696), (256, 256, 256)], ids=str)
+def test_direct_loads_make_no_chain_of_roundings_longer(m, n, k):
+    """A wave adds half of its part of a slice in a row; staged in registers it is a whole slice."""
+    from jaxjs_hip import gemm, tuner
+    from jaxjs_hip.lowering import matmulKernel
+
+    kernel = matmulKernel(m, n, k, DType.Float32)
+    assert gemm.is_direct_product(kernel)
+    g = tuner.tuneHip(kernel).gemm
+    staged, direct = gemm.choose_tile(dict(g, direct=False)), gemm.choose_tile(dict(g, direct=True))
+    assert not staged.get("DLDS") and direct["DLDS"]
+    assert 2 * direct["WK"] * direct.get("SPLITK", 1) >= staged.get("SPLITK", 1)
