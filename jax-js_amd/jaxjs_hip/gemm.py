@@ -390,20 +390,38 @@ def is_sliced_product(kernel: Kernel) -> bool:
     265 x 3843 (weights along k) 68.7 -> 24.1, 4070 x 448 x 5184 31.9 -> 29.0.  In one slice, copies of both operands in one launch
     instead of two (1984 x 1543 x 1281 26.4 -> 23.1), and behind fewer than 512 rows, where the general template's element loads cost
     18 ns per k (379 x 5964 x 6175 111 -> 66), from k = 1024 on (3520 x 355 x 666 12.8 against 15.2).  Of 60 shapes drawn, 27 take it, none
-    slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4)."""
+    slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4).
+
+    Whole operands that the tile plan gives eight waves stay with it: blocks of 128 to 1536 rows and width 192 or 224, whose second MLP product
+    has a k axis of 768 or 896, were all slower or no faster with it cut (768 x 192 35.4 and 36.1 us for the block, 1344 x 224 41.7 and 43.8).  With
+    four waves, from a k axis of 1024 on, blocks are faster by up to a quarter (448 x 704 66.8 -> 49.1, 768 x 768 60.5 -> 54.7, 462 x 256 37.0 -> 35.4), also
+    where the tile plan folds two slices inside the launch.  With an epilogue that reads nothing one plain launch takes less, half a
+    microsecond or, of operands that both run along k, one, and partial sums whose rows are off the 16-byte grid cost more: alone,
+    384 x 1664 x 1344 9.6 us and 11.4 cut, along k 512 x 821 x 1280 8.8 and 12.6, 256 x 3008 x 1792 11.0 and 12.5, 1024 x 285 x 1344 9.1 and 9.9, but
+    421 x 2112 x 1984 15.1 and 14.1, and 640 x 320 x 1088 8.6 and 8.3."""
     if kernel.reduction is None or kernel.size == 0:
         return False
     t = tuner.tuneHip(kernel)
     if t.klass != "gemm" or t.gemm["dtype"] != DType.Float16 or few_plan(t) is not None:
         return False
-    p = sliced_plan(t.gemm)
-    return p is not None and (p["slices"] > 1 or (p["repack"] == "ab" and (t.gemm["K"] >= 1024 or _repack_operand(t.gemm) is not None)))
+    g, p = t.gemm, sliced_plan(t.gemm)
+    if p is None:
+        return False
+    if p["slices"] > 1 and not p["repack"]:
+        tile = choose_tile(g)
+        if tile.get("WM", 2) * tile.get("WN", 2) == 8:
+            return False
+        if tile.get("SPLITK", 1) == 1:
+            reads = bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex))
+            return p["gain"] >= (0.0 if reads else 1.05 if g["a_sk"] == 1 and g["b_sk"] == 1 else 0.5) + (1e-6 * p["slices"] * g["M"] * g["N"] if g["N"] % 4 else 0.0)
+    return p["slices"] > 1 or (p["repack"] == "ab" and (g["K"] >= 1024 or _repack_operand(g) is not None))
 
 
 def sliced_plan(g: dict) -> Optional[dict]:
-    """Copies (`repack`, see `_repack_operand`, or ""), padded k axis, slab depth and slices of the k axis for a float16 product of up to
+    """Copies (`repack`, see `_repack_operand`, or ""), padded k axis, slab depth and slices of the k axis, and what the slices gain, for a float16 product of up to
     one 128x128 tile per CU; None where the tile plan stands.  Slice z walks the slabs from z * slabs / slices on.  The number of
-    slices is the cheapest by 6 ns per element of k, and 2 us and the partial sums at 5 TB/s for the fold's launch."""
+    slices is the cheapest by 6 ns per element of k, and 2.2 us and the partial sums at 5 TB/s for the fold's launch (2.0 cut 1536 x 256 x 1024: a
+    block of 49.0 us took 49.7; with 2.2, 1680 x 288 x 1152 is still cut, 52.6 -> 51.5)."""
     if g["dtype"] != DType.Float16 or g["batch"] or g.get("a_gather") or g.get("b_gather") or g["a_k0"] != g["K"] or g["b_k0"] != g["K"]:
         return None
     M, N, K = g["M"], g["N"], g["K"]
@@ -417,8 +435,8 @@ def sliced_plan(g: dict) -> Optional[dict]:
     if sum(M if t == "a" else N for t in tags) * slabs * deep * 2 > (1 << 30):
         return None
     most = max(1, min(slabs // 4, tuner.CU_COUNT // count))
-    us = [-(-slabs // n) * deep * 0.006 + (2.0 + n * M * N * 8 / 5e6 if n > 1 else 0.0) for n in range(1, most + 1)]
-    return dict(slices=us.index(min(us)) + 1, repack=tags, deep=deep, k=slabs * deep)
+    us = [-(-slabs // n) * deep * 0.006 + (2.2 + n * M * N * 8 / 5e6 if n > 1 else 0.0) for n in range(1, most + 1)]
+    return dict(slices=us.index(min(us)) + 1, repack=tags, deep=deep, k=slabs * deep, gain=us[0] - min(us))
 
 
 def _edge_ok(extent: int, tile: int, k_contiguous: bool) -> bool:

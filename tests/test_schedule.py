@@ -624,6 +624,23 @@ def test_float16_products_in_front_of_rotations_keep_their_order_of_sums(m, n):
         assert is_sliced_product(units[0].source) and not any(u.options for u in units[:at])
 
 
+@pytest.mark.parametrize("m,n,k,alone,block", [(192, 224, 896, False, False), (1344, 224, 896, False, False), (768, 192, 768, False, False), (1536, 256, 1024, False, False),
+                                               (462, 256, 1024, True, True), (1680, 288, 1152, False, True), (512, 821, 1280, False, False), (384, 1664, 1344, False, True),
+                                               (768, 640, 2560, True, True), (615, 768, 3072, True, True), (2240, 576, 2304, True, True)], ids=str)
+def test_whole_operands_are_cut_only_where_the_slices_are_worth_the_fold(m, n, k, alone, block):
+    """As a product of its own, and behind the bias and the residual of a transformer block's second MLP product."""
+    from jaxjs_hip import jit as J, library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.schedule import plan_units
+
+    a, b, bt, bias, rest = (ShapedArray(s, DType.Float16) for s in ((m, k), (k, n), (n, k), (n,), (m, n)))
+    plain, = plan_units(J.jit(L.matmul, [a, b]) if n % 4 == 0 else J.jit(lambda a, b: L.matmul(a, L.swapaxes(b, 0, 1)), [a, bt]))
+    assert bool(plain.options) == alone
+    if n % 4 == 0:
+        behind, = plan_units(J.jit(lambda a, b, bias, rest: rest.add(L.matmul(a, b).add(bias)), [a, b, bias, rest]))
+        assert bool(behind.options) == block
+
+
 def test_schedules_ask_for_uneven_slices_of_float16_products():
     from jaxjs_hip import DType, jit as J, library as L
     from jaxjs_hip.jit import ShapedArray
