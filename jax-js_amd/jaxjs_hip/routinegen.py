@@ -166,14 +166,27 @@ def _gen_cholesky(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, scratch, "cholesky", need, dict(n=n, batch=batch, launches=len(steps), **info))
 
 
-def _trisolve_few(n: int, total: int) -> Optional[Tuple[int, int]]:
-    """Right-hand sides of a workgroup and rows of a staged block where `total` right-hand sides of order n are few enough to
-    keep theirs and the solved entries in LDS, a workgroup to a CU; None where they are not."""
-    from . import tuner
-    width = -(-n // 8) * 8
-    for rhs in (8, 16, 32, 64):
-        rb = min(32, n, (160 * 1024 - 64 - 8 * width * rhs) // (16 * width + 16))
-        if rb >= 1 and total <= rhs * tuner.CU_COUNT:
+TRISOLVE_FEW = 64  # right-hand sides for every CU up to which they are few
+
+
+def _trisolve_few(n: int, m: int, mats: int) -> Optional[Tuple[int, int]]:
+    """Right-hand sides of a workgroup and rows of a staged block where m right-hand sides each of `mats` matrices of order n are few
+    enough to keep theirs and the solved entries in LDS; None where they are not.
+
+    As few for a workgroup as leave a CU to each, with blocks of up to 32 rows; for more matrices than that no more than one of them has,
+    and blocks of at most four rows, eight below order 64, so that two to eight workgroups fit a CU, which hide each other's barriers.  float32, one right-hand side each,
+    in microseconds, the other kernels, 32 rows, these: 300 of order 256 487, 575, 288; 512 of 512 1736, 1942, 1014; 4096 of 128 826, 1460 (16 to
+    a workgroup), 469; 16384 of 100 1915, 4405 (64), 1260; 600 of 48 48, 28, 27 (37 with four rows).  With 20 right-hand sides each, 512 of order 256 783, 585 (64), 586 (32).
+    Fewer where more do not fit, up to two rounds of workgroups."""
+    if mats * m > TRISOLVE_FEW * tuner.CU_COUNT:
+        return None
+    width, offered = -(-n // 8) * 8, (8, 16, 32, 64)
+    wanted = next((r for r in offered if mats * -(-m // r) <= tuner.CU_COUNT), None)
+    rows = 32 if wanted is not None else 8 if n < 64 else 4
+    wanted = wanted or next((r for r in offered if r >= m), 64)
+    for rhs in reversed(offered[:offered.index(wanted) + 1]):
+        rb = min(rows, n, (160 * 1024 - 64 - 8 * width * rhs) // (16 * width + 16))
+        if rb >= 1 and (rhs == wanted or mats * -(-m // rhs) <= 2 * tuner.CU_COUNT):
             return rhs, rb
     return None
 
@@ -199,7 +212,7 @@ def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
         return _empty("trisolve", n=n, m=m, batch=mats)
     unit = 1 if (routine.params or {}).get("unitDiagonal", False) else 0
     need = {0: mats * n * n * eb, 1: mats * m * n * eb}
-    few = _trisolve_few(n, mats * m)
+    few = _trisolve_few(n, m, mats)
     if few is not None:
         rhs, rb = few
         src = _linalg_source(numerics, ROUTINE=1, N=n, M=m, THREADS=256, UNIT=unit, STAGED=2, RB=rb, RHS=rhs, ELEM=ctype, CMP=cmp_t)

@@ -351,3 +351,12 @@ def test_direct_loads_make_no_chain_of_roundings_longer(m, n, k):
     staged, direct = gemm.choose_tile(dict(g, direct=False)), gemm.choose_tile(dict(g, direct=True))
     assert not staged.get("DLDS") and direct["DLDS"]
     assert 2 * direct["WK"] * direct.get("SPLITK", 1) >= staged.get("SPLITK", 1)
+
+
+@pytest.mark.parametrize("n,m,mats,plan", [(256, 1, 300, (8, 4)), (128, 1, 4096, (8, 4)), (100, 1, 16384, (8, 4)), (48, 1, 600, (8, 8)), (256, 20, 512, (32, 4)), (128, 1, 256, (8, 32)),
+                                           (609, 14, 1, (8, 12)), (1284, 28, 68, (8, 3)), (64, 65, 250, (64, 4)), (100, 1, 16385, None), (2048, 8, 1, None)], ids=str)
+def test_few_right_hand_sides_are_counted_by_workgroup(n, m, mats, plan):
+    """No workgroup holds right-hand sides of two matrices: what makes them few is how many workgroups that is."""
+    from jaxjs_hip import routinegen
+
+    assert routinegen._trisolve_few(n, m, mats) == plan

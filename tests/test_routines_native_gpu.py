@@ -561,7 +561,8 @@ def test_lu_strips_in_several_launches(shape, monkeypatch):
 
 
 @pytest.mark.parametrize("n,m,mats,dt", [(1, 1, 1, F32), (7, 8, 1, F32), (8, 9, 3, F32), (9, 1, 2, F32), (17, 2049, 1, F32), (25, 4100, 1, F32), (40, 8200, 1, F32), (127, 17, 1, F32),
-                                         (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16)],
+                                         (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16),
+                                         (70, 1, 600, F32), (45, 11, 300, F32), (261, 2, 270, F32), (90, 40, 280, np.float64)],
                          ids=lambda v: np.dtype(v).name if isinstance(v, type) else str(v))
 def test_triangular_solve_of_few_right_hand_sides(n, m, mats, dt):
     """Groups of eight entries and rows of a staged block that are not whole, 8 to 64 right-hand sides a workgroup, lanes without one; a zero, an infinite and
