@@ -38,6 +38,7 @@ SORT_LOCAL, SORT_TILES = 16, 1024  # words of a lane in a tile's register runs, 
 SORT_HELD = 8     # pieces of 16 bytes that a lane hands to others at a time: whole lines of 128 bytes (float32 32768 x 1024: 70.6 us, 83 with 4)
 SORT_GROUP = 8    # elements a thread sorts in registers at the end of every stage (4 for rows of <= 256: more threads stay busy)
 LAUNCH_THREADS = (1 << 32) - 1  # of a launch, along one axis
+LU_SCRATCH = 1 << 28  # bytes of unrounded multipliers
 CHOLESKY_PANEL_FROM = 192  # matrix order from which many matrices may take two launches a panel, and a plan counts its panels
 CHOLESKY_WAVE_BELOW = {2: 44, 4: 28, 8: 28}  # matrix order, by bytes per element, below which many matrices take a wave each
 
@@ -250,16 +251,20 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     if m <= 4096:
         rows = -(-m // 1024)  # of a thread of the panel's workgroup, in registers with as many columns as fit
         width = min(32, 1 << (64 // (rows * (2 if eb == 8 else 1))).bit_length() - 1, max(8, 1 << (min(m, n) - 1).bit_length()))
-        src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb, BLOCK="unsigned" if batch * -(-n // 8) + batch < 1 << 32 else "unsigned long long")
+        # the multipliers of a panel, of as many matrices at a time as LU_SCRATCH holds: at least 512, which fill the chip
+        at_once = min(batch, LU_SCRATCH // (width * m * 8))
+        src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb, BLOCK="unsigned" if (at_once + 1) * (-(-n // 8) + 1) < 1 << 32 else "unsigned long long")
         steps = []
-        for j in range(0, max(min(m, n), 1), width):
-            steps.append(LaunchStep("jh_lu_panel", (batch, 1, 1), (_round64(m - j), 1, 1), 0,
-                                    [("in", 0), ("out", 0), ("out", 1), ("out", 2), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j)]))
-            strips = -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
-            for first in range(0, batch * strips, LAUNCH_THREADS // 512):
-                steps.append(LaunchStep("jh_lu_strip", (min(batch * strips - first, LAUNCH_THREADS // 512), 1, 1), (512, 1, 1), 0,
-                                        [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", j), ("const", first)]))
-        return KernelSource([src], steps, [batch * width * m * 8, batch * m * 4, max(batch * 4, 16)], "lu", {0: batch * m * n * eb},
+        for mat in range(0, batch, at_once):
+            mats = min(at_once, batch - mat)
+            for j in range(0, max(min(m, n), 1), width):
+                steps.append(LaunchStep("jh_lu_panel", (mats, 1, 1), (_round64(m - j), 1, 1), 0,
+                                        [("in", 0), ("out", 0), ("out", 1), ("out", 2), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", mat), ("const", j)]))
+                strips = -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
+                for first in range(0, mats * strips, LAUNCH_THREADS // 512):
+                    steps.append(LaunchStep("jh_lu_strip", (min(mats * strips - first, LAUNCH_THREADS // 512), 1, 1), (512, 1, 1), 0,
+                                            [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", mat), ("const", j), ("const", first)]))
+        return KernelSource([src], steps, [at_once * width * m * 8, at_once * m * 4, max(at_once * 4, 16)], "lu", {0: batch * m * n * eb},
                             dict(m=m, n=n, batch=batch, launches=len(steps), **({"variant": "by columns"} if min(m, n) >= LU_BY_COLUMNS_FROM else {})))
     if min(m, n) >= LU_BY_COLUMNS_FROM and batch * m * n < (1 << 31):
         # Large matrices: two launches per column, the rank-1 update of the trailing block over the whole chip; the same

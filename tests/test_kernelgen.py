@@ -329,13 +329,29 @@ def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
     done = {}
     for s in ks.steps:
         if s.name == "jh_lu_strip":
-            j, first = s.args[-2][1], s.args[-1][1]
-            assert first == done.get(j, 0)
-            done[j] = first + s.grid[0]
+            mat, j, first = (c for kind, c in s.args if kind == "const")
+            assert first == done.get((mat, j), 0)
+            done[mat, j] = first + s.grid[0]
     width = max(8, min(32, 1 << (min(m, n) - 1).bit_length()))
-    for j, blocks in done.items():
-        assert blocks == batch * (-(-j // 8) + -(-(n - min(j + width, m, n)) // 8))
-    assert ("(unsigned long long)first + blockIdx.x" in ks.sources[0]) == (max(done.values(), default=0) >= 1 << 32)
+    panels = [(s.args[-2][1], s.args[-1][1], s.grid[0]) for s in ks.steps if s.name == "jh_lu_panel"]
+    assert sum(mats for _mat, j, mats in panels if j == 0) == batch
+    for mat, j, mats in panels:
+        assert done.get((mat, j), 0) == mats * (-(-j // 8) + -(-(n - min(j + width, m, n)) // 8))
+    assert max(done.values(), default=0) < 1 << 32 or "(unsigned long long)first + blockIdx.x" in ks.sources[0]
+
+
+@pytest.mark.parametrize("shape", [(1 << 20, 4096, 1), (2_000_000, 64, 64), (500_000, 130, 200), (1 << 22, 9, 7), (3, 4096, 4096)], ids=str)
+@pytest.mark.parametrize("dtype", [DType.Float16, DType.Float32, DType.Float64], ids=str)
+def test_lu_s_workspace_does_not_grow_with_the_batch(shape, dtype):
+    """Multipliers of a panel in double are up to sixteen times as large as a batch of thin matrices."""
+    from jaxjs_hip.routine import Routine, Routines, RoutineType
+    from jaxjs_hip.routinegen import LU_SCRATCH, generateRoutine
+
+    batch, m, n = shape
+    ks = generateRoutine(Routine(Routines.LU, RoutineType([shape], [dtype], [shape, (batch, min(m, n)), (batch, m)], [dtype, DType.Int32, DType.Int32])))
+    assert ks.scratch_bytes[0] <= LU_SCRATCH and sum(ks.scratch_bytes) <= 1.2 * LU_SCRATCH
+    sizes = [s.grid[0] for s in ks.steps if s.name == "jh_lu_panel"]
+    assert min(sizes[:1]) >= min(batch, 512)
 
 
 @pytest.mark.parametrize("m,n,k", [(652, 896, 704), (512, 1408, 768), (192, 3904, 832), (448, 1536, 576), (2072, 256, 640), (608, 832, 576), (1080, 512, 640), (1024, 1024, 1024),

@@ -560,6 +560,17 @@ def test_lu_strips_in_several_launches(shape, monkeypatch):
     assert_bits(got, want, f"lu {shape} {ks.info}")
 
 
+@pytest.mark.parametrize("shape,dt", [((5, 41, 70), F32), ((7, 9, 3), np.float16)], ids=str)
+def test_lu_of_matrices_a_few_at_a_time(shape, dt, monkeypatch):
+    """The workspace lowered to the multipliers of two matrices: the last launches have one."""
+    from jaxjs_hip import routinegen
+    monkeypatch.setattr(routinegen, "LU_SCRATCH", 2 * (32 if shape[1] > 16 else 8) * shape[1] * 8)
+    a = RNG.uniform(-1, 1, shape).astype(dt)
+    got, want, ks = both(R.lu(a), [a])
+    assert {s.grid[0] for s in ks.steps if s.name == "jh_lu_panel"} == {1, 2}
+    assert_bits(got, want, f"lu {shape} {ks.info}")
+
+
 @pytest.mark.parametrize("n,m,mats,dt", [(1, 1, 1, F32), (7, 8, 1, F32), (8, 9, 3, F32), (9, 1, 2, F32), (17, 2049, 1, F32), (25, 4100, 1, F32), (40, 8200, 1, F32), (127, 17, 1, F32),
                                          (640, 9, 1, F32), (900, 20, 1, F32), (1300, 3, 1, F32), (1900, 5, 1, F32), (500, 10, 1, np.float64), (333, 12, 1, np.float16),
                                          (70, 1, 600, F32), (45, 11, 300, F32), (261, 2, 270, F32), (90, 40, 280, np.float64)],
