@@ -218,7 +218,7 @@ def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
         rhs, rb = few
         src = _linalg_source(numerics, ROUTINE=1, N=n, M=m, THREADS=256, UNIT=unit, STAGED=2, RB=rb, RHS=rhs, ELEM=ctype, CMP=cmp_t)
         steps = [LaunchStep("jh_trisolve_few", (mats * -(-m // rhs), 1, 1), (256, 1, 1), 0, [("in", 0), ("in", 1), ("out", 0)])]
-        return KernelSource([src], steps, [], "trisolve", need, dict(n=n, m=m, batch=mats, threads=256, staged=n >= TRISOLVE_STAGED_FROM, rows_per_block=rb))
+        return KernelSource([src], steps, [], "trisolve", need, dict(n=n, m=m, batch=mats, variant="few", rhs=rhs, rows_per_block=rb))
     if TRISOLVE_STAGED_FROM <= n <= TRISOLVE_STAGED_MAX_N:
         # one wave of 64 right-hand sides + three waves staging blocks of rows in LDS as doubles (two buffers <= 128 KB)
         rb = max(1, min(8, TRISOLVE_STAGED_MAX_N // n))
@@ -227,12 +227,12 @@ def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
         steps = [LaunchStep("jh_trisolve_staged", (mats * ((m + 63) // 64), 1, 1), (256, 1, 1), 0,
                             [("in", 0), ("in", 1), ("out", 0), ("scratch", 0)])]
         return KernelSource([src], steps, [mats * m * n * 8], "trisolve", need,
-                            dict(n=n, m=m, batch=mats, threads=256, staged=True, rows_per_block=rb))
+                            dict(n=n, m=m, batch=mats, variant="staged", rows_per_block=rb))
     threads = 64 if m <= 64 else 256
     src = _linalg_source(numerics, ROUTINE=1, N=n, M=m, THREADS=threads, UNIT=unit, AHEAD=TRISOLVE_AHEAD, ELEM=ctype, CMP=cmp_t)
     blocks = mats * ((m + threads - 1) // threads)
     steps = [LaunchStep("jh_trisolve", (blocks, 1, 1), (threads, 1, 1), 0, [("in", 0), ("in", 1), ("out", 0), ("scratch", 0)])]
-    return KernelSource([src], steps, [mats * m * n * eb], "trisolve", need, dict(n=n, m=m, batch=mats, threads=threads, staged=False))
+    return KernelSource([src], steps, [mats * m * n * eb], "trisolve", need, dict(n=n, m=m, batch=mats, variant="plain", threads=threads))
 
 
 def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
@@ -265,10 +265,10 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
                     steps.append(LaunchStep("jh_lu_strip", (min(mats * strips - first, LAUNCH_THREADS // 512), 1, 1), (512, 1, 1), 0,
                                             [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", mat), ("const", j), ("const", first)]))
         return KernelSource([src], steps, [at_once * width * m * 8, at_once * m * 4, max(at_once * 4, 16)], "lu", {0: batch * m * n * eb},
-                            dict(m=m, n=n, batch=batch, launches=len(steps), **({"variant": "by columns"} if min(m, n) >= LU_BY_COLUMNS_FROM else {})))
+                            dict(m=m, n=n, batch=batch, launches=len(steps), variant="by panels"))
     if min(m, n) >= LU_BY_COLUMNS_FROM and batch * m * n < (1 << 31):
-        # Large matrices: two launches per column, the rank-1 update of the trailing block over the whole chip; the same
-        # operations per element as the single-workgroup kernel (bit-identical).
+        # More rows than a workgroup holds a panel of: two launches per column, the rank-1 update of the trailing block over the whole
+        # chip; the same operations per element as the panels.
         src = _linalg_source(numerics, ROUTINE=6, N=n, M=m, THREADS=1024, BATCH=batch, ELEM=ctype, CMP=cmp_t)
         grid1 = lambda count: (max(1, min((count + 255) // 256, 1 << 16)), 1, 1)  # noqa: E731
         steps = [LaunchStep("jh_lu_init", grid1(batch * m * n), (256, 1, 1), 0, [("in", 0), ("out", 0), ("out", 2)])]
@@ -348,7 +348,7 @@ ATTENTION_FEW_QUERIES = 4     # queries per sequence up to which a query may be 
 TRISOLVE_STAGED_FROM = 128    # matrix size from which TriangularSolve stages the matrix in LDS with helper waves
 TRISOLVE_STAGED_MAX_N = 8192   # two one-row buffers of doubles still fit in LDS
 TRISOLVE_AHEAD = 8       # entries of a row that a right-hand side's thread fetches ahead of its subtraction chain
-LU_BY_COLUMNS_FROM = 192  # smaller dimension from which LU runs two launches per column over the whole chip
+LU_BY_COLUMNS_FROM = 192  # smaller dimension from which LU of more than 4096 rows runs, two launches per column over the whole chip
 CHOLESKY_RIGHT_LOOKING_MAX_BYTES = 1 << 30  # the double-precision working copy of all matrices
 FFT_FUSED_MAX_N = 8192  # 16 bytes of LDS per point: 128 KiB
 

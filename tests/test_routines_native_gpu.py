@@ -152,7 +152,7 @@ def test_triangular_solve(case, unit):
          + np.tril(RNG.standard_normal(ashape), -1)).astype(F32)  # the strictly lower part must not matter
     b = RNG.standard_normal(ashape[:-2] + (m, n)).astype(F32)
     got, want, ks = both(R.triangular_solve(a, b, unit), [a, b])
-    assert ks.info["staged"] == (n >= 128)  # from 128 on helper waves stage the matrix in LDS as doubles
+    assert ks.info["variant"] == "few"
     assert_bits(got, want, f"triangular_solve {case} {ks.info}")
 
 
@@ -161,21 +161,23 @@ def test_triangular_solve(case, unit):
 def test_lu(shape):
     a = RNG.uniform(-1, 1, shape).astype(F32)
     got, want, ks = both(R.lu(a), [a])
-    # from 192 rows and columns on: two launches per column, the trailing update over the whole chip
-    assert (ks.info.get("variant") == "by columns") == (min(shape[-2:]) >= 192)
+    assert ks.info["variant"] == "by panels"
     assert_bits(got, want, f"lu {shape} {ks.info}")
 
 
-def test_lu_by_columns_zero_pivot_and_nan_columns():
-    """The special cases of the small kernel's test, embedded in matrices large enough for the by-columns variant: a zero
-    pivot column (that step eliminates nothing), equal magnitudes (the first row wins), a NaN that must not win."""
-    a = RNG.uniform(-1, 1, (2, 260, 260)).astype(F32)
+@pytest.mark.parametrize("shape,dt", [((2, 260, 260), F32), ((1, 4100, 200), F32), ((2, 4099, 193), F32), ((1, 4100, 200), np.float64), ((1, 4100, 200), np.float16)],
+                         ids=lambda v: np.dtype(v).name if isinstance(v, type) else str(v))
+def test_lu_zero_pivot_and_nan_columns_of_larger_matrices(shape, dt):
+    """The special cases of the test below, in panels and, of more than 4096 rows, column by column: a zero pivot column
+    (that step eliminates nothing), equal magnitudes (the first row wins), a NaN that must not win."""
+    a = RNG.uniform(-1, 1, shape).astype(dt)
     a[0, :, 3] = 0.0   # stays zero through every update: step 3 meets a zero pivot
-    a[1, 10, 5] = np.nan
-    a[1, 20:23, 7] = [0.75, -0.75, 0.75]
+    a[-1, 10, 5] = np.nan
+    a[-1, 20:23, 7] = [0.75, -0.75, 0.75]
+    a[-1, :, 11] = np.sign(a[-1, :, 11])
     got, want, ks = both(R.lu(a), [a])
-    assert ks.info["variant"] == "by columns"
-    assert_bits(got, want, "lu by columns, special columns")
+    assert ks.info["variant"] == ("by panels" if shape[1] <= 4096 else "by columns")
+    assert_bits(got, want, "lu, special columns")
 
 
 def test_lu_ties_zero_pivots_and_nans():
@@ -352,7 +354,7 @@ def test_triangular_solve_other_element_types(case, unit, dt):
          + np.tril(RNG.standard_normal(ashape), -1)).astype(dt)
     b = RNG.standard_normal(ashape[:-2] + (m, n)).astype(dt)
     got, want, ks = both(R.triangular_solve(a, b, unit), [a, b])
-    assert got[0].dtype == dt and ks.info["staged"] == (n >= 128)
+    assert got[0].dtype == dt and ks.info["variant"] == "few"
     assert_bits(got, want, f"triangular_solve {case} {np.dtype(dt).name} {ks.info}")
 
 
@@ -365,7 +367,7 @@ def test_lu_other_element_types(shape, dt):
         a[10, 5] = np.nan  # a NaN that must not win the pivot search
         a[20:23, 7] = [0.75, -0.75, 0.75]
     got, want, ks = both(R.lu(a), [a])
-    assert got[0].dtype == dt and (ks.info.get("variant") == "by columns") == (min(shape[-2:]) >= 192)
+    assert got[0].dtype == dt and ks.info["variant"] == "by panels"
     assert_bits(got, want, f"lu {shape} {np.dtype(dt).name} {ks.info}")
 
 
@@ -558,6 +560,20 @@ def test_lu_strips_in_several_launches(shape, monkeypatch):
     got, want, ks = both(R.lu(a), [a])
     assert max(s.grid[0] for s in ks.steps if s.name == "jh_lu_strip") == 7
     assert_bits(got, want, f"lu {shape} {ks.info}")
+
+
+@pytest.mark.parametrize("dt", [F32, np.float64, np.float16], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("n,m,mats,variant", [(9, 16400, 1, "plain"), (21, 19, 900, "plain"), (130, 16400, 1, "staged"), (2050, 3, 1, "staged")], ids=str)
+def test_triangular_solve_of_many_right_hand_sides(n, m, mats, variant, dt):
+    """More than LDS takes, of a workgroup or of all CUs; the diagonal and right-hand sides of the test of few."""
+    a = (np.triu(RNG.standard_normal((mats, n, n))) + np.sqrt(n) * np.eye(n)).astype(dt)
+    b = RNG.standard_normal((mats, m, n)).astype(dt)
+    a[0, 1, 1], a[0, 2, 2], a[0, 3, 3] = 0.0, np.inf, np.finfo(dt).smallest_subnormal
+    b[0, 0, 0], b[0, m - 1, n // 2] = np.inf, np.nan
+    a += np.tril(np.full((n, n), np.nan), -1).astype(dt)  # the strictly lower part must not matter
+    got, want, ks = both(R.triangular_solve(a, b), [a, b])
+    assert ks.info["variant"] == variant
+    assert_bits(got, want, f"triangular_solve {mats} x {n} x {m} {np.dtype(dt).name} {ks.info}")
 
 
 @pytest.mark.parametrize("shape,dt", [((5, 41, 70), F32), ((7, 9, 3), np.float16)], ids=str)
