@@ -1,5 +1,6 @@
 """pytest configuration: import path for the in-tree package and the `gpu` marker."""
 import os
+import subprocess
 import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -20,3 +21,35 @@ if _SHIFT:
 
     _default_rng = _np.random.default_rng
     _np.random.default_rng = lambda seed=None: _default_rng(seed + _SHIFT if isinstance(seed, int) else seed)
+
+
+# A kernel cache without kernels: the 4000 that the GPU tests compile take 11 minutes one after the other.  Processes beside the run,
+# which do not see the GPU, compile those of the tests ahead of it (JAXHIP_WARM=1), each a part of them.
+_warmers = []
+
+
+def pytest_collection_modifyitems(items):
+    part = os.environ.get("JAXHIP_WARM_PART")
+    if part:
+        i, n = map(int, part.split("/"))
+        items[:] = [t for t in items if hasattr(t.module, "WARM_ONLY") or t.module.__name__ in ("test_parity_gpu", "test_fuzz_gpu", "test_conv")][i::n]
+
+
+def pytest_collection_finish(session):
+    if os.environ.get("JAXHIP_WARM") or session.config.option.collectonly or len(session.items) < 1000 or not os.path.exists("/dev/kfd"):
+        return
+    from jaxjs_hip.runtime import CACHE_DIR
+
+    if os.path.isdir(CACHE_DIR) and len(os.listdir(CACHE_DIR)) > 2000:
+        return
+    n = max(1, int(os.environ.get("MAX_JOBS", "8")) - 4)
+    for i in range(n):
+        env = dict(os.environ, JAXHIP_WARM="1", JAXHIP_WARM_PART=f"{i}/{n}", HIP_VISIBLE_DEVICES="-1", OMP_NUM_THREADS="1")
+        _warmers.append(subprocess.Popen([sys.executable, "-m", "pytest", os.path.join(ROOT, "tests"), "-q", "-m", "gpu", "-p", "no:cacheprovider"],
+                                         cwd=ROOT, env=env, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL))
+
+
+def pytest_sessionfinish():
+    for p in _warmers:
+        p.kill()
+        p.wait()

@@ -46,6 +46,25 @@ def fast_backend():
     return _backends["fast"]
 
 
+def compile_units(prog, numerics=None):
+    """Compile the launches of the program's schedule into the on-disk cache."""
+    from jaxjs_hip.alu import Kernel
+    from jaxjs_hip.jit import jitCompile
+    from jaxjs_hip.kernelgen import generate
+    from jaxjs_hip.rewrite import fuse_attention
+    from jaxjs_hip.routine import Routine
+    from jaxjs_hip.routinegen import generateRoutine
+    from jaxjs_hip.runtime import compile_source
+    from jaxjs_hip.schedule import plan_units
+
+    numerics = numerics or NUMERICS
+    fused = fuse_attention(prog.jaxpr, prog.consts) if prog.jaxpr is not None else None
+    for u in plan_units(prog if fused is None else jitCompile(fused, prog.consts)):
+        ks = generate(u.source, numerics, **u.options) if isinstance(u.source, Kernel) else generateRoutine(u.source, numerics) if isinstance(u.source, Routine) else u.source.generate(numerics)
+        for src in ks.sources if ks is not None else []:
+            compile_source(src)
+
+
 def device_run(kernel, inputs, **tune_opts):
     """Upload inputs, dispatch the kernel once, read the typed result back."""
     if WARM_ONLY:

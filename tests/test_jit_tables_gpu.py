@@ -4,7 +4,7 @@ kernel and routine on the GPU (Wasm-faithful numerics, so the tables' own tolera
 import pytest
 
 import test_jit as T
-from gpu_util import WARM_ONLY, backend
+from gpu_util import WARM_ONLY, backend, compile_units
 
 pytestmark = pytest.mark.gpu
 
@@ -49,6 +49,11 @@ def _hip():
 
 class _CompileOnly(T.OracleBackend):
     """Warm-up stand-in: compiles what the hip backend would run into the on-disk cache, computes on the CPU checker."""
+
+    @property
+    def scheduleProgram(self):
+        """Of a program that is executed: the launches of its schedule.  (No schedule to run by: the checker takes its dispatches.)"""
+        return lambda prog: compile_units(prog, "wasm")
 
     def prepareKernelSync(self, kernel):
         from jaxjs_hip.kernelgen import generate

@@ -14,7 +14,7 @@ from jaxjs_hip.jit import ShapedArray
 from jaxjs_hip.patches import Layouts
 from jaxjs_hip.schedule import plan_units
 
-from gpu_util import backend
+from gpu_util import WARM_ONLY, backend, compile_units
 
 CASES = [  # dtype, batch, channels in and out, size, window, stride, padding, dilation
     ("f32", 2, 41, 50, 16, 3, 1, 1, 1),
@@ -43,6 +43,13 @@ def programs(dtype, B, C, O, S, W, stride, pad, dilation):
                 filter=(J.jit(lambda x, ct: J.convTransposeRhs(x, ct, list(ws), p), [x, ct]), (xs, (B, O, out, out)))), (xs, ws, (B, O, out, out))
 
 
+def warm(progs):
+    if WARM_ONLY:
+        for prog in progs:
+            compile_units(prog)
+        pytest.skip("warm-up run: compiled only")
+
+
 def expected(which, args, shapes, stride, pad, dilation):
     xs, ws, _ = shapes
     t = [torch.from_numpy(a.astype(np.float64)) for a in args]
@@ -58,9 +65,10 @@ def expected(which, args, shapes, stride, pad, dilation):
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_laid_out_operands_give_the_convolution(case):
     dtype, stride, pad, dilation = case[0], *case[6:]
+    made, shapes = programs(*case)
+    warm(prog for prog, _operands in made.values())
     be = backend()
     rng = np.random.default_rng(len(str(case)))
-    made, shapes = programs(*case)
     packed = 0
     for which, (prog, operands) in made.items():
         args = [rng.standard_normal(s).astype(NP[dtype]) for s in operands]
@@ -85,11 +93,12 @@ def test_laid_out_operands_give_the_convolution(case):
 @pytest.mark.gpu
 def test_an_operand_that_the_epilogue_reads_too():
     """The image joins the result behind the convolution: it is laid out beside its own buffer, which the epilogue reads."""
-    be = backend()
     p = ConvParams(0, [1, 1], [(1, 1), (1, 1)], [1, 1], [1, 1])
     x, w = ShapedArray((3, 41, 19, 19), DType.Float32), ShapedArray((41, 41, 3, 3), DType.Float32)
     prog = J.jit(lambda x, w: J.conv(x, w, p).add(x), [x, w])
     assert any(isinstance(u.source, Layouts) for u in plan_units(prog))
+    warm([prog])
+    be = backend()
     rng = np.random.default_rng(5)
     args = [rng.standard_normal(a.shape).astype(np.float32) for a in (x, w)]
     slots = [be.malloc(a.nbytes, a) for a in args]
@@ -170,6 +179,7 @@ def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
     """Replays of a graph with other values in between, and the dispatches of a traced run, against the launch list."""
     from jaxjs_hip.graph import GraphedProgram
 
+    warm(prog for prog, _operands in programs(*case)[0].values())
     be = backend()
     for prog, operands in programs(*case)[0].values():
         prepared = prog.prepare(be)
@@ -201,9 +211,10 @@ def test_programs_without_room_for_layouts(case, monkeypatch):
     from jaxjs_hip.graph import GraphedProgram
     from jaxjs_hip.schedule import Schedule
 
-    be = backend()
     made, shapes = programs(*case)
     prog, operands = made["forward"]
+    warm([prog])
+    be = backend()
     rng = np.random.default_rng(11)
     slots = [be.malloc(a.nbytes, a) for a in (rng.standard_normal(s).astype(NP[case[0]]) for s in operands)]
     want, = Schedule(be, prog, layouts=False).run(slots)

@@ -28,6 +28,7 @@ def numerics_mode(request):
 
 
 def warm(prog):
+    gpu_util.compile_units(prog)
     from jaxjs_hip.kernelgen import generate
     from jaxjs_hip.runtime import compile_source
     from jaxjs_hip.routinegen import generateRoutine

@@ -3,13 +3,13 @@ vector width, the lane counts and the register limit."""
 import numpy as np
 import pytest
 
-from gpu_util import WARM_ONLY, backend
+from gpu_util import WARM_ONLY, backend, compile_units
 from jaxjs_hip import DType
 from jaxjs_hip import jit as J
 from jaxjs_hip import library as L
 from jaxjs_hip import workloads as W
 from jaxjs_hip.jit import ShapedArray
-from jaxjs_hip.rowchain import RowChain, gen_rows
+from jaxjs_hip.rowchain import RowChain
 from jaxjs_hip.rowproduct import ProductRows, RowProduct
 from jaxjs_hip.schedule import plan_units
 from jit_util import run_program
@@ -29,9 +29,7 @@ def check(prog, arrays, f16, chained=True, terms=0):
     chains = [u.source for u in plan_units(prog) if isinstance(u.source, RowChain)]
     assert len(chains) == 1 or not chained, [type(u.source).__name__ for u in plan_units(prog)]
     if WARM_ONLY:
-        from jaxjs_hip.runtime import compile_source
-        for c in chains:
-            compile_source(gen_rows(c, "wasm").sources[0])
+        compile_units(prog)
         pytest.skip("warm-up run: compiled only")
     be = backend()
     before = be.live_slots()
