@@ -389,8 +389,8 @@ def is_sliced_product(kernel: Kernel) -> bool:
     halves and cuts no copies: 343 x 896 x 7104 40.2 -> 18.5 us, 448 x 395 x 3264 18.8 -> 10.9, 1125 x 768 x 4800 28.7 -> 18.4, 2176 x
     265 x 3843 (weights along k) 68.7 -> 24.1, 4070 x 448 x 5184 31.9 -> 29.0.  In one slice, copies of both operands in one launch
     instead of two (1984 x 1543 x 1281 26.4 -> 23.1), and behind fewer than 512 rows, where the general template's element loads cost
-    18 ns per k (379 x 5964 x 6175 111 -> 66), from k = 1024 on (3520 x 355 x 666 12.8 against 15.2).  Of 60 shapes drawn, 27 take it, none
-    slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4).
+    18 ns per k (379 x 5964 x 6175 111 -> 66), from k = 1024 on (3520 x 355 x 666 12.8 against 15.2).  Of 105 products drawn that it
+    could take alone none that it takes is more than 3 per cent slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4).
 
     Whole operands that the tile plan gives eight waves stay with it: blocks of 128 to 1536 rows and width 192 or 224, whose second MLP product
     has a k axis of 768 or 896, were all slower or no faster with it cut (768 x 192 35.4 and 36.1 us for the block, 1344 x 224 41.7 and 43.8).  With
