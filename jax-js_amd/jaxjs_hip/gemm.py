@@ -393,7 +393,7 @@ def is_sliced_product(kernel: Kernel) -> bool:
     could take alone none that it takes is more than 3 per cent slower.  Shapes of the kernel for few rows or tiles stay there (704 x 320 x 3600 13.6 against 19.5, 406 x 448 x 962 7.2 and 12.4).
 
     Whole operands that the tile plan gives eight waves stay with it: blocks of 128 to 1536 rows and width 192 or 224, whose second MLP product
-    has a k axis of 768 or 896, were all slower or no faster with it cut (768 x 192 35.4 and 36.1 us for the block, 1344 x 224 41.7 and 43.8).  With
+    has a k axis of 768 or 896, were slower by up to 5 per cent with it cut (768 x 192 35.4 and 36.1 us for the block, 1344 x 224 41.7 and 43.8), but for 128 x 224, 33.5 and 32.8.  With
     four waves, from a k axis of 1024 on, blocks are faster by up to a quarter (448 x 704 66.8 -> 49.1, 768 x 768 60.5 -> 54.7, 462 x 256 37.0 -> 35.4), also
     where the tile plan folds two slices inside the launch.  With an epilogue that reads nothing one plain launch takes less, half a
     microsecond or, of operands that both run along k, one, and partial sums whose rows are off the 16-byte grid cost more: alone,
