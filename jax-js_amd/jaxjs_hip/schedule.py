@@ -423,17 +423,16 @@ class Schedule:
             self._lean = Schedule(self.backend, self.source, layouts=False)
         return self._lean
 
-    def run(self, inputs: Sequence[int]) -> List[int]:
-        if not self._no_room:
-            try:
-                return self._run(inputs)
-            except DeviceMemoryError:
-                if not self.laid_out:
-                    raise
-                self._no_room = True
-        return self.without_layouts().run(inputs)
+    def _gives_way(self, error: BaseException) -> bool:
+        """Whether `error` is that the device has no room, with layouts in the schedule: this call and later ones do without."""
+        if not self.laid_out or not isinstance(error, DeviceMemoryError):
+            return False
+        self._no_room = True
+        return True
 
-    def _run(self, inputs: Sequence[int]) -> List[int]:
+    def run(self, inputs: Sequence[int]) -> List[int]:
+        if self._no_room:
+            return self.without_layouts().run(inputs)
         be, prog = self.backend, self.prog
         if len(inputs) != prog.nargs:
             raise ValueError(f"jit program takes {prog.nargs} inputs, got {len(inputs)}")
@@ -466,10 +465,12 @@ class Schedule:
                         for u in self.units:
                             u.exe.data.rezero(be.dev)
                     check(rc, "jh_launch_list")
-        except BaseException:
+        except BaseException as e:
             for m in made:
                 be.decRef(m)
-            raise
+            if not self._gives_way(e):
+                raise
+            return self.without_layouts().run(inputs)  # (nothing was launched, and the workspace not allocated)
         finally:
             be._release(space, self._work[-1])  # a later owner's work is queued behind this program's on the one stream
         scope = dict(zip(self._made, made))
@@ -487,10 +488,12 @@ class Schedule:
                 for o in u.outputs:
                     scope[o] = made[o] = be.malloc(self._sizes[o])
                 be.dispatch(u.exe, [scope[i] for i in u.inputs], [scope[o] for o in u.outputs])
-        except BaseException:
+        except BaseException as e:
             for s in made.values():
                 be.decRef(s)
-            raise
+            if not self._gives_way(e):
+                raise
+            return self.without_layouts().run(inputs)
         for o, s in made.items():
             if o not in self._made:
                 be.decRef(s)
