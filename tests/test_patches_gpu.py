@@ -229,7 +229,7 @@ def test_programs_without_room_for_layouts(case, monkeypatch):
     schedule = Schedule(be, prog)
     monkeypatch.setattr(be, "scheduleProgram", lambda p: Schedule(be, p))
     assert schedule.laid_out
-    outs = schedule.run(slots) + schedule.run(slots)
+    outs = schedule.run(slots) + schedule.run(slots) + Schedule(be, prog)._run_by_unit(slots)
     graph = GraphedProgram(be, prog, slots)
     for _ in range(2):
         graph.launch()

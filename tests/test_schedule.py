@@ -607,6 +607,8 @@ def test_a_program_without_room_for_layouts_runs_without_them():
     assert be.live_slots() == 4 and not graph._owned
     graph._make_room(lean)
     assert be.live_slots() == 4 + len(graph._owned)
+    before, be.dispatch = be.live_slots(), lambda exe, ins, outs: None
+    assert len(Schedule(be, prog)._run_by_unit(inputs)) == 1 and be.live_slots() == before + 1 and len(launched) == 3
 
 
 @pytest.mark.parametrize("m,n", [(1024, 128), (2048, 256), (4096, 136), (3264, 400)], ids=str)
