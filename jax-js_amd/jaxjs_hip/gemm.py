@@ -94,7 +94,7 @@ _F32_PLANS = ((dict(BM=64, BN=64, WM=2, WN=2, WK=2, STAGES=4), 2.18, 71.0, 274.5
               (dict(BM=128, BN=128, WM=4, WN=2, WK=1, STAGES=2), 3.10, 12.2, 281.9e3, 0.988, 1.130, 0.993))
 
 
-def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Dict[str, int]:
+def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Optional[Dict[str, int]]:
     """Plan of a float32 product whose slabs go to LDS by direct loads (`_f32_direct`), by an estimate: a launch, the tiles of the
     CU that gets most of them at the plan's rate, and the fold of slices of the k axis inside the launch.  It is a fit to 132
     products of 64 to 8192 rows, columns and k in both orders of B under all plans, within 1.7 per cent of the fastest one in
@@ -102,7 +102,8 @@ def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Dict[str, int]:
     150 -> 124, 4096 1080 -> 946 (145 TFLOP/s), 8192 8596 -> 7565, 3632 x 3088 x 144 49.6 -> 37.0, 1280 x 640 x 320 10.5 -> 7.6, 960 x 384 x
     3696 95.9 -> 41.5, 3672 x 768 x 1408 86.9 -> 69.4.
     `parts`: slices of the k axis that staging in registers takes, each a chain of roundings as long as itself.  Here a chain is half
-    of what a wave has of a slice, and only plans that make it no longer are taken.  The others grew the error of four in 400 drawn products."""
+    of what a wave has of a slice, and only plans that make it no longer are taken.  The others grew the error of four in 400 drawn products.  None where there are none:
+    batches, which are not cut here, and products that staging cuts in up to 64."""
     best = None
     for plan, launch, fill, rate, alone, fold, sums in _F32_PLANS:
         count = tiles(plan["BM"], plan["BN"])
@@ -115,7 +116,7 @@ def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Dict[str, int]:
                 us += fold * split + sums * 1e-6 * split * g["M"] * g["N"]
             if best is None or us < best[0]:
                 best = (us, dict(plan, BK=32, DLDS=1, **(dict(SPLITK=split, FUSEK=1) if split > 1 else {})))
-    return best[1]
+    return best and best[1]
 
 
 def is_direct_product(kernel: Kernel) -> bool:
@@ -125,7 +126,8 @@ def is_direct_product(kernel: Kernel) -> bool:
     if kernel.reduction is None or kernel.size == 0:
         return False
     t = tuner.tuneHip(kernel)
-    return t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and few_plan(t) is None
+    return (t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and few_plan(t) is None
+            and bool(choose_tile(dict(t.gemm, direct=True)).get("DLDS")))
 
 
 def _f32_direct(g: dict) -> bool:
@@ -190,7 +192,9 @@ def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
         # Direct loads where a schedule asks for them, and for any Kernel of at least two 128x128 tiles per CU, whose plans nothing pins
         # (8192^3 8596 -> 7565 us; 4096^3 1080 -> 946).
         if _f32_direct(g) and (g.get("direct") or tiles(128, 128) >= 2 * CU):
-            return _f32_tile(g, tiles, nb, 1 if tiles(128, 128) >= 2 * CU else choose_tile(dict(g, direct=False)).get("SPLITK", 1))
+            plan = _f32_tile(g, tiles, nb, 1 if tiles(128, 128) >= 2 * CU else choose_tile(dict(g, direct=False)).get("SPLITK", 1))
+            if plan is not None:
+                return plan
         if plain_k and not loose_ops and g["M"] >= 128 and g["N"] >= 64 and tiles(128, 64) * 4 > CU:
             return _f32_staged_tile(g, tiles, nb)
         # Among the shapes that do, the cheapest by (rounds of two workgroups per CU) x (tile area) / (rate of the

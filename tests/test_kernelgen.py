@@ -369,6 +369,24 @@ def test_direct_loads_make_no_chain_of_roundings_longer(m, n, k):
     assert 2 * direct["WK"] * direct.get("SPLITK", 1) >= staged.get("SPLITK", 1)
 
 
+@pytest.mark.parametrize("batch,m,n,k", [(2, 224, 128, 1792), (3, 192, 256, 512), (6, 96, 224, 2048), (1, 256, 48, 30720), (1, 32, 576, 26624), (1, 60, 192, 18432), (2, 64, 64, 128),
+                                         (2, 512, 512, 512), (24, 128, 128, 512), (1, 64, 33, 16384)], ids=str)
+def test_products_cut_finer_than_direct_loads_cut_them_keep_their_plan(batch, m, n, k):
+    """Batches, which direct loads cut into no slices, and few rows behind a long axis, staged in up to 64 of them."""
+    from jaxjs_hip import gemm, jit as J, library as L, tuner
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.kernelgen import generate
+    from jaxjs_hip.schedule import plan_units
+
+    lead = (batch,) if batch > 1 else ()
+    unit, = plan_units(J.jit(lambda a, b: L.matmul(a, b), [ShapedArray(lead + (m, k), DType.Float32), ShapedArray(lead + (k, n), DType.Float32)]))
+    generate(unit.source, **unit.options)
+    g = tuner.tuneHip(unit.source).gemm
+    staged, taken = gemm.choose_tile(dict(g, direct=False)), gemm.choose_tile(dict(g, direct=bool(unit.options)))
+    assert unit.options == (dict(direct_f32=True) if taken.get("DLDS") else {})
+    assert taken == staged or 2 * taken["WK"] * taken.get("SPLITK", 1) >= staged.get("SPLITK", 1)
+
+
 @pytest.mark.parametrize("n,m,mats,plan", [(256, 1, 300, (8, 4)), (128, 1, 4096, (8, 4)), (100, 1, 16384, (8, 4)), (48, 1, 600, (8, 8)), (256, 20, 512, (32, 4)), (128, 1, 256, (8, 32)),
                                            (609, 14, 1, (8, 12)), (1284, 28, 68, (8, 3)), (64, 65, 250, (64, 4)), (100, 1, 16385, None), (2048, 8, 1, None)], ids=str)
 def test_few_right_hand_sides_are_counted_by_workgroup(n, m, mats, plan):
