@@ -103,7 +103,12 @@ def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Optional[Dict[str, int]]:
     3696 95.9 -> 41.5, 3672 x 768 x 1408 86.9 -> 69.4.
     `parts`: slices of the k axis that staging in registers takes, each a chain of roundings as long as itself.  Here a chain is half
     of what a wave has of a slice, and only plans that make it no longer are taken.  The others grew the error of four in 400 drawn products.  None where there are none:
-    batches, which are not cut here, and products that staging cuts in up to 64."""
+    batches, which are not cut here, and products that staging cuts in up to 64.  And none where staging has the shorter walk along k: for a batch that
+    it cuts in two behind k = 512, in four behind 256 (2 x 256 x 512 x 256 7.1 us staged, 6.5 here, x 512 8.8 and 10.0, x 2048 18.6 and 34.2; 2 x 512 x 512 x 512 11.3
+    and 11.0, x 1024 18.1 and 18.7), and where it cuts in more than eight and all slices have a CU to themselves (48 x 320 x 17408 27.7 and 38.7; with 288 slices
+    32 x 576 x 17408 41.0 and 38.8)."""
+    if (nb > 1 and parts > 1 and parts * g["K"] > 1024) or (parts > 8 and parts * tiles(64, 64) <= tuner.CU_COUNT):
+        return None
     best = None
     for plan, launch, fill, rate, alone, fold, sums in _F32_PLANS:
         count = tiles(plan["BM"], plan["BN"])
@@ -122,11 +127,12 @@ def _f32_tile(g: dict, tiles, nb: int, parts: int) -> Optional[Dict[str, int]]:
 def is_direct_product(kernel: Kernel) -> bool:
     """Whether `kernel` is better prepared with the option `direct_f32`: a float32 product that no other kernel takes.  (Why it is an
     option, which programs' schedules set, and not the plan of every such Kernel: the plans of smaller products, slabs staged in registers,
-    are pinned by tests/test_kernelgen.py.)"""
+    are pinned by tests/test_kernelgen.py.)  Batches of one slab stay staged, there is nothing to fetch ahead (12 x 512 x 512 x 32 6.2 us and
+    6.5 by direct loads, 36 x 128 x 128 x 32 5.0 and 5.4; of k = 64 24 x 256 x 256 5.8 and 5.3)."""
     if kernel.reduction is None or kernel.size == 0:
         return False
     t = tuner.tuneHip(kernel)
-    return (t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and few_plan(t) is None
+    return (t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and not (t.gemm["batch"] and t.gemm["K"] <= 32) and few_plan(t) is None
             and bool(choose_tile(dict(t.gemm, direct=True)).get("DLDS")))
 
 

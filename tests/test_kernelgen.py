@@ -369,9 +369,11 @@ def test_direct_loads_make_no_chain_of_roundings_longer(m, n, k):
     assert 2 * direct["WK"] * direct.get("SPLITK", 1) >= staged.get("SPLITK", 1)
 
 
-@pytest.mark.parametrize("batch,m,n,k", [(2, 224, 128, 1792), (3, 192, 256, 512), (6, 96, 224, 2048), (1, 256, 48, 30720), (1, 32, 576, 26624), (1, 60, 192, 18432), (2, 64, 64, 128),
-                                         (2, 512, 512, 512), (24, 128, 128, 512), (1, 64, 33, 16384)], ids=str)
-def test_products_cut_finer_than_direct_loads_cut_them_keep_their_plan(batch, m, n, k):
+@pytest.mark.parametrize("batch,m,n,k,direct", [
+    (2, 224, 128, 1792, False), (3, 192, 256, 512, False), (6, 96, 224, 2048, False), (1, 256, 48, 30720, False), (1, 32, 576, 26624, False), (1, 60, 192, 18432, False), (2, 64, 64, 128, False),
+    (2, 256, 512, 256, True), (2, 256, 512, 512, False), (2, 512, 512, 512, True), (2, 512, 512, 1024, False), (24, 128, 128, 512, False), (24, 256, 256, 512, True), (12, 512, 512, 32, False), (12, 512, 512, 64, True), (1, 48, 320, 17408, False), (1, 32, 576, 17408, True)],
+    ids=str)
+def test_products_cut_finer_than_direct_loads_cut_them_keep_their_plan(batch, m, n, k, direct):
     """Batches, which direct loads cut into no slices, and few rows behind a long axis, staged in up to 64 of them."""
     from jaxjs_hip import gemm, jit as J, library as L, tuner
     from jaxjs_hip.jit import ShapedArray
@@ -383,7 +385,7 @@ def test_products_cut_finer_than_direct_loads_cut_them_keep_their_plan(batch, m,
     generate(unit.source, **unit.options)
     g = tuner.tuneHip(unit.source).gemm
     staged, taken = gemm.choose_tile(dict(g, direct=False)), gemm.choose_tile(dict(g, direct=bool(unit.options)))
-    assert unit.options == (dict(direct_f32=True) if taken.get("DLDS") else {})
+    assert unit.options == (dict(direct_f32=True) if direct else {}) and bool(taken.get("DLDS")) == direct
     assert taken == staged or 2 * taken["WK"] * taken.get("SPLITK", 1) >= staged.get("SPLITK", 1)
 
 
