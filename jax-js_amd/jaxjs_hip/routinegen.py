@@ -235,6 +235,36 @@ def _gen_trisolve(routine: Routine, numerics: str) -> Optional[KernelSource]:
     return KernelSource([src], steps, [mats * m * n * eb], "trisolve", need, dict(n=n, m=m, batch=mats, variant="plain", threads=threads))
 
 
+def _lu_width(m: int, n: int, eb: int) -> int:
+    """Columns of a panel: as many as fit a thread's registers with its rows of 1024."""
+    rows = -(-m // 1024)
+    return min(32, 1 << (64 // (rows * (2 if eb == 8 else 1))).bit_length() - 1, max(8, 1 << (min(m, n) - 1).bit_length()))
+
+
+def _lu_strips(m: int, n: int, width: int, j: int) -> int:
+    """Strips of eight columns beside the panel from column j on."""
+    return -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
+
+
+def _lu_by_matrix(m: int, n: int, batch: int, eb: int) -> bool:
+    """Whether matrices take a workgroup each for all their columns, in one launch, and not panels.
+
+    A panel's column is the faster one, but every eight columns beside a panel cost a workgroup of 512 threads, few of which have an
+    element where there are few rows.  Matrices of at most five rows go by matrix where anything is beside their panel (7.5 us for one launch, 11 for two; float32
+    1202 x [3, 272] 10.0 us, 82 by panels, 8484 x [2, 445] 62 and 828) unless they are few and long, and others up to 64 (48 in float64) where many strips meet many
+    matrices: float32 829 x [12, 1078] 164 and 647, 262 x [46, 310] 272 and 421, 13646 x [34, 34] 535 and 932, but float64 21 x [75, 262] 528 and 161, 125 x [16, 238] 53 and
+    37, float16 855 x [57, 57] 507 and 383.  With more rows than columns panels are twice to five times as fast.  In float16, whose elements a panel's threads convert in every
+    step, also very many small ones without strips: 11900 x [3, 3] 14.6 and 19.3, 10728 x [24, 24] 326 and 413.  Of 434 batches of all three types the choice is 0.7 per
+    cent from the faster one in the mean."""
+    if m > n or batch * _round64(n) > LAUNCH_THREADS:
+        return False
+    width = _lu_width(m, n, eb)
+    strips = batch * sum(_lu_strips(m, n, width, j) for j in range(0, m, width))
+    if strips and ((m <= 5 and (n <= 256 or batch >= 16 * m)) or (m <= (48 if eb == 8 else 64) and batch >= 48 and strips >= (128 if eb == 2 else 200) * m)):
+        return True
+    return eb == 2 and m <= 32 and batch >= 8192
+
+
 def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     t = routine.type
     shape = list(t.inputShapes[0])
@@ -248,9 +278,13 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
     batch = prod(shape[:-2])
     if batch == 0 or m == 0:
         return _empty("lu", m=m, n=n, batch=batch)
+    if m <= 4096 and _lu_by_matrix(m, n, batch, eb):
+        threads = _round64(max(m, n))
+        src = _linalg_source(numerics, ROUTINE=2, N=n, M=m, THREADS=threads, ELEM=ctype, CMP=cmp_t)
+        steps = [LaunchStep("jh_lu", (batch, 1, 1), (threads, 1, 1), 0, [("in", 0), ("out", 0), ("out", 1), ("out", 2)])]
+        return KernelSource([src], steps, [], "lu", {0: batch * m * n * eb}, dict(m=m, n=n, batch=batch, launches=1, variant="by matrix"))
     if m <= 4096:
-        rows = -(-m // 1024)  # of a thread of the panel's workgroup, in registers with as many columns as fit
-        width = min(32, 1 << (64 // (rows * (2 if eb == 8 else 1))).bit_length() - 1, max(8, 1 << (min(m, n) - 1).bit_length()))
+        width = _lu_width(m, n, eb)
         # the multipliers of a panel, of as many matrices at a time as LU_SCRATCH holds: at least 512, which fill the chip
         at_once = min(batch, LU_SCRATCH // (width * m * 8))
         src = _linalg_source(numerics, ROUTINE=10, N=n, M=m, RB=width, ELEM=ctype, CMP=cmp_t, ELEM_BYTES=eb, BLOCK="unsigned" if (at_once + 1) * (-(-n // 8) + 1) < 1 << 32 else "unsigned long long")
@@ -260,7 +294,7 @@ def _gen_lu(routine: Routine, numerics: str) -> Optional[KernelSource]:
             for j in range(0, max(min(m, n), 1), width):
                 steps.append(LaunchStep("jh_lu_panel", (mats, 1, 1), (_round64(m - j), 1, 1), 0,
                                         [("in", 0), ("out", 0), ("out", 1), ("out", 2), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", mat), ("const", j)]))
-                strips = -(-j // 8) + -(-(n - min(j + width, m, n)) // 8)
+                strips = _lu_strips(m, n, width, j)
                 for first in range(0, mats * strips, LAUNCH_THREADS // 512):
                     steps.append(LaunchStep("jh_lu_strip", (min(mats * strips - first, LAUNCH_THREADS // 512), 1, 1), (512, 1, 1), 0,
                                             [("in", 0), ("out", 0), ("out", 1), ("scratch", 0), ("scratch", 1), ("scratch", 2), ("const", mat), ("const", j), ("const", first)]))

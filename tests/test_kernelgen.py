@@ -317,7 +317,7 @@ def test_attention_takes_a_workgroup_per_query_only_for_few_queries_of_few_heads
     assert [s.name for s in ks.steps] == ["jh_attention_few" if by_queries else "jh_attention"]
 
 
-@pytest.mark.parametrize("shape", [(140000, 8, 512), (3, 8, 100_000_000), (9_000_000, 8, 16), (2_000_000, 70, 33), (1 << 25, 1, 1200)], ids=str)
+@pytest.mark.parametrize("shape", [(140000, 8, 512), (3, 8, 100_000_000), (9_000_000, 8, 16), (2_000_000, 70, 33), (1 << 25, 1, 1200), (70000, 65, 800)], ids=str)
 def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
     """Every strip of every matrix once, in launches of the size that the device takes."""
     from jaxjs_hip.routine import Routine, Routines, RoutineType
@@ -326,6 +326,9 @@ def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
     batch, m, n = shape
     ks = generateRoutine(Routine(Routines.LU, RoutineType([shape], [DType.Float32], [shape, (batch, min(m, n)), (batch, m)], [DType.Float32, DType.Int32, DType.Int32])))
     assert all(s.grid[0] * s.block[0] < 1 << 32 for s in ks.steps)
+    if ks.info["variant"] == "by matrix":
+        assert [s.grid for s in ks.steps] == [(batch, 1, 1)]
+        return
     done = {}
     for s in ks.steps:
         if s.name == "jh_lu_strip":
@@ -340,6 +343,15 @@ def test_lu_s_launches_hold_fewer_than_2_to_the_32_threads(shape):
     assert max(done.values(), default=0) < 1 << 32 or "(unsigned long long)first + blockIdx.x" in ks.sources[0]
 
 
+@pytest.mark.parametrize("batch,m,n,eb,by_matrix", [(1202, 3, 272, 4, True), (1, 5, 256, 4, True), (24, 3, 2000, 4, False), (829, 12, 1078, 4, True), (40, 12, 1078, 4, False), (13646, 34, 34, 4, True),
+                                                    (855, 57, 57, 2, False), (21, 75, 262, 8, False), (500, 49, 900, 8, False), (500, 49, 900, 4, True), (5000, 100, 64, 4, False),
+                                                    (11900, 3, 3, 2, True), (11900, 3, 3, 4, False), (5681, 14, 3, 2, False), (1 << 25, 1, 1200, 4, False), (9000, 27, 6, 2, False)], ids=str)
+def test_which_lu_goes_by_matrix(batch, m, n, eb, by_matrix):
+    from jaxjs_hip import routinegen
+
+    assert routinegen._lu_by_matrix(m, n, batch, eb) == by_matrix
+
+
 @pytest.mark.parametrize("shape", [(1 << 20, 4096, 1), (2_000_000, 64, 64), (500_000, 130, 200), (1 << 22, 9, 7), (3, 4096, 4096)], ids=str)
 @pytest.mark.parametrize("dtype", [DType.Float16, DType.Float32, DType.Float64], ids=str)
 def test_lu_s_workspace_does_not_grow_with_the_batch(shape, dtype):
@@ -349,6 +361,9 @@ def test_lu_s_workspace_does_not_grow_with_the_batch(shape, dtype):
 
     batch, m, n = shape
     ks = generateRoutine(Routine(Routines.LU, RoutineType([shape], [dtype], [shape, (batch, min(m, n)), (batch, m)], [dtype, DType.Int32, DType.Int32])))
+    if ks.info["variant"] == "by matrix":
+        assert not ks.scratch_bytes
+        return
     assert ks.scratch_bytes[0] <= LU_SCRATCH and sum(ks.scratch_bytes) <= 1.2 * LU_SCRATCH
     sizes = [s.grid[0] for s in ks.steps if s.name == "jh_lu_panel"]
     assert min(sizes[:1]) >= min(batch, 512)

@@ -161,7 +161,7 @@ def test_triangular_solve(case, unit):
 def test_lu(shape):
     a = RNG.uniform(-1, 1, shape).astype(F32)
     got, want, ks = both(R.lu(a), [a])
-    assert ks.info["variant"] == "by panels"
+    assert ks.info["variant"] == ("by matrix" if shape == (1, 5) else "by panels")
     assert_bits(got, want, f"lu {shape} {ks.info}")
 
 
@@ -548,6 +548,19 @@ def test_lu_panels_at_their_edges(shape, dt):
         a[shape[0] // 2:, :] *= 0.5
         a[:, 2] = a[:, 1]  # cancels: a zero pivot column
     got, want, ks = both(R.lu(a), [a])
+    assert_bits(got, want, f"lu {shape} {np.dtype(dt).name} {ks.info}")
+
+
+@pytest.mark.parametrize("dt", ELEMS, ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("shape", [(1, 2), (40, 2, 300), (90, 5, 257), (70, 9, 3000), (300, 17, 130), (900, 33, 65), (64, 48, 1100), (8192, 3, 4), (7, 1, 65)], ids=str)
+def test_lu_of_many_wide_matrices(shape, dt):
+    """A workgroup per matrix, of one wave to sixteen: rows and columns that are not whole waves, few values of which the first row has to win, a zero column, a NaN."""
+    a = RNG.integers(-2, 3, shape).astype(dt)
+    if a.ndim == 3:
+        a[0, :, 0], a[-1, -1, 1] = 0.0, np.nan
+        a[len(a) // 2] = RNG.uniform(-1, 1, shape[1:]).astype(dt)
+    got, want, ks = both(R.lu(a), [a])
+    assert ks.info["variant"] == "by matrix"
     assert_bits(got, want, f"lu {shape} {np.dtype(dt).name} {ks.info}")
 
 
