@@ -133,7 +133,7 @@ def is_direct_product(kernel: Kernel) -> bool:
         return False
     t = tuner.tuneHip(kernel)
     return (t.klass == "gemm" and t.gemm["dtype"] == DType.Float32 and _f32_direct(t.gemm) and not (t.gemm["batch"] and t.gemm["K"] <= 32) and few_plan(t) is None
-            and bool(choose_tile(dict(t.gemm, direct=True)).get("DLDS")))
+            and bool(choose_tile(dict(t.gemm, direct=True), bool(t.epilogue.collect(lambda n: n.op == AluOp.GlobalIndex))).get("DLDS")))
 
 
 def _f32_direct(g: dict) -> bool:
@@ -197,7 +197,11 @@ def choose_tile(g: dict, reads: bool = False) -> Dict[str, int]:
         bk = 32 if plain_k else 16
         # Direct loads where a schedule asks for them, and for any Kernel of at least two 128x128 tiles per CU, whose plans nothing pins
         # (8192^3 8596 -> 7565 us; 4096^3 1080 -> 946).
-        if _f32_direct(g) and (g.get("direct") or tiles(128, 128) >= 2 * CU):
+        # Short k axes behind an epilogue that reads buffers stay staged where there is more than a round of tiles: four workgroups have a
+        # place on a CU then and hide each other's epilogues, where direct loads leave it to two (with a residual 784 x 3664 x 64 11.6 us staged, 15.7 by direct loads, 3220 x
+        # 924 x 96 12.7 and 16.2, 3852 x 684 x 184 18.9 and 22.7, 3020 x 668 x 240 20.3 and 19.9; 1900 x 484 x 88, one round, 6.8 and 6.4).
+        exposed = reads and g["K"] <= 256 and tiles(64, 64) > 2 * CU
+        if _f32_direct(g) and (g.get("direct") or tiles(128, 128) >= 2 * CU) and not exposed:
             plan = _f32_tile(g, tiles, nb, 1 if tiles(128, 128) >= 2 * CU else choose_tile(dict(g, direct=False)).get("SPLITK", 1))
             if plan is not None:
                 return plan

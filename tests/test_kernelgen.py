@@ -404,6 +404,19 @@ def test_products_cut_finer_than_direct_loads_cut_them_keep_their_plan(batch, m,
     assert taken == staged or 2 * taken["WK"] * taken.get("SPLITK", 1) >= staged.get("SPLITK", 1)
 
 
+@pytest.mark.parametrize("m,n,k,reads,direct", [(784, 3664, 64, True, False), (784, 3664, 64, False, True), (3852, 684, 184, True, False), (1900, 484, 88, True, True),
+                                                (3300, 2144, 352, True, True), (2264, 3808, 60, True, False), (4096, 4096, 64, True, False), (4096, 4096, 64, False, True)], ids=str)
+def test_epilogues_that_read_behind_short_axes_keep_products_staged(m, n, k, reads, direct):
+    from jaxjs_hip import jit as J, library as L
+    from jaxjs_hip.jit import ShapedArray
+    from jaxjs_hip.kernelgen import generate
+    from jaxjs_hip.schedule import plan_units
+
+    a, b, c = (ShapedArray(s, DType.Float32) for s in ((m, k), (k, n), (m, n)))
+    unit, = plan_units(J.jit(lambda a, b, *c: L.matmul(a, b).add(c[0]) if c else L.matmul(a, b), [a, b, c] if reads else [a, b]))
+    assert ("global_load_lds_dwordx4" in generate(unit.source, **unit.options).sources[0]) == direct
+
+
 @pytest.mark.parametrize("n,m,mats,plan", [(256, 1, 300, (8, 4)), (128, 1, 4096, (8, 4)), (100, 1, 16384, (8, 4)), (48, 1, 600, (8, 8)), (256, 20, 512, (32, 4)), (128, 1, 256, (8, 32)),
                                            (609, 14, 1, (8, 12)), (1284, 28, 68, (8, 3)), (64, 65, 250, (64, 4)), (100, 1, 16385, None), (2048, 8, 1, None)], ids=str)
 def test_few_right_hand_sides_are_counted_by_workgroup(n, m, mats, plan):
