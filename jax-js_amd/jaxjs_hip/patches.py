@@ -199,7 +199,9 @@ def _us_gathered(kernel: Kernel) -> float:
 
     A fit to 180 Kernels of drawn convolutions.  The templates' time is their walk over k, by how many operands have vector loads,
     and goes on with the workgroups of a CU, which hide each other's loads in part; that of the reductions by rows and columns is the
-    products, 0.3 to 1.7 million a microsecond where windows are walked and eight where both operands come in vectors."""
+    products, 0.3 to 1.7 million a microsecond where windows are walked and eight where both operands come in vectors.  An image whose windows' rows come
+    in whole groups of four or eight has vector loads too, for a walk of 6 to 10 ns an element of k in float16 and 37 in float32 (94 convolutions with windows of 4 to 16: float16 [6, 20, 28, 28] to 461, 4 x 4, stride 4, 6.1 us, laid
+    out 8.2; 171 to 299 channels of 60 x 60, 4 x 4, 20.6 and 35.9; [2, 388, 40, 40] to 65, stride 2, 11.7 and 29.0)."""
     t = tuner.tuneHip(kernel)
     K = kernel.reduction.size
     if t.klass != "gemm":
@@ -220,7 +222,13 @@ def _us_gathered(kernel: Kernel) -> float:
     rounds = max(1.0, info["tiles"] * split / tuner.CU_COUNT) ** 0.5  # workgroups that share a CU hide each other's loads
     single = sum(x == "element" for x in info.get("gather", {}).values())  # operands without vector loads
     per_k = (0.045 + 0.0275 * single + (0.03 if g.get("a_loose") or g.get("b_loose") else 0.0)) if half else 0.05 + 0.01 * single
-    return max(3.0, per_k * K / split * rounds - 1.0) + (2.0 if split > 1 else 0.0)
+    fold = 2.0 if split > 1 else 0.0
+    us = max(3.0, per_k * K / split * rounds - 1.0) + fold
+    gather = info.get("gather", {})
+    if gather.get("a") == "none" and gather.get("b") in ("k4", "k8"):
+        area = info["BM"] * info["BN"] / 4096
+        us = min(us, (4.7 + (0.0063 + 0.0036 * (area - 1)) * K / split * rounds if half else 3.4 + 0.0373 * K / split * rounds) + fold)
+    return us
 
 
 def _us_packed(packed: Packed, sums_stay: bool) -> float:

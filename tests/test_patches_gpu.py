@@ -173,6 +173,14 @@ def test_operands_past_32_bit_indices_are_not_laid_out(stride, taken):
     assert (found is not None) == taken
 
 
+@pytest.mark.parametrize("B,ci,co,size,window,stride,laid_out", [(6, 20, 461, 28, 4, 4, False), (1, 171, 299, 60, 4, 1, False), (2, 388, 65, 40, 4, 2, False), (2, 3, 713, 32, 8, 8, False),
+                                                                 (8, 11, 652, 24, 3, 2, True)], ids=str)
+def test_windows_with_vector_loads_are_not_laid_out(B, ci, co, size, window, stride, laid_out):
+    p = ConvParams(0, [stride] * 2, [(0, 0)] * 2, [1, 1], [1, 1])
+    prog = J.jit(lambda x, w: J.conv(x, w, p), [ShapedArray((B, ci, size, size), DType.Float16), ShapedArray((co, ci, window, window), DType.Float16)])
+    assert any(isinstance(u.source, Layouts) for u in plan_units(prog)) == laid_out
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", [CASES[0], CASES[6]], ids=str)
 def test_laid_out_operands_under_capture_and_one_dispatch_at_a_time(case):
